@@ -139,6 +139,7 @@ size_t dsalt_bwd_args_size(void) { return sizeof(dsalt_bwd_args); }
 size_t dsalt_select_args_size(void) { return sizeof(dsalt_select_args); }
 size_t dsalt_scores_args_size(void) { return sizeof(dsalt_scores_args); }
 size_t dsalt_rope_args_size(void) { return sizeof(dsalt_rope_args); }
+size_t dsalt_lmk_weights_args_size(void) { return sizeof(dsalt_lmk_weights_args); }
 
 int dsalt_fwd_check(const dsalt_fwd_args *a) {
     if (!a) return fail(DSALT_ERR_INVALID, "args is NULL");
@@ -330,6 +331,78 @@ int dsalt_select_hybrid(const dsalt_scores_args *sa, const dsalt_select_args *a,
     hipError_t e = dsalt::launch_norms_for_select(*sa, src, st);
     if (e == hipSuccess) e = dsalt::launch_select(*a, st, &src);
     if (e != hipSuccess) return fail(DSALT_ERR_LAUNCH, "dsalt_select_hybrid launch failed: %s", hipGetErrorString(e));
+    return DSALT_OK;
+}
+
+int64_t dsalt_lmk_weights_workspace_size(int32_t total_len, int32_t n_heads) {
+    if (total_len < 0 || n_heads < 1) return -1;
+    return dsalt::lmk_weights_workspace_bytes(total_len, n_heads);
+}
+
+int dsalt_lmk_weights_check(const dsalt_lmk_weights_args *a, int32_t backward) {
+    if (!a) return fail(DSALT_ERR_INVALID, "args is NULL");
+    if (a->total_len < 0 || a->num_seqs < 1 || a->n_heads < 1 || a->n_kv_heads < 1)
+        return fail(DSALT_ERR_INVALID, "total_len must be >= 0, num_seqs, n_heads and n_kv_heads >= 1");
+    if (a->n_heads % a->n_kv_heads || a->n_kv_heads > dsalt::scores_max_kv())
+        return fail(DSALT_ERR_INVALID, "n_kv_heads (%d) must divide n_heads (%d) and be <= %d", a->n_kv_heads,
+                    a->n_heads, dsalt::scores_max_kv());
+    if (a->k_lmk < 0 || a->k_lmk > DSALT_MAX_K_LMK)
+        return fail(DSALT_ERR_UNSUPPORTED, "k_lmk must be in [0, %d] (got %d)", DSALT_MAX_K_LMK, a->k_lmk);
+    if (a->table && a->num_seqs != 1) return fail(DSALT_ERR_INVALID, "table = 1 takes one sequence");
+    if ((int64_t)a->num_seqs * a->n_heads > (int64_t)INT32_MAX || (int64_t)a->num_seqs * a->k_lmk > (int64_t)INT32_MAX)
+        return fail(DSALT_ERR_UNSUPPORTED, "too many (head, sequence) pairs or slots");
+    if (!(a->tau > 0.f)) return fail(DSALT_ERR_INVALID, "tau must be > 0 (got %g)", (double)a->tau);
+    if (a->total_len == 0) return DSALT_OK;
+    const int64_t need = dsalt::scores_workspace_bytes(a->total_len, a->n_kv_heads);
+    if (!a->norms || a->norms_bytes < need || !aligned(a->norms, 256))
+        return fail(DSALT_ERR_INVALID, "norms must be a 256-byte aligned scores workspace of %lld bytes", (long long)need);
+    if (!a->alpha || !a->cu_seqlens || (a->k_lmk > 0 && !a->lmk_pos))
+        return fail(DSALT_ERR_INVALID, "alpha, cu_seqlens and lmk_pos must be non-NULL");
+    if (!backward) {
+        if (!a->weight && (a->table || a->k_lmk > 0)) return fail(DSALT_ERR_INVALID, "weight is NULL");
+        return DSALT_OK;
+    }
+    if (!a->d_weight && (a->table || a->k_lmk > 0)) return fail(DSALT_ERR_INVALID, "d_weight is NULL");
+    const int64_t ws = dsalt::lmk_weights_workspace_bytes(a->total_len, a->n_heads);
+    if (!a->workspace || a->workspace_bytes < ws || !aligned(a->workspace, 256))
+        return fail(DSALT_ERR_INVALID, "workspace must be 256-byte aligned and hold %lld bytes", (long long)ws);
+    for (int dt : {a->x_dtype, a->v_dtype})
+        if (dt != DSALT_DTYPE_BF16 && dt != DSALT_DTYPE_F16 && dt != DSALT_DTYPE_F32)
+            return fail(DSALT_ERR_INVALID, "x_dtype and v_dtype must be DSALT_DTYPE_BF16, _F16 or _F32 (got %d, %d)",
+                        a->x_dtype, a->v_dtype);
+    const int ex = a->x_dtype == DSALT_DTYPE_F32 ? 4 : 8, ev = a->v_dtype == DSALT_DTYPE_F32 ? 4 : 8;
+    if (a->dx) {
+        if (a->d_model < 1 || a->d_model % ex) return fail(DSALT_ERR_UNSUPPORTED, "d_model must be a multiple of %d", ex);
+        if (!a->x || !aligned(a->x, 16) || !aligned(a->dx, 16) || a->x_stride_t < a->d_model || a->x_stride_t % ex)
+            return fail(DSALT_ERR_INVALID, "x and dx must be 16-byte aligned, x's row stride a multiple of %d", ex);
+    }
+    if (a->dv) {
+        if (a->head_dim < 1 || a->head_dim % ev)
+            return fail(DSALT_ERR_UNSUPPORTED, "head_dim must be a multiple of %d", ev);
+        if (!a->v || !aligned(a->v, 16) || !aligned(a->dv, 16) || a->v_stride_t < 0 || a->v_stride_h < 0 ||
+            a->v_stride_t % ev || a->v_stride_h % ev)
+            return fail(DSALT_ERR_INVALID, "v and dv must be 16-byte aligned, v's strides multiples of %d", ev);
+        if (a->dv_in && (!aligned(a->dv_in, 16) || a->dv_in_stride_t < 0 || a->dv_in_stride_h < 0 ||
+                         a->dv_in_stride_t % ev || a->dv_in_stride_h % ev))
+            return fail(DSALT_ERR_INVALID, "dv_in must be 16-byte aligned with strides multiples of %d", ev);
+    }
+    return DSALT_OK;
+}
+
+int dsalt_lmk_weights(const dsalt_lmk_weights_args *a, void *stream) {
+    int rc = dsalt_lmk_weights_check(a, 0);
+    if (rc) return rc;
+    hipError_t e = dsalt::launch_lmk_weights(*a, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(DSALT_ERR_LAUNCH, "dsalt_lmk_weights launch failed: %s", hipGetErrorString(e));
+    return DSALT_OK;
+}
+
+int dsalt_lmk_weights_bwd(const dsalt_lmk_weights_args *a, void *stream) {
+    int rc = dsalt_lmk_weights_check(a, 1);
+    if (rc) return rc;
+    hipError_t e = dsalt::launch_lmk_weights_bwd(*a, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess)
+        return fail(DSALT_ERR_LAUNCH, "dsalt_lmk_weights_bwd launch failed: %s", hipGetErrorString(e));
     return DSALT_OK;
 }
 

@@ -45,6 +45,17 @@ hipError_t launch_rope(const dsalt_rope_args &a, hipStream_t stream);
 hipError_t launch_scores(const dsalt_scores_args &a, hipStream_t stream);
 int64_t scores_workspace_bytes(int total_len, int n_kv);
 int scores_max_kv();
+// The sections of a scores workspace (norms [T] and [T, n_kv], fp64 partials, statistics).
+struct NormsView {
+    float *xn, *vn;
+    double *part;  // [nblk][1 + n_kv][2]
+    float *stats;  // [1 + n_kv][2]
+    int nblk;
+};
+NormsView scores_workspace_view(void *workspace, int total_len, int n_kv);
+hipError_t launch_lmk_weights(const dsalt_lmk_weights_args &a, hipStream_t stream);
+hipError_t launch_lmk_weights_bwd(const dsalt_lmk_weights_args &a, hipStream_t stream);
+int64_t lmk_weights_workspace_bytes(int total_len, int n_heads);
 hipError_t launch_quantize(const float *w_cont, int64_t n, float *w_out, int32_t *w_int,
                            hipStream_t stream);
 hipError_t launch_swiglu(const void *gate, const void *up, void *out, int64_t n, int dtype, hipStream_t stream);

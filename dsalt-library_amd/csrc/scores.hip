@@ -300,6 +300,20 @@ int64_t scores_workspace_bytes(int total_len, int n_kv) {
 
 int scores_max_kv() { return kMaxKvScores; }
 
+NormsView scores_workspace_view(void *workspace, int total_len, int n_kv) {
+    NormsView n;
+    n.nblk = (total_len + kNormTokens - 1) / kNormTokens;
+    char *ws = static_cast<char *>(workspace);
+    n.xn = reinterpret_cast<float *>(ws);
+    ws += align256((size_t)total_len * 4);
+    n.vn = reinterpret_cast<float *>(ws);
+    ws += align256((size_t)total_len * n_kv * 4);
+    n.part = reinterpret_cast<double *>(ws);
+    ws += align256((size_t)n.nblk * (1 + n_kv) * 2 * 8);
+    n.stats = reinterpret_cast<float *>(ws);
+    return n;
+}
+
 namespace {
 
 ScoreParams make_params(const dsalt_scores_args &a) {
@@ -315,16 +329,13 @@ ScoreParams make_params(const dsalt_scores_args &a) {
     p.n_kv = a.n_kv_heads;
     p.D = a.head_dim;
     p.H = a.n_heads;
-    p.nblk = (a.total_len + kNormTokens - 1) / kNormTokens;
+    const NormsView n = scores_workspace_view(a.workspace, a.total_len, a.n_kv_heads);
+    p.nblk = n.nblk;
     p.norms_f32 = a.norms_f32 != 0;
-    char *ws = static_cast<char *>(a.workspace);
-    p.xn = reinterpret_cast<float *>(ws);
-    ws += align256((size_t)p.T * 4);
-    p.vn = reinterpret_cast<float *>(ws);
-    ws += align256((size_t)p.T * p.n_kv * 4);
-    p.part = reinterpret_cast<double *>(ws);
-    ws += align256((size_t)p.nblk * (1 + p.n_kv) * 2 * 8);
-    p.stats = reinterpret_cast<float *>(ws);
+    p.xn = n.xn;
+    p.vn = n.vn;
+    p.part = n.part;
+    p.stats = n.stats;
     p.x_st = a.x_stride_t;
     p.v_st = a.v_stride_t;
     p.v_sh = a.v_stride_h;

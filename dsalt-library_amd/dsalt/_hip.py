@@ -129,6 +129,22 @@ class RopeArgs(ctypes.Structure):
     ]
 
 
+class LmkWeightsArgs(ctypes.Structure):
+    _fields_ = [
+        ("total_len", c_int32), ("num_seqs", c_int32), ("n_heads", c_int32), ("n_kv_heads", c_int32),
+        ("head_dim", c_int32), ("d_model", c_int32), ("k_lmk", c_int32),
+        ("x_dtype", c_int32), ("v_dtype", c_int32), ("table", c_int32), ("tau", c_float),
+        ("norms", c_void_p), ("norms_bytes", c_int64),
+        ("alpha", c_void_p), ("lmk_pos", c_void_p), ("cu_seqlens", c_void_p),
+        ("weight", c_void_p), ("d_weight", c_void_p), ("d_alpha", c_void_p),
+        ("x", c_void_p), ("x_stride_t", c_int64),
+        ("v", c_void_p), ("v_stride_t", c_int64), ("v_stride_h", c_int64),
+        ("dv_in", c_void_p), ("dv_in_stride_t", c_int64), ("dv_in_stride_h", c_int64),
+        ("dx", c_void_p), ("dv", c_void_p),
+        ("workspace", c_void_p), ("workspace_bytes", c_int64),
+    ]
+
+
 EXPORTED_SYMBOLS = (
     "dsalt_fwd", "dsalt_fwd_check", "dsalt_bwd", "dsalt_bwd_check", "dsalt_bwd_workspace_size",
     "dsalt_select_landmarks", "dsalt_select_check", "dsalt_quantize_windows",
@@ -136,7 +152,8 @@ EXPORTED_SYMBOLS = (
     "dsalt_select_args_size", "dsalt_hybrid_scores", "dsalt_scores_check", "dsalt_scores_workspace_size",
     "dsalt_scores_args_size", "dsalt_rope", "dsalt_rope_check", "dsalt_rope_args_size",
     "dsalt_bwd_noalloc", "dsalt_select_workspace_size", "dsalt_select_hybrid", "dsalt_swiglu",
-    "dsalt_add_rms_norm",
+    "dsalt_add_rms_norm", "dsalt_lmk_weights", "dsalt_lmk_weights_bwd", "dsalt_lmk_weights_check",
+    "dsalt_lmk_weights_workspace_size", "dsalt_lmk_weights_args_size",
 )
 NOALLOC_SCRATCH_BYTES = 76 << 20  # DSALT_NOALLOC_SCRATCH_BYTES
 SELECT_SPLIT_MIN = 4096  # longer sequences can be selected chunk-wise
@@ -167,6 +184,9 @@ def lib() -> ctypes.CDLL:
         ("dsalt_select_hybrid", [ctypes.POINTER(ScoresArgs), ctypes.POINTER(SelectArgs), c_void_p]),
         ("dsalt_rope", [ctypes.POINTER(RopeArgs), c_void_p]),
         ("dsalt_rope_check", [ctypes.POINTER(RopeArgs)]),
+        ("dsalt_lmk_weights", [ctypes.POINTER(LmkWeightsArgs), c_void_p]),
+        ("dsalt_lmk_weights_bwd", [ctypes.POINTER(LmkWeightsArgs), c_void_p]),
+        ("dsalt_lmk_weights_check", [ctypes.POINTER(LmkWeightsArgs), c_int32]),
         ("dsalt_quantize_windows", [c_void_p, c_int64, c_void_p, c_void_p, c_void_p]),
         ("dsalt_swiglu", [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_void_p]),
         ("dsalt_add_rms_norm", [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_float, c_int32,
@@ -181,10 +201,12 @@ def lib() -> ctypes.CDLL:
     h.dsalt_scores_workspace_size.restype = c_int64
     h.dsalt_select_workspace_size.argtypes = [c_int32] * 4
     h.dsalt_select_workspace_size.restype = c_int64
+    h.dsalt_lmk_weights_workspace_size.argtypes = [c_int32] * 2
+    h.dsalt_lmk_weights_workspace_size.restype = c_int64
     h.dsalt_abi_version.restype = ctypes.c_int
     h.dsalt_last_error.restype = ctypes.c_char_p
     for n in ("dsalt_fwd_args_size", "dsalt_bwd_args_size", "dsalt_select_args_size", "dsalt_scores_args_size",
-              "dsalt_rope_args_size"):
+              "dsalt_rope_args_size", "dsalt_lmk_weights_args_size"):
         getattr(h, n).restype = c_size_t
     _lib = h
     check_abi()
@@ -197,7 +219,7 @@ def check_abi() -> None:
         raise DsaltError(f"ABI version mismatch: library {h.dsalt_abi_version()} vs binding {ABI_VERSION}")
     for struct, fn in ((FwdArgs, h.dsalt_fwd_args_size), (BwdArgs, h.dsalt_bwd_args_size),
                        (SelectArgs, h.dsalt_select_args_size), (ScoresArgs, h.dsalt_scores_args_size),
-                       (RopeArgs, h.dsalt_rope_args_size)):
+                       (RopeArgs, h.dsalt_rope_args_size), (LmkWeightsArgs, h.dsalt_lmk_weights_args_size)):
         if ctypes.sizeof(struct) != fn():
             raise DsaltError(f"{struct.__name__} layout mismatch: {ctypes.sizeof(struct)} vs {fn()} bytes")
 
@@ -753,7 +775,7 @@ class SelectHybridLauncher:
     def __init__(self, x: torch.Tensor, v: torch.Tensor, alpha: torch.Tensor, n_heads: int,
                  w_cont: torch.Tensor | None, cu_seqlens: torch.Tensor, k_lmk: int, chunked: bool = True,
                  max_seqlen: int | None = None, gate=None, norms_f32: bool | None = None, rope_k=None,
-                 gate_linear=None):
+                 gate_linear=None, quantize: bool = True):
         if norms_f32 is None:
             norms_f32 = autocast_norms()
         if gate_linear is not None and (gate is not None or w_cont is not None):
@@ -783,7 +805,9 @@ class SelectHybridLauncher:
             self._sa.gate_out = self.logit.data_ptr()
         self.k_out, keep_k = _rope_k_args(self._sa, v, rope_k)
         self.out = torch.empty((n_heads, cu.shape[0] - 1, k_lmk), device=self.device, dtype=torch.int64)
-        self.w_out = torch.empty(T, device=self.device, dtype=torch.float32)
+        # quantize=False: w_cont is taken as the windows themselves (select_landmarks' test)
+        self.w_out = torch.empty(T, device=self.device, dtype=torch.float32) if quantize else None
+        self.norms, self.cu = ws, cu
         self._a, keep_s = _select_args(None, w_cont, cu, k_lmk, self.out, chunked, max_seqlen, self.w_out, gate,
                                        shape=(T, n_heads))
         self._keep = (x, v, alpha, cu, ws, keep_k, keep_s, keep_g)
@@ -792,6 +816,63 @@ class SelectHybridLauncher:
 
     def __call__(self) -> None:
         _raise(self._fn(*self._refs, stream_handle(self.device)), "dsalt_select_hybrid")
+
+
+def _lmk_weights_args(norms, alpha, lmk_pos, cu, T, n_kv, tau, table):
+    H, S, k = lmk_pos.shape
+    a = LmkWeightsArgs()
+    a.total_len, a.num_seqs, a.n_heads, a.n_kv_heads, a.k_lmk = T, S, H, n_kv, k
+    a.table, a.tau = int(table), float(tau)
+    a.norms, a.norms_bytes = norms.data_ptr(), norms.numel()
+    a.alpha, a.lmk_pos, a.cu_seqlens = alpha.data_ptr(), lmk_pos.data_ptr(), cu.data_ptr()
+    return a
+
+
+def lmk_weights(norms: torch.Tensor, alpha: torch.Tensor, lmk_pos: torch.Tensor, cu: torch.Tensor, T: int, n_kv: int,
+                tau: float, table: bool = False) -> torch.Tensor:
+    """Weights log(max(sigmoid(s / tau), 1e-20)) of the landmarks that a SelectHybridLauncher
+    selected (``norms``, ``cu``: its attributes; ``alpha`` [H] fp32): [H, S, k] fp32 with
+    -inf in empty slots, or with ``table`` (one sequence) [H, T] with -inf off the landmarks."""
+    dev = require_gpu(norms, alpha, lmk_pos, cu)
+    H, S, k = lmk_pos.shape
+    weight = torch.empty((H, T) if table else (H, S, k), device=dev, dtype=torch.float32)
+    a = _lmk_weights_args(norms, alpha, lmk_pos, cu, T, n_kv, tau, table)
+    a.weight = weight.data_ptr()
+    _raise(lib().dsalt_lmk_weights(ctypes.byref(a), stream_handle(dev)), "dsalt_lmk_weights")
+    return weight
+
+
+def lmk_weights_bwd(d_weight: torch.Tensor, norms: torch.Tensor, alpha: torch.Tensor, lmk_pos: torch.Tensor,
+                    cu: torch.Tensor, x: torch.Tensor, v: torch.Tensor, dv_in: torch.Tensor | None, tau: float,
+                    table: bool = False, need_dx: bool = True, need_dv: bool = True):
+    """Backward of ``lmk_weights`` through the scores: (dx [T, d] in x's dtype or None, dv
+    [T, n_kv, D] in v's dtype (plus ``dv_in``) or None, d_alpha [H] fp32)."""
+    dev = require_gpu(d_weight, norms, alpha, lmk_pos, cu, x, v, dv_in)
+    x, v, _ = _score_operands(x, v, alpha, alpha.shape[0])
+    T, n_kv, D = v.shape
+    H = alpha.shape[0]
+    d_weight = d_weight.to(torch.float32).contiguous()
+    a = _lmk_weights_args(norms, alpha, lmk_pos, cu, T, n_kv, tau, table)
+    a.head_dim, a.d_model = D, x.shape[1]
+    a.x_dtype, a.v_dtype = _SCORE_DTYPES[x.dtype], _SCORE_DTYPES[v.dtype]
+    a.x, a.x_stride_t = x.data_ptr(), x.stride(0)
+    a.v, a.v_stride_t, a.v_stride_h = v.data_ptr(), v.stride(0), v.stride(1)
+    if dv_in is not None and need_dv:
+        ev = 4 if v.dtype == torch.float32 else 8
+        if (dv_in.dtype != v.dtype or dv_in.stride(2) != 1 or dv_in.stride(0) % ev or dv_in.stride(1) % ev
+                or dv_in.data_ptr() % 16):
+            dv_in = dv_in.to(v.dtype).contiguous()
+        if dv_in.data_ptr() % 16:
+            dv_in = dv_in.clone()
+        a.dv_in, a.dv_in_stride_t, a.dv_in_stride_h = dv_in.data_ptr(), dv_in.stride(0), dv_in.stride(1)
+    dx = torch.empty(x.shape, device=dev, dtype=x.dtype) if need_dx else None
+    dv = torch.empty(v.shape, device=dev, dtype=v.dtype) if need_dv else None
+    d_alpha = torch.empty((H,), device=dev, dtype=torch.float32)
+    ws = torch.empty((lib().dsalt_lmk_weights_workspace_size(T, H),), device=dev, dtype=torch.uint8)
+    a.d_weight, a.d_alpha, a.dx, a.dv = d_weight.data_ptr(), d_alpha.data_ptr(), _ptr(dx), _ptr(dv)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+    _raise(lib().dsalt_lmk_weights_bwd(ctypes.byref(a), stream_handle(dev)), "dsalt_lmk_weights_bwd")
+    return dx, dv, d_alpha
 
 
 _SCORE_DTYPES = {torch.bfloat16: DTYPE_BF16, torch.float16: DTYPE_F16, torch.float32: DTYPE_F32}

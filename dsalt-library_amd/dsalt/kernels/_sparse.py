@@ -57,9 +57,9 @@ def _backward(ctx, grad_out, need_dw: bool):
         ctx.dsalt_mode, q_c, k_c, v_c, out, lse, grad_out, w_f, lp, lb, cu,
         ctx.dsalt_scale, ctx.dsalt_tau, ctx.dsalt_edge, need_dw=need_dw, grad_dtype=gdt)
     dk, dv = _hip.group_sum(dk, n_kv), _hip.group_sum(dv, n_kv)
-    return (dq.to(od), dk.to(od), dv.to(od),
-            None if d_bias is None else d_bias.to(od),
-            None if d_w is None else d_w.to(od))
+    # the landmark-weight and window gradients stay fp32, as the kernels sum them (autograd
+    # casts each to its input's dtype)
+    return dq.to(od), dk.to(od), dv.to(od), d_bias, d_w
 
 
 class _SparseAttention(torch.autograd.Function):

@@ -39,6 +39,7 @@ import torch.nn.functional as F
 
 from .. import _hip
 from ..kernels._dense import dense_attention, dense_probabilities
+from ..kernels._lmk_weights import landmark_weights
 from ..kernels._sparse import sparse_attention
 from ..kernels.landmark_tokens_ker import hybrid_scores_from_v, hybrid_scores_per_head
 from ..kernels.selectors import _compute_landmark_indices, _landmarks_and_windows
@@ -262,7 +263,12 @@ class DSALTAttention(nn.Module):
 
         # grouped K/V heads go to the kernels as they are (query head h reads K/V head
         # h // n_rep); no repeated copy
-        w_cont, lmk_bias, lmk_pos = self._dense_selectors(xs, T, device, v_sel)
+        if self._hip_weights(xs, v_sel):
+            w_cont = self._window_continuous(xs)
+            v, lmk_bias, lmk_pos, _ = landmark_weights(xs, v, self._alpha(), xs.new_zeros(1, dtype=torch.float32).expand(T), cu,
+                                                       min(self.k_lmk, T), T, self.tau_lmk, table=True)
+        else:
+            w_cont, lmk_bias, lmk_pos = self._dense_selectors(xs, T, device, v_sel)
         out = dense_attention(q, k, v, w_cont, lmk_bias, self.tau_win, float(self.win_edge))
         if not self.training and getattr(self, "_collect_last_P", True):
             self._last_P = dense_probabilities(q, self._repeat_kv(k), w_cont, lmk_bias, self.tau_win,
@@ -272,6 +278,13 @@ class DSALTAttention(nn.Module):
         self._last_selection = (w_cont.detach(), lmk_pos)
         aux = x.new_zeros(())
         return self._apply_out_proj(out.reshape(1, T, self.d_model)), aux
+
+    def _hip_weights(self, x: torch.Tensor, v: torch.Tensor | None) -> bool:
+        """Whether the selection and its differentiable weights run on the HIP passes over x
+        and the value projection v (``_hip_scores`` and ``_fused_selector`` set, no
+        projection bias, operands that the passes take)."""
+        return (v is not None and self._fused_selector and self._hip_scores and x.shape[0] > 0
+                and _hip.scores_supported(x, v))
 
     @_dynamo_opaque
     def _dense_selectors(self, x, T, device, v=None):
@@ -304,9 +317,21 @@ class DSALTAttention(nn.Module):
         the selection is detached; ``w_cont`` and ``lmk_logw`` carry the gradients.
         With ``v`` (the pre-RoPE value projection ``[T, n_kv, dh]``, equal to ``x @ W_V.T``
         when the projection has no bias) the scores are formed from it instead of a second
-        GEMM; the selection sees bit-identical scores either way."""
+        GEMM; the selection sees bit-identical scores either way on the torch route."""
+        return self._select_train(x, cu_seqlens, total_len, device, cu_list, v)[:3]
+
+    @_dynamo_opaque
+    def _select_train(self, x, cu_seqlens, total_len, device, cu_list=None, v=None):
+        """``_train_selectors`` and the ``v`` to attend with: on the HIP route the one whose
+        gradient passes through the weights' backward (``landmark_weights``)."""
         w_cont = self._window_continuous(x)
         alpha = self._alpha()
+        if self._hip_weights(x, v):
+            max_len = None if cu_list is None else max((b - a for a, b in zip(cu_list[:-1], cu_list[1:])), default=0)
+            v, lmk_logw, lmk_pos, w_disc = landmark_weights(x, v, alpha, w_cont, cu_seqlens, self.k_lmk, max_len,
+                                                            self.tau_lmk)
+            self._last_selection = (w_disc, lmk_pos)
+            return w_cont, lmk_pos, lmk_logw, v
         route_v = v if self._fused_selector else None
         with torch.no_grad():  # windows quantised by the selection launch
             w_disc, lmk_pos = _landmarks_and_windows(
@@ -326,7 +351,7 @@ class DSALTAttention(nn.Module):
         lmk_logw = torch.sigmoid(s_sel / self.tau_lmk).clamp(min=1e-20).log()
         lmk_logw = lmk_logw.masked_fill(lmk_pos < 0, float("-inf"))
         self._last_selection = (w_disc, lmk_pos)
-        return w_cont, lmk_pos, lmk_logw
+        return w_cont, lmk_pos, lmk_logw, v
 
     def _packed(self, x: torch.Tensor, cu_seqlens: torch.Tensor, total_len: int, device: torch.device,
                 rope_cs: tuple | None = None, cu_list: list | None = None, need_aux: bool = True):
@@ -363,7 +388,8 @@ class DSALTAttention(nn.Module):
 
         if self.training:
             self._last_P = None
-            w_cont, lmk_pos, lmk_logw = self._train_selectors(x, cu_seqlens, total_len, device, cu_list, v_sel)
+            w_cont, lmk_pos, lmk_logw, v_train = self._select_train(x, cu_seqlens, total_len, device, cu_list, v_sel)
+            v = v if v_train is None else v_train
             out = sparse_attention(_hip.MODE_SOFT, q, k, v, lmk_pos, lmk_logw, w_cont, cu_seqlens,
                                    self.tau_win, float(self.win_edge))
             return self._apply_out_proj(out.reshape(total_len, self.d_model)), aux

@@ -416,6 +416,53 @@ int dsalt_swiglu(const void *gate, const void *up, void *out, int64_t n, int32_t
 int dsalt_add_rms_norm(const void *x, const void *h, void *x_out, void *y, const void *weight, int64_t rows,
                        int32_t d, float eps, int32_t dtype, void *stream);
 
+/*
+ * Differentiable weights of the selected landmarks, forward and backward, from the norms
+ * that dsalt_select_hybrid (or dsalt_hybrid_scores) left in its scores workspace.
+ * Replaces the differentiable score and weight ops of _train_selectors
+ * (dsalt/modules/dsalt_attention.py:457-487) and _diff_logbias (:403-438) and their
+ * autograd backward.
+ * dsalt_lmk_weights: weight = log(max(sigmoid(s / tau), 1e-20)) of the hybrid score s of
+ * each selected token: [H, S, k] contiguous (-inf in slots without a position), or with
+ * table = 1 (num_seqs = 1) the [H, T] row of each head, -inf off its landmarks. Writes the
+ * statistics into `norms`; d_*, x, v, dx, dv and workspace are not read.
+ * dsalt_lmk_weights_bwd (after dsalt_lmk_weights on the same norms): from d_weight (the
+ * layout of weight, contiguous) d_alpha [H] (may be NULL), dx [T, d_model] contiguous in
+ * x_dtype and dv [T, n_kv, D] contiguous in v_dtype (either may be NULL) through the
+ * norms; dv_in (may be NULL: 0) in v_dtype is added to dv. Every sum has a fixed order;
+ * one rounding per result. Positions must be distinct within a (head, sequence). x, v and
+ * dv_in as dsalt_hybrid_scores takes x and v. workspace: >= dsalt_lmk_weights_workspace_size
+ * bytes, 256-byte aligned (backward only).
+ */
+typedef struct dsalt_lmk_weights_args {
+    int32_t total_len, num_seqs, n_heads, n_kv_heads, head_dim, d_model, k_lmk;
+    int32_t x_dtype, v_dtype;
+    int32_t table;
+    float tau;
+    void *norms; /* the scores workspace of that call, for total_len and n_kv_heads */
+    int64_t norms_bytes;
+    const float *alpha;     /* [H], as that call had it */
+    const int64_t *lmk_pos; /* [H, S, k] contiguous */
+    const int32_t *cu_seqlens;
+    float *weight;
+    const float *d_weight;
+    float *d_alpha;
+    const void *x;
+    int64_t x_stride_t;
+    const void *v;
+    int64_t v_stride_t, v_stride_h;
+    const void *dv_in;
+    int64_t dv_in_stride_t, dv_in_stride_h;
+    void *dx, *dv;
+    void *workspace;
+    int64_t workspace_bytes;
+} dsalt_lmk_weights_args;
+
+int64_t dsalt_lmk_weights_workspace_size(int32_t total_len, int32_t n_heads);
+int dsalt_lmk_weights(const dsalt_lmk_weights_args *args, void *stream);
+int dsalt_lmk_weights_bwd(const dsalt_lmk_weights_args *args, void *stream);
+int dsalt_lmk_weights_check(const dsalt_lmk_weights_args *args, int32_t backward);
+
 int dsalt_abi_version(void);
 const char *dsalt_last_error(void);
 /* sizeof of the argument structs as compiled into the library (ABI layout check). */
@@ -424,6 +471,7 @@ size_t dsalt_bwd_args_size(void);
 size_t dsalt_select_args_size(void);
 size_t dsalt_scores_args_size(void);
 size_t dsalt_rope_args_size(void);
+size_t dsalt_lmk_weights_args_size(void);
 
 #ifdef __cplusplus
 }
