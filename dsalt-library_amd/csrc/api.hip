@@ -139,6 +139,8 @@ size_t dsalt_bwd_args_size(void) { return sizeof(dsalt_bwd_args); }
 size_t dsalt_select_args_size(void) { return sizeof(dsalt_select_args); }
 size_t dsalt_scores_args_size(void) { return sizeof(dsalt_scores_args); }
 size_t dsalt_rope_args_size(void) { return sizeof(dsalt_rope_args); }
+size_t dsalt_rope_tables_size(void) { return sizeof(dsalt_rope_tables); }
+size_t dsalt_qkv_args_size(void) { return sizeof(dsalt_qkv_args); }
 size_t dsalt_lmk_weights_args_size(void) { return sizeof(dsalt_lmk_weights_args); }
 
 int dsalt_fwd_check(const dsalt_fwd_args *a) {
@@ -319,19 +321,54 @@ int dsalt_hybrid_scores(const dsalt_scores_args *a, void *stream) {
     return DSALT_OK;
 }
 
-int dsalt_select_hybrid(const dsalt_scores_args *sa, const dsalt_select_args *a, void *stream) {
+namespace {
+
+int check_operands(const dsalt_scores_args *sa, const dsalt_qkv_args *o) {
+    if (!sa->k) return fail(DSALT_ERR_INVALID, "q needs k (and the RoPE tables) in the score arguments");
+    const bool cast = sa->v_dtype == DSALT_DTYPE_F32 && o->out_dtype == DSALT_DTYPE_F16;
+    if (!cast && o->out_dtype != sa->v_dtype)
+        return fail(DSALT_ERR_INVALID, "out_dtype must be v_dtype, or F16 for fp32 operands (got %d)", o->out_dtype);
+    if (cast != (o->v_out != nullptr)) return fail(DSALT_ERR_INVALID, "v_out goes with fp16 outputs of fp32 operands");
+    if (sa->total_len == 0) return DSALT_OK;
+    if (!o->q || !o->q_out) return fail(DSALT_ERR_INVALID, "q and q_out must be non-NULL");
+    const int ev = sa->v_dtype == DSALT_DTYPE_F32 ? 4 : 8;
+    if (!aligned(o->q, 16) || !aligned(o->q_out, 16) || !aligned(o->v_out, 16))
+        return fail(DSALT_ERR_INVALID, "q, q_out and v_out must be 16-byte aligned");
+    for (int64_t st : {o->q_stride_t, o->q_stride_h, o->q_out_stride_t, o->q_out_stride_h, o->v_out_stride_t,
+                       o->v_out_stride_h})
+        if (st < 0 || st % ev) return fail(DSALT_ERR_INVALID, "operand strides must be non-negative multiples of %d", ev);
+    if (cast && (o->q_out == o->q || o->v_out == sa->v || sa->k_out == sa->k))
+        return fail(DSALT_ERR_INVALID, "fp16 outputs must not alias the fp32 operands");
+    return DSALT_OK;
+}
+
+int select_hybrid(const dsalt_scores_args *sa, const dsalt_select_args *a, const dsalt_qkv_args *o, void *stream,
+                  const char *what) {
     int rc = check_scores(sa, true);
     if (rc) return rc;
     if ((rc = check_select(a, true))) return rc;
     if (sa->total_len != a->total_len || sa->n_heads != a->n_heads)
         return fail(DSALT_ERR_INVALID, "score and selection arguments disagree: total_len %d / %d, n_heads %d / %d",
                     sa->total_len, a->total_len, sa->n_heads, a->n_heads);
+    if (o && (rc = check_operands(sa, o))) return rc;
     const hipStream_t st = static_cast<hipStream_t>(stream);
     dsalt::HybridSrc src;
-    hipError_t e = dsalt::launch_norms_for_select(*sa, src, st);
+    hipError_t e = dsalt::launch_norms_for_select(*sa, o, src, st);
     if (e == hipSuccess) e = dsalt::launch_select(*a, st, &src);
-    if (e != hipSuccess) return fail(DSALT_ERR_LAUNCH, "dsalt_select_hybrid launch failed: %s", hipGetErrorString(e));
+    if (e != hipSuccess) return fail(DSALT_ERR_LAUNCH, "%s launch failed: %s", what, hipGetErrorString(e));
     return DSALT_OK;
+}
+
+}  // namespace
+
+int dsalt_select_hybrid(const dsalt_scores_args *sa, const dsalt_select_args *a, void *stream) {
+    return select_hybrid(sa, a, nullptr, stream, "dsalt_select_hybrid");
+}
+
+int dsalt_select_hybrid_qkv(const dsalt_scores_args *sa, const dsalt_select_args *a, const dsalt_qkv_args *o,
+                            void *stream) {
+    if (!o) return fail(DSALT_ERR_INVALID, "operands is NULL");
+    return select_hybrid(sa, a, o, stream, "dsalt_select_hybrid_qkv");
 }
 
 int64_t dsalt_lmk_weights_workspace_size(int32_t total_len, int32_t n_heads) {
@@ -533,8 +570,28 @@ int dsalt_bwd_check(const dsalt_bwd_args *a) {
 int dsalt_bwd(const dsalt_bwd_args *a, void *stream) {
     int rc = dsalt_bwd_check(a);
     if (rc) return rc;
-    hipError_t e = dsalt::launch_bwd(*a, static_cast<hipStream_t>(stream));
+    hipError_t e = dsalt::launch_bwd(*a, nullptr, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(DSALT_ERR_LAUNCH, "dsalt_bwd launch failed: %s", hipGetErrorString(e));
+    return DSALT_OK;
+}
+
+int dsalt_bwd_rope(const dsalt_bwd_args *a, const dsalt_rope_tables *r, void *stream) {
+    int rc = dsalt_bwd_check(a);
+    if (rc) return rc;
+    if (r) {
+        if (a->mode == DSALT_MODE_DENSE && a->head_dim != 64)
+            return fail(DSALT_ERR_UNSUPPORTED, "DSALT_MODE_DENSE un-rotates its gradients at head_dim 64 only (got %d)",
+                        a->head_dim);
+        if (!r->cos || !r->sin || !aligned(r->cos, 16) || !aligned(r->sin, 16) || r->rows < 1 ||
+            r->stride < a->head_dim || r->stride % 4)
+            return fail(DSALT_ERR_INVALID,
+                        "RoPE tables need rows >= 1, stride >= head_dim and a multiple of 4, 16-byte alignment "
+                        "(rows %d, stride %lld)", r->rows, (long long)r->stride);
+        if (r->round_dtype != DSALT_DTYPE_BF16 && r->round_dtype != DSALT_DTYPE_F16 && r->round_dtype != DSALT_DTYPE_F32)
+            return fail(DSALT_ERR_INVALID, "round_dtype must be DSALT_DTYPE_BF16, _F16 or _F32 (got %d)", r->round_dtype);
+    }
+    hipError_t e = dsalt::launch_bwd(*a, r, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(DSALT_ERR_LAUNCH, "dsalt_bwd_rope launch failed: %s", hipGetErrorString(e));
     return DSALT_OK;
 }
 
@@ -554,7 +611,7 @@ int dsalt_bwd_noalloc(const dsalt_bwd_args *a, void *stream) {
     b.workspace = scratch_ptr;
     b.workspace_bytes = DSALT_NOALLOC_SCRATCH_BYTES;
     if ((rc = dsalt_bwd_check(&b))) return rc;
-    hipError_t e = dsalt::launch_bwd(b, static_cast<hipStream_t>(stream));
+    hipError_t e = dsalt::launch_bwd(b, nullptr, static_cast<hipStream_t>(stream));
     if (e != hipSuccess)
         return fail(DSALT_ERR_LAUNCH, "dsalt_bwd_noalloc launch failed: %s", hipGetErrorString(e));
     return DSALT_OK;

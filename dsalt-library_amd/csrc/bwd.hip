@@ -32,7 +32,10 @@
 // a lane owns one column (query or key) of each 32x32 block and 16 rows of it.
 #include "common.h"
 #include "launch.h"
+#include "rotary.h"
 #include "tiles.h"
+
+#include <stddef.h>
 
 #include <algorithm>
 #include <type_traits>
@@ -93,6 +96,7 @@ struct BwdParams {
     int kv_rep;  // query heads per K/V head
     float scale, scale_log2, inv_tau, win_edge;
     float inv_c2;  // 1 / scale_log2: log2-unit bias -> raw q.k units
+    RopeRows rope; // q and k were rotated with these tables: dq and dk are returned un-rotated
 };
 
 __device__ __forceinline__ uint4 ld16(const uint16_t *p) { return *reinterpret_cast<const uint4 *>(p); }
@@ -555,7 +559,15 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
         for (; t < nb; ++t) tile(t, std::integral_constant<int, kEdgeTile>());
     for (; t < nt; ++t) tile(t, std::integral_constant<int, kLmkTile>());
 
-    if (qvalid) store_row<DT, ND>(p.dq, tok_i * p.dq_st + (int64_t)head * p.dq_sh, p.grad_f32, dqacc, p.scale, hh);
+    if (qvalid) {
+        float mul = p.scale;
+        const RopeRows rope = late_rope_rows(offsetof(BwdParams, rope));
+        if (rope.cos) {
+            rotate_acc_transposed<ND>(dqacc, mul, rope, i, hh);
+            mul = 1.f;
+        }
+        store_row<DT, ND>(p.dq, tok_i * p.dq_st + (int64_t)head * p.dq_sh, p.grad_f32, dqacc, mul, hh);
+    }
     if (MODE == kSoft && p.ws_dwh) {
         const float dwt = half_sum(dw) * p.inv_tau;
         if (hh == 0 && qvalid) p.ws_dwh[tok_i * p.n_heads + head] = dwt;
@@ -1313,7 +1325,13 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
     if (!LMK) {
         if (kvalid) {
             const int64_t tok = (int64_t)seq_start + key;
-            store_row<DT, ND>(p.dk, tok * p.dk_st + (int64_t)head * p.dk_sh, p.grad_f32, dk, p.scale, hh);
+            float mul = p.scale;
+            const RopeRows rope = late_rope_rows(offsetof(BwdParams, rope));
+            if (rope.cos) {
+                rotate_acc_transposed<ND>(dk, mul, rope, key, hh);
+                mul = 1.f;
+            }
+            store_row<DT, ND>(p.dk, tok * p.dk_st + (int64_t)head * p.dk_sh, p.grad_f32, dk, mul, hh);
             store_row<DT, ND>(p.dv, tok * p.dv_st + (int64_t)head * p.dv_sh, p.grad_f32, dv, 1.f, hh);
         }
         if (MODE == kSoft && p.d_w && p.ws_dwh && head == 0 && tid < kBM) {
@@ -1451,8 +1469,8 @@ int64_t bwd_workspace_bytes(int total_len, int num_seqs, int n_heads, int head_d
     return sparse;
 }
 
-hipError_t launch_bwd(const dsalt_bwd_args &a, hipStream_t stream) {
-    if (a.mode == DSALT_MODE_DENSE) return launch_dense_bwd(a, stream);
+hipError_t launch_bwd(const dsalt_bwd_args &a, const dsalt_rope_tables *rope, hipStream_t stream) {
+    if (a.mode == DSALT_MODE_DENSE) return launch_dense_bwd(a, rope, stream);
     if (a.total_len == 0) {
         return hipSuccess;
     }
@@ -1511,6 +1529,7 @@ hipError_t launch_bwd(const dsalt_bwd_args &a, hipStream_t stream) {
     p.inv_c2 = 1.f / p.scale_log2;
     p.inv_tau = 1.f / a.tau_win;
     p.win_edge = a.win_edge;
+    p.rope = rope_rows(rope);
     if (a.dtype == DSALT_DTYPE_BF16) return launch_dt<BF16>(p, a.head_dim, a.mode, stream);
     return launch_dt<F16>(p, a.head_dim, a.mode, stream);
 }

@@ -34,7 +34,10 @@
 // Every output element is written by one thread: the results are deterministic.
 #include "common.h"
 #include "launch.h"
+#include "rotary.h"
 #include "tiles.h"
+
+#include <stddef.h>
 
 #include <type_traits>
 
@@ -72,6 +75,7 @@ struct DenseParams {
     float scale;
     float inv_tau, win_edge;
     int edge_fast;   // the window tail from per-tile factors (13.5 / tau < 40)
+    RopeRows rope;   // q and k were rotated with these tables: dq and dk are returned un-rotated
 };
 
 // First key of the zero-bias core (d <= w~ - win_edge, i.e. j >= i - floor(w~ - win_edge))
@@ -554,13 +558,21 @@ __global__ void __launch_bounds__(128 * dense_bwd_groups(D), 1) dense_dq_kernel(
     const float dw = half_sum(dwl) * p.inv_tau;
     if (qvalid) {
         const int64_t off = (int64_t)i * p.dq_st + (int64_t)head * p.dq_sh;
+        float mul = p.scale;
+        if constexpr (D == 64) {  // at D = 128 the rotation costs dq its second wave per SIMD
+            const RopeRows rope = late_rope_rows(offsetof(DenseParams, rope));
+            if (rope.cos) {
+                rotate_acc_transposed<ND>(dq, mul, rope, i, hh);
+                mul = 1.f;
+            }
+        }
 #pragma unroll
         for (int d = 0; d < ND; ++d)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int dd = d * 32 + g * 8 + hh * 4;
-                const float a0 = dq[d][g * 4] * p.scale, a1 = dq[d][g * 4 + 1] * p.scale;
-                const float a2 = dq[d][g * 4 + 2] * p.scale, a3 = dq[d][g * 4 + 3] * p.scale;
+                const float a0 = dq[d][g * 4] * mul, a1 = dq[d][g * 4 + 1] * mul;
+                const float a2 = dq[d][g * 4 + 2] * mul, a3 = dq[d][g * 4 + 3] * mul;
                 if (p.grad_f32) {
                     *reinterpret_cast<float4 *>(static_cast<float *>(p.dq) + off + dd) = make_float4(a0, a1, a2, a3);
                 } else {
@@ -774,13 +786,21 @@ __global__ void __launch_bounds__(128 * dense_bwd_groups(D), 1) dense_kv_kernel(
     if (kvalid) {
         const int64_t ok = (int64_t)j * p.dk_st + (int64_t)head * p.dk_sh;
         const int64_t ov = (int64_t)j * p.dv_st + (int64_t)head * p.dv_sh;
+        float mul = p.scale;
+        if constexpr (D == 64) {  // at D = 128 the rotation costs dq its second wave per SIMD
+            const RopeRows rope = late_rope_rows(offsetof(DenseParams, rope));
+            if (rope.cos) {
+                rotate_acc_transposed<ND>(dk, mul, rope, j, hh);
+                mul = 1.f;
+            }
+        }
 #pragma unroll
         for (int d = 0; d < ND; ++d)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int dd = d * 32 + g * 8 + hh * 4;
-                const float k0_ = dk[d][g * 4] * p.scale, k1 = dk[d][g * 4 + 1] * p.scale;
-                const float k2 = dk[d][g * 4 + 2] * p.scale, k3 = dk[d][g * 4 + 3] * p.scale;
+                const float k0_ = dk[d][g * 4] * mul, k1 = dk[d][g * 4 + 1] * mul;
+                const float k2 = dk[d][g * 4 + 2] * mul, k3 = dk[d][g * 4 + 3] * mul;
                 const float v0 = dv[d][g * 4], v1 = dv[d][g * 4 + 1], v2 = dv[d][g * 4 + 2], v3 = dv[d][g * 4 + 3];
                 if (p.grad_f32) {
                     *reinterpret_cast<float4 *>(static_cast<float *>(p.dk) + ok + dd) = make_float4(k0_, k1, k2, k3);
@@ -885,7 +905,7 @@ int64_t dense_bwd_workspace_bytes(int total_len, int n_heads) {
            al((int64_t)n_heads * total_len * 4);
 }
 
-hipError_t launch_dense_bwd(const dsalt_bwd_args &a, hipStream_t stream) {
+hipError_t launch_dense_bwd(const dsalt_bwd_args &a, const dsalt_rope_tables *rope, hipStream_t stream) {
     if (a.total_len == 0) return hipSuccess;
     DenseParams p = dense_params(a.total_len, a.n_heads, a.head_dim);
     p.kv_rep = a.n_kv_heads > 0 ? a.n_heads / a.n_kv_heads : 1;
@@ -923,6 +943,7 @@ hipError_t launch_dense_bwd(const dsalt_bwd_args &a, hipStream_t stream) {
     p.dk_st = a.dk_stride_t; p.dk_sh = a.dk_stride_h;
     p.dv_st = a.dv_stride_t; p.dv_sh = a.dv_stride_h;
     set_common(p, a.scale, a.tau_win, a.win_edge);
+    p.rope = rope_rows(rope);
     return a.dtype == DSALT_DTYPE_BF16 ? dense_bwd_dt<BF16>(p, a.head_dim, stream)
                                        : dense_bwd_dt<F16>(p, a.head_dim, stream);
 }

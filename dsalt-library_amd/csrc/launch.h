@@ -29,7 +29,7 @@ constexpr int fwd_waves_per_simd(int head_dim, bool wide_edge) { return head_dim
 constexpr int fwd_ring(int) { return 2; }  // K / V ring depth
 
 hipError_t launch_fwd(const dsalt_fwd_args &a, hipStream_t stream);
-hipError_t launch_bwd(const dsalt_bwd_args &a, hipStream_t stream);
+hipError_t launch_bwd(const dsalt_bwd_args &a, const dsalt_rope_tables *rope, hipStream_t stream);
 // Selection scores formed on the fly from the norms pass's outputs (scores workspace):
 // per-token norms, per-block fp64 partial sums, and the per-head balance alpha.
 struct HybridSrc {
@@ -39,7 +39,8 @@ struct HybridSrc {
     int nblk, n_kv, n_heads, total_len;
 };
 hipError_t launch_select(const dsalt_select_args &a, hipStream_t stream, const HybridSrc *hy = nullptr);
-hipError_t launch_norms_for_select(const dsalt_scores_args &a, HybridSrc &src, hipStream_t stream);
+hipError_t launch_norms_for_select(const dsalt_scores_args &a, const dsalt_qkv_args *operands, HybridSrc &src,
+                                   hipStream_t stream);
 int64_t select_workspace_bytes(int total_len, int num_seqs, int n_heads, int k);
 hipError_t launch_rope(const dsalt_rope_args &a, hipStream_t stream);
 hipError_t launch_scores(const dsalt_scores_args &a, hipStream_t stream);
@@ -74,7 +75,7 @@ int64_t bwd_workspace_bytes(int total_len, int num_seqs, int n_heads, int head_d
 // Dense batched mode (dense.hip): one sequence, every causal key, the [H, T] landmark
 // bias table.
 hipError_t launch_dense_fwd(const dsalt_fwd_args &a, hipStream_t stream);
-hipError_t launch_dense_bwd(const dsalt_bwd_args &a, hipStream_t stream);
+hipError_t launch_dense_bwd(const dsalt_bwd_args &a, const dsalt_rope_tables *rope, hipStream_t stream);
 int64_t dense_bwd_workspace_bytes(int total_len, int n_heads);
 
 }  // namespace dsalt

@@ -11,6 +11,7 @@
 //   dx[j + D/2] = g[j + D/2] c[j + D/2] - g[j] s[j]
 #pragma once
 
+#include "../../include/dsalt_hip.h"
 #include "common.h"
 
 namespace dsalt {
@@ -151,10 +152,12 @@ __device__ __forceinline__ int seq_offset(const int32_t *cu, int S, int T, int t
 // an FMA), and each fp32 result is made opaque before its conversion to the 16-bit type:
 // otherwise the backend may fold the sum and the conversion into one mixed-precision
 // v_fma_mix{lo,hi}_f16, which rounds the exact sum once instead of to fp32 first.
-template <typename DT, int VW>
+// DO: element type of the output (the rotated value rounded to DT, then to DO).
+template <typename DT, int VW, typename DO = DT>
 __device__ __forceinline__ void rotate_vec(const void *in, int64_t ib, void *out, int64_t ob, const float *cr,
                                            const float *sr, int half, int j0, bool in_table, bool transpose) {
     typedef Elem<DT> E;
+    typedef Elem<DO> EO;
     float a[VW], b[VW], c0[VW], c1[VW], s0[VW], s1[VW], o0[VW], o1[VW];
     E::template ldv<VW>(in, ib + j0, a);
     E::template ldv<VW>(in, ib + j0 + half, b);
@@ -175,8 +178,82 @@ __device__ __forceinline__ void rotate_vec(const void *in, int64_t ib, void *out
         }
         asm volatile("" : "+v"(o0[e]), "+v"(o1[e]));
     }
-    E::template stv<VW>(out, ob + j0, o0);
-    E::template stv<VW>(out, ob + j0 + half, o1);
+    EO::template stv<VW>(out, ob + j0, o0);
+    EO::template stv<VW>(out, ob + j0 + half, o1);
+}
+
+// RoPE tables of a gradient epilogue (dsalt_rope_tables): rows of head_dim fp32 entries,
+// each rounded to `round_dtype` as it is read; cos = null: no rotation.
+struct RopeRows {
+    const float *cos, *sin;
+    int64_t st;
+    int rows, half, round_dtype;
+};
+
+// The RopeRows at byte offset `off` of the kernel's argument block, read here: through the
+// parameter itself the compiler loads the six fields at kernel entry and holds them in
+// scalar registers across the tile loops, which have none to spare.
+__device__ __forceinline__ RopeRows late_rope_rows(size_t off) {
+    typedef const __attribute__((address_space(4))) char *kptr;
+    uint64_t a = (uint64_t)(kptr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(a));
+    const __attribute__((address_space(4))) RopeRows *r = (const __attribute__((address_space(4))) RopeRows *)(a + off);
+    RopeRows t;
+    t.cos = r->cos;
+    t.sin = r->sin;
+    t.st = r->st;
+    t.rows = r->rows;
+    t.half = r->half;
+    t.round_dtype = r->round_dtype;
+    return t;
+}
+
+inline RopeRows rope_rows(const dsalt_rope_tables *t) {
+    RopeRows r{};
+    if (t) {
+        r.cos = t->cos;
+        r.sin = t->sin;
+        r.st = t->stride;
+        r.rows = t->rows;
+        r.half = t->half;
+        r.round_dtype = t->round_dtype;
+    }
+    return r;
+}
+
+// The transposed rotation of one gradient row held as D/32 transposed 32x32 accumulator
+// blocks (registers = head-dim d*32 + (r/4)*8 + hh*4 + r%4: a lane holds both elements of
+// each of its pairs, in blocks d and d + ND/2), scaled by `mul` first; `pos` the row's
+// position in its sequence (NaN outside the table, as rotate_vec). fp32 throughout: the
+// caller's store rounds once.
+template <int ND>
+__device__ __forceinline__ void rotate_acc_transposed(f32x16 (&acc)[ND], float mul, const RopeRows &t, int pos, int hh) {
+    const bool in_table = pos >= 0 && pos < t.rows;
+    const float *cr = t.cos + (int64_t)(in_table ? pos : 0) * t.st, *sr = t.sin + (int64_t)(in_table ? pos : 0) * t.st;
+    auto rnd = [&](float x) {
+        if (!in_table) return NAN;
+        return t.round_dtype == 0 ? Elem<BF16>::round(x) : t.round_dtype == 1 ? Elem<F16>::round(x) : x;
+    };
+#pragma unroll
+    for (int d = 0; d < ND / 2; ++d) {
+        // one block pair's table loads in flight at a time: all of them at D = 128 cost the
+        // kernels around this a wave per SIMD
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int lo = d * 32 + g * 8 + hh * 4, hi = t.half ? lo : lo + ND * 16;
+            const float4 c0 = *reinterpret_cast<const float4 *>(cr + lo), s0 = *reinterpret_cast<const float4 *>(sr + lo);
+            const float4 c1 = *reinterpret_cast<const float4 *>(cr + hi), s1 = *reinterpret_cast<const float4 *>(sr + hi);
+            const float ca[4] = {c0.x, c0.y, c0.z, c0.w}, cb[4] = {c1.x, c1.y, c1.z, c1.w};
+            const float sa[4] = {s0.x, s0.y, s0.z, s0.w}, sb[4] = {s1.x, s1.y, s1.z, s1.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float a = acc[d][g * 4 + e] * mul, b = acc[d + ND / 2][g * 4 + e] * mul;
+                acc[d][g * 4 + e] = a * rnd(ca[e]) + b * rnd(sb[e]);
+                acc[d + ND / 2][g * 4 + e] = b * rnd(cb[e]) - a * rnd(sa[e]);
+            }
+        }
+    }
 }
 
 }  // namespace dsalt

@@ -129,6 +129,20 @@ class RopeArgs(ctypes.Structure):
     ]
 
 
+class RopeTables(ctypes.Structure):
+    _fields_ = [("cos", c_void_p), ("sin", c_void_p), ("stride", c_int64), ("rows", c_int32), ("half", c_int32),
+                ("round_dtype", c_int32), ("reserved", c_int32)]
+
+
+class QkvArgs(ctypes.Structure):
+    _fields_ = [
+        ("out_dtype", c_int32), ("reserved", c_int32),
+        ("q", c_void_p), ("q_stride_t", c_int64), ("q_stride_h", c_int64),
+        ("q_out", c_void_p), ("q_out_stride_t", c_int64), ("q_out_stride_h", c_int64),
+        ("v_out", c_void_p), ("v_out_stride_t", c_int64), ("v_out_stride_h", c_int64),
+    ]
+
+
 class LmkWeightsArgs(ctypes.Structure):
     _fields_ = [
         ("total_len", c_int32), ("num_seqs", c_int32), ("n_heads", c_int32), ("n_kv_heads", c_int32),
@@ -153,7 +167,8 @@ EXPORTED_SYMBOLS = (
     "dsalt_scores_args_size", "dsalt_rope", "dsalt_rope_check", "dsalt_rope_args_size",
     "dsalt_bwd_noalloc", "dsalt_select_workspace_size", "dsalt_select_hybrid", "dsalt_swiglu",
     "dsalt_add_rms_norm", "dsalt_lmk_weights", "dsalt_lmk_weights_bwd", "dsalt_lmk_weights_check",
-    "dsalt_lmk_weights_workspace_size", "dsalt_lmk_weights_args_size",
+    "dsalt_lmk_weights_workspace_size", "dsalt_lmk_weights_args_size", "dsalt_bwd_rope", "dsalt_rope_tables_size",
+    "dsalt_select_hybrid_qkv", "dsalt_qkv_args_size",
 )
 NOALLOC_SCRATCH_BYTES = 76 << 20  # DSALT_NOALLOC_SCRATCH_BYTES
 SELECT_SPLIT_MIN = 4096  # longer sequences can be selected chunk-wise
@@ -184,6 +199,9 @@ def lib() -> ctypes.CDLL:
         ("dsalt_select_hybrid", [ctypes.POINTER(ScoresArgs), ctypes.POINTER(SelectArgs), c_void_p]),
         ("dsalt_rope", [ctypes.POINTER(RopeArgs), c_void_p]),
         ("dsalt_rope_check", [ctypes.POINTER(RopeArgs)]),
+        ("dsalt_bwd_rope", [ctypes.POINTER(BwdArgs), ctypes.POINTER(RopeTables), c_void_p]),
+        ("dsalt_select_hybrid_qkv", [ctypes.POINTER(ScoresArgs), ctypes.POINTER(SelectArgs), ctypes.POINTER(QkvArgs),
+                                     c_void_p]),
         ("dsalt_lmk_weights", [ctypes.POINTER(LmkWeightsArgs), c_void_p]),
         ("dsalt_lmk_weights_bwd", [ctypes.POINTER(LmkWeightsArgs), c_void_p]),
         ("dsalt_lmk_weights_check", [ctypes.POINTER(LmkWeightsArgs), c_int32]),
@@ -206,7 +224,7 @@ def lib() -> ctypes.CDLL:
     h.dsalt_abi_version.restype = ctypes.c_int
     h.dsalt_last_error.restype = ctypes.c_char_p
     for n in ("dsalt_fwd_args_size", "dsalt_bwd_args_size", "dsalt_select_args_size", "dsalt_scores_args_size",
-              "dsalt_rope_args_size", "dsalt_lmk_weights_args_size"):
+              "dsalt_rope_args_size", "dsalt_lmk_weights_args_size", "dsalt_rope_tables_size", "dsalt_qkv_args_size"):
         getattr(h, n).restype = c_size_t
     _lib = h
     check_abi()
@@ -219,7 +237,8 @@ def check_abi() -> None:
         raise DsaltError(f"ABI version mismatch: library {h.dsalt_abi_version()} vs binding {ABI_VERSION}")
     for struct, fn in ((FwdArgs, h.dsalt_fwd_args_size), (BwdArgs, h.dsalt_bwd_args_size),
                        (SelectArgs, h.dsalt_select_args_size), (ScoresArgs, h.dsalt_scores_args_size),
-                       (RopeArgs, h.dsalt_rope_args_size), (LmkWeightsArgs, h.dsalt_lmk_weights_args_size)):
+                       (RopeArgs, h.dsalt_rope_args_size), (LmkWeightsArgs, h.dsalt_lmk_weights_args_size),
+                       (RopeTables, h.dsalt_rope_tables_size), (QkvArgs, h.dsalt_qkv_args_size)):
         if ctypes.sizeof(struct) != fn():
             raise DsaltError(f"{struct.__name__} layout mismatch: {ctypes.sizeof(struct)} vs {fn()} bytes")
 
@@ -424,13 +443,14 @@ def bwd_workspace_size(T: int, S: int, H: int, D: int, k: int) -> int:
 
 def bwd(mode: int, q, k, v, out, lse, dout, w, lmk_pos, lmk_bias, cu_seqlens, scale: float,
         tau_win: float = 1.0, win_edge: float = 4.0, need_dw: bool = False,
-        grad_dtype: torch.dtype | None = None):
-    """Sparse-attention backward. Returns (dq, dk, dv, d_lmk_bias [H,S,k] fp32 or None,
+        grad_dtype: torch.dtype | None = None, rope=None):
+    """Sparse-attention backward. ``rope = (cos, sin, dtype)``: q and k are rotated with these
+    tables (rounded to dtype); dq and dk come back for the un-rotated ones. Returns (dq, dk, dv, d_lmk_bias [H,S,k] fp32 or None,
     d_w [T] fp32 or None); dq/dk/dv are [T, H, D] per query head in ``grad_dtype`` (q.dtype
     or torch.float32, default q.dtype): with grouped K/V heads ``group_sum`` gives the K/V
     gradients."""
     launcher = BwdLauncher(mode, q, k, v, out, lse, dout, w, lmk_pos, lmk_bias, cu_seqlens, scale,
-                           tau_win, win_edge, need_dw, grad_dtype)
+                           tau_win, win_edge, need_dw, grad_dtype, rope)
     launcher()
     return launcher.results
 
@@ -441,15 +461,32 @@ class BwdLauncher:
 
     def __init__(self, mode: int, q, k, v, out, lse, dout, w, lmk_pos, lmk_bias, cu_seqlens, scale: float,
                  tau_win: float = 1.0, win_edge: float = 4.0, need_dw: bool = False,
-                 grad_dtype: torch.dtype | None = None):
+                 grad_dtype: torch.dtype | None = None, rope=None):
         self.args, self._keep, self.results, self.device = _bwd_args(
             mode, q, k, v, out, lse, dout, w, lmk_pos, lmk_bias, cu_seqlens, scale, tau_win, win_edge,
             need_dw, grad_dtype)
-        self._fn = lib().dsalt_bwd
+        self._rope, keep = _rope_tables_arg(rope, q.shape[2])
+        self._keep += (keep,)
+        self._fn = lib().dsalt_bwd_rope
         self._ref = ctypes.byref(self.args)
 
     def __call__(self) -> None:
-        _raise(self._fn(self._ref, stream_handle(self.device)), "dsalt_bwd")
+        _raise(self._fn(self._ref, self._rope, stream_handle(self.device)), "dsalt_bwd")
+
+
+def _rope_tables_arg(rope, D: int):
+    """(pointer to a RopeTables block or None, tensors to keep alive) of rope = (cos, sin, dtype)."""
+    if rope is None:
+        return None, None
+    cos, sin, dtype = rope
+    require_gpu(cos, sin)
+    cos, sin, half = rope_tables(cos, sin)
+    if cos.dim() != 2 or cos.shape != sin.shape or cos.shape[1] != D:
+        raise DsaltError(f"RoPE tables must be [rows, {D}] (got {tuple(cos.shape)}, {tuple(sin.shape)})")
+    t = RopeTables()
+    t.cos, t.sin, t.stride, t.rows = cos.data_ptr(), sin.data_ptr(), cos.stride(0), cos.shape[0]
+    t.half, t.round_dtype = int(half), _SCORE_DTYPES[dtype]
+    return ctypes.byref(t), (t, cos, sin)
 
 
 def _bwd_args(mode, q, k, v, out, lse, dout, w, lmk_pos, lmk_bias, cu_seqlens, scale, tau_win, win_edge,
@@ -584,11 +621,12 @@ class DenseFwdLauncher:
 
 
 def dense_bwd(q, k, v, out, lse, dout, w_cont, lmk_bias, scale: float, tau_win: float = 1.0,
-              win_edge: float = 4.0, need_dw: bool = True, grad_dtype: torch.dtype | None = None):
+              win_edge: float = 4.0, need_dw: bool = True, grad_dtype: torch.dtype | None = None, rope=None):
     """Dense-mode backward. Returns (dq, dk, dv in ``grad_dtype`` (default q.dtype),
-    d_lmk_bias [H, T] fp32 or None (when lmk_bias is None), d_w [T] fp32 or None)."""
+    d_lmk_bias [H, T] fp32 or None (when lmk_bias is None), d_w [T] fp32 or None).
+    ``rope``: as for ``bwd`` (head_dim 64)."""
     launcher = DenseBwdLauncher(q, k, v, out, lse, dout, w_cont, lmk_bias, scale, tau_win, win_edge,
-                                need_dw, grad_dtype)
+                                need_dw, grad_dtype, rope)
     launcher()
     return launcher.results
 
@@ -597,7 +635,7 @@ class DenseBwdLauncher:
     """A dense-mode backward with its argument block, outputs and workspace built once."""
 
     def __init__(self, q, k, v, out, lse, dout, w_cont, lmk_bias, scale: float, tau_win: float = 1.0,
-                 win_edge: float = 4.0, need_dw: bool = True, grad_dtype: torch.dtype | None = None):
+                 win_edge: float = 4.0, need_dw: bool = True, grad_dtype: torch.dtype | None = None, rope=None):
         self.device = require_gpu(q, k, v, out, lse, dout, w_cont, lmk_bias)
         T, H, D, n_kv, w, lb = _dense_common(q, k, v, w_cont, lmk_bias)
         if tuple(out.shape) != (T, H, D) or tuple(dout.shape) != (T, H, D):
@@ -641,13 +679,14 @@ class DenseBwdLauncher:
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws_bytes
         a.scale, a.tau_win, a.win_edge = float(scale), float(tau_win), float(win_edge)
         self.args = a
-        self._keep = (q, k, v, out, lse, dout, w, lb, ws)
+        self._rope, keep = _rope_tables_arg(rope, D)
+        self._keep = (q, k, v, out, lse, dout, w, lb, ws, keep)
         self.results = (dq, dk, dv, d_lb, d_w)
-        self._fn = lib().dsalt_bwd
+        self._fn = lib().dsalt_bwd_rope
         self._ref = ctypes.byref(self.args)
 
     def __call__(self) -> None:
-        _raise(self._fn(self._ref, stream_handle(self.device)), "dsalt_bwd (dense)")
+        _raise(self._fn(self._ref, self._rope, stream_handle(self.device)), "dsalt_bwd (dense)")
 
 
 def _select_args(scores, w, cu, k_lmk, out, chunked, max_seqlen=None, w_out=None, gate=None, shape=None):
@@ -775,7 +814,7 @@ class SelectHybridLauncher:
     def __init__(self, x: torch.Tensor, v: torch.Tensor, alpha: torch.Tensor, n_heads: int,
                  w_cont: torch.Tensor | None, cu_seqlens: torch.Tensor, k_lmk: int, chunked: bool = True,
                  max_seqlen: int | None = None, gate=None, norms_f32: bool | None = None, rope_k=None,
-                 gate_linear=None, quantize: bool = True):
+                 gate_linear=None, quantize: bool = True, rope_q: torch.Tensor | None = None):
         if norms_f32 is None:
             norms_f32 = autocast_norms()
         if gate_linear is not None and (gate is not None or w_cont is not None):
@@ -803,7 +842,14 @@ class SelectHybridLauncher:
             self._sa.gate_w = keep_g[0].data_ptr()
             self._sa.gate_b = _ptr(keep_g[1])
             self._sa.gate_out = self.logit.data_ptr()
-        self.k_out, keep_k = _rope_k_args(self._sa, v, rope_k)
+        # rope_q (with rope_k): the norms pass forms the attention's operands q_out, k_out and
+        # v_out - q rotated like k, and for fp32 operands all three in fp16
+        cast = rope_q is not None and v.dtype == torch.float32
+        self.k_out, keep_k = _rope_k_args(self._sa, v, rope_k, torch.float16 if cast else None)
+        self._qkv, self.q_out, self.v_out = None, None, v
+        if rope_q is not None:
+            self._qkv, self.q_out, self.v_out, keep_q = _qkv_args(rope_q, v, n_heads, cast)
+            keep_k = (keep_k, keep_q)
         self.out = torch.empty((n_heads, cu.shape[0] - 1, k_lmk), device=self.device, dtype=torch.int64)
         # quantize=False: w_cont is taken as the windows themselves (select_landmarks' test)
         self.w_out = torch.empty(T, device=self.device, dtype=torch.float32) if quantize else None
@@ -813,6 +859,9 @@ class SelectHybridLauncher:
         self._keep = (x, v, alpha, cu, ws, keep_k, keep_s, keep_g)
         self._refs = (ctypes.byref(self._sa), ctypes.byref(self._a))
         self._fn = lib().dsalt_select_hybrid
+        if self._qkv is not None:
+            self._refs += (ctypes.byref(self._qkv),)
+            self._fn = lib().dsalt_select_hybrid_qkv
 
     def __call__(self) -> None:
         _raise(self._fn(*self._refs, stream_handle(self.device)), "dsalt_select_hybrid")
@@ -982,7 +1031,38 @@ def _score_operands(x, v, alpha, n_heads):
     return x, v, alpha
 
 
-def _rope_k_args(a: ScoresArgs, v: torch.Tensor, rope_k):
+def _qkv_args(q: torch.Tensor, v: torch.Tensor, n_heads: int, cast: bool):
+    """The operand block of a norms pass that rotates q [T, H, D] too, its outputs q_out and
+    v_out (v itself without a cast) and the tensors to keep alive until the launch."""
+    T, _, D = v.shape
+    if q.dtype != v.dtype or tuple(q.shape) != (T, n_heads, D):
+        raise DsaltError(f"q must be [{T}, {n_heads}, {D}] in v's dtype (got {tuple(q.shape)} {q.dtype})")
+    q = q if q.stride(2) == 1 else q.contiguous()
+    dt = torch.float16 if cast else q.dtype
+    q_out = torch.empty((T, n_heads, D), device=q.device, dtype=dt)
+    o = QkvArgs()
+    o.out_dtype = _SCORE_DTYPES[dt]
+    o.q, o.q_stride_t, o.q_stride_h = q.data_ptr(), q.stride(0), q.stride(1)
+    o.q_out, o.q_out_stride_t, o.q_out_stride_h = q_out.data_ptr(), q_out.stride(0), q_out.stride(1)
+    v_out = v
+    if cast:
+        v_out = torch.empty(v.shape, device=v.device, dtype=dt)
+        o.v_out, o.v_out_stride_t, o.v_out_stride_h = v_out.data_ptr(), v_out.stride(0), v_out.stride(1)
+    return o, q_out, v_out, q
+
+
+def rope_operands_supported(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether the norms pass can rotate q and k beside v's norms (the rules of dsalt_scores_check
+    for k): one dtype, unit inner strides, 16-byte aligned rows, D / 2 a multiple of one
+    16-byte load."""
+    ev = 4 if v.dtype == torch.float32 else 8
+    return (q.dtype == k.dtype == v.dtype and k.shape == v.shape and q.shape[2] == v.shape[2]
+            and (v.shape[2] // 2) % ev == 0
+            and all(t.stride(2) == 1 and t.stride(0) % ev == 0 and t.stride(1) % ev == 0 and t.data_ptr() % 16 == 0
+                    for t in (q, k)))
+
+
+def _rope_k_args(a: ScoresArgs, v: torch.Tensor, rope_k, out_dtype: torch.dtype | None = None):
     """Fill the k-rotation fields of a score argument block from rope_k = (k, cos, sin,
     cu_seqlens) or leave them empty (rope_k None); returns (k_out or None, tensors to keep
     alive until the launch)."""
@@ -993,7 +1073,7 @@ def _rope_k_args(a: ScoresArgs, v: torch.Tensor, rope_k):
         raise DsaltError(f"k must match v's shape and dtype (got {tuple(k.shape)} {k.dtype}, "
                          f"{tuple(v.shape)} {v.dtype})")
     k = k if k.stride(2) == 1 else k.contiguous()
-    k_out = torch.empty_like(k)
+    k_out = torch.empty(k.shape, device=k.device, dtype=out_dtype) if out_dtype is not None else torch.empty_like(k)
     cos = cos.to(torch.float32).contiguous()
     sin = sin.to(torch.float32).contiguous()
     cu = _cu_i32(cu) if cu is not None else None

@@ -40,6 +40,7 @@ import torch.nn.functional as F
 from .. import _hip
 from ..kernels._dense import dense_attention, dense_probabilities
 from ..kernels._lmk_weights import landmark_weights
+from ..kernels._module_attention import module_attention
 from ..kernels._sparse import sparse_attention
 from ..kernels.landmark_tokens_ker import hybrid_scores_from_v, hybrid_scores_per_head
 from ..kernels.selectors import _compute_landmark_indices, _landmarks_and_windows
@@ -258,26 +259,32 @@ class DSALTAttention(nn.Module):
         k = self.k_proj(xs).view(T, self.n_kv_heads, self.head_dim)
         v = self.v_proj(xs).view(T, self.n_kv_heads, self.head_dim)
         v_sel = v if (self.v_proj.bias is None and self._fused_selector) else None
-        cu = torch.tensor([0, T], dtype=torch.int32, device=device)
-        q, k = apply_rotary_emb_packed(q, k, *self._rope_tables(), cu)
-
-        # grouped K/V heads go to the kernels as they are (query head h reads K/V head
-        # h // n_rep); no repeated copy
-        if self._hip_weights(xs, v_sel):
+        collect_P = not self.training and getattr(self, "_collect_last_P", True)
+        self._last_P = None
+        if T > 0 and not collect_P and self._hip_attention(xs, q, k, v_sel):
+            cu = torch.arange(0, T + 1, T, dtype=torch.int32, device=device)  # [0, T], made on the GPU
             w_cont = self._window_continuous(xs)
-            v, lmk_bias, lmk_pos, _ = landmark_weights(xs, v, self._alpha(), xs.new_zeros(1, dtype=torch.float32).expand(T), cu,
-                                                       min(self.k_lmk, T), T, self.tau_lmk, table=True)
+            out, lmk_pos, _ = module_attention(xs, q, k, v, w_cont, self._alpha(), *self._rope_tables(), cu,
+                                               min(self.k_lmk, T), T, self.tau_lmk, self.tau_win, float(self.win_edge),
+                                               dense=True)
         else:
+            cu = torch.tensor([0, T], dtype=torch.int32, device=device)
+            q, k = apply_rotary_emb_packed(q, k, *self._rope_tables(), cu)
+            # grouped K/V heads go to the kernels as they are (query head h reads K/V head
+            # h // n_rep); no repeated copy
             w_cont, lmk_bias, lmk_pos = self._dense_selectors(xs, T, device, v_sel)
-        out = dense_attention(q, k, v, w_cont, lmk_bias, self.tau_win, float(self.win_edge))
-        if not self.training and getattr(self, "_collect_last_P", True):
-            self._last_P = dense_probabilities(q, self._repeat_kv(k), w_cont, lmk_bias, self.tau_win,
-                                               float(self.win_edge))
-        else:
-            self._last_P = None
+            out = dense_attention(q, k, v, w_cont, lmk_bias, self.tau_win, float(self.win_edge))
+            if collect_P:
+                self._last_P = dense_probabilities(q, self._repeat_kv(k), w_cont, lmk_bias, self.tau_win,
+                                                   float(self.win_edge))
         self._last_selection = (w_cont.detach(), lmk_pos)
         aux = x.new_zeros(())
         return self._apply_out_proj(out.reshape(1, T, self.d_model)), aux
+
+    def _hip_attention(self, x: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor | None) -> bool:
+        """Whether RoPE, selection, weights and attention run as one function
+        (``module_attention``): the HIP score route, operands that its norms pass takes."""
+        return self._hip_weights(x, v) and _hip.rope_operands_supported(q, k, v)
 
     def _hip_weights(self, x: torch.Tensor, v: torch.Tensor | None) -> bool:
         """Whether the selection and its differentiable weights run on the HIP passes over x
@@ -363,6 +370,16 @@ class DSALTAttention(nn.Module):
         # x W_V^T before RoPE and the kv repeat: the selector's value norms come from it
         # (only without a projection bias, where v is exactly x W_V^T)
         v_sel = v if self.v_proj.bias is None else None
+
+        if self.training and rope_cs is None and self._hip_attention(x, q, k, v_sel):
+            self._last_P = None
+            max_len = None if cu_list is None else max((b - a for a, b in zip(cu_list[:-1], cu_list[1:])), default=0)
+            out, lmk_pos, w_disc = module_attention(x, q, k, v, self._window_continuous(x), self._alpha(),
+                                                    *self._rope_tables(), cu_seqlens, self.k_lmk, max_len, self.tau_lmk,
+                                                    self.tau_win, float(self.win_edge))
+            self._last_selection = (w_disc, lmk_pos)
+            return (self._apply_out_proj(out.reshape(total_len, self.d_model)),
+                    x.new_zeros(()) if need_aux else None)
 
         # RoPE in one HIP pass (dsalt_attention.py:570-585): positions from cu_seqlens
         # in-kernel, cos/sin rounded to q's dtype as the reference's cos.to(q.dtype). At

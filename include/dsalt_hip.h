@@ -192,6 +192,27 @@ int dsalt_bwd(const dsalt_bwd_args *args, void *stream);
 int dsalt_bwd_check(const dsalt_bwd_args *args);
 
 /*
+ * dsalt_bwd for queries and keys that were rotated by RoPE (dsalt_rope or the norms pass):
+ * args->q and args->k are the rotated ones, dq and dk come back for the un-rotated ones
+ * (the transposed rotation in fp32 as the gradients are stored, one rounding). Replaces
+ * the backward of apply_rotary_emb (dsalt/kernels/window_utils.py:73-88) after the
+ * attention's. Table rows are positions inside a sequence (the token in DSALT_MODE_DENSE);
+ * a position past the table gives NaN. rope = NULL: dsalt_bwd. DSALT_MODE_DENSE takes
+ * tables at head_dim 64 only (DSALT_ERR_UNSUPPORTED otherwise: rotate with dsalt_rope).
+ */
+typedef struct dsalt_rope_tables {
+    const float *cos, *sin; /* rows of >= head_dim entries, 16-byte aligned */
+    int64_t stride;         /* row stride (elements), a multiple of 4 */
+    int32_t rows;
+    int32_t half;           /* 1: every row repeats its first half (half of it is read) */
+    int32_t round_dtype;    /* element type that the entries are rounded to (F32: none) */
+    int32_t reserved;
+} dsalt_rope_tables;
+
+int dsalt_bwd_rope(const dsalt_bwd_args *args, const dsalt_rope_tables *rope, void *stream);
+size_t dsalt_rope_tables_size(void);
+
+/*
  * dsalt_bwd without a caller workspace and without any allocation.
  * No counterpart in the reference: it is for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
@@ -343,6 +364,28 @@ int dsalt_scores_check(const dsalt_scores_args *args);
  * except that select->scores is not read (may be NULL). total_len and n_heads must agree.
  */
 int dsalt_select_hybrid(const dsalt_scores_args *scores, const dsalt_select_args *select, void *stream);
+
+/*
+ * dsalt_select_hybrid whose norms pass also forms the attention's operands: q rotated like
+ * k (scores->k must be set; same tables and rules, n_heads heads of v_dtype), and with
+ * out_dtype = DSALT_DTYPE_F16 for v_dtype = DSALT_DTYPE_F32 the rotated q and k and the
+ * unrotated v written as fp16 (rounded from the fp32 values, as a cast after the rotation
+ * would). Otherwise out_dtype = v_dtype and v_out = NULL (v is its own operand). The
+ * k_out of `scores` has out_dtype. Outputs alias no input when out_dtype != v_dtype.
+ */
+typedef struct dsalt_qkv_args {
+    int32_t out_dtype, reserved;
+    const void *q;
+    int64_t q_stride_t, q_stride_h;
+    void *q_out;
+    int64_t q_out_stride_t, q_out_stride_h;
+    void *v_out;
+    int64_t v_out_stride_t, v_out_stride_h;
+} dsalt_qkv_args;
+
+int dsalt_select_hybrid_qkv(const dsalt_scores_args *scores, const dsalt_select_args *select,
+                            const dsalt_qkv_args *operands, void *stream);
+size_t dsalt_qkv_args_size(void);
 
 /*
  * Rotary position embedding of q and k (half-split convention) in one pass.

@@ -1,0 +1,151 @@
+"""The attention module's core as one function (RoPE, selection, weights, attention): its
+operands against dsalt_rope and a cast, the un-rotated gradients of the backward kernels
+against rotating them afterwards, and the module's output and gradients against the
+composed route (separate RoPE, selection and attention functions)."""
+import math
+
+import pytest
+import torch
+
+from dsalt import _hip
+from dsalt.kernels.window_utils import build_rope_cache
+from dsalt.modules import DSALTAttention
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+def tables(rows, D, cat=True, seed=0):
+    if cat:
+        return tuple(t.to(DEV) for t in build_rope_cache(rows, D, torch.device("cpu")))
+    g = torch.Generator().manual_seed(seed)
+    return tuple(torch.randn(rows, D, generator=g).to(DEV) for _ in range(2))
+
+
+@pytest.mark.parametrize("H,n_kv,D,dtype,strided,cat,rows", [
+    (4, 4, 64, torch.bfloat16, True, True, 300), (6, 2, 128, torch.float16, False, False, 300),
+    (8, 4, 64, torch.float32, False, True, 300), (3, 1, 128, torch.float32, True, False, 300),
+    (2, 2, 64, torch.bfloat16, False, True, 100)], ids=["bf16-strided", "fp16-d128-gqa", "fp32", "fp32-mqa-strided", "past"])
+def test_norms_pass_operands_equal_rope_then_cast(H, n_kv, D, dtype, strided, cat, rows):
+    print(f"operands H={H} n_kv={n_kv} D={D} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(H + D)
+    lens, d = [257, 0, 30], 192
+    T = sum(lens)
+    cu = torch.tensor([0, 257, 257, 287], dtype=torch.int32, device=DEV)
+    wide = torch.randn(T, H + 2 * n_kv, D, generator=g).to(DEV, dtype)
+    q, k, v = wide[:, :H], wide[:, H:H + n_kv], wide[:, H + n_kv:]
+    if not strided:
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    x = torch.randn(T, d, generator=g).to(DEV, dtype)
+    w = (1 + 60 * torch.rand(T, generator=g)).to(DEV)
+    alpha = torch.rand(H, generator=g).to(DEV)
+    cos, sin = tables(rows, D, cat)
+    f = _hip.SelectHybridLauncher(x, v, alpha, H, w, cu, 16, max_seqlen=257, rope_k=(k, cos, sin, cu), rope_q=q)
+    f()
+    q_r, k_r = _hip.rope(q, k, cos, sin, cu)
+    w_ref, pos_ref, _ = _hip.select_hybrid(x, v, alpha, H, w, cu, 16, max_seqlen=257)
+    cdt = _hip.compute_dtype(dtype)
+    assert f.q_out.dtype == f.k_out.dtype == f.v_out.dtype == cdt
+    for got, want in ((f.q_out, q_r.to(cdt)), (f.k_out, k_r.to(cdt)), (f.v_out, v.to(cdt))):
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+    assert torch.equal(f.out, pos_ref) and torch.equal(f.w_out, w_ref)
+
+
+@pytest.mark.parametrize("cat,rows", [(True, 400), (False, 400), (True, 200)], ids=["module-tables", "any-tables", "past"])
+@pytest.mark.parametrize("mode,D,dtype", [(_hip.MODE_HARD, 64, torch.bfloat16), (_hip.MODE_SOFT, 64, torch.float16),
+                                          (_hip.MODE_SOFT, 128, torch.bfloat16), (_hip.MODE_DENSE, 64, torch.bfloat16)])
+def test_backward_unrotates_like_rope(mode, D, dtype, cat, rows):
+    """dq and dk returned un-rotated against dsalt_rope's transposed rotation of the plain
+    backward's, in fp32 (the two contract products differently: a few ulp of each pair)."""
+    print(f"bwd rope mode={mode} D={D} {dtype} cat={cat} rows={rows}", flush=True)
+    g = torch.Generator().manual_seed(D + mode)
+    H, lens = 2, [331] if mode == _hip.MODE_DENSE else [331, 1, 96]
+    T = sum(lens)
+    cu_list = [0, 331] if mode == _hip.MODE_DENSE else [0, 331, 332, 428]
+    cu = torch.tensor(cu_list, dtype=torch.int32, device=DEV)
+    q, k, v, do = (torch.randn(T, H, D, generator=g).to(DEV, dtype) for _ in range(4))
+    w = (2 + 80 * torch.rand(T, generator=g)).to(DEV)
+    cos, sin = tables(rows, D, cat)
+    scale = 1 / math.sqrt(D)
+    # the tables rounded as the forward's rotation rounds them
+    cos_r, sin_r = cos.to(dtype).float(), sin.to(dtype).float()
+    if mode == _hip.MODE_DENSE:
+        out, lse = _hip.dense_fwd(q, k, v, w, None, scale)
+        run = lambda rope: _hip.dense_bwd(q, k, v, out, lse, do, w, None, scale, grad_dtype=torch.float32, rope=rope)  # noqa: E731
+    else:
+        if mode == _hip.MODE_HARD:
+            w = w.floor()
+        pos = _hip.select_landmarks(torch.randn(T, H, generator=g).to(DEV), w.floor(), cu, 12)
+        out, lse = _hip.fwd(mode, q, k, v, w, pos, None, cu, scale)
+        run = lambda rope: _hip.bwd(mode, q, k, v, out, lse, do, w, pos, None, cu, scale,  # noqa: E731
+                                    need_dw=mode == _hip.MODE_SOFT, grad_dtype=torch.float32, rope=rope)
+    plain, fused = run(None), run((cos, sin, dtype))
+    dq, dk = _hip.rope(plain[0], plain[1], cos_r, sin_r, cu, transpose=True)
+    for got, want in ((fused[0], dq), (fused[1], dk)):
+        assert torch.equal(got.isnan(), want.isnan()) and bool(got.isnan().any()) == (rows < 331)
+        got, want = got.nan_to_num(), want.nan_to_num()
+        assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())
+    for got, want in zip(fused[2:], plain[2:]):
+        assert (got is None and want is None) or torch.equal(got, want)
+
+
+CASES = {
+    # heads, n_kv, D, lens (None: unpacked), dtype, k, autocast
+    "bf16": (4, 4, 64, [300, 77, 512], torch.bfloat16, 16, False),
+    "bf16-gqa-d128": (4, 2, 128, [260, 65], torch.bfloat16, 8, False),
+    "fp32": (3, 3, 64, [200, 130], torch.float32, 8, False),
+    "autocast": (4, 4, 64, [300, 77], torch.float32, 16, True),
+    "no-landmarks": (2, 2, 64, [150], torch.bfloat16, 0, False),
+    "dense-bf16": (4, 4, 64, None, torch.bfloat16, 16, False),
+    "dense-fp32-gqa": (4, 1, 64, None, torch.float32, 16, False),
+    "dense-d128": (2, 2, 128, None, torch.bfloat16, 8, False),
+}
+
+
+@pytest.mark.parametrize("case", list(CASES))
+def test_module_training_equals_composed_route(case):
+    """Output and every gradient against the route of separate functions. Both round their
+    operands and outputs alike; the composed route also rounds dq and dk before rotating
+    them back, so the difference is bounded by a few roundings of the compute type."""
+    H, n_kv, D, lens, dtype, k, autocast = CASES[case]
+    print(f"module attention {case}", flush=True)
+    torch.manual_seed(3)
+    T = 333 if lens is None else sum(lens)
+    mod = DSALTAttention(H * D, H, 8, 100, k, max_seq_len=600, n_kv_heads=n_kv).to(DEV, dtype).train()
+    x = torch.randn(T, H * D, device=DEV).to(dtype)
+    dy = torch.randn(T, H * D, device=DEV)
+    packed = {}
+    if lens is None:
+        x, dy = x[None], dy[None]
+    else:
+        cu = torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
+        packed = {"cu_seqlens": cu, "cu_list": cu.tolist()}
+    got = {}
+    for route in ("one", "composed"):
+        if route == "composed":
+            mod._hip_attention = lambda *a: False
+        mod.zero_grad(set_to_none=True)
+        xx = x.clone().requires_grad_()
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+            y, _ = mod(xx, **packed)
+        y.backward(dy.to(y.dtype))
+        got[route] = {"y": y.detach(), "x": xx.grad, **{n: p.grad for n, p in mod.named_parameters()}}
+        got[route]["sel"] = mod._last_selection[1]
+    assert torch.equal(got["one"].pop("sel"), got["composed"].pop("sel"))
+    tol = 1e-2 if dtype == torch.bfloat16 or autocast else 2e-3
+    for name, a in got["one"].items():
+        b = got["composed"][name]
+        if a is None or b is None:  # no landmark: alpha takes no gradient
+            assert k == 0 and name == "alpha_w"
+            continue
+        assert a.dtype == b.dtype
+        if name == "win_gate.bias":  # a sum of cancelling terms: on the scale of its weight's gradient
+            assert abs(float(a - b)) <= tol * float(got["composed"]["win_gate.weight"].double().norm())
+            continue
+        bar = tol
+        if name == "alpha_w" and lens is None and dtype == torch.bfloat16:
+            # the composed dense route takes torch's norms: where their fp32 sum rounds to the
+            # other bf16 neighbour a z moves by ulp / std = 2^-5 / 0.4, one of H k terms here
+            bar = 4 * 2 ** -5 / 0.4 / math.sqrt(H * k)
+        a, b = a.double(), b.double()
+        assert float((a - b).norm()) <= bar * float(b.norm()), name
