@@ -140,6 +140,7 @@ size_t dsalt_select_args_size(void) { return sizeof(dsalt_select_args); }
 size_t dsalt_scores_args_size(void) { return sizeof(dsalt_scores_args); }
 size_t dsalt_rope_args_size(void) { return sizeof(dsalt_rope_args); }
 size_t dsalt_rope_tables_size(void) { return sizeof(dsalt_rope_tables); }
+size_t dsalt_module_grads_args_size(void) { return sizeof(dsalt_module_grads_args); }
 size_t dsalt_qkv_args_size(void) { return sizeof(dsalt_qkv_args); }
 size_t dsalt_lmk_weights_args_size(void) { return sizeof(dsalt_lmk_weights_args); }
 
@@ -323,21 +324,33 @@ int dsalt_hybrid_scores(const dsalt_scores_args *a, void *stream) {
 
 namespace {
 
-int check_operands(const dsalt_scores_args *sa, const dsalt_qkv_args *o) {
-    if (!sa->k) return fail(DSALT_ERR_INVALID, "q needs k (and the RoPE tables) in the score arguments");
+int check_operands(const dsalt_scores_args *sa, const dsalt_select_args *a, const dsalt_qkv_args *o) {
+    if (!sa->k) return fail(DSALT_ERR_INVALID, "the operands need k (and the RoPE tables) in the score arguments");
     const bool cast = sa->v_dtype == DSALT_DTYPE_F32 && o->out_dtype == DSALT_DTYPE_F16;
     if (!cast && o->out_dtype != sa->v_dtype)
         return fail(DSALT_ERR_INVALID, "out_dtype must be v_dtype, or F16 for fp32 operands (got %d)", o->out_dtype);
     if (cast != (o->v_out != nullptr)) return fail(DSALT_ERR_INVALID, "v_out goes with fp16 outputs of fp32 operands");
+    if (o->win_w) {
+        const bool low = o->win_dtype == DSALT_DTYPE_BF16 || o->win_dtype == DSALT_DTYPE_F16;
+        if (o->win_dtype != sa->x_dtype && !(low && sa->x_dtype == DSALT_DTYPE_F32))
+            return fail(DSALT_ERR_INVALID, "win_dtype must be x_dtype, or a 16-bit type for fp32 x (got %d)", o->win_dtype);
+        if (sa->gate_w) return fail(DSALT_ERR_INVALID, "win_w replaces gate_w");
+        if (!o->win_logit || !o->win_out) return fail(DSALT_ERR_INVALID, "win_w needs win_logit and win_out");
+        if (!aligned(o->win_w, 16) || !aligned(o->win_b, sa->x_dtype == DSALT_DTYPE_F32 ? 4 : 2))
+            return fail(DSALT_ERR_INVALID, "win_w must be 16-byte aligned, win_b to its element");
+        if (!(o->n_min == o->n_min) || !(o->n_max == o->n_max))
+            return fail(DSALT_ERR_INVALID, "n_min and n_max must not be NaN");
+        if (a->w_logit) return fail(DSALT_ERR_INVALID, "win_w forms the windows: w_logit must be NULL");
+    }
     if (sa->total_len == 0) return DSALT_OK;
-    if (!o->q || !o->q_out) return fail(DSALT_ERR_INVALID, "q and q_out must be non-NULL");
+    if (o->q && !o->q_out) return fail(DSALT_ERR_INVALID, "q needs q_out");
     const int ev = sa->v_dtype == DSALT_DTYPE_F32 ? 4 : 8;
     if (!aligned(o->q, 16) || !aligned(o->q_out, 16) || !aligned(o->v_out, 16))
         return fail(DSALT_ERR_INVALID, "q, q_out and v_out must be 16-byte aligned");
     for (int64_t st : {o->q_stride_t, o->q_stride_h, o->q_out_stride_t, o->q_out_stride_h, o->v_out_stride_t,
                        o->v_out_stride_h})
         if (st < 0 || st % ev) return fail(DSALT_ERR_INVALID, "operand strides must be non-negative multiples of %d", ev);
-    if (cast && (o->q_out == o->q || o->v_out == sa->v || sa->k_out == sa->k))
+    if (cast && ((o->q && o->q_out == o->q) || o->v_out == sa->v || sa->k_out == sa->k))
         return fail(DSALT_ERR_INVALID, "fp16 outputs must not alias the fp32 operands");
     return DSALT_OK;
 }
@@ -350,7 +363,7 @@ int select_hybrid(const dsalt_scores_args *sa, const dsalt_select_args *a, const
     if (sa->total_len != a->total_len || sa->n_heads != a->n_heads)
         return fail(DSALT_ERR_INVALID, "score and selection arguments disagree: total_len %d / %d, n_heads %d / %d",
                     sa->total_len, a->total_len, sa->n_heads, a->n_heads);
-    if (o && (rc = check_operands(sa, o))) return rc;
+    if (o && (rc = check_operands(sa, a, o))) return rc;
     const hipStream_t st = static_cast<hipStream_t>(stream);
     dsalt::HybridSrc src;
     hipError_t e = dsalt::launch_norms_for_select(*sa, o, src, st);
@@ -440,6 +453,73 @@ int dsalt_lmk_weights_bwd(const dsalt_lmk_weights_args *a, void *stream) {
     hipError_t e = dsalt::launch_lmk_weights_bwd(*a, static_cast<hipStream_t>(stream));
     if (e != hipSuccess)
         return fail(DSALT_ERR_LAUNCH, "dsalt_lmk_weights_bwd launch failed: %s", hipGetErrorString(e));
+    return DSALT_OK;
+}
+
+int64_t dsalt_module_grads_workspace_size(int32_t total_len, int32_t n_heads, int32_t d_model) {
+    if (total_len < 0 || n_heads < 1 || d_model < 1) return -1;
+    return dsalt::module_grads_workspace_bytes(total_len, n_heads, d_model);
+}
+
+namespace {
+
+int check_module_grads(const dsalt_module_grads_args *a, bool x_step) {
+    if (!a) return fail(DSALT_ERR_INVALID, "args is NULL");
+    const dsalt_lmk_weights_args &w = a->weights;
+    int rc = dsalt_lmk_weights_check(&w, 1);
+    if (rc) return rc;
+    if (w.total_len == 0) return DSALT_OK;
+    if (w.d_model < 1) return fail(DSALT_ERR_INVALID, "d_model must be >= 1");
+    const int64_t need = dsalt::module_grads_workspace_bytes(w.total_len, w.n_heads, w.d_model);
+    if (w.workspace_bytes < need)
+        return fail(DSALT_ERR_INVALID, "workspace too small: %lld < %lld bytes", (long long)w.workspace_bytes,
+                    (long long)need);
+    const int ex = w.x_dtype == DSALT_DTYPE_F32 ? 4 : 8, ev = w.v_dtype == DSALT_DTYPE_F32 ? 4 : 8;
+    if (!x_step) {
+        const bool grouped = w.n_heads != w.n_kv_heads;
+        if (a->heads_dtype != w.v_dtype && a->heads_dtype != DSALT_DTYPE_F32)
+            return fail(DSALT_ERR_INVALID, "heads_dtype must be v_dtype or F32 (got %d)", a->heads_dtype);
+        if (w.head_dim < 1 || w.head_dim % ev) return fail(DSALT_ERR_UNSUPPORTED, "head_dim must be a multiple of %d", ev);
+        if (!w.v || !aligned(w.v, 16) || w.v_stride_t < 0 || w.v_stride_h < 0 || w.v_stride_t % ev || w.v_stride_h % ev)
+            return fail(DSALT_ERR_INVALID, "v must be 16-byte aligned with strides multiples of %d", ev);
+        if (!a->dv || !a->dv_heads || (grouped && (!a->dk || !a->dk_heads)))
+            return fail(DSALT_ERR_INVALID, "dv and dv_heads (and with grouped heads dk and dk_heads) must be non-NULL");
+        if (!aligned(a->dv, 16) || !aligned(a->dv_heads, 16) || (grouped && (!aligned(a->dk, 16) || !aligned(a->dk_heads, 16))))
+            return fail(DSALT_ERR_INVALID, "the gradients must be 16-byte aligned");
+        for (int64_t st : {a->dkh_stride_t, a->dkh_stride_h, a->dvh_stride_t, a->dvh_stride_h, a->dk_stride_t,
+                           a->dk_stride_h, a->dv_stride_t, a->dv_stride_h})
+            if (st < 0 || st % ev)
+                return fail(DSALT_ERR_INVALID, "gradient strides must be non-negative multiples of %d", ev);
+        return DSALT_OK;
+    }
+    if (w.d_model % ex) return fail(DSALT_ERR_UNSUPPORTED, "d_model must be a multiple of %d", ex);
+    if (!w.x || !aligned(w.x, 16) || w.x_stride_t < w.d_model || w.x_stride_t % ex)
+        return fail(DSALT_ERR_INVALID, "x must be 16-byte aligned, its row stride a multiple of %d", ex);
+    if (!aligned(a->dx, 16) || !aligned(a->dx_in, 16)) return fail(DSALT_ERR_INVALID, "dx and dx_in must be 16-byte aligned");
+    for (int dt : {a->in_dtype, a->win_dtype})
+        if (dt != DSALT_DTYPE_BF16 && dt != DSALT_DTYPE_F16 && dt != DSALT_DTYPE_F32)
+            return fail(DSALT_ERR_INVALID, "in_dtype and win_dtype must be DSALT_DTYPE_BF16, _F16 or _F32 (got %d, %d)",
+                        a->in_dtype, a->win_dtype);
+    if (a->win_w && (!a->win_logit || !a->d_w || !aligned(a->win_w, 16)))
+        return fail(DSALT_ERR_INVALID, "win_w (16-byte aligned) needs win_logit and d_w");
+    return DSALT_OK;
+}
+
+}  // namespace
+
+int dsalt_module_grads_v(const dsalt_module_grads_args *a, void *stream) {
+    int rc = check_module_grads(a, false);
+    if (rc) return rc;
+    hipError_t e = dsalt::launch_module_grads_v(*a, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(DSALT_ERR_LAUNCH, "dsalt_module_grads_v launch failed: %s", hipGetErrorString(e));
+    return DSALT_OK;
+}
+
+int dsalt_module_grads_x(const dsalt_module_grads_args *a, void *stream) {
+    int rc = check_module_grads(a, true);
+    if (rc) return rc;
+    hipError_t e = dsalt::launch_module_grads_x(*a, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(DSALT_ERR_LAUNCH, "dsalt_module_grads_x launch failed: %s", hipGetErrorString(e));
     return DSALT_OK;
 }
 
@@ -587,8 +667,8 @@ int dsalt_bwd_rope(const dsalt_bwd_args *a, const dsalt_rope_tables *r, void *st
             return fail(DSALT_ERR_INVALID,
                         "RoPE tables need rows >= 1, stride >= head_dim and a multiple of 4, 16-byte alignment "
                         "(rows %d, stride %lld)", r->rows, (long long)r->stride);
-        if (r->round_dtype != DSALT_DTYPE_BF16 && r->round_dtype != DSALT_DTYPE_F16 && r->round_dtype != DSALT_DTYPE_F32)
-            return fail(DSALT_ERR_INVALID, "round_dtype must be DSALT_DTYPE_BF16, _F16 or _F32 (got %d)", r->round_dtype);
+        if (r->round_dtype != a->dtype && r->round_dtype != DSALT_DTYPE_F32)
+            return fail(DSALT_ERR_INVALID, "round_dtype must equal dtype or be DSALT_DTYPE_F32 (got %d)", r->round_dtype);
     }
     hipError_t e = dsalt::launch_bwd(*a, r, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(DSALT_ERR_LAUNCH, "dsalt_bwd_rope launch failed: %s", hipGetErrorString(e));

@@ -563,7 +563,7 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
         float mul = p.scale;
         const RopeRows rope = late_rope_rows(offsetof(BwdParams, rope));
         if (rope.cos) {
-            rotate_acc_transposed<ND>(dqacc, mul, rope, i, hh);
+            rotate_acc_transposed<DT, ND>(dqacc, mul, rope, i, hh);
             mul = 1.f;
         }
         store_row<DT, ND>(p.dq, tok_i * p.dq_st + (int64_t)head * p.dq_sh, p.grad_f32, dqacc, mul, hh);
@@ -1328,7 +1328,7 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
             float mul = p.scale;
             const RopeRows rope = late_rope_rows(offsetof(BwdParams, rope));
             if (rope.cos) {
-                rotate_acc_transposed<ND>(dk, mul, rope, key, hh);
+                rotate_acc_transposed<DT, ND>(dk, mul, rope, key, hh);
                 mul = 1.f;
             }
             store_row<DT, ND>(p.dk, tok * p.dk_st + (int64_t)head * p.dk_sh, p.grad_f32, dk, mul, hh);

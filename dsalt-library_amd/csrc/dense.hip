@@ -562,7 +562,7 @@ __global__ void __launch_bounds__(128 * dense_bwd_groups(D), 1) dense_dq_kernel(
         if constexpr (D == 64) {  // at D = 128 the rotation costs dq its second wave per SIMD
             const RopeRows rope = late_rope_rows(offsetof(DenseParams, rope));
             if (rope.cos) {
-                rotate_acc_transposed<ND>(dq, mul, rope, i, hh);
+                rotate_acc_transposed<DT, ND>(dq, mul, rope, i, hh);
                 mul = 1.f;
             }
         }
@@ -756,7 +756,7 @@ __global__ void __launch_bounds__(128 * dense_bwd_groups(D), 1) dense_kv_kernel(
         }
         __syncthreads();
         if (grp == 0) {
-#pragma unroll
+#pragma unroll 1  // one group's partials in registers at a time
             for (int g = 1; g < NG; ++g) {
 #pragma unroll
                 for (int d = 0; d < ND; ++d)
@@ -775,7 +775,7 @@ __global__ void __launch_bounds__(128 * dense_bwd_groups(D), 1) dense_kv_kernel(
         }
         __syncthreads();
         if (grp > 0) return;
-#pragma unroll
+#pragma unroll 1
         for (int g = 1; g < NG; ++g)
 #pragma unroll
             for (int d = 0; d < ND; ++d)
@@ -790,7 +790,7 @@ __global__ void __launch_bounds__(128 * dense_bwd_groups(D), 1) dense_kv_kernel(
         if constexpr (D == 64) {  // at D = 128 the rotation costs dq its second wave per SIMD
             const RopeRows rope = late_rope_rows(offsetof(DenseParams, rope));
             if (rope.cos) {
-                rotate_acc_transposed<ND>(dk, mul, rope, j, hh);
+                rotate_acc_transposed<DT, ND>(dk, mul, rope, j, hh);
                 mul = 1.f;
             }
         }

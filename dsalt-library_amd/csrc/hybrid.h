@@ -57,4 +57,15 @@ __device__ __forceinline__ float hybrid_mix(float zx, float zv, float alpha) {
     return __fadd_rn(__fmul_rn(alpha, zv), __fmul_rn(__fsub_rn(1.0f, alpha), zx));
 }
 
+// The module's continuous window of a gate logit, in torch's
+// operation order and roundings: sigmoid(x) = 1 / (1 + exp(-x)) in fp32 (expf, IEEE
+// division), rounded to the logit's dtype by rnd; times span, rounded; plus n_min, rounded
+// (dsalt_attention.py:270-276 of the reference: n_min + sigmoid(win_gate(x)) * (n_max - n_min)).
+template <typename R>
+__device__ __forceinline__ float gate_window(float x, float n_min, float span, R rnd) {
+    const float sg = rnd(1.f / (1.f + expf(-x)));
+    const float t = rnd(__fmul_rn(sg, span));
+    return rnd(__fadd_rn(n_min, t));
+}
+
 }  // namespace dsalt

@@ -57,6 +57,9 @@ NormsView scores_workspace_view(void *workspace, int total_len, int n_kv);
 hipError_t launch_lmk_weights(const dsalt_lmk_weights_args &a, hipStream_t stream);
 hipError_t launch_lmk_weights_bwd(const dsalt_lmk_weights_args &a, hipStream_t stream);
 int64_t lmk_weights_workspace_bytes(int total_len, int n_heads);
+hipError_t launch_module_grads_v(const dsalt_module_grads_args &a, hipStream_t stream);
+hipError_t launch_module_grads_x(const dsalt_module_grads_args &a, hipStream_t stream);
+int64_t module_grads_workspace_bytes(int total_len, int n_heads, int d_model);
 hipError_t launch_quantize(const float *w_cont, int64_t n, float *w_out, int32_t *w_int,
                            hipStream_t stream);
 hipError_t launch_swiglu(const void *gate, const void *up, void *out, int64_t n, int dtype, hipStream_t stream);

@@ -24,10 +24,13 @@
 // forms the window gate's logit x_t . w + b (win_gate, dsalt_attention.py:270-276) from
 // the x chunks it loads: fp32 products and sums in a fixed order, the bias added, one
 // rounding to x's dtype; this replaces the module's GEMV and its bias copy.
-// With q given as well (dsalt_select_hybrid_qkv), the same pass rotates q, and for fp32
-// operands it writes q, k and v as the fp16 operands that the attention takes: training
-// and the dense variant then need no RoPE launch and no casts (9290 tokens x 16 heads x 64
-// in bf16: RoPE pass 22.2 + norms 11.6 us before).
+// The module form (dsalt_select_hybrid_qkv) also rotates q, forms the windows and, for fp32
+// operands, writes q, k and v as the fp16 operands that the attention takes: training and
+// the dense variant then need no RoPE launch, gate GEMV, window ops or casts. 9290 tokens x
+// 16 heads x 64 in bf16: 34.4 us against 22.2 (RoPE) + 11.6 (norms) + 30 (gate, windows).
+// A pass is bound by each wave's chain of loads at the waves that its registers allow: with
+// one table read per token, 16-bit rows and tables kept packed and reductions by DPP the
+// inference form (8192 tokens: x, v, k) went 20.0 -> 15.3 us, 5.5 TB/s.
 #include "common.h"
 #include "launch.h"
 #include "hybrid.h"
@@ -36,6 +39,29 @@
 #include <type_traits>
 
 namespace dsalt {
+
+// Sum over the aligned groups of W lanes (W a power of two <= 64; every lane of a group
+// receives it), with the same tree as a butterfly of lane exchanges by 1, 2, 4, ..., hence
+// the same bits: the first four levels are DPP adds (quad permutes and row mirrors: after a
+// level the lanes of a pair hold equal sums, so a mirror reaches the partner group as well
+// as an exchange does), which cost no LDS round trip; the last two exchange rows through
+// v_permlane{16,32}_swap.
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float x) {
+    return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float group_sum_lanes(float x, int width) {
+    if (width > 1) x = dpp_add<0xB1>(x);   // quad_perm [1,0,3,2]
+    if (width > 2) x = dpp_add<0x4E>(x);   // quad_perm [2,3,0,1]
+    if (width > 4) x = dpp_add<0x141>(x);  // row_half_mirror
+    if (width > 8) x = dpp_add<0x140>(x);  // row_mirror
+    if (width > 16) {
+        auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    if (width > 32) x = half_sum(x);
+    return x;
+}
 namespace {
 
 constexpr int kNormTokens = 16;    // tokens (= waves) per workgroup of norms_kernel
@@ -66,8 +92,19 @@ struct ScoreParams {
     const void *q;
     void *q_out, *v_out;
     int64_t q_st, q_sh, qo_st, qo_sh, vo_st, vo_sh;
-    int out_f16;
+    int out_f16, rope_rep;
+    // optional window gate (module form): logit = x . win_w + win_b on operands rounded to
+    // win_dt, rounded to win_dt; w~ = n_min + sigmoid(logit) span with every step so rounded
+    const void *win_w, *win_b;  // in x's dtype
+    float *win_logit, *win_out; // [T]
+    int win_dt;
+    float n_min, span;
 };
+
+// v rounded to element type `dt` (a DSALT_DTYPE_*)
+__device__ __forceinline__ float round_to(float v, int dt) {
+    return dt == DSALT_DTYPE_BF16 ? BF16::round(v) : dt == DSALT_DTYPE_F16 ? F16::round(v) : v;
+}
 
 // Element loads and the dtype rounding of a norm, per storage type.
 struct LdBF16 {
@@ -155,19 +192,17 @@ template <> struct ElemOf<LdBF16> { typedef BF16 T; };
 template <> struct ElemOf<LdF16> { typedef F16 T; };
 template <> struct ElemOf<LdF32> { typedef F32 T; };
 
-// Sum over the `width` lanes of each aligned lane group (width a power of two <= 64);
-// every lane of the group receives it.
-__device__ __forceinline__ float group_sum(float x, int width) {
-    for (int o = 1; o < width; o <<= 1) x += __shfl_xor(x, o);
-    return x;
-}
-
-template <typename LX, typename LV>
-__global__ void __launch_bounds__(64 * kNormTokens) norms_kernel(const ScoreParams p) {
+// FULL: the module form (q rotated too, fp16 operands, the windows). Without it the kernel is
+// held to 64 registers, 8 waves per SIMD: a workgroup has 16 waves, so one register more
+// would halve the resident workgroups (the module form spills there).
+template <typename LX, typename LV, bool FULL>
+__global__ void __launch_bounds__(64 * kNormTokens, FULL ? 4 : 8) norms_kernel(const ScoreParams p) {
     constexpr int EX = LX::E, EV = LV::E;
+    typedef typename ElemOf<LX>::T DX;
     constexpr int BX = EX == 8 ? 2 : 4, BV = EV == 8 ? 2 : 4;  // bytes per element
     __shared__ float s_n[kNormTokens][1 + kMaxKvScores];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // the wave id as a scalar: row addresses and the position then cost no vector registers
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int t0 = blockIdx.x * kNormTokens;
     const int G = p.D / EV;         // lanes per v row
     const int rows_per = 64 / G;    // v rows per load instruction
@@ -176,10 +211,41 @@ __global__ void __launch_bounds__(64 * kNormTokens) norms_kernel(const ScorePara
         // ||x_t||: lanes stride the row in 16-byte chunks
         const char *xr = static_cast<const char *>(p.x) + (int64_t)t * p.x_st * BX;
         float sx = 0.f;
-        if constexpr (EX == 8) {
-            if (p.gate_w) {
-                // the window gate's logit from the same chunks: each lane sums its chunks'
-                // products in order, then the lanes' sums are added by a fixed butterfly
+        if (FULL && p.win_w) {
+            // the module's gate: products of the rounded operands summed in fp64 (16-bit products
+            // are exact), so that the logit's one rounding is the correctly rounded one
+            const char *gw = static_cast<const char *>(p.win_w);
+            double gd = 0.0;
+#pragma unroll 1
+            for (int c = lane * EX; c < p.d; c += 64 * EX) {
+                float xa[EX], ga[EX];
+                Elem<DX>::template ldv<EX>(xr, c, xa);
+                Elem<DX>::template ldv<EX>(gw, c, ga);
+                if constexpr (EX == 8) {
+                    sx += LX::sumsq(*reinterpret_cast<const uint4 *>(xr + (int64_t)c * BX));
+                } else {
+                    sx += LX::sumsq16(xr + (int64_t)c * BX);
+#pragma unroll
+                    for (int e = 0; e < EX; ++e) {
+                        xa[e] = round_to(xa[e], p.win_dt);
+                        ga[e] = round_to(ga[e], p.win_dt);
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < EX; ++e) gd = fma((double)xa[e], (double)ga[e], gd);
+            }
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) gd += __shfl_xor(gd, o);
+            if (lane == 0) {
+                if (p.win_b) gd += (double)round_to(Elem<DX>::ld(p.win_b, 0), p.win_dt);
+                const float logit = round_to((float)gd, p.win_dt);
+                p.win_logit[t] = logit;
+                p.win_out[t] = gate_window(logit, p.n_min, p.span, [&](float v) { return round_to(v, p.win_dt); });
+            }
+        } else if (!FULL && EX == 8 && p.gate_w) {
+            // the window gate's logit from the same chunks: each lane sums its chunks'
+            // products in order, then the lanes' sums are added by a fixed butterfly
+            if constexpr (EX == 8) {
                 const char *gw = static_cast<const char *>(p.gate_w);
                 float gd = 0.f;
                 for (int c = lane * EX; c < p.d; c += 64 * EX) {
@@ -187,20 +253,18 @@ __global__ void __launch_bounds__(64 * kNormTokens) norms_kernel(const ScorePara
                     sx += LX::sumsq(xv);
                     gd = LX::dot(xv, *reinterpret_cast<const uint4 *>(gw + (int64_t)c * BX), gd);
                 }
-                gd = group_sum(gd, 64);
+                gd = group_sum_lanes(gd, 64);
                 if (lane == 0) {
                     float logit = p.gate_b ? gd + LX::ld1(p.gate_b) : gd;
                     // rounded to fp32 first: no mixed-precision fold of the sum and the conversion
                     asm volatile("" : "+v"(logit));
                     LX::st1(static_cast<char *>(p.gate_out) + (int64_t)t * BX, LX::round(logit));
                 }
-            } else {
-                for (int c = lane * EX; c < p.d; c += 64 * EX) sx += LX::sumsq16(xr + (int64_t)c * BX);
             }
         } else {
             for (int c = lane * EX; c < p.d; c += 64 * EX) sx += LX::sumsq16(xr + (int64_t)c * BX);
         }
-        sx = group_sum(sx, 64);
+        sx = group_sum_lanes(sx, 64);
         const float xn = p.norms_f32 ? sqrtf(sx) : LX::round(sqrtf(sx));
         if (lane == 0) {
             p.xn[t] = xn;
@@ -212,7 +276,7 @@ __global__ void __launch_bounds__(64 * kNormTokens) norms_kernel(const ScorePara
             const int g = g0 + lane / G;
             float sv = 0.f;
             if (g < p.n_kv) sv = LV::sumsq16(vr + ((int64_t)g * p.v_sh + (lane % G) * EV) * BV);
-            sv = group_sum(sv, G);
+            sv = group_sum_lanes(sv, G);
             const float vn = p.norms_f32 ? sqrtf(sv) : LV::round(sqrtf(sv));
             if (g < p.n_kv && lane % G == 0) {
                 p.vn[(int64_t)t * p.n_kv + g] = vn;
@@ -228,24 +292,34 @@ __global__ void __launch_bounds__(64 * kNormTokens) norms_kernel(const ScorePara
             const float *cr = p.cos + (int64_t)(in_table ? pos : 0) * p.cs_st;
             const float *sr = p.sin + (int64_t)(in_table ? pos : 0) * p.cs_st;
             typedef typename ElemOf<LV>::T DT;
-            auto rotate = [&](const void *in, int64_t ib, int64_t ih, void *out, int64_t ob, int64_t oh, int heads) {
-                for (int r = lane; r < heads * nj; r += 64) {
-                    const int h = r / nj, j0 = (r - h * nj) * VW;
-                    const int64_t i0 = ib + (int64_t)h * ih, o0 = ob + (int64_t)h * oh;
-                    if constexpr (std::is_same<DT, F32>::value) {
-                        if (p.out_f16) {
-                            rotate_vec<DT, VW, F16>(in, i0, out, o0, cr, sr, half, j0, in_table, false);
-                            continue;
-                        }
+            // nj divides 64: a lane rotates the same pairs of every head row, so its table
+            // entries are read and rounded once a token (they are 4 to 16 times the bytes of
+            // the pairs themselves)
+            const int j0 = (lane & (nj - 1)) * VW;
+            RopeVec<DT, VW> tv;
+            tv.template load<true>(cr, sr, half, j0, in_table, p.rope_rep != 0);
+            const int rows = (p.n_kv + (FULL && p.q ? p.H : 0)) * nj;
+#pragma unroll 1  // unrolled, the addresses and rows of two steps cost half the waves
+            for (int r = lane; r < rows; r += 64) {  // k's heads, then q's
+                tv.pin();
+                const bool isq = FULL && r >= p.n_kv * nj;
+                const int h = (isq ? r - p.n_kv * nj : r) / nj;
+                const void *in = isq ? p.q : p.k;
+                void *out = isq ? p.q_out : p.k_out;
+                const int64_t ib = (int64_t)t * (isq ? p.q_st : p.k_st) + (int64_t)h * (isq ? p.q_sh : p.k_sh);
+                const int64_t ob = (int64_t)t * (isq ? p.qo_st : p.ko_st) + (int64_t)h * (isq ? p.qo_sh : p.ko_sh);
+                if constexpr (FULL && std::is_same<DT, F32>::value) {
+                    if (p.out_f16) {
+                        rotate_pairs<DT, VW, F16>(in, ib, out, ob, tv, half, j0, false);
+                        continue;
                     }
-                    rotate_vec<DT, VW>(in, i0, out, o0, cr, sr, half, j0, in_table, false);
                 }
-            };
-            rotate(p.k, (int64_t)t * p.k_st, p.k_sh, p.k_out, (int64_t)t * p.ko_st, p.ko_sh, p.n_kv);
-            if (p.q) rotate(p.q, (int64_t)t * p.q_st, p.q_sh, p.q_out, (int64_t)t * p.qo_st, p.qo_sh, p.H);
-            if constexpr (std::is_same<DT, F32>::value) {
+                rotate_pairs<DT, VW>(in, ib, out, ob, tv, half, j0, false);
+            }
+            if constexpr (FULL && std::is_same<DT, F32>::value) {
                 if (p.v_out) {
                     const int nv = p.D / VW;
+#pragma unroll 1
                     for (int r = lane; r < p.n_kv * nv; r += 64) {
                         const int h = r / nv, j0 = (r - h * nv) * VW;
                         float a[VW];
@@ -307,20 +381,19 @@ __global__ void __launch_bounds__(256) standardize_kernel(const ScoreParams p) {
 
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
-template <typename LX>
+template <typename LX, bool FULL>
 void launch_norms_x(int v_dtype, const ScoreParams &p, hipStream_t stream) {
-    if (v_dtype == DSALT_DTYPE_BF16)
-        hipLaunchKernelGGL((norms_kernel<LX, LdBF16>), dim3(p.nblk), dim3(64 * kNormTokens), 0, stream, p);
-    else if (v_dtype == DSALT_DTYPE_F16)
-        hipLaunchKernelGGL((norms_kernel<LX, LdF16>), dim3(p.nblk), dim3(64 * kNormTokens), 0, stream, p);
-    else
-        hipLaunchKernelGGL((norms_kernel<LX, LdF32>), dim3(p.nblk), dim3(64 * kNormTokens), 0, stream, p);
+    const dim3 grid(p.nblk), block(64 * kNormTokens);
+    if (v_dtype == DSALT_DTYPE_BF16) hipLaunchKernelGGL((norms_kernel<LX, LdBF16, FULL>), grid, block, 0, stream, p);
+    else if (v_dtype == DSALT_DTYPE_F16) hipLaunchKernelGGL((norms_kernel<LX, LdF16, FULL>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((norms_kernel<LX, LdF32, FULL>), grid, block, 0, stream, p);
 }
 
+template <bool FULL>
 void launch_norms(int x_dtype, int v_dtype, const ScoreParams &p, hipStream_t stream) {
-    if (x_dtype == DSALT_DTYPE_BF16) launch_norms_x<LdBF16>(v_dtype, p, stream);
-    else if (x_dtype == DSALT_DTYPE_F16) launch_norms_x<LdF16>(v_dtype, p, stream);
-    else launch_norms_x<LdF32>(v_dtype, p, stream);
+    if (x_dtype == DSALT_DTYPE_BF16) launch_norms_x<LdBF16, FULL>(v_dtype, p, stream);
+    else if (x_dtype == DSALT_DTYPE_F16) launch_norms_x<LdF16, FULL>(v_dtype, p, stream);
+    else launch_norms_x<LdF32, FULL>(v_dtype, p, stream);
 }
 
 }  // namespace
@@ -399,7 +472,7 @@ ScoreParams make_params(const dsalt_scores_args &a) {
 hipError_t launch_scores(const dsalt_scores_args &a, hipStream_t stream) {
     if (a.total_len == 0) return hipSuccess;
     const ScoreParams p = make_params(a);
-    launch_norms(a.x_dtype, a.v_dtype, p, stream);
+    launch_norms<false>(a.x_dtype, a.v_dtype, p, stream);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(stats_kernel, dim3(1), dim3(1024), 0, stream, p);
@@ -422,6 +495,14 @@ hipError_t launch_norms_for_select(const dsalt_scores_args &a, const dsalt_qkv_a
         p.vo_st = o->v_out_stride_t;
         p.vo_sh = o->v_out_stride_h;
         p.out_f16 = o->out_dtype == DSALT_DTYPE_F16 && a.v_dtype == DSALT_DTYPE_F32;
+        p.rope_rep = o->rope_half;
+        p.win_w = o->win_w;
+        p.win_b = o->win_b;
+        p.win_logit = o->win_logit;
+        p.win_out = o->win_out;
+        p.win_dt = o->win_dtype;
+        p.n_min = o->n_min;
+        p.span = o->n_max - o->n_min;
     }
     src.xn = p.xn;
     src.vn = p.vn;
@@ -432,7 +513,8 @@ hipError_t launch_norms_for_select(const dsalt_scores_args &a, const dsalt_qkv_a
     src.n_heads = p.H;
     src.total_len = p.T;
     if (a.total_len == 0) return hipSuccess;
-    launch_norms(a.x_dtype, a.v_dtype, p, stream);
+    if (o) launch_norms<true>(a.x_dtype, a.v_dtype, p, stream);
+    else launch_norms<false>(a.x_dtype, a.v_dtype, p, stream);
     return hipGetLastError();
 }
 

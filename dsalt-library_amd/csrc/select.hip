@@ -148,16 +148,6 @@ __device__ __forceinline__ void block_excl_scan2(int a, int b, int lane, int wav
 // max(1, floor(w)), NaN kept: DSALTAttention._window_sizes(floor=True)
 __device__ __forceinline__ float quantize_window(float x) { return (x != x) ? x : fmaxf(floorf(x), 1.f); }
 
-// The module's continuous window of token `tok` from its 16-bit gate logit, in torch's
-// operation order and roundings: sigmoid(x) = 1 / (1 + exp(-x)) in fp32 (expf, IEEE
-// division), rounded to the logit's dtype; times span, rounded; plus n_min, rounded
-// (dsalt_attention.py:270-276 of the reference: n_min + sigmoid(win_gate(x)) * (n_max - n_min)).
-template <typename R>
-__device__ __forceinline__ float gate_window(float x, float n_min, float span, R rnd) {
-    const float sg = rnd(1.f / (1.f + expf(-x)));
-    const float t = rnd(__fmul_rn(sg, span));
-    return rnd(__fadd_rn(n_min, t));
-}
 __device__ __forceinline__ float window_of(const float *w, int64_t w_st, const void *logit, int64_t l_st, int l_dt,
                                            float n_min, float span, int64_t tok) {
     if (!logit) return w[tok * w_st];

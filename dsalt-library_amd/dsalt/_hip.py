@@ -136,10 +136,12 @@ class RopeTables(ctypes.Structure):
 
 class QkvArgs(ctypes.Structure):
     _fields_ = [
-        ("out_dtype", c_int32), ("reserved", c_int32),
+        ("out_dtype", c_int32), ("rope_half", c_int32),
         ("q", c_void_p), ("q_stride_t", c_int64), ("q_stride_h", c_int64),
         ("q_out", c_void_p), ("q_out_stride_t", c_int64), ("q_out_stride_h", c_int64),
         ("v_out", c_void_p), ("v_out_stride_t", c_int64), ("v_out_stride_h", c_int64),
+        ("win_w", c_void_p), ("win_b", c_void_p), ("win_logit", c_void_p), ("win_out", c_void_p),
+        ("win_dtype", c_int32), ("n_min", c_float), ("n_max", c_float), ("reserved", c_int32),
     ]
 
 
@@ -159,6 +161,22 @@ class LmkWeightsArgs(ctypes.Structure):
     ]
 
 
+class ModuleGradsArgs(ctypes.Structure):
+    _fields_ = [
+        ("weights", LmkWeightsArgs),
+        ("heads_dtype", c_int32), ("in_dtype", c_int32), ("win_dtype", c_int32), ("alpha_sigmoid", c_int32),
+        ("d_alpha", c_void_p),
+        ("dk_heads", c_void_p), ("dv_heads", c_void_p),
+        ("dkh_stride_t", c_int64), ("dkh_stride_h", c_int64), ("dvh_stride_t", c_int64), ("dvh_stride_h", c_int64),
+        ("dk", c_void_p), ("dv", c_void_p),
+        ("dk_stride_t", c_int64), ("dk_stride_h", c_int64), ("dv_stride_t", c_int64), ("dv_stride_h", c_int64),
+        ("dx_in", c_void_p), ("dx", c_void_p),
+        ("win_w", c_void_p), ("win_logit", c_void_p), ("d_w", c_void_p),
+        ("d_win_w", c_void_p), ("d_win_b", c_void_p),
+        ("n_min", c_float), ("n_max", c_float),
+    ]
+
+
 EXPORTED_SYMBOLS = (
     "dsalt_fwd", "dsalt_fwd_check", "dsalt_bwd", "dsalt_bwd_check", "dsalt_bwd_workspace_size",
     "dsalt_select_landmarks", "dsalt_select_check", "dsalt_quantize_windows",
@@ -168,7 +186,8 @@ EXPORTED_SYMBOLS = (
     "dsalt_bwd_noalloc", "dsalt_select_workspace_size", "dsalt_select_hybrid", "dsalt_swiglu",
     "dsalt_add_rms_norm", "dsalt_lmk_weights", "dsalt_lmk_weights_bwd", "dsalt_lmk_weights_check",
     "dsalt_lmk_weights_workspace_size", "dsalt_lmk_weights_args_size", "dsalt_bwd_rope", "dsalt_rope_tables_size",
-    "dsalt_select_hybrid_qkv", "dsalt_qkv_args_size",
+    "dsalt_select_hybrid_qkv", "dsalt_qkv_args_size", "dsalt_module_grads_v", "dsalt_module_grads_x",
+    "dsalt_module_grads_workspace_size", "dsalt_module_grads_args_size",
 )
 NOALLOC_SCRATCH_BYTES = 76 << 20  # DSALT_NOALLOC_SCRATCH_BYTES
 SELECT_SPLIT_MIN = 4096  # longer sequences can be selected chunk-wise
@@ -202,6 +221,8 @@ def lib() -> ctypes.CDLL:
         ("dsalt_bwd_rope", [ctypes.POINTER(BwdArgs), ctypes.POINTER(RopeTables), c_void_p]),
         ("dsalt_select_hybrid_qkv", [ctypes.POINTER(ScoresArgs), ctypes.POINTER(SelectArgs), ctypes.POINTER(QkvArgs),
                                      c_void_p]),
+        ("dsalt_module_grads_v", [ctypes.POINTER(ModuleGradsArgs), c_void_p]),
+        ("dsalt_module_grads_x", [ctypes.POINTER(ModuleGradsArgs), c_void_p]),
         ("dsalt_lmk_weights", [ctypes.POINTER(LmkWeightsArgs), c_void_p]),
         ("dsalt_lmk_weights_bwd", [ctypes.POINTER(LmkWeightsArgs), c_void_p]),
         ("dsalt_lmk_weights_check", [ctypes.POINTER(LmkWeightsArgs), c_int32]),
@@ -219,12 +240,15 @@ def lib() -> ctypes.CDLL:
     h.dsalt_scores_workspace_size.restype = c_int64
     h.dsalt_select_workspace_size.argtypes = [c_int32] * 4
     h.dsalt_select_workspace_size.restype = c_int64
+    h.dsalt_module_grads_workspace_size.argtypes = [c_int32] * 3
+    h.dsalt_module_grads_workspace_size.restype = c_int64
     h.dsalt_lmk_weights_workspace_size.argtypes = [c_int32] * 2
     h.dsalt_lmk_weights_workspace_size.restype = c_int64
     h.dsalt_abi_version.restype = ctypes.c_int
     h.dsalt_last_error.restype = ctypes.c_char_p
     for n in ("dsalt_fwd_args_size", "dsalt_bwd_args_size", "dsalt_select_args_size", "dsalt_scores_args_size",
-              "dsalt_rope_args_size", "dsalt_lmk_weights_args_size", "dsalt_rope_tables_size", "dsalt_qkv_args_size"):
+              "dsalt_rope_args_size", "dsalt_lmk_weights_args_size", "dsalt_rope_tables_size", "dsalt_qkv_args_size",
+              "dsalt_module_grads_args_size"):
         getattr(h, n).restype = c_size_t
     _lib = h
     check_abi()
@@ -238,7 +262,8 @@ def check_abi() -> None:
     for struct, fn in ((FwdArgs, h.dsalt_fwd_args_size), (BwdArgs, h.dsalt_bwd_args_size),
                        (SelectArgs, h.dsalt_select_args_size), (ScoresArgs, h.dsalt_scores_args_size),
                        (RopeArgs, h.dsalt_rope_args_size), (LmkWeightsArgs, h.dsalt_lmk_weights_args_size),
-                       (RopeTables, h.dsalt_rope_tables_size), (QkvArgs, h.dsalt_qkv_args_size)):
+                       (RopeTables, h.dsalt_rope_tables_size), (QkvArgs, h.dsalt_qkv_args_size),
+                       (ModuleGradsArgs, h.dsalt_module_grads_args_size)):
         if ctypes.sizeof(struct) != fn():
             raise DsaltError(f"{struct.__name__} layout mismatch: {ctypes.sizeof(struct)} vs {fn()} bytes")
 
@@ -443,14 +468,15 @@ def bwd_workspace_size(T: int, S: int, H: int, D: int, k: int) -> int:
 
 def bwd(mode: int, q, k, v, out, lse, dout, w, lmk_pos, lmk_bias, cu_seqlens, scale: float,
         tau_win: float = 1.0, win_edge: float = 4.0, need_dw: bool = False,
-        grad_dtype: torch.dtype | None = None, rope=None):
-    """Sparse-attention backward. ``rope = (cos, sin, dtype)``: q and k are rotated with these
+        grad_dtype: torch.dtype | None = None, rope=None, grads=None):
+    """Sparse-attention backward. ``grads``: the tensors to write dq, dk and dv into (any
+    16-byte aligned strides). ``rope = (cos, sin, dtype)``: q and k are rotated with these
     tables (rounded to dtype); dq and dk come back for the un-rotated ones. Returns (dq, dk, dv, d_lmk_bias [H,S,k] fp32 or None,
     d_w [T] fp32 or None); dq/dk/dv are [T, H, D] per query head in ``grad_dtype`` (q.dtype
     or torch.float32, default q.dtype): with grouped K/V heads ``group_sum`` gives the K/V
     gradients."""
     launcher = BwdLauncher(mode, q, k, v, out, lse, dout, w, lmk_pos, lmk_bias, cu_seqlens, scale,
-                           tau_win, win_edge, need_dw, grad_dtype, rope)
+                           tau_win, win_edge, need_dw, grad_dtype, rope, grads)
     launcher()
     return launcher.results
 
@@ -461,10 +487,10 @@ class BwdLauncher:
 
     def __init__(self, mode: int, q, k, v, out, lse, dout, w, lmk_pos, lmk_bias, cu_seqlens, scale: float,
                  tau_win: float = 1.0, win_edge: float = 4.0, need_dw: bool = False,
-                 grad_dtype: torch.dtype | None = None, rope=None):
+                 grad_dtype: torch.dtype | None = None, rope=None, grads=None):
         self.args, self._keep, self.results, self.device = _bwd_args(
             mode, q, k, v, out, lse, dout, w, lmk_pos, lmk_bias, cu_seqlens, scale, tau_win, win_edge,
-            need_dw, grad_dtype)
+            need_dw, grad_dtype, grads)
         self._rope, keep = _rope_tables_arg(rope, q.shape[2])
         self._keep += (keep,)
         self._fn = lib().dsalt_bwd_rope
@@ -489,8 +515,19 @@ def _rope_tables_arg(rope, D: int):
     return ctypes.byref(t), (t, cos, sin)
 
 
+def _grad_outputs(q: torch.Tensor, dtype: torch.dtype, grads):
+    """dq, dk and dv [T, H, D]: new ones, or the caller's (checked)."""
+    if grads is None:
+        return tuple(torch.empty(q.shape, device=q.device, dtype=dtype) for _ in range(3))
+    for g in grads:
+        if g.shape != q.shape or g.dtype != dtype or g.device != q.device or g.stride(2) != 1:
+            raise DsaltError(f"gradient outputs must be {tuple(q.shape)} {dtype} with unit inner stride, got "
+                             f"{tuple(g.shape)} {g.dtype}")
+    return grads
+
+
 def _bwd_args(mode, q, k, v, out, lse, dout, w, lmk_pos, lmk_bias, cu_seqlens, scale, tau_win, win_edge,
-              need_dw, grad_dtype):
+              need_dw, grad_dtype, grads=None):
     dev = require_gpu(q, k, v, out, lse, dout, w, cu_seqlens)
     if q.dim() != 3:
         raise DsaltError(f"q must be [T, H, D], got {tuple(q.shape)}")
@@ -522,9 +559,7 @@ def _bwd_args(mode, q, k, v, out, lse, dout, w, lmk_pos, lmk_bias, cu_seqlens, s
     gdt = q.dtype if grad_dtype is None else grad_dtype
     if gdt not in (q.dtype, torch.float32):
         raise DsaltError(f"grad_dtype must be {q.dtype} or torch.float32, got {gdt}")
-    dq = torch.empty(q.shape, device=dev, dtype=gdt)
-    dk = torch.empty(q.shape, device=dev, dtype=gdt)
-    dv = torch.empty(q.shape, device=dev, dtype=gdt)
+    dq, dk, dv = _grad_outputs(q, gdt, grads)
     d_bias = torch.empty((H, S, kl), device=dev, dtype=torch.float32) if kl > 0 else None
     d_w = torch.empty((T,), device=dev, dtype=torch.float32) if need_dw else None
     ws_bytes = bwd_workspace_size(T, S, H, D, kl)
@@ -621,12 +656,13 @@ class DenseFwdLauncher:
 
 
 def dense_bwd(q, k, v, out, lse, dout, w_cont, lmk_bias, scale: float, tau_win: float = 1.0,
-              win_edge: float = 4.0, need_dw: bool = True, grad_dtype: torch.dtype | None = None, rope=None):
+              win_edge: float = 4.0, need_dw: bool = True, grad_dtype: torch.dtype | None = None, rope=None,
+              grads=None):
     """Dense-mode backward. Returns (dq, dk, dv in ``grad_dtype`` (default q.dtype),
     d_lmk_bias [H, T] fp32 or None (when lmk_bias is None), d_w [T] fp32 or None).
-    ``rope``: as for ``bwd`` (head_dim 64)."""
+    ``rope``, ``grads``: as for ``bwd`` (``rope`` at head_dim 64)."""
     launcher = DenseBwdLauncher(q, k, v, out, lse, dout, w_cont, lmk_bias, scale, tau_win, win_edge,
-                                need_dw, grad_dtype, rope)
+                                need_dw, grad_dtype, rope, grads)
     launcher()
     return launcher.results
 
@@ -635,7 +671,8 @@ class DenseBwdLauncher:
     """A dense-mode backward with its argument block, outputs and workspace built once."""
 
     def __init__(self, q, k, v, out, lse, dout, w_cont, lmk_bias, scale: float, tau_win: float = 1.0,
-                 win_edge: float = 4.0, need_dw: bool = True, grad_dtype: torch.dtype | None = None, rope=None):
+                 win_edge: float = 4.0, need_dw: bool = True, grad_dtype: torch.dtype | None = None, rope=None,
+                 grads=None):
         self.device = require_gpu(q, k, v, out, lse, dout, w_cont, lmk_bias)
         T, H, D, n_kv, w, lb = _dense_common(q, k, v, w_cont, lmk_bias)
         if tuple(out.shape) != (T, H, D) or tuple(dout.shape) != (T, H, D):
@@ -649,9 +686,7 @@ class DenseBwdLauncher:
         if gdt not in (q.dtype, torch.float32):
             raise DsaltError(f"grad_dtype must be {q.dtype} or torch.float32, got {gdt}")
         dev = self.device
-        dq = torch.empty(q.shape, device=dev, dtype=gdt)
-        dk = torch.empty(q.shape, device=dev, dtype=gdt)
-        dv = torch.empty(q.shape, device=dev, dtype=gdt)
+        dq, dk, dv = _grad_outputs(q, gdt, grads)
         d_lb = torch.empty((H, T), device=dev, dtype=torch.float32) if lb is not None else None
         d_w = torch.empty((T,), device=dev, dtype=torch.float32) if need_dw else None
         ws_bytes = bwd_workspace_size(T, 1, H, D, 0)
@@ -814,13 +849,14 @@ class SelectHybridLauncher:
     def __init__(self, x: torch.Tensor, v: torch.Tensor, alpha: torch.Tensor, n_heads: int,
                  w_cont: torch.Tensor | None, cu_seqlens: torch.Tensor, k_lmk: int, chunked: bool = True,
                  max_seqlen: int | None = None, gate=None, norms_f32: bool | None = None, rope_k=None,
-                 gate_linear=None, quantize: bool = True, rope_q: torch.Tensor | None = None):
+                 gate_linear=None, quantize: bool = True, rope_q: torch.Tensor | None = None, window=None,
+                 free_windows: bool = False):
         if norms_f32 is None:
             norms_f32 = autocast_norms()
         if gate_linear is not None and (gate is not None or w_cont is not None):
             raise DsaltError("gate_linear replaces gate and w_cont: pass neither with it")
-        self.device = require_gpu(x, v, alpha, cu_seqlens,
-                                  gate_linear[0] if gate_linear is not None else w_cont if gate is None else gate[0])
+        self.device = require_gpu(x, v, alpha, cu_seqlens, gate_linear[0] if gate_linear is not None else
+                                  window[0] if window is not None else w_cont if gate is None else gate[0])
         x, v, alpha = _score_operands(x, v, alpha, n_heads)
         cu = _cu_i32(cu_seqlens)
         T = x.shape[0]
@@ -835,6 +871,15 @@ class SelectHybridLauncher:
             self.logit = torch.empty(T, device=self.device, dtype=x.dtype)
             gate = (self.logit, n_min, n_max)
             keep_g = (weight, bias)
+        # window = (weight, bias or None, dtype, n_min, n_max), with rope_q: the norms pass forms the
+        # gate's logits and w~ (win_logit, win_out); the selection excludes their windows, or
+        # with free_windows (one sequence, the dense variant) nothing
+        self.win_logit = self.win_out = None
+        if window is not None:
+            self.win_logit, self.win_out = torch.empty((2, T), device=self.device, dtype=torch.float32).unbind(0)
+            w_cont = self.win_out
+            if free_windows:
+                w_cont = torch.zeros(1, device=self.device, dtype=torch.float32).expand(T)
         w_cont, gate = _window_source(w_cont, gate)
         ws = torch.empty((scores_workspace_size(T, v.shape[1]),), device=self.device, dtype=torch.uint8)
         self._sa = scores_args(x, v, alpha, n_heads, None, None, None, ws, norms_f32)
@@ -843,13 +888,15 @@ class SelectHybridLauncher:
             self._sa.gate_b = _ptr(keep_g[1])
             self._sa.gate_out = self.logit.data_ptr()
         # rope_q (with rope_k): the norms pass forms the attention's operands q_out, k_out and
-        # v_out - q rotated like k, and for fp32 operands all three in fp16
+        # v_out - q and k rotated in place, or for fp32 operands all three in fp16
         cast = rope_q is not None and v.dtype == torch.float32
-        self.k_out, keep_k = _rope_k_args(self._sa, v, rope_k, torch.float16 if cast else None)
+        self.k_out, keep_k = _rope_k_args(self._sa, v, rope_k, torch.float16 if cast else None, rope_q is not None)
         self._qkv, self.q_out, self.v_out = None, None, v
         if rope_q is not None:
-            self._qkv, self.q_out, self.v_out, keep_q = _qkv_args(rope_q, v, n_heads, cast)
-            keep_k = (keep_k, keep_q)
+            self._qkv, self.q_out, self.v_out, keep_q = _qkv_args(rope_q, v, n_heads, cast, rope_k, window)
+            if window is not None:
+                self._qkv.win_logit, self._qkv.win_out = self.win_logit.data_ptr(), self.win_out.data_ptr()
+            keep_k = (keep_k, keep_q, window)
         self.out = torch.empty((n_heads, cu.shape[0] - 1, k_lmk), device=self.device, dtype=torch.int64)
         # quantize=False: w_cont is taken as the windows themselves (select_landmarks' test)
         self.w_out = torch.empty(T, device=self.device, dtype=torch.float32) if quantize else None
@@ -889,6 +936,59 @@ def lmk_weights(norms: torch.Tensor, alpha: torch.Tensor, lmk_pos: torch.Tensor,
     a.weight = weight.data_ptr()
     _raise(lib().dsalt_lmk_weights(ctypes.byref(a), stream_handle(dev)), "dsalt_lmk_weights")
     return weight
+
+
+class ModuleGrads:
+    """The gradients of the module's states, value projection, gate and alpha besides the
+    attention's own kernels (dsalt_module_grads_v, then dsalt_module_grads_x): ``x`` [T, d],
+    ``v`` [T, n_kv, D], ``norms`` ... ``cu`` as the forward left them, ``d_weight`` the gradient
+    of its landmark weights."""
+
+    def __init__(self, x, v, norms, alpha, lmk_pos, cu, d_weight, tau: float, table: bool):
+        self.device = require_gpu(x, v, norms, alpha, lmk_pos, cu, d_weight)
+        T, n_kv, D = v.shape
+        H, d = alpha.shape[0], x.shape[1]
+        w = _lmk_weights_args(norms, alpha, lmk_pos, cu, T, n_kv, tau, table)
+        w.head_dim, w.d_model = D, d
+        w.x_dtype, w.v_dtype = _SCORE_DTYPES[x.dtype], _SCORE_DTYPES[v.dtype]
+        w.x, w.x_stride_t = x.data_ptr(), x.stride(0)
+        w.v, w.v_stride_t, w.v_stride_h = v.data_ptr(), v.stride(0), v.stride(1)
+        ws = torch.empty((lib().dsalt_module_grads_workspace_size(T, H, d),), device=self.device, dtype=torch.uint8)
+        w.d_weight, w.workspace, w.workspace_bytes = d_weight.data_ptr(), ws.data_ptr(), ws.numel()
+        self.a = ModuleGradsArgs()
+        self.a.weights = w
+        self._x = x
+        self._keep = (x, v, norms, alpha, lmk_pos, cu, d_weight, ws)
+
+    def values(self, dk_heads, dv_heads, dk, dv, alpha_sigmoid: bool):
+        """dv (and for grouped heads dk) [T, n_kv, D], written from the attention's per-head
+        gradients [T, H, D] with the value norms' share added; returns d_alpha [H] fp32
+        (of alpha_w with ``alpha_sigmoid``: alpha = sigmoid(alpha_w))."""
+        a = self.a
+        d_alpha = torch.empty((a.weights.n_heads,), device=self.device, dtype=torch.float32)
+        a.d_alpha, a.alpha_sigmoid, a.heads_dtype = d_alpha.data_ptr(), int(alpha_sigmoid), _SCORE_DTYPES[dv_heads.dtype]
+        a.dv_heads, a.dvh_stride_t, a.dvh_stride_h = dv_heads.data_ptr(), dv_heads.stride(0), dv_heads.stride(1)
+        a.dk_heads, a.dkh_stride_t, a.dkh_stride_h = dk_heads.data_ptr(), dk_heads.stride(0), dk_heads.stride(1)
+        a.dv, a.dv_stride_t, a.dv_stride_h = dv.data_ptr(), dv.stride(0), dv.stride(1)
+        a.dk, a.dk_stride_t, a.dk_stride_h = dk.data_ptr(), dk.stride(0), dk.stride(1)
+        _raise(lib().dsalt_module_grads_v(ctypes.byref(a), stream_handle(self.device)), "dsalt_module_grads_v")
+        return d_alpha
+
+    def states(self, dx_in, need_dx: bool, window):
+        """(dx [T, d] in x's dtype or None, d_weight [1, d] and d_bias [1] of the gate in x's
+        dtype): ``dx_in`` [T, d] contiguous plus the state norm's and the gate's shares.
+        ``window = (weight, win_logit, d_w [T] fp32, dtype, n_min, n_max)``."""
+        a, x = self.a, self._x
+        weight, logit, d_w, dtype, n_min, n_max = window
+        dx = torch.empty(x.shape, device=self.device, dtype=x.dtype) if need_dx else None
+        dwg = torch.empty((1, x.shape[1]), device=self.device, dtype=x.dtype)
+        dbg = torch.empty((1,), device=self.device, dtype=x.dtype)
+        a.dx_in, a.dx, a.in_dtype = _ptr(dx_in), _ptr(dx), _SCORE_DTYPES[x.dtype if dx_in is None else dx_in.dtype]
+        a.win_w, a.win_logit, a.d_w, a.win_dtype = weight.data_ptr(), logit.data_ptr(), d_w.data_ptr(), _SCORE_DTYPES[dtype]
+        a.d_win_w, a.d_win_b = dwg.data_ptr(), dbg.data_ptr()
+        a.n_min, a.n_max = float(n_min), float(n_max)
+        _raise(lib().dsalt_module_grads_x(ctypes.byref(a), stream_handle(self.device)), "dsalt_module_grads_x")
+        return dx, dwg, dbg
 
 
 def lmk_weights_bwd(d_weight: torch.Tensor, norms: torch.Tensor, alpha: torch.Tensor, lmk_pos: torch.Tensor,
@@ -1031,38 +1131,33 @@ def _score_operands(x, v, alpha, n_heads):
     return x, v, alpha
 
 
-def _qkv_args(q: torch.Tensor, v: torch.Tensor, n_heads: int, cast: bool):
-    """The operand block of a norms pass that rotates q [T, H, D] too, its outputs q_out and
-    v_out (v itself without a cast) and the tensors to keep alive until the launch."""
+def _qkv_args(q: torch.Tensor, v: torch.Tensor, n_heads: int, cast: bool, rope_k, window):
+    """The operand block of a norms pass that rotates q [T, H, D] too (in place without a cast)
+    and forms the windows, its outputs q_out and v_out (v itself without a cast) and the
+    tensors to keep alive until the launch."""
     T, _, D = v.shape
-    if q.dtype != v.dtype or tuple(q.shape) != (T, n_heads, D):
-        raise DsaltError(f"q must be [{T}, {n_heads}, {D}] in v's dtype (got {tuple(q.shape)} {q.dtype})")
-    q = q if q.stride(2) == 1 else q.contiguous()
+    if q.dtype != v.dtype or tuple(q.shape) != (T, n_heads, D) or q.stride(2) != 1:
+        raise DsaltError(f"q must be [{T}, {n_heads}, {D}] in v's dtype with unit inner stride (got {tuple(q.shape)} "
+                         f"{q.dtype})")
     dt = torch.float16 if cast else q.dtype
-    q_out = torch.empty((T, n_heads, D), device=q.device, dtype=dt)
+    q_out = torch.empty((T, n_heads, D), device=q.device, dtype=dt) if cast else q
     o = QkvArgs()
     o.out_dtype = _SCORE_DTYPES[dt]
+    o.rope_half = int(rope_tables(rope_k[1], rope_k[2])[2])
     o.q, o.q_stride_t, o.q_stride_h = q.data_ptr(), q.stride(0), q.stride(1)
     o.q_out, o.q_out_stride_t, o.q_out_stride_h = q_out.data_ptr(), q_out.stride(0), q_out.stride(1)
     v_out = v
     if cast:
         v_out = torch.empty(v.shape, device=v.device, dtype=dt)
         o.v_out, o.v_out_stride_t, o.v_out_stride_h = v_out.data_ptr(), v_out.stride(0), v_out.stride(1)
+    if window is not None:
+        weight, bias, dtype, n_min, n_max = window
+        o.win_w, o.win_b, o.win_dtype = weight.data_ptr(), _ptr(bias), _SCORE_DTYPES[dtype]
+        o.n_min, o.n_max = float(n_min), float(n_max)
     return o, q_out, v_out, q
 
 
-def rope_operands_supported(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
-    """Whether the norms pass can rotate q and k beside v's norms (the rules of dsalt_scores_check
-    for k): one dtype, unit inner strides, 16-byte aligned rows, D / 2 a multiple of one
-    16-byte load."""
-    ev = 4 if v.dtype == torch.float32 else 8
-    return (q.dtype == k.dtype == v.dtype and k.shape == v.shape and q.shape[2] == v.shape[2]
-            and (v.shape[2] // 2) % ev == 0
-            and all(t.stride(2) == 1 and t.stride(0) % ev == 0 and t.stride(1) % ev == 0 and t.data_ptr() % 16 == 0
-                    for t in (q, k)))
-
-
-def _rope_k_args(a: ScoresArgs, v: torch.Tensor, rope_k, out_dtype: torch.dtype | None = None):
+def _rope_k_args(a: ScoresArgs, v: torch.Tensor, rope_k, out_dtype: torch.dtype | None = None, in_place: bool = False):
     """Fill the k-rotation fields of a score argument block from rope_k = (k, cos, sin,
     cu_seqlens) or leave them empty (rope_k None); returns (k_out or None, tensors to keep
     alive until the launch)."""
@@ -1073,7 +1168,10 @@ def _rope_k_args(a: ScoresArgs, v: torch.Tensor, rope_k, out_dtype: torch.dtype 
         raise DsaltError(f"k must match v's shape and dtype (got {tuple(k.shape)} {k.dtype}, "
                          f"{tuple(v.shape)} {v.dtype})")
     k = k if k.stride(2) == 1 else k.contiguous()
-    k_out = torch.empty(k.shape, device=k.device, dtype=out_dtype) if out_dtype is not None else torch.empty_like(k)
+    if out_dtype is not None:
+        k_out = torch.empty(k.shape, device=k.device, dtype=out_dtype)
+    else:
+        k_out = k if in_place else torch.empty_like(k)
     cos = cos.to(torch.float32).contiguous()
     sin = sin.to(torch.float32).contiguous()
     cu = _cu_i32(cu) if cu is not None else None

@@ -1,12 +1,14 @@
-"""Autograd glue of the attention module's core: RoPE, landmark selection and weights, and
-SOFT (packed) or dense attention as one differentiable function of x, q, k, v, w~ and alpha
-(dsalt/modules/dsalt_attention.py:371-438, :440-487, :570-585 of the reference).
+"""Autograd glue of the attention module's core: q/k/v projections, window gate, RoPE,
+landmark selection and weights, and SOFT (packed) or dense attention as one differentiable
+function of the states and the parameters (dsalt/modules/dsalt_attention.py:270-284,
+:371-438, :440-487, :566-585 of the reference).
 
-Forward: the norms pass (which rotates q and k and, for fp32 modules, writes the fp16
-operands), the selection, the landmark weights and the attention. Backward: the attention's
-kernels, which return dq and dk un-rotated, then the weights' backward, which adds the
-norms' share to dv. Nothing of it runs as torch elementwise ops, and no rotated or cast
-copy is made besides the operands the attention reads.
+Forward: one GEMM against the three projection weights concatenated; the norms pass, which
+also forms the gate's logits and windows, rotates q and k in place and, for fp32 modules,
+writes the fp16 operands; the selection; the landmark weights; the attention. Backward: the
+attention's kernels write dq, dk (un-rotated) and dv into one [T, d + 2 kv] buffer, the
+norms' share is added to dv, two GEMMs give the weights' gradients and dx, and one pass adds
+the norm and gate shares to dx and sums the gate's gradients.
 """
 from __future__ import annotations
 
@@ -19,73 +21,108 @@ from .. import _hip
 
 class _ModuleAttention(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, q, k, v, w_cont, alpha, cos, sin, cu_seqlens, k_lmk, max_seqlen, tau_lmk, tau_win, win_edge,
-                dense):
-        a32 = alpha.detach().to(torch.float32).contiguous()
-        T, H, D = q.shape
-        w32 = w_cont.detach().to(torch.float32)
-        # the dense variant excludes no key from the selection (its exclusion is per query)
-        w_sel = w32.new_zeros(1).expand(T) if dense else w32
-        sel = _hip.SelectHybridLauncher(x.detach(), v.detach(), a32, H, w_sel, cu_seqlens, k_lmk,
-                                        max_seqlen=max_seqlen, quantize=not dense,
-                                        rope_k=(k.detach(), cos, sin, cu_seqlens), rope_q=q.detach())
+    def forward(ctx, x, wq, wk, wv, wg, bg, alpha_w, cos, sin, cu_seqlens, opt):
+        cdt, H, n_kv, D = opt["dtype"], opt["n_heads"], opt["n_kv_heads"], opt["head_dim"]
+        T, dense, k_lmk = x.shape[0], opt["dense"], opt["k_lmk"]
+        xd = x.detach()
+        xb = xd if xd.dtype == cdt else xd.to(cdt)
+        ws = [w.detach() for w in (wq, wk, wv)]
+        if wq.dtype == cdt:
+            w_cat = torch.cat(ws)
+        else:
+            w_cat = torch.empty((sum(w.shape[0] for w in ws), x.shape[1]), device=x.device, dtype=cdt)
+            for dst, w in zip(w_cat.split([w.shape[0] for w in ws]), ws):
+                dst.copy_(w)
+        qkv = torch.mm(xb, w_cat.t())
+        q, k, v = _split(qkv, H, n_kv, D)
+        a32 = torch.sigmoid(alpha_w.detach()).to(torch.float32)
+        sel = _hip.SelectHybridLauncher(
+            xd, v, a32, H, None, cu_seqlens, k_lmk, max_seqlen=opt["max_seqlen"], quantize=not dense,
+            rope_k=(k, cos, sin, cu_seqlens), rope_q=q, window=(wg.detach(), None if bg is None else bg.detach(), cdt,
+                                                                opt["n_min"], opt["n_max"]), free_windows=dense)
         sel()
-        weight = _hip.lmk_weights(sel.norms, a32, sel.out, sel.cu, T, v.shape[1], tau_lmk, dense)
+        weight = _hip.lmk_weights(sel.norms, a32, sel.out, sel.cu, T, n_kv, opt["tau_lmk"], dense)
         scale = 1.0 / math.sqrt(D)
         if dense:
-            out, lse = _hip.dense_fwd(sel.q_out, sel.k_out, sel.v_out, w32, weight, scale, tau_win, win_edge)
+            out, lse = _hip.dense_fwd(sel.q_out, sel.k_out, sel.v_out, sel.win_out, weight, scale, opt["tau_win"],
+                                      opt["win_edge"])
         else:
             pos, logw = (sel.out, weight) if k_lmk > 0 else (None, None)
-            out, lse = _hip.fwd(_hip.MODE_SOFT, sel.q_out, sel.k_out, sel.v_out, w32, pos, logw, sel.cu, scale, tau_win,
-                                win_edge)
-        # without a cast the attention's v is the input itself
-        cast = sel.v_out.dtype != v.dtype
-        ctx.save_for_backward(x, v, sel.q_out, sel.k_out, sel.v_out if cast else None, out, lse, w32, weight, a32,
-                              sel.norms, sel.out, sel.cu, cos, sin)
-        ctx.dsalt = (k_lmk, tau_lmk, tau_win, win_edge, dense, scale, q.dtype, w_cont.dtype, alpha.dtype)
+            out, lse = _hip.fwd(_hip.MODE_SOFT, sel.q_out, sel.k_out, sel.v_out, sel.win_out, pos, logw, sel.cu, scale,
+                                opt["tau_win"], opt["win_edge"])
+        cast = cdt == torch.float32  # separate fp16 operands; otherwise q and k were rotated in place
+        ops = (sel.q_out, sel.k_out, sel.v_out) if cast else (None, None, None)
+        ctx.save_for_backward(x, None if xb is xd else xb, qkv, *ops, w_cat, wg, out, lse, sel.win_logit, sel.win_out,
+                              weight, a32, sel.norms, sel.out, sel.cu, cos, sin)
+        ctx.dsalt = opt, scale, wq.dtype, alpha_w.dtype
         if dense:
-            ctx.mark_non_differentiable(sel.out)
+            ctx.mark_non_differentiable(sel.out, sel.win_out)
         else:
-            ctx.mark_non_differentiable(sel.out, sel.w_out)
-        return out, sel.out, sel.w_out
+            ctx.mark_non_differentiable(sel.out, sel.win_out, sel.w_out)
+        return out, sel.out, sel.win_out, sel.w_out
 
     @staticmethod
-    def backward(ctx, grad_out, _d_pos, _d_w):
-        x, v, q_r, k_r, v_c, out, lse, w32, weight, a32, norms, pos, cu, cos, sin = ctx.saved_tensors
-        k_lmk, tau_lmk, tau_win, win_edge, dense, scale, od, w_dtype, a_dtype = ctx.dsalt
-        v_c = v.detach() if v_c is None else v_c
-        H, D, n_kv = q_r.shape[1], q_r.shape[2], k_r.shape[1]
-        # grouped K/V heads: per-query-head gradients in fp32, summed over each group
-        gdt = torch.float32 if (od == torch.float32 or n_kv != H) else q_r.dtype
-        need_x, _, _, need_v, need_w, need_a = ctx.needs_input_grad[:6]
+    def backward(ctx, grad_out, *_):
+        (x, xb, qkv, q_r, k_r, v_r, w_cat, wg, out, lse, logit, w32, weight, a32, norms, pos, cu, cos,
+         sin) = ctx.saved_tensors
+        opt, scale, w_dtype, a_dtype = ctx.dsalt
+        H, n_kv, D, dense, od = opt["n_heads"], opt["n_kv_heads"], opt["head_dim"], opt["dense"], qkv.dtype
+        T, grouped = x.shape[0], n_kv != H
+        xb = x.detach() if xb is None else xb
+        need_x, *need_w = ctx.needs_input_grad[:4]
+        need_gate = ctx.needs_input_grad[4] or ctx.needs_input_grad[5]
+        q, k, v = _split(qkv, H, n_kv, D)
+        if q_r is None:
+            q_r, k_r, v_r = q, k, v
+        dqkv = torch.empty_like(qkv)
+        dq, dk, dv = _split(dqkv, H, n_kv, D)
+        # grouped K/V heads: per-query-head gradients in fp32, summed over each group below
+        gdt, grads = (torch.float32, None) if grouped else (od, (dq, dk, dv))
+        fused = not dense or D == 64  # the dense kernels un-rotate their gradients at D = 64
+        rope = (cos, sin, od) if fused else None
         if dense:
-            fused = D == 64  # the dense kernels un-rotate their gradients at D = 64
-            dq, dk, dv, d_weight, dw = _hip.dense_bwd(q_r, k_r, v_c, out, lse, grad_out, w32, weight, scale, tau_win,
-                                                      win_edge, need_dw=need_w, grad_dtype=gdt,
-                                                      rope=(cos, sin, od) if fused else None)
+            dq_h, dk_h, dv_h, d_weight, dw = _hip.dense_bwd(q_r, k_r, v_r, out, lse, grad_out, w32, weight, scale,
+                                                            opt["tau_win"], opt["win_edge"], True, gdt, rope, grads)
         else:
-            fused = True
-            lp, lw = (pos, weight) if k_lmk > 0 else (None, None)
-            dq, dk, dv, d_weight, dw = _hip.bwd(_hip.MODE_SOFT, q_r, k_r, v_c, out, lse, grad_out, w32, lp, lw, cu, scale,
-                                                tau_win, win_edge, need_dw=need_w, grad_dtype=gdt, rope=(cos, sin, od))
-        dk, dv = _hip.group_sum(dk, n_kv), _hip.group_sum(dv, n_kv)
-        dq, dk, dv = dq.to(od), dk.to(od), dv.to(od)
+            lp, lw = (pos, weight) if opt["k_lmk"] > 0 else (None, None)
+            dq_h, dk_h, dv_h, d_weight, dw = _hip.bwd(_hip.MODE_SOFT, q_r, k_r, v_r, out, lse, grad_out, w32, lp, lw, cu,
+                                                      scale, opt["tau_win"], opt["win_edge"], True, gdt, rope, grads)
+        if grouped:
+            dq.copy_(dq_h)
+        g = _hip.ModuleGrads(x.detach(), v, norms, a32, pos, cu, weight if d_weight is None else d_weight,
+                             opt["tau_lmk"], dense)
+        d_alpha = g.values(dk_h, dv_h, dk, dv, alpha_sigmoid=True)
         if not fused:
-            dq, dk = _hip.rope(dq, dk, cos, sin, cu, transpose=True, q_out=dq, k_out=dk)
-        dx = da = None
-        if d_weight is not None and (need_x or need_v or need_a):
-            dx, dv_all, da = _hip.lmk_weights_bwd(d_weight, norms, a32, pos, cu, x, v, dv, tau_lmk, dense, need_x, need_v)
-            dv = dv if dv_all is None else dv_all
-            da = da.to(a_dtype) if need_a else None
-        return (dx, dq, dk, dv, None if dw is None else dw.to(w_dtype), da, None, None, None, None, None, None, None, None,
-                None)
+            _hip.rope(dq, dk, cos, sin, cu, transpose=True, q_out=dq, k_out=dk)
+        dws = [None, None, None]
+        if all(need_w):
+            d_cat = torch.mm(dqkv.t(), xb)
+            dws = (d_cat if w_dtype == od else d_cat.to(w_dtype)).split([H * D, n_kv * D, n_kv * D])
+        elif any(need_w):
+            parts = dqkv.split([H * D, n_kv * D, n_kv * D], 1)
+            dws = [torch.mm(p.t(), xb).to(w_dtype) if n else None for p, n in zip(parts, need_w)]
+        dx = dwg = dbg = None
+        if need_x or need_gate:
+            dx_in = torch.mm(dqkv, w_cat) if need_x else None
+            dx, dwg, dbg = g.states(dx_in, need_x, (wg, logit, dw, od, opt["n_min"], opt["n_max"]))
+        if not ctx.needs_input_grad[5]:
+            dbg = None
+        return (dx, *dws, dwg if ctx.needs_input_grad[4] else None, dbg,
+                d_alpha.to(a_dtype) if ctx.needs_input_grad[6] else None, None, None, None, None)
 
 
-def module_attention(x, q, k, v, w_cont, alpha, cos, sin, cu_seqlens, k_lmk: int, max_seqlen, tau_lmk: float,
-                     tau_win: float, win_edge: float, dense: bool = False):
-    """``(out [T, H, D] in the compute dtype, lmk_pos [H, S, k], w)`` from un-rotated q [T, H, D],
-    k and v [T, n_kv, D] (operands that ``_hip.scores_supported`` and
-    ``_hip.rope_operands_supported`` take), the states x [T, d], the windows w~ [T] and the
-    heads' alpha; ``w`` are the quantised windows (None with ``dense``: one sequence)."""
-    return _ModuleAttention.apply(x, q, k, v, w_cont, alpha, cos, sin, cu_seqlens, k_lmk, max_seqlen, tau_lmk, tau_win,
-                                  win_edge, dense)
+def _split(qkv: torch.Tensor, H: int, n_kv: int, D: int):
+    """q [T, H, D], k and v [T, n_kv, D]: the column views of qkv [T, (H + 2 n_kv) D]."""
+    T = qkv.shape[0]
+    q, k, v = qkv.split([H * D, n_kv * D, n_kv * D], 1)
+    return q.view(T, H, D), k.view(T, n_kv, D), v.view(T, n_kv, D)
+
+
+def module_attention(x, q_proj, k_proj, v_proj, win_gate, alpha_w, cos, sin, cu_seqlens, opt: dict):
+    """``(out [T, H, D] in the compute dtype, lmk_pos [H, S, k], w~ [T], quantised w or None)`` of
+    packed states x [T, d]. The four projections are plain nn.Linear modules (q, k and v
+    without bias); ``opt``: dtype (of the projections' results), n_heads, n_kv_heads,
+    head_dim, k_lmk, max_seqlen, tau_lmk, tau_win, win_edge, n_min, n_max, dense (one
+    sequence, the dense variant). Operands: as DSALTAttention._one_function checks them."""
+    return _ModuleAttention.apply(x, q_proj.weight, k_proj.weight, v_proj.weight, win_gate.weight, win_gate.bias, alpha_w,
+                                  cos, sin, cu_seqlens, opt)

@@ -6,9 +6,11 @@ RoPE buffers, fixed attributes (tau_win = 1, tau_lmk = 2, win_edge = 4) and
 ``forward(x, cu_seqlens=None, max_seqlen=None, rope_cs=None, cu_list=None) -> (out, aux)``.
 
 Packed input (``cu_seqlens`` given) runs the sparse path:
-  * training: ``_train_selectors`` (continuous window, HIP landmark top-k, soft landmark
-    weight log sigmoid(s/tau_lmk)) then the SOFT HIP kernels (forward + deterministic
-    backward carrying d_w~ to win_gate and d_logw to alpha_w), dsalt_attention.py:440-487;
+  * training: projections, continuous window, HIP landmark top-k, soft landmark weight
+    log sigmoid(s/tau_lmk) and the SOFT HIP kernels (forward + deterministic backward
+    carrying d_w~ to win_gate and d_logw to alpha_w) as one function
+    (``module_attention``) where ``_one_function`` holds, otherwise as separate ones
+    (``_train_selectors``), dsalt_attention.py:440-487;
   * inference: two HIP launches select (dsalt_select_hybrid: a norms pass over x and the
     value projection that also rotates k, then one launch forming the hybrid scores, the
     floor-quantised windows from the gate logits and the landmark top-k), then the HARD
@@ -69,7 +71,8 @@ class DSALTAttention(nn.Module):
     the landmark sets of configs 2, 3 and 4 (fp32, bf16, autocast) are the reference
     route's, set for set, but a near-tie could move. ``_hip_scores = False`` keeps torch's own norm
     and standardisation ops on v, whose fp32 scores are bit-identical to the reference's
-    route. The differentiable landmark weights of training always use the torch ops.
+    route. The differentiable landmark weights of training follow the same switch (HIP
+    passes forward and backward, or torch's ops).
     ``_fuse_gate`` (default True): on that route's inference path, with 16-bit x and
     ``win_gate`` parameters of x's dtype, the norms pass also forms the window gate's
     logits (an fp32 dot product in its own fixed order, rounded once) instead of torch's
@@ -85,6 +88,7 @@ class DSALTAttention(nn.Module):
     follows each weight's pointer and version counter: in-place updates (optimizer steps,
     ``load_state_dict``, ``copy_`` under no_grad) are seen, but a change made through
     ``weight.data`` does not bump the counter - call ``invalidate_qkv_cache()`` after one.
+    Training and the dense variant concatenate the weights on each call (nothing is kept).
     ``_last_selection`` holds the ``(windows, landmark positions)`` of the last forward.
     """
 
@@ -160,14 +164,19 @@ class DSALTAttention(nn.Module):
                 and self.v_proj.bias is None and all(w.dtype == x.dtype and w.device == x.device for w in ws)
                 and self.d_model % 8 == 0 and self.kv_dim % 8 == 0):
             return self.q_proj(x), self.k_proj(x), self.v_proj(x)
+        qkv = F.linear(x, self._qkv_weight())
+        d, kv = self.d_model, self.kv_dim
+        return qkv[:, :d], qkv[:, d:d + kv], qkv[:, d + kv:]
+
+    def _qkv_weight(self) -> torch.Tensor:
+        """The q, k and v weights concatenated, kept until one of them changes."""
+        ws = (self.q_proj.weight, self.k_proj.weight, self.v_proj.weight)
         key = tuple((w.data_ptr(), w._version, w.dtype, w.device) for w in ws)
         cache = getattr(self, "_qkv_weight_cache", None)
         if cache is None or cache[0] != key:
             cache = (key, torch.cat([w.detach() for w in ws], 0))
             self._qkv_weight_cache = cache
-        qkv = F.linear(x, cache[1])
-        d, kv = self.d_model, self.kv_dim
-        return qkv[:, :d], qkv[:, d:d + kv], qkv[:, d + kv:]
+        return cache[1]
 
     def _alpha(self) -> torch.Tensor:
         return torch.sigmoid(self.alpha_w)
@@ -255,19 +264,16 @@ class DSALTAttention(nn.Module):
         if self.training and self.dropout > 0:
             raise NotImplementedError("attention dropout is not supported by the dense HIP path")
         xs = x[0]
-        q = self.q_proj(xs).view(T, self.n_heads, self.head_dim)
-        k = self.k_proj(xs).view(T, self.n_kv_heads, self.head_dim)
-        v = self.v_proj(xs).view(T, self.n_kv_heads, self.head_dim)
-        v_sel = v if (self.v_proj.bias is None and self._fused_selector) else None
         collect_P = not self.training and getattr(self, "_collect_last_P", True)
         self._last_P = None
-        if T > 0 and not collect_P and self._hip_attention(xs, q, k, v_sel):
+        if not collect_P and self._one_function(xs):
             cu = torch.arange(0, T + 1, T, dtype=torch.int32, device=device)  # [0, T], made on the GPU
-            w_cont = self._window_continuous(xs)
-            out, lmk_pos, _ = module_attention(xs, q, k, v, w_cont, self._alpha(), *self._rope_tables(), cu,
-                                               min(self.k_lmk, T), T, self.tau_lmk, self.tau_win, float(self.win_edge),
-                                               dense=True)
+            out, lmk_pos, w_cont, _ = self._attend(xs, cu, min(self.k_lmk, T), T, dense=True)
         else:
+            q = self.q_proj(xs).view(T, self.n_heads, self.head_dim)
+            k = self.k_proj(xs).view(T, self.n_kv_heads, self.head_dim)
+            v = self.v_proj(xs).view(T, self.n_kv_heads, self.head_dim)
+            v_sel = v if (self.v_proj.bias is None and self._fused_selector) else None
             cu = torch.tensor([0, T], dtype=torch.int32, device=device)
             q, k = apply_rotary_emb_packed(q, k, *self._rope_tables(), cu)
             # grouped K/V heads go to the kernels as they are (query head h reads K/V head
@@ -281,10 +287,53 @@ class DSALTAttention(nn.Module):
         aux = x.new_zeros(())
         return self._apply_out_proj(out.reshape(1, T, self.d_model)), aux
 
-    def _hip_attention(self, x: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor | None) -> bool:
-        """Whether RoPE, selection, weights and attention run as one function
-        (``module_attention``): the HIP score route, operands that its norms pass takes."""
-        return self._hip_weights(x, v) and _hip.rope_operands_supported(q, k, v)
+    def _one_function(self, x: torch.Tensor) -> bool:
+        """Whether projections, gate, RoPE, selection and attention of x [T, d] run as one function
+        (``module_attention``): the HIP score route; projections that are plain nn.Linear
+        modules without hooks (a wrapped, parametrised or hooked one is called as it is, on the
+        route of separate functions), q, k and v without bias; one element type for x and the
+        weights, or fp32 for all of them under a 16-bit autocast; rows that the norms pass
+        loads in 16-byte pieces."""
+        lin = (self.q_proj, self.k_proj, self.v_proj, self.win_gate)
+        if not (self._fused_selector and self._hip_scores and self._fuse_qkv and all(type(m) is nn.Linear for m in lin)):
+            return False
+        if any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+               or "forward" in m.__dict__ for m in lin):
+            return False
+        g = nn.modules.module
+        if (g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks
+                or g._global_backward_pre_hooks):
+            return False
+        if any(m.bias is not None for m in lin[:3]) or x.dim() != 2 or x.shape[0] == 0 or x.shape[1] != self.d_model:
+            return False
+        ps = [m.weight for m in lin] + ([] if self.win_gate.bias is None else [self.win_gate.bias])
+        if any(p.dtype != x.dtype or p.device != x.device or not p.is_contiguous() for p in ps):
+            return False
+        if self.alpha_w.device != x.device or self.alpha_w.shape != (self.n_heads,):
+            return False
+        if x.dtype not in (torch.bfloat16, torch.float16, torch.float32):
+            return False
+        cdt = self._compute_dtype(x)
+        if cdt not in (torch.bfloat16, torch.float16, torch.float32) or (cdt != x.dtype and x.dtype != torch.float32):
+            return False
+        per = 4 if x.dtype == torch.float32 else 8  # elements per 16-byte load
+        return (self.head_dim in (64, 128) and self.n_kv_heads <= _hip.SCORES_MAX_KV and x.stride(1) == 1
+                and x.stride(0) >= self.d_model and x.stride(0) % per == 0 and x.data_ptr() % 16 == 0
+                and self.win_gate.weight.data_ptr() % 16 == 0)
+
+    @staticmethod
+    def _compute_dtype(x: torch.Tensor) -> torch.dtype:
+        """Element type of the projections' results: autocast's where it is on."""
+        return torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
+
+    @_dynamo_opaque
+    def _attend(self, x, cu_seqlens, k_lmk, max_seqlen, dense=False):
+        cos, sin = self._rope_tables()
+        opt = dict(dtype=self._compute_dtype(x), n_heads=self.n_heads, n_kv_heads=self.n_kv_heads,
+                   head_dim=self.head_dim, k_lmk=k_lmk, max_seqlen=max_seqlen, tau_lmk=self.tau_lmk,
+                   tau_win=self.tau_win, win_edge=float(self.win_edge), n_min=self.n_min, n_max=self.n_max, dense=dense)
+        return module_attention(x, self.q_proj, self.k_proj, self.v_proj, self.win_gate, self.alpha_w, cos, sin,
+                                cu_seqlens, opt)
 
     def _hip_weights(self, x: torch.Tensor, v: torch.Tensor | None) -> bool:
         """Whether the selection and its differentiable weights run on the HIP passes over x
@@ -363,6 +412,13 @@ class DSALTAttention(nn.Module):
     def _packed(self, x: torch.Tensor, cu_seqlens: torch.Tensor, total_len: int, device: torch.device,
                 rope_cs: tuple | None = None, cu_list: list | None = None, need_aux: bool = True):
         _hip.require_gpu(x, cu_seqlens)
+        if self.training and rope_cs is None and self._one_function(x):
+            self._last_P = None
+            max_len = None if cu_list is None else max((b - a for a, b in zip(cu_list[:-1], cu_list[1:])), default=0)
+            out, lmk_pos, _, w_disc = self._attend(x, cu_seqlens, self.k_lmk, max_len)
+            self._last_selection = (w_disc, lmk_pos)
+            return (self._apply_out_proj(out.reshape(total_len, self.d_model)),
+                    x.new_zeros(()) if need_aux else None)
         q, k, v = self._project_qkv(x)
         q = q.view(total_len, self.n_heads, self.head_dim)
         k = k.view(total_len, self.n_kv_heads, self.head_dim)
@@ -370,16 +426,6 @@ class DSALTAttention(nn.Module):
         # x W_V^T before RoPE and the kv repeat: the selector's value norms come from it
         # (only without a projection bias, where v is exactly x W_V^T)
         v_sel = v if self.v_proj.bias is None else None
-
-        if self.training and rope_cs is None and self._hip_attention(x, q, k, v_sel):
-            self._last_P = None
-            max_len = None if cu_list is None else max((b - a for a, b in zip(cu_list[:-1], cu_list[1:])), default=0)
-            out, lmk_pos, w_disc = module_attention(x, q, k, v, self._window_continuous(x), self._alpha(),
-                                                    *self._rope_tables(), cu_seqlens, self.k_lmk, max_len, self.tau_lmk,
-                                                    self.tau_win, float(self.win_edge))
-            self._last_selection = (w_disc, lmk_pos)
-            return (self._apply_out_proj(out.reshape(total_len, self.d_model)),
-                    x.new_zeros(()) if need_aux else None)
 
         # RoPE in one HIP pass (dsalt_attention.py:570-585): positions from cu_seqlens
         # in-kernel, cos/sin rounded to q's dtype as the reference's cos.to(q.dtype). At

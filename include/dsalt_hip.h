@@ -205,7 +205,7 @@ typedef struct dsalt_rope_tables {
     int64_t stride;         /* row stride (elements), a multiple of 4 */
     int32_t rows;
     int32_t half;           /* 1: every row repeats its first half (half of it is read) */
-    int32_t round_dtype;    /* element type that the entries are rounded to (F32: none) */
+    int32_t round_dtype;    /* what the entries are rounded to: args->dtype, or F32 (not at all) */
     int32_t reserved;
 } dsalt_rope_tables;
 
@@ -366,21 +366,35 @@ int dsalt_scores_check(const dsalt_scores_args *args);
 int dsalt_select_hybrid(const dsalt_scores_args *scores, const dsalt_select_args *select, void *stream);
 
 /*
- * dsalt_select_hybrid whose norms pass also forms the attention's operands: q rotated like
- * k (scores->k must be set; same tables and rules, n_heads heads of v_dtype), and with
- * out_dtype = DSALT_DTYPE_F16 for v_dtype = DSALT_DTYPE_F32 the rotated q and k and the
- * unrotated v written as fp16 (rounded from the fp32 values, as a cast after the rotation
- * would). Otherwise out_dtype = v_dtype and v_out = NULL (v is its own operand). The
- * k_out of `scores` has out_dtype. Outputs alias no input when out_dtype != v_dtype.
+ * dsalt_select_hybrid whose norms pass also forms the attention's operands and windows.
+ * Operands (scores->k must be set; q may be NULL): q rotated like k (same tables and rules,
+ * n_heads heads of v_dtype), and with out_dtype = DSALT_DTYPE_F16 for v_dtype =
+ * DSALT_DTYPE_F32 the rotated q and k and the unrotated v written as fp16 (rounded from the
+ * fp32 values, as a cast after the rotation would). Otherwise out_dtype = v_dtype and
+ * v_out = NULL (v is its own operand). The k_out of `scores` has out_dtype. Outputs alias
+ * no input when out_dtype != v_dtype; q_out may alias q otherwise.
+ * Windows (win_w NULL: none): logit = x . win_w + win_b[0] over operands rounded to
+ * win_dtype (x_dtype, or a 16-bit type for fp32 x: autocast), fp32 sums in a fixed order,
+ * rounded to win_dtype; w~ = n_min + sigmoid(logit) (n_max - n_min), every step rounded to
+ * win_dtype. win_w [d_model] (16-byte aligned) and win_b [1] (may be NULL) in x_dtype;
+ * win_logit and win_out [T] fp32. Replaces _window_continuous
+ * (dsalt/modules/dsalt_attention.py:270-276); `select` takes its windows from win_out
+ * (w = win_out; scores->gate_w must be NULL).
  */
 typedef struct dsalt_qkv_args {
-    int32_t out_dtype, reserved;
+    int32_t out_dtype;
+    int32_t rope_half; /* 1: every table row repeats its first half (half of it is read) */
     const void *q;
     int64_t q_stride_t, q_stride_h;
     void *q_out;
     int64_t q_out_stride_t, q_out_stride_h;
     void *v_out;
     int64_t v_out_stride_t, v_out_stride_h;
+    const void *win_w, *win_b;
+    float *win_logit, *win_out;
+    int32_t win_dtype;
+    float n_min, n_max;
+    int32_t reserved;
 } dsalt_qkv_args;
 
 int dsalt_select_hybrid_qkv(const dsalt_scores_args *scores, const dsalt_select_args *select,
@@ -500,6 +514,46 @@ typedef struct dsalt_lmk_weights_args {
     void *workspace;
     int64_t workspace_bytes;
 } dsalt_lmk_weights_args;
+
+/*
+ * Gradients of the attention module's inputs besides the attention's own kernels, in two
+ * steps around the projections' GEMMs. Replaces, with dsalt_bwd, autograd's backward of
+ * win_gate, of the hybrid scores and of the grouped K/V heads, and the sums of their
+ * contributions (dsalt/modules/dsalt_attention.py:270-276, :440-487).
+ * dsalt_module_grads_v: weights.d_weight to d_alpha and the per-token sums (workspace), then
+ *   dv [T, n_kv, D] in v_dtype, any 16-byte aligned strides = the value norms' share + the
+ *   attention's dv: `dv_heads` [T, H, D] summed over each group of heads, in heads_dtype
+ *   (v_dtype or F32); with dk_heads (grouped heads), dk likewise without a norm share.
+ *   With n_kv_heads = n_heads dv may alias dv_heads.
+ * dsalt_module_grads_x (same weights and workspace, later): dx [T, d_model] contiguous in
+ *   x_dtype = dx_in (in in_dtype, contiguous; NULL: 0) + the state norm's share + d_logit
+ *   win_w, with d_logit = d_w (n_max - n_min) sg (1 - sg), sg the gate as the forward
+ *   rounded it, and d_win_w [d_model], d_win_b [1] in x_dtype (win_w NULL: no gate; d_win_w
+ *   and d_win_b may be NULL).
+ * weights: as dsalt_lmk_weights_bwd takes them; dx, dv, dv_in and d_alpha of it are not
+ * written, its workspace must hold dsalt_module_grads_workspace_size bytes. fp32 sums in
+ * fixed orders, one rounding per result.
+ */
+typedef struct dsalt_module_grads_args {
+    dsalt_lmk_weights_args weights;
+    int32_t heads_dtype, in_dtype, win_dtype, alpha_sigmoid;
+    float *d_alpha;  /* [H]; alpha_sigmoid: of alpha_w, alpha = sigmoid(alpha_w); may be NULL */
+    const void *dk_heads, *dv_heads;
+    int64_t dkh_stride_t, dkh_stride_h, dvh_stride_t, dvh_stride_h;
+    void *dk, *dv;
+    int64_t dk_stride_t, dk_stride_h, dv_stride_t, dv_stride_h;
+    const void *dx_in;
+    void *dx;
+    const void *win_w;
+    const float *win_logit, *d_w;
+    void *d_win_w, *d_win_b;
+    float n_min, n_max;
+} dsalt_module_grads_args;
+
+int64_t dsalt_module_grads_workspace_size(int32_t total_len, int32_t n_heads, int32_t d_model);
+int dsalt_module_grads_v(const dsalt_module_grads_args *args, void *stream);
+int dsalt_module_grads_x(const dsalt_module_grads_args *args, void *stream);
+size_t dsalt_module_grads_args_size(void);
 
 int64_t dsalt_lmk_weights_workspace_size(int32_t total_len, int32_t n_heads);
 int dsalt_lmk_weights(const dsalt_lmk_weights_args *args, void *stream);

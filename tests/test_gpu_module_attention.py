@@ -40,9 +40,9 @@ def test_norms_pass_operands_equal_rope_then_cast(H, n_kv, D, dtype, strided, ca
     w = (1 + 60 * torch.rand(T, generator=g)).to(DEV)
     alpha = torch.rand(H, generator=g).to(DEV)
     cos, sin = tables(rows, D, cat)
-    f = _hip.SelectHybridLauncher(x, v, alpha, H, w, cu, 16, max_seqlen=257, rope_k=(k, cos, sin, cu), rope_q=q)
-    f()
     q_r, k_r = _hip.rope(q, k, cos, sin, cu)
+    f = _hip.SelectHybridLauncher(x, v, alpha, H, w, cu, 16, max_seqlen=257, rope_k=(k, cos, sin, cu), rope_q=q)
+    f()  # rotates q and k in place unless they are fp32
     w_ref, pos_ref, _ = _hip.select_hybrid(x, v, alpha, H, w, cu, 16, max_seqlen=257)
     cdt = _hip.compute_dtype(dtype)
     assert f.q_out.dtype == f.k_out.dtype == f.v_out.dtype == cdt
@@ -123,7 +123,7 @@ def test_module_training_equals_composed_route(case):
     got = {}
     for route in ("one", "composed"):
         if route == "composed":
-            mod._hip_attention = lambda *a: False
+            mod._one_function = lambda *a: False
         mod.zero_grad(set_to_none=True)
         xx = x.clone().requires_grad_()
         with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
@@ -149,3 +149,67 @@ def test_module_training_equals_composed_route(case):
             bar = 4 * 2 ** -5 / 0.4 / math.sqrt(H * k)
         a, b = a.double(), b.double()
         assert float((a - b).norm()) <= bar * float(b.norm()), name
+
+
+def small_module(dtype=torch.bfloat16):
+    torch.manual_seed(9)
+    mod = DSALTAttention(256, 4, 8, 100, 16, max_seq_len=400, n_kv_heads=2).to(DEV, dtype).train()
+    cu = torch.tensor([0, 250, 333], dtype=torch.int32, device=DEV)
+    return mod, torch.randn(333, 256, device=DEV).to(dtype), {"cu_seqlens": cu, "cu_list": [0, 250, 333]}
+
+
+def test_hooked_projections_are_called():
+    """A hook on a projection takes the route of separate functions, where it runs."""
+    print("module attention hooks", flush=True)
+    mod, x, packed = small_module()
+    assert mod._one_function(x)
+    seen = []
+    h = mod.k_proj.register_forward_hook(lambda m, a, o: seen.append(o.shape))
+    assert not mod._one_function(x)
+    mod(x, **packed)[0].float().sum().backward()
+    assert seen == [(333, 128)]
+    h.remove()
+    assert mod._one_function(x)
+
+
+@pytest.mark.parametrize("frozen", [("q_proj.weight",), ("k_proj.weight", "v_proj.weight", "alpha_w"),
+                                    ("win_gate.weight", "win_gate.bias"), ("q_proj.weight", "k_proj.weight", "v_proj.weight")])
+@pytest.mark.parametrize("x_grad", [True, False])
+def test_frozen_parameters_take_no_gradient(frozen, x_grad):
+    """The other gradients are what they are without the freezing (the weights' GEMMs are
+    taken apart, so up to their rounding)."""
+    print(f"module attention frozen {frozen} x_grad={x_grad}", flush=True)
+    mod, x, packed = small_module()
+    dy = torch.randn(333, 256, device=DEV).to(x.dtype)
+    want = {}
+    for pas in ("all", "frozen"):
+        mod.zero_grad(set_to_none=True)
+        for n, p in mod.named_parameters():
+            p.requires_grad_(pas == "all" or n not in frozen)
+        xx = x.clone().requires_grad_(pas == "all" or x_grad)
+        mod(xx, **packed)[0].backward(dy)
+        got = {"x": xx.grad, **{n: p.grad for n, p in mod.named_parameters()}}
+        if pas == "all":
+            want = got
+    for n, g in got.items():
+        if n in frozen or (n == "x" and not x_grad):
+            assert g is None, n
+        else:
+            w = want[n].double()
+            assert float((g.double() - w).norm()) <= 2 ** -8 * float(w.norm()), n
+
+
+@pytest.mark.parametrize("dtype,autocast", [(torch.bfloat16, False), (torch.float16, False), (torch.float32, True)])
+def test_training_windows_are_the_rounded_gate(dtype, autocast):
+    """The windows of the norms pass are torch's formula on the correctly rounded logits."""
+    print(f"module attention windows {dtype} autocast={autocast}", flush=True)
+    mod, x, packed = small_module(dtype)
+    with torch.no_grad():
+        mod.win_gate.weight.mul_(8)
+    cdt = torch.bfloat16 if autocast else dtype
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+        mod(x, **packed)
+    w, b = mod.win_gate.weight.to(cdt).double(), mod.win_gate.bias.to(cdt).double()
+    logit = (x.to(cdt).double() @ w.t() + b).squeeze(-1).to(cdt)
+    want = mod.n_min + torch.sigmoid(logit) * (mod.n_max - mod.n_min)
+    assert torch.equal(mod._last_selection[0], want.float().floor().clamp(min=1))
