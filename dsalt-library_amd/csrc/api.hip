@@ -559,6 +559,84 @@ int dsalt_add_rms_norm(const void *x, const void *h, void *x_out, void *y, const
     return DSALT_OK;
 }
 
+int dsalt_swiglu_rows(const void *gate_up, const void *d_out, void *out, int64_t rows, int32_t f, int32_t dtype,
+                      void *stream) {
+    if (rows < 0) return fail(DSALT_ERR_INVALID, "rows must be >= 0 (got %lld)", (long long)rows);
+    if (dtype != DSALT_DTYPE_BF16 && dtype != DSALT_DTYPE_F16 && dtype != DSALT_DTYPE_F32)
+        return fail(DSALT_ERR_INVALID, "dtype must be DSALT_DTYPE_BF16, _F16 or _F32 (got %d)", dtype);
+    const int per = dtype == DSALT_DTYPE_F32 ? 4 : 8;
+    if (f < per || f % per || f > (1 << 24))
+        return fail(DSALT_ERR_UNSUPPORTED, "f must be a multiple of %d in [%d, 2^24] (got %d)", per, per, f);
+    if (rows > ((int64_t)1 << 31) / (f / per) * 128)
+        return fail(DSALT_ERR_UNSUPPORTED, "rows * f is too large (%lld x %d)", (long long)rows, f);
+    if (rows == 0) return DSALT_OK;
+    if (!gate_up || !out) return fail(DSALT_ERR_INVALID, "gate_up and out must be non-NULL");
+    if (!aligned(gate_up, 16) || !aligned(d_out, 16) || !aligned(out, 16))
+        return fail(DSALT_ERR_INVALID, "gate_up, d_out and out must be 16-byte aligned");
+    if (out == gate_up || out == d_out) return fail(DSALT_ERR_INVALID, "out must not alias an input");
+    hipError_t e = dsalt::launch_swiglu_rows(gate_up, d_out, out, rows, f, dtype, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(DSALT_ERR_LAUNCH, "dsalt_swiglu_rows launch failed: %s", hipGetErrorString(e));
+    return DSALT_OK;
+}
+
+namespace {
+bool float_dtype(int dt) { return dt == DSALT_DTYPE_BF16 || dt == DSALT_DTYPE_F16 || dt == DSALT_DTYPE_F32; }
+
+int check_norm_train(const dsalt_norm_train_args *a, bool bwd) {
+    if (!a) return fail(DSALT_ERR_INVALID, "args must be non-NULL");
+    if (a->rows < 0 || a->rows > ((int64_t)1 << 31))
+        return fail(DSALT_ERR_INVALID, "rows must be in [0, 2^31] (got %lld)", (long long)a->rows);
+    if (a->d < 8 || a->d % 8 || a->d > dsalt::rms_norm_max_dim())
+        return fail(DSALT_ERR_UNSUPPORTED, "d must be a multiple of 8 in [8, %d] (got %d)", dsalt::rms_norm_max_dim(), a->d);
+    if (!float_dtype(a->x_dtype)) return fail(DSALT_ERR_INVALID, "x_dtype %d is not a float dtype", a->x_dtype);
+    const bool x32 = a->x_dtype == DSALT_DTYPE_F32;
+    const auto branch = [&](int dt) { return x32 ? float_dtype(dt) : dt == a->x_dtype; };
+    const bool norm = bwd || a->rstd || a->y || a->y_cast;
+    if (norm && a->w_dtype != DSALT_DTYPE_F32 && a->w_dtype != a->x_dtype)
+        return fail(DSALT_ERR_UNSUPPORTED, "weight dtype %d with x dtype %d", a->w_dtype, a->x_dtype);
+    if ((a->h || a->dh) && !branch(a->h_dtype))
+        return fail(DSALT_ERR_UNSUPPORTED, "h dtype %d with x dtype %d", a->h_dtype, a->x_dtype);
+    if (!bwd && a->y_cast && a->cast_dtype != DSALT_DTYPE_BF16 && a->cast_dtype != DSALT_DTYPE_F16)
+        return fail(DSALT_ERR_INVALID, "cast_dtype must be DSALT_DTYPE_BF16 or _F16 (got %d)", a->cast_dtype);
+    if (bwd && !branch(a->dy_dtype))
+        return fail(DSALT_ERR_UNSUPPORTED, "dy dtype %d with x dtype %d", a->dy_dtype, a->x_dtype);
+    if (a->rows == 0) return DSALT_OK;
+    if (!a->x || (norm && !a->weight)) return fail(DSALT_ERR_INVALID, "x and weight must be non-NULL");
+    for (const void *q : {a->x, a->h, a->weight, (const void *)a->x_out, (const void *)a->y, (const void *)a->y_cast, a->dy,
+                          a->dx_out, (const void *)a->dx, (const void *)a->dh, (const void *)a->workspace})
+        if (!aligned(q, 16)) return fail(DSALT_ERR_INVALID, "row tensors must be 16-byte aligned");
+    if (!aligned(a->rstd, 4)) return fail(DSALT_ERR_INVALID, "rstd must be 4-byte aligned");
+    if (!bwd) {
+        if (a->h && !a->x_out) return fail(DSALT_ERR_INVALID, "h needs x_out");
+        if (!a->h && !norm) return fail(DSALT_ERR_INVALID, "nothing to compute: no h and no output");
+    } else {
+        if (!a->dy || !a->rstd) return fail(DSALT_ERR_INVALID, "dy and rstd must be non-NULL");
+        if (a->d_weight && (!a->workspace || a->workspace_bytes < dsalt::norm_train_workspace_bytes(a->rows, a->d)))
+            return fail(DSALT_ERR_INVALID, "d_weight needs workspace of dsalt_norm_train_workspace_size bytes");
+    }
+    return DSALT_OK;
+}
+}  // namespace
+
+int dsalt_norm_train(const dsalt_norm_train_args *args, void *stream) {
+    if (int rc = check_norm_train(args, false)) return rc;
+    hipError_t e = dsalt::launch_norm_train(*args, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(DSALT_ERR_LAUNCH, "dsalt_norm_train launch failed: %s", hipGetErrorString(e));
+    return DSALT_OK;
+}
+
+int dsalt_norm_train_bwd(const dsalt_norm_train_args *args, void *stream) {
+    if (int rc = check_norm_train(args, true)) return rc;
+    hipError_t e = dsalt::launch_norm_train_bwd(*args, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(DSALT_ERR_LAUNCH, "dsalt_norm_train_bwd launch failed: %s", hipGetErrorString(e));
+    return DSALT_OK;
+}
+
+int64_t dsalt_norm_train_workspace_size(int64_t rows, int32_t d) {
+    return rows <= 0 || d <= 0 ? 0 : dsalt::norm_train_workspace_bytes(rows, d);
+}
+size_t dsalt_norm_train_args_size(void) { return sizeof(dsalt_norm_train_args); }
+
 int dsalt_rope_check(const dsalt_rope_args *a) {
     if (!a) return fail(DSALT_ERR_INVALID, "args is NULL");
     if (a->total_len < 0 || a->n_q_heads < 0 || a->n_k_heads < 0)

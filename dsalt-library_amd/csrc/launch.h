@@ -66,6 +66,11 @@ hipError_t launch_swiglu(const void *gate, const void *up, void *out, int64_t n,
 hipError_t launch_add_rms_norm(const void *x, const void *h, void *x_out, void *y, const void *weight, int64_t rows,
                                int d, float eps, int dtype, hipStream_t stream);
 int rms_norm_max_dim();
+hipError_t launch_swiglu_rows(const void *gate_up, const void *d_out, void *out, int64_t rows, int f, int dtype,
+                              hipStream_t stream);
+hipError_t launch_norm_train(const dsalt_norm_train_args &a, hipStream_t stream);
+hipError_t launch_norm_train_bwd(const dsalt_norm_train_args &a, hipStream_t stream);
+int64_t norm_train_workspace_bytes(int64_t rows, int d);
 
 // Number of query blocks of `bm` tokens over a packed batch, as an upper bound that is
 // computable without reading cu_seqlens: sum_s ceil(L_s/bm) <= ceil(T/bm) + S.

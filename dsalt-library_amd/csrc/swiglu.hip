@@ -84,7 +84,89 @@ __global__ void __launch_bounds__(256) swiglu_kernel(const uint4 *__restrict__ g
     if (i < n16) o[i] = swiglu_word<DT>(g[i], u[i]);
 }
 
+// Training: gu [rows, 2F] holds gate | up, the output of one GEMM against both weights
+// concatenated. Forward: out [rows, F] as above. Backward, with da = d out: dgu [rows, 2F] =
+//   dgate = da * u * sig * (1 + g * (1 - sig)),  dup = da * silu(g)
+// each formed in fp32 and rounded once (torch rounds silu, da * u and each factor's gradient
+// to 16 bits on the way); dup takes the rounded silu(g) that the forward multiplied with.
+// A thread takes one 16-byte word of each half. 6473 x 2816 in bf16: forward 21.5 us (109 MB,
+// 5.1 TB/s), backward 35.5 us (182 MB, 5.1 TB/s), as fast as a copy of the bytes; torch's
+// passes took 18 + 17 and 21 + 17 + 17 us.
+template <typename DT>
+__device__ __forceinline__ void swiglu_grad(float g, float u, float da, float &dg, float &du) {
+    const float sig = 1.f / (1.f + expf(-g));
+    // where g * (1 - sig) is inf * 0 (g = +inf) or sig * g is 0 * inf (g = -inf) this is NaN,
+    // as torch's formula is
+    dg = da * u * (sig * (1.f + g * (1.f - sig)));
+    du = da * silu_rounded<DT>(g);
+    asm volatile("" : "+v"(dg), "+v"(du));
+}
+
+template <typename DT>
+__device__ __forceinline__ void swiglu_grad_word(uint4 g, uint4 u, uint4 da, uint4 &dg, uint4 &du) {
+    const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, uw[4] = {u.x, u.y, u.z, u.w}, aw[4] = {da.x, da.y, da.z, da.w};
+    uint32_t og[4], ou[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if constexpr (std::is_same<DT, F32>::value) {
+            float a, b;
+            swiglu_grad<F32>(__uint_as_float(gw[e]), __uint_as_float(uw[e]), __uint_as_float(aw[e]), a, b);
+            og[e] = __float_as_uint(a);
+            ou[e] = __float_as_uint(b);
+        } else {
+            float a0, b0, a1, b1;
+            swiglu_grad<DT>(DT::lo_f32(gw[e]), DT::lo_f32(uw[e]), DT::lo_f32(aw[e]), a0, b0);
+            swiglu_grad<DT>(DT::hi_f32(gw[e]), DT::hi_f32(uw[e]), DT::hi_f32(aw[e]), a1, b1);
+            og[e] = DT::pack2(a0, a1);
+            ou[e] = DT::pack2(b0, b1);
+        }
+    }
+    dg = make_uint4(og[0], og[1], og[2], og[3]);
+    du = make_uint4(ou[0], ou[1], ou[2], ou[3]);
+}
+
+// fw: words of F elements; n = rows * fw. The row of a workgroup's first word is a scalar
+// division, the row of a thread's word from there a 32-bit one.
+template <typename DT, bool BWD>
+__global__ void __launch_bounds__(256) swiglu_rows_kernel(const uint4 *__restrict__ gu, const uint4 *__restrict__ da,
+                                                          uint4 *__restrict__ o, int64_t n, uint32_t fw) {
+    const int64_t first = (int64_t)blockIdx.x * 256;
+    const int64_t row0 = first / fw;
+    const uint32_t w = (uint32_t)(first - row0 * fw) + threadIdx.x, r = w / fw, col = w - r * fw;
+    const int64_t i = first + threadIdx.x, row = row0 + r;
+    if (i >= n) return;
+    const int64_t at = row * 2 * fw + col;
+    const uint4 g = gu[at], u = gu[at + fw];
+    if constexpr (BWD) {
+        uint4 dg, du;
+        swiglu_grad_word<DT>(g, u, da[i], dg, du);
+        o[at] = dg;
+        o[at + fw] = du;
+    } else {
+        o[i] = swiglu_word<DT>(g, u);
+    }
+}
+
+template <typename DT>
+void launch_rows(const uint4 *gu, const uint4 *da, uint4 *o, int64_t n, uint32_t fw, hipStream_t stream) {
+    const dim3 grid((unsigned)((n + 255) / 256));
+    if (da) hipLaunchKernelGGL((swiglu_rows_kernel<DT, true>), grid, dim3(256), 0, stream, gu, da, o, n, fw);
+    else hipLaunchKernelGGL((swiglu_rows_kernel<DT, false>), grid, dim3(256), 0, stream, gu, da, o, n, fw);
+}
+
 }  // namespace
+
+hipError_t launch_swiglu_rows(const void *gate_up, const void *d_out, void *out, int64_t rows, int f, int dtype,
+                              hipStream_t stream) {
+    if (rows == 0) return hipSuccess;
+    const int fw = f / (dtype == DSALT_DTYPE_F32 ? 4 : 8);
+    const uint4 *gu = static_cast<const uint4 *>(gate_up), *da = static_cast<const uint4 *>(d_out);
+    uint4 *o = static_cast<uint4 *>(out);
+    if (dtype == DSALT_DTYPE_BF16) launch_rows<BF16>(gu, da, o, rows * fw, fw, stream);
+    else if (dtype == DSALT_DTYPE_F16) launch_rows<F16>(gu, da, o, rows * fw, fw, stream);
+    else launch_rows<F32>(gu, da, o, rows * fw, fw, stream);
+    return hipGetLastError();
+}
 
 hipError_t launch_swiglu(const void *gate, const void *up, void *out, int64_t n, int dtype, hipStream_t stream) {
     if (n == 0) return hipSuccess;

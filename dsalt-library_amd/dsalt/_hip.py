@@ -177,6 +177,19 @@ class ModuleGradsArgs(ctypes.Structure):
     ]
 
 
+class NormTrainArgs(ctypes.Structure):
+    _fields_ = [
+        ("rows", c_int64), ("d", c_int32),
+        ("x_dtype", c_int32), ("h_dtype", c_int32), ("w_dtype", c_int32), ("cast_dtype", c_int32), ("dy_dtype", c_int32),
+        ("eps", c_float),
+        ("x", c_void_p), ("h", c_void_p), ("weight", c_void_p),
+        ("x_out", c_void_p), ("y", c_void_p), ("y_cast", c_void_p), ("rstd", c_void_p),
+        ("dy", c_void_p), ("dx_out", c_void_p),
+        ("dx", c_void_p), ("dh", c_void_p), ("d_weight", c_void_p),
+        ("workspace", c_void_p), ("workspace_bytes", c_int64),
+    ]
+
+
 EXPORTED_SYMBOLS = (
     "dsalt_fwd", "dsalt_fwd_check", "dsalt_bwd", "dsalt_bwd_check", "dsalt_bwd_workspace_size",
     "dsalt_select_landmarks", "dsalt_select_check", "dsalt_quantize_windows",
@@ -187,7 +200,8 @@ EXPORTED_SYMBOLS = (
     "dsalt_add_rms_norm", "dsalt_lmk_weights", "dsalt_lmk_weights_bwd", "dsalt_lmk_weights_check",
     "dsalt_lmk_weights_workspace_size", "dsalt_lmk_weights_args_size", "dsalt_bwd_rope", "dsalt_rope_tables_size",
     "dsalt_select_hybrid_qkv", "dsalt_qkv_args_size", "dsalt_module_grads_v", "dsalt_module_grads_x",
-    "dsalt_module_grads_workspace_size", "dsalt_module_grads_args_size",
+    "dsalt_module_grads_workspace_size", "dsalt_module_grads_args_size", "dsalt_swiglu_rows", "dsalt_norm_train",
+    "dsalt_norm_train_bwd", "dsalt_norm_train_workspace_size", "dsalt_norm_train_args_size",
 )
 NOALLOC_SCRATCH_BYTES = 76 << 20  # DSALT_NOALLOC_SCRATCH_BYTES
 SELECT_SPLIT_MIN = 4096  # longer sequences can be selected chunk-wise
@@ -227,6 +241,9 @@ def lib() -> ctypes.CDLL:
         ("dsalt_lmk_weights_bwd", [ctypes.POINTER(LmkWeightsArgs), c_void_p]),
         ("dsalt_lmk_weights_check", [ctypes.POINTER(LmkWeightsArgs), c_int32]),
         ("dsalt_quantize_windows", [c_void_p, c_int64, c_void_p, c_void_p, c_void_p]),
+        ("dsalt_norm_train", [ctypes.POINTER(NormTrainArgs), c_void_p]),
+        ("dsalt_norm_train_bwd", [ctypes.POINTER(NormTrainArgs), c_void_p]),
+        ("dsalt_swiglu_rows", [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_void_p]),
         ("dsalt_swiglu", [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_void_p]),
         ("dsalt_add_rms_norm", [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_float, c_int32,
                                 c_void_p]),
@@ -242,13 +259,15 @@ def lib() -> ctypes.CDLL:
     h.dsalt_select_workspace_size.restype = c_int64
     h.dsalt_module_grads_workspace_size.argtypes = [c_int32] * 3
     h.dsalt_module_grads_workspace_size.restype = c_int64
+    h.dsalt_norm_train_workspace_size.argtypes = [c_int64, c_int32]
+    h.dsalt_norm_train_workspace_size.restype = c_int64
     h.dsalt_lmk_weights_workspace_size.argtypes = [c_int32] * 2
     h.dsalt_lmk_weights_workspace_size.restype = c_int64
     h.dsalt_abi_version.restype = ctypes.c_int
     h.dsalt_last_error.restype = ctypes.c_char_p
     for n in ("dsalt_fwd_args_size", "dsalt_bwd_args_size", "dsalt_select_args_size", "dsalt_scores_args_size",
               "dsalt_rope_args_size", "dsalt_lmk_weights_args_size", "dsalt_rope_tables_size", "dsalt_qkv_args_size",
-              "dsalt_module_grads_args_size"):
+              "dsalt_module_grads_args_size", "dsalt_norm_train_args_size"):
         getattr(h, n).restype = c_size_t
     _lib = h
     check_abi()
@@ -263,7 +282,8 @@ def check_abi() -> None:
                        (SelectArgs, h.dsalt_select_args_size), (ScoresArgs, h.dsalt_scores_args_size),
                        (RopeArgs, h.dsalt_rope_args_size), (LmkWeightsArgs, h.dsalt_lmk_weights_args_size),
                        (RopeTables, h.dsalt_rope_tables_size), (QkvArgs, h.dsalt_qkv_args_size),
-                       (ModuleGradsArgs, h.dsalt_module_grads_args_size)):
+                       (ModuleGradsArgs, h.dsalt_module_grads_args_size),
+                       (NormTrainArgs, h.dsalt_norm_train_args_size)):
         if ctypes.sizeof(struct) != fn():
             raise DsaltError(f"{struct.__name__} layout mismatch: {ctypes.sizeof(struct)} vs {fn()} bytes")
 
@@ -1352,3 +1372,91 @@ def add_rms_norm(x: torch.Tensor, h: torch.Tensor | None, weight: torch.Tensor, 
                                     x.numel() // d, d, float(eps), _SCORE_DTYPES[x.dtype], stream_handle(dev)),
            "dsalt_add_rms_norm")
     return x_out, y
+
+
+def _rows_aligned(*ts: torch.Tensor | None) -> bool:
+    return all(t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0) for t in ts)
+
+
+def aligned_rows(t: torch.Tensor) -> torch.Tensor:
+    """t itself when it is contiguous and 16-byte aligned, otherwise a copy that is."""
+    return t if _rows_aligned(t) else t.clone(memory_format=torch.contiguous_format)
+
+
+def norm_train_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether dsalt_norm_train takes rows of x [..., d] with this weight [d]: GPU tensors,
+    contiguous and 16-byte aligned, d a multiple of 8 up to 4096, x bf16, fp16 or fp32, the
+    weight of x's dtype or (16-bit x) fp32."""
+    if x.device.type != "cuda" or x.dtype not in _SCORE_DTYPES or x.dim() < 1 or x.numel() == 0:
+        return False
+    d = x.shape[-1]
+    return (8 <= d <= RMS_NORM_MAX_DIM and d % 8 == 0 and _rows_aligned(x, weight) and weight.device == x.device
+            and weight.dtype in (x.dtype, torch.float32) and weight.shape == (d,))
+
+
+def norm_train_branch_supported(x: torch.Tensor, h: torch.Tensor) -> bool:
+    """Whether h can be added to x by dsalt_norm_train: its shape, contiguous and aligned, in
+    x's dtype or (fp32 x) 16-bit, so that the sum has x's dtype."""
+    return (h.shape == x.shape and h.device == x.device and _rows_aligned(h)
+            and (h.dtype == x.dtype or (x.dtype == torch.float32 and h.dtype in (torch.bfloat16, torch.float16))))
+
+
+def norm_train(x, h, weight, eps: float, want_y: bool = True, cast: torch.dtype | None = None):
+    """``(x_out, y, y_cast, rstd)`` of x (+ h): see dsalt_norm_train. weight None: the sum only
+    (y, y_cast and rstd None). h None: x_out is None."""
+    dev = require_gpu(x, h, weight)
+    d = x.shape[-1]
+    a = NormTrainArgs(rows=x.numel() // d, d=d, eps=float(eps), x_dtype=_SCORE_DTYPES[x.dtype], x=x.data_ptr())
+    x_out = y = y_cast = rstd = None
+    if h is not None:
+        x_out = torch.empty_like(x)
+        a.h, a.h_dtype, a.x_out = h.data_ptr(), _SCORE_DTYPES[h.dtype], x_out.data_ptr()
+    if weight is not None:
+        a.weight, a.w_dtype = weight.data_ptr(), _SCORE_DTYPES[weight.dtype]
+        rstd = torch.empty(a.rows, device=dev, dtype=torch.float32)
+        a.rstd = rstd.data_ptr()
+        if want_y:
+            y = torch.empty_like(x)
+            a.y = y.data_ptr()
+        if cast is not None:
+            y_cast = torch.empty_like(x, dtype=cast)
+            a.y_cast, a.cast_dtype = y_cast.data_ptr(), _SCORE_DTYPES[cast]
+    _raise(lib().dsalt_norm_train(ctypes.byref(a), stream_handle(dev)), "dsalt_norm_train")
+    return x_out, y, y_cast, rstd
+
+
+def norm_train_bwd(x, weight, rstd, dy, dx_out, h_dtype: torch.dtype | None, want_dx: bool, want_dw: bool):
+    """``(dx, dh, d_weight)``: see dsalt_norm_train_bwd; dh in h_dtype (None: not formed)."""
+    dev = require_gpu(x, weight, rstd, dy, dx_out)
+    d = x.shape[-1]
+    a = NormTrainArgs(rows=x.numel() // d, d=d, x_dtype=_SCORE_DTYPES[x.dtype], w_dtype=_SCORE_DTYPES[weight.dtype],
+                      dy_dtype=_SCORE_DTYPES[dy.dtype], x=x.data_ptr(), weight=weight.data_ptr(), rstd=rstd.data_ptr(),
+                      dy=dy.data_ptr(), dx_out=_ptr(dx_out))
+    dx = dh = dw = ws = None
+    if want_dx:
+        dx = torch.empty_like(x)
+        a.dx = dx.data_ptr()
+    if h_dtype is not None:
+        dh = torch.empty_like(x, dtype=h_dtype)
+        a.dh, a.h_dtype = dh.data_ptr(), _SCORE_DTYPES[h_dtype]
+    if want_dw:
+        a.workspace_bytes = lib().dsalt_norm_train_workspace_size(a.rows, d)
+        ws = torch.empty(a.workspace_bytes, device=dev, dtype=torch.uint8)
+        dw = torch.empty_like(weight)
+        a.d_weight, a.workspace = dw.data_ptr(), ws.data_ptr()
+    _raise(lib().dsalt_norm_train_bwd(ctypes.byref(a), stream_handle(dev)), "dsalt_norm_train_bwd")
+    return dx, dh, dw
+
+
+def swiglu_rows(gate_up: torch.Tensor, d_out: torch.Tensor | None = None) -> torch.Tensor:
+    """``silu(gate) * up`` [T, f] of contiguous gate_up [T, 2 f] (gate | up), or with d_out [T, f]
+    the gradient of gate_up. One HIP pass."""
+    dev = require_gpu(gate_up, d_out)
+    rows, f = gate_up.shape[0], gate_up.shape[1] // 2
+    if not _rows_aligned(gate_up, d_out) or (d_out is not None and (d_out.shape != (rows, f)
+                                                                    or d_out.dtype != gate_up.dtype)):
+        raise DsaltError("dsalt_swiglu_rows needs contiguous, 16-byte aligned gate_up [T, 2f] and d_out [T, f]")
+    out = torch.empty_like(gate_up) if d_out is not None else gate_up.new_empty(rows, f)
+    _raise(lib().dsalt_swiglu_rows(gate_up.data_ptr(), _ptr(d_out), out.data_ptr(), rows, f,
+                                   _SCORE_DTYPES[gate_up.dtype], stream_handle(dev)), "dsalt_swiglu_rows")
+    return out

@@ -21,11 +21,11 @@ from .. import _hip
 
 class _ModuleAttention(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, wq, wk, wv, wg, bg, alpha_w, cos, sin, cu_seqlens, opt):
+    def forward(ctx, x, wq, wk, wv, wg, bg, alpha_w, cos, sin, cu_seqlens, opt, x_cast):
         cdt, H, n_kv, D = opt["dtype"], opt["n_heads"], opt["n_kv_heads"], opt["head_dim"]
         T, dense, k_lmk = x.shape[0], opt["dense"], opt["k_lmk"]
         xd = x.detach()
-        xb = xd if xd.dtype == cdt else xd.to(cdt)
+        xb = xd if xd.dtype == cdt else xd.to(cdt) if x_cast is None else x_cast.detach()
         ws = [w.detach() for w in (wq, wk, wv)]
         if wq.dtype == cdt:
             w_cat = torch.cat(ws)
@@ -108,7 +108,7 @@ class _ModuleAttention(torch.autograd.Function):
         if not ctx.needs_input_grad[5]:
             dbg = None
         return (dx, *dws, dwg if ctx.needs_input_grad[4] else None, dbg,
-                d_alpha.to(a_dtype) if ctx.needs_input_grad[6] else None, None, None, None, None)
+                d_alpha.to(a_dtype) if ctx.needs_input_grad[6] else None, *[None] * 5)
 
 
 def _split(qkv: torch.Tensor, H: int, n_kv: int, D: int):
@@ -118,11 +118,12 @@ def _split(qkv: torch.Tensor, H: int, n_kv: int, D: int):
     return q.view(T, H, D), k.view(T, n_kv, D), v.view(T, n_kv, D)
 
 
-def module_attention(x, q_proj, k_proj, v_proj, win_gate, alpha_w, cos, sin, cu_seqlens, opt: dict):
+def module_attention(x, q_proj, k_proj, v_proj, win_gate, alpha_w, cos, sin, cu_seqlens, opt: dict, x_cast=None):
     """``(out [T, H, D] in the compute dtype, lmk_pos [H, S, k], w~ [T], quantised w or None)`` of
     packed states x [T, d]. The four projections are plain nn.Linear modules (q, k and v
     without bias); ``opt``: dtype (of the projections' results), n_heads, n_kv_heads,
     head_dim, k_lmk, max_seqlen, tau_lmk, tau_win, win_edge, n_min, n_max, dense (one
-    sequence, the dense variant). Operands: as DSALTAttention._one_function checks them."""
+    sequence, the dense variant). ``x_cast``: x rounded to dtype, if the caller has it.
+    Operands: as DSALTAttention._one_function checks them."""
     return _ModuleAttention.apply(x, q_proj.weight, k_proj.weight, v_proj.weight, win_gate.weight, win_gate.bias, alpha_w,
-                                  cos, sin, cu_seqlens, opt)
+                                  cos, sin, cu_seqlens, opt, x_cast)

@@ -41,6 +41,7 @@ import torch.nn.functional as F
 
 from .. import _hip
 from ..kernels._dense import dense_attention, dense_probabilities
+from ..kernels._block_train import autocast_dtype, eager, plain
 from ..kernels._lmk_weights import landmark_weights
 from ..kernels._module_attention import module_attention
 from ..kernels._sparse import sparse_attention
@@ -247,15 +248,17 @@ class DSALTAttention(nn.Module):
     # ---- forward -----------------------------------------------------------------------
     def forward(self, x: torch.Tensor, cu_seqlens: torch.Tensor | None = None,
                 max_seqlen: int | None = None, rope_cs: tuple | None = None,
-                cu_list: list | None = None, *, _need_aux: bool = True) -> tuple[torch.Tensor, torch.Tensor]:
+                cu_list: list | None = None, *, _need_aux: bool = True,
+                _x_cast: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
         # _need_aux=False (internal, packed path): return None instead of the zero aux loss,
-        # so that a caller that discards it launches no fill for it
+        # so that a caller that discards it launches no fill for it. _x_cast (internal): x rounded to
+        # the autocast type, if the caller has it
         if cu_seqlens is not None:
-            return self._packed(x, cu_seqlens, x.shape[0], x.device, rope_cs, cu_list, need_aux=_need_aux)
+            return self._packed(x, cu_seqlens, x.shape[0], x.device, rope_cs, cu_list, need_aux=_need_aux, x_cast=_x_cast)
         B, T, _ = x.shape
-        return self._batched(x, B, T, x.device)
+        return self._batched(x, B, T, x.device, _x_cast)
 
-    def _batched(self, x: torch.Tensor, B: int, T: int, device: torch.device):
+    def _batched(self, x: torch.Tensor, B: int, T: int, device: torch.device, x_cast: torch.Tensor | None = None):
         """Dense batched forward of ``x [1, T, d]`` (dsalt_attention.py:371-438)."""
         _hip.require_gpu(x)
         if B != 1:
@@ -268,7 +271,8 @@ class DSALTAttention(nn.Module):
         self._last_P = None
         if not collect_P and self._one_function(xs):
             cu = torch.arange(0, T + 1, T, dtype=torch.int32, device=device)  # [0, T], made on the GPU
-            out, lmk_pos, w_cont, _ = self._attend(xs, cu, min(self.k_lmk, T), T, dense=True)
+            out, lmk_pos, w_cont, _ = self._attend(xs, cu, min(self.k_lmk, T), T, dense=True,
+                                                     x_cast=None if x_cast is None else x_cast[0])
         else:
             q = self.q_proj(xs).view(T, self.n_heads, self.head_dim)
             k = self.k_proj(xs).view(T, self.n_kv_heads, self.head_dim)
@@ -295,14 +299,11 @@ class DSALTAttention(nn.Module):
         weights, or fp32 for all of them under a 16-bit autocast; rows that the norms pass
         loads in 16-byte pieces."""
         lin = (self.q_proj, self.k_proj, self.v_proj, self.win_gate)
+        if not eager(x, self.alpha_w):
+            return False
         if not (self._fused_selector and self._hip_scores and self._fuse_qkv and all(type(m) is nn.Linear for m in lin)):
             return False
-        if any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-               or "forward" in m.__dict__ for m in lin):
-            return False
-        g = nn.modules.module
-        if (g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks
-                or g._global_backward_pre_hooks):
+        if not plain(*lin) or not eager(*(p for m in lin for p in m.parameters())):
             return False
         if any(m.bias is not None for m in lin[:3]) or x.dim() != 2 or x.shape[0] == 0 or x.shape[1] != self.d_model:
             return False
@@ -313,7 +314,7 @@ class DSALTAttention(nn.Module):
             return False
         if x.dtype not in (torch.bfloat16, torch.float16, torch.float32):
             return False
-        cdt = self._compute_dtype(x)
+        cdt = autocast_dtype(x)
         if cdt not in (torch.bfloat16, torch.float16, torch.float32) or (cdt != x.dtype and x.dtype != torch.float32):
             return False
         per = 4 if x.dtype == torch.float32 else 8  # elements per 16-byte load
@@ -321,19 +322,14 @@ class DSALTAttention(nn.Module):
                 and x.stride(0) >= self.d_model and x.stride(0) % per == 0 and x.data_ptr() % 16 == 0
                 and self.win_gate.weight.data_ptr() % 16 == 0)
 
-    @staticmethod
-    def _compute_dtype(x: torch.Tensor) -> torch.dtype:
-        """Element type of the projections' results: autocast's where it is on."""
-        return torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
-
     @_dynamo_opaque
-    def _attend(self, x, cu_seqlens, k_lmk, max_seqlen, dense=False):
+    def _attend(self, x, cu_seqlens, k_lmk, max_seqlen, dense=False, x_cast=None):
         cos, sin = self._rope_tables()
-        opt = dict(dtype=self._compute_dtype(x), n_heads=self.n_heads, n_kv_heads=self.n_kv_heads,
+        opt = dict(dtype=autocast_dtype(x), n_heads=self.n_heads, n_kv_heads=self.n_kv_heads,
                    head_dim=self.head_dim, k_lmk=k_lmk, max_seqlen=max_seqlen, tau_lmk=self.tau_lmk,
                    tau_win=self.tau_win, win_edge=float(self.win_edge), n_min=self.n_min, n_max=self.n_max, dense=dense)
         return module_attention(x, self.q_proj, self.k_proj, self.v_proj, self.win_gate, self.alpha_w, cos, sin,
-                                cu_seqlens, opt)
+                                cu_seqlens, opt, x_cast)
 
     def _hip_weights(self, x: torch.Tensor, v: torch.Tensor | None) -> bool:
         """Whether the selection and its differentiable weights run on the HIP passes over x
@@ -410,12 +406,13 @@ class DSALTAttention(nn.Module):
         return w_cont, lmk_pos, lmk_logw, v
 
     def _packed(self, x: torch.Tensor, cu_seqlens: torch.Tensor, total_len: int, device: torch.device,
-                rope_cs: tuple | None = None, cu_list: list | None = None, need_aux: bool = True):
+                rope_cs: tuple | None = None, cu_list: list | None = None, need_aux: bool = True,
+                x_cast: torch.Tensor | None = None):
         _hip.require_gpu(x, cu_seqlens)
         if self.training and rope_cs is None and self._one_function(x):
             self._last_P = None
             max_len = None if cu_list is None else max((b - a for a, b in zip(cu_list[:-1], cu_list[1:])), default=0)
-            out, lmk_pos, _, w_disc = self._attend(x, cu_seqlens, self.k_lmk, max_len)
+            out, lmk_pos, _, w_disc = self._attend(x, cu_seqlens, self.k_lmk, max_len, x_cast=x_cast)
             self._last_selection = (w_disc, lmk_pos)
             return (self._apply_out_proj(out.reshape(total_len, self.d_model)),
                     x.new_zeros(()) if need_aux else None)

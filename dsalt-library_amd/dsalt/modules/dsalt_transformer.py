@@ -4,8 +4,9 @@ The LM consumer of the attention path: x + attn(norm(x)), then x + ffn(norm(x)),
 SwiGLU feed-forward. Parameter names and creation order follow the reference
 (attn_norm, ffn_norm, attn, ffn; gate_proj, up_proj, down_proj) so state dicts load and
 seeded initialisations agree. The attention runs on the HIP kernels; the projections are
-torch (hipBLASLt GEMMs). Without autograd on the GPU, the FFN's gated product and each
-residual add with the norm after it are HIP passes too; with autograd they are torch ops.
+torch (hipBLASLt GEMMs). On the GPU the FFN's gated product and each residual add with the
+norm after it are HIP passes too, with autograd forward and backward (rows or modules that
+those do not take run torch's ops).
 """
 from __future__ import annotations
 
@@ -15,14 +16,16 @@ import torch.nn.functional as F
 import torch.utils.checkpoint
 
 from .. import _hip
+from ..kernels import _block_train
 from ..kernels.RMSENorm import RMSENorm
 from .dsalt_attention import DSALTAttention
 
 
 class SwiGLUFFN(nn.Module):
-    """``down_proj(silu(gate_proj(x)) * up_proj(x))`` (dsalt_transformer.py:10-21). Without
-    autograd, on the GPU, the gated product is one HIP pass (``dsalt_swiglu``) with torch's
-    roundings, instead of torch's silu and product passes."""
+    """``down_proj(silu(gate_proj(x)) * up_proj(x))`` (dsalt_transformer.py:10-21). On the GPU
+    the gated product is one HIP pass with torch's roundings (``dsalt_swiglu``), instead of
+    torch's silu and product passes; with autograd, and projections that are plain nn.Linear
+    modules, the whole is one function with a HIP pass for the product's gradients."""
 
     def __init__(self, d_model: int, d_ff: int, dropout: float = 0.0):
         super().__init__()
@@ -32,6 +35,8 @@ class SwiGLUFFN(nn.Module):
         self.drop = nn.Dropout(dropout)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if torch.is_grad_enabled() and _block_train.swiglu_supported(self, x):
+            return self.drop(_block_train.swiglu_ffn(self, x))
         g, u = self.gate_proj(x), self.up_proj(x)
         if not torch.is_grad_enabled() and _hip.swiglu_supported(g, u):
             h = _hip.swiglu(g, u)  # one pass, the same bits as the two torch ops below
@@ -46,7 +51,9 @@ class DSALTTransformerBlock(nn.Module):
     the FFN in the backward when training. ``_fuse_norms`` (default True): at inference
     without autograd, with 16-bit rows, a residual add and the norm after it run as one
     HIP pass (``dsalt_add_rms_norm``: the sum is torch's add bit for bit, the norm can
-    differ from F.rms_norm in an output's last bit)."""
+    differ from F.rms_norm in an output's last bit); with autograd, in fp32 or 16-bit, as one
+    pass forward and one backward (``dsalt_norm_train``), which under autocast also writes
+    the norm in the projections' type."""
 
     _fuse_norms = True
 
@@ -67,23 +74,48 @@ class DSALTTransformerBlock(nn.Module):
                 gradient_checkpointing: bool = False, rope_cs: tuple | None = None,
                 cu_list: list | None = None) -> tuple[torch.Tensor, torch.Tensor]:
         aux_box = []
+        train_norms = torch.is_grad_enabled() and self._fuse_norms
 
-        def attend(h):
-            o, a = self.attn(h, cu_seqlens=cu_seqlens, max_seqlen=max_seqlen, rope_cs=rope_cs, cu_list=cu_list)
+        def attend(h, h_cast=None):
+            more = {} if h_cast is None else {"_x_cast": h_cast}
+            o, a = self.attn(h, cu_seqlens=cu_seqlens, max_seqlen=max_seqlen, rope_cs=rope_cs, cu_list=cu_list, **more)
             aux_box.append(a)
             return o
 
         recompute = gradient_checkpointing and self.training
-        h = self.attn_norm(x)
-        x_attn = torch.utils.checkpoint.checkpoint(attend, h, use_reentrant=False) if recompute else attend(h)
+        # under autocast the projections' operand is written by the norm itself
+        cast = _block_train.autocast_dtype(x) if x.is_cuda else x.dtype
+        cast = cast if cast != x.dtype and x.dtype == torch.float32 else None
+        h_cast = None
+        if train_norms and self._train_norm(x, None, self.attn_norm):
+            if cast is not None and type(self.attn) is DSALTAttention and _block_train.plain(self.attn):
+                x, h, h_cast = _block_train.add_norm(x, None, self.attn_norm, cast)
+            else:
+                x, h = _block_train.add_norm(x, None, self.attn_norm)
+        else:
+            h = self.attn_norm(x)
+        x_attn = (torch.utils.checkpoint.checkpoint(attend, h, h_cast, use_reentrant=False) if recompute
+                  else attend(h, h_cast))
         if self._norms_fusable(x, x_attn, self.ffn_norm):
             # the residual add and the FFN's norm in one HIP pass (inference)
             x, h = _hip.add_rms_norm(x, x_attn, self.ffn_norm.weight, self.ffn_norm.eps)
+        elif train_norms and self._train_norm(x, x_attn, self.ffn_norm):
+            low = (cast is not None and type(self.ffn) is SwiGLUFFN and _block_train.plain(self.ffn)
+                   and _block_train.swiglu_supported(self.ffn, x))
+            x, h = _block_train.add_norm(x, x_attn, self.ffn_norm, cast if low else None, low)
         else:
             x = x + x_attn
             h = self.ffn_norm(x)
-        x = x + (torch.utils.checkpoint.checkpoint(self.ffn, h, use_reentrant=False) if recompute else self.ffn(h))
+        f = torch.utils.checkpoint.checkpoint(self.ffn, h, use_reentrant=False) if recompute else self.ffn(h)
+        x = _block_train.residual_add(x, f) if train_norms else x + f
         return x, aux_box[0]
+
+    @staticmethod
+    def _train_norm(x: torch.Tensor, h: torch.Tensor | None, norm: nn.Module) -> bool:
+        """Whether x (+ h) and the RMSENorm `norm` can run as one differentiable pass."""
+        return (_block_train.eager(x, norm.weight) and type(norm) is RMSENorm and _block_train.plain(norm) and _hip.norm_train_supported(x, norm.weight)
+                and norm.normalized_shape == (x.shape[-1],)
+                and (h is None or _hip.norm_train_branch_supported(x, h)))
 
     def _norms_fusable(self, x: torch.Tensor, h: torch.Tensor | None, norm: nn.Module) -> bool:
         """Whether x (+ h) and the RMSENorm `norm` can run as one dsalt_add_rms_norm pass:

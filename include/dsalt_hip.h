@@ -474,6 +474,51 @@ int dsalt_add_rms_norm(const void *x, const void *h, void *x_out, void *y, const
                        int32_t d, float eps, int32_t dtype, void *stream);
 
 /*
+ * Training form of the gated product. gate_up [rows, 2 f] (gate | up, contiguous), out
+ * [rows, f]: the bits of dsalt_swiglu. With d_out [rows, f] in the same dtype (backward):
+ * out is [rows, 2 f], the gradients of gate and up, each formed in fp32 and rounded once.
+ * f a multiple of 8 (4 for fp32) up to 2^24; 16-byte aligned pointers; out aliases nothing.
+ * Replaces F.silu(gate_proj(x)) * up_proj(x) (dsalt/modules/dsalt_transformer.py:20-21)
+ * under autograd.
+ */
+int dsalt_swiglu_rows(const void *gate_up, const void *d_out, void *out, int64_t rows, int32_t f, int32_t dtype,
+                      void *stream);
+
+/*
+ * Residual add and RMSNorm of a training step, forward (dsalt_norm_train) and backward
+ * (dsalt_norm_train_bwd), of rows [rows, d], contiguous.
+ * Forward: x_out = x + h (h NULL: x is normalised as it is, x_out not written), rstd [rows],
+ * and y (x's dtype) and/or y_cast (cast_dtype, bf16 or fp16) = (x_out * rstd) * weight; with
+ * rstd, y and y_cast all NULL only the sum is formed. Backward: x is the normalised tensor,
+ * dy the gradient of y or y_cast, dx_out that of x_out (or NULL); writes dx (x's dtype), dh
+ * (h_dtype) and d_weight (w_dtype), each of which may be NULL; d_weight needs workspace of
+ * dsalt_norm_train_workspace_size(rows, d) bytes, dead when the launches end. Sums in fp32
+ * in a fixed order.
+ * dtypes: x fp32 with fp32 weight and h and dy in fp32, bf16 or fp16; or x, h and dy all
+ * bf16 or all fp16 with the weight of that dtype or fp32. d a multiple of 8 up to 4096;
+ * 16-byte aligned pointers (rstd 4); outputs alias no input.
+ * Replaces the torch ops of dsalt/modules/dsalt_transformer.py:81-84 and RMSENorm.forward
+ * (dsalt/kernels/RMSENorm.py:21-23) with their autograd.
+ */
+typedef struct dsalt_norm_train_args {
+    int64_t rows;
+    int32_t d;
+    int32_t x_dtype, h_dtype, w_dtype, cast_dtype, dy_dtype;
+    float eps;
+    const void *x, *h, *weight;
+    void *x_out, *y, *y_cast;
+    float *rstd;
+    const void *dy, *dx_out;
+    void *dx, *dh, *d_weight;
+    void *workspace;
+    int64_t workspace_bytes;
+} dsalt_norm_train_args;
+int dsalt_norm_train(const dsalt_norm_train_args *args, void *stream);
+int dsalt_norm_train_bwd(const dsalt_norm_train_args *args, void *stream);
+int64_t dsalt_norm_train_workspace_size(int64_t rows, int32_t d);
+size_t dsalt_norm_train_args_size(void);
+
+/*
  * Differentiable weights of the selected landmarks, forward and backward, from the norms
  * that dsalt_select_hybrid (or dsalt_hybrid_scores) left in its scores workspace.
  * Replaces the differentiable score and weight ops of _train_selectors
