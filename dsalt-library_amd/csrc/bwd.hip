@@ -17,7 +17,7 @@
 //           on MFMA. Computes
 //           Delta = rowsum(O * dO) for its queries and writes dQ, the per-head soft-edge
 //           d_w~, the per-query records of the key-parallel passes and (head 0) the
-//           block's smallest band start, which bounds the query scan of `kv` (workspace).
+//           smallest band start of each 64 queries, which bounds the scan of `kv` (workspace).
 //   lmk_kv  key-parallel over landmark slots: one workgroup per (head, 64 slots, chunk of
 //           512 queries of one sequence); 4 waves = 2 slot groups x 2 query sub-blocks scan
 //           the chunk's queries in 64-query LDS tiles. Writes landmark dK/dV and d_bias
@@ -50,13 +50,31 @@ constexpr int kv_bm(int d) { return 32 * kv_waves(d); }  // keys per band kv wor
 constexpr int kv_qt(int d) { return d == 64 ? 32 : 64; }
 constexpr int kv_stages(int) { return 4; }
 constexpr int kTN = 64;     // queries per lmk_kv tile
-constexpr int kDqW = 2;     // waves per dq workgroup
-constexpr int kDqBM = 64;   // queries per dq workgroup (32 per wave)
+constexpr int kDqW = 4;     // waves per dq workgroup
+constexpr int kDqBM = 32 * kDqW;  // queries per dq workgroup (32 per wave)
 constexpr int kDqBN = 32;   // keys per dq tile
-constexpr int kDqStages = 3;  // dq LDS ring depth
+constexpr int kMinBM = 64;  // queries per smallest-band-start entry (bounds the scan of kv)
+constexpr int kDqStages = 4;  // dq LDS ring depth
 constexpr int kLC = 512;  // queries per lmk_kv chunk (chunks are numbered like query blocks)
 
-enum { kCoreTile = 0, kEdgeTile = 1, kLmkTile = 2 };  // tile kinds of the dq loop phases
+// Tile kinds of the dq loop phases (kDiagTile, kRowTile: initial-value rows, see below).
+enum { kCoreTile = 0, kEdgeTile = 1, kLmkTile = 2, kDiagTile = 3, kRowTile = 4 };
+
+// How the kernels apply the SOFT window edge. kEdgeTab (win_edge <= kEdgeKeys, as the
+// forward's edge rows): at most kEdgeKeys keys of a query are edge keys, so its scores start
+// from a few initial values - minus infinity below the band, the edge bias, nothing in the
+// core, all with minus its LSE - and no band element needs a mask or an edge factor. Wider
+// edges form them per element: as factors while those stay in the fp32 range (kEdgeFast),
+// else one exp per element (kEdgeExact). HARD windows have no edge (kEdgeExact).
+enum { kEdgeExact = 0, kEdgeFast = 1, kEdgeTab = 2 };
+constexpr int kEdgeKeys = 4;
+// dq: a query's row of initial values holds keys lo - 4 .. lo + 7 (read four consecutive keys
+// at a time from a start clamped to lo - 4 .. lo + 4); rows start in 32 different banks
+constexpr int kIniLen = kEdgeKeys + 8;
+__host__ __device__ constexpr int ini_row(int q) { return q * kIniLen + (q >> 3); }
+// dq: the dS of a query's keys lo - 4 .. lo + 7, written like the rows are read; what lies
+// outside lo .. lo + 3 is never read, so that a row's end is the next one's start
+__host__ __device__ constexpr int ds_row(int q) { return q * 8 + (q >> 3); }
 
 // Per-(head, query) record written by dq and streamed by kv next to the Q / dO tiles,
 // field-major ([H][field][T]) so that one field of a 64-query tile is one 256-byte
@@ -74,6 +92,16 @@ enum {
     kRecGClo = 7,    // INT_MAX - max corelo over the query's 32-query group
     kRecFields = 8
 };
+// kEdgeTab: the initial values of a query's scores at keys lo, lo + 1, .. lo + 3 and in the
+// core (kTabLse2 = kTabIni + kEdgeKeys, as kRecLse2). The key-parallel band pass keeps a
+// field of minus infinity before them in LDS: key - lo clamped to -1 .. 4 is the field.
+enum {
+    kTabIni = 0,
+    kTabLse2 = 4,
+    kTabDelta = 5,
+    kTabLo = 6,
+    kTabPmax = 7
+};
 
 struct BwdParams {
     const uint16_t *q, *k, *v, *dout;
@@ -85,7 +113,7 @@ struct BwdParams {
     void *dq, *dk, *dv;  // gradient outputs: fp32 if grad_f32, else the compute dtype
     float *d_bias, *d_w;
     float *ws_qrec;          // per-query records [H][kRecFields][T], written by bwd_dq_kernel
-    int *ws_minlo;           // [n_dqblk]: smallest band start of each dq query block
+    int *ws_minlo;           // smallest band start of each block of kMinBM queries
     float *ws_dwh;           // [T*H] or null
     float *ws_ldk, *ws_ldv;  // landmark dK/dV partials [H][n_lchunk][k_pad][D] or null
     float *ws_ldb;           // landmark d_bias partials [H][n_lchunk][k_pad] or null
@@ -146,13 +174,23 @@ __device__ __forceinline__ void pack_block(const f32x16 &x, uint32_t (&pk)[8]) {
 // The forward's structure: one workgroup = kDqW waves x 32 queries of one (sequence,
 // head); K and V tiles of kDqBN keys stream through a kDqStages-deep LDS ring by direct
 // global->LDS loads (band tiles from the diagonal down, then the gathered landmark
-// tiles). Small workgroups and tiles keep the LDS ring (24 KB at D = 64) and the
-// registers small enough for 3 workgroups per SIMD set at D = 64. Per tile a wave
+// tiles). Four waves share a ring of four stages (32 KB at D = 64), so that with the rows below
+// three workgroups, 12 waves, fit a CU's LDS as they fit its registers (two waves on three
+// stages: 5 workgroups, 10 waves). Per tile a wave
 // computes S^T = K.Q^T and dP^T = V.dO^T (lane = query column), P = 2^(S c + bias - lse2)
 // on admitted pairs, dS = P (dP - Delta), and dQ^T += K^T.dS^T with K read transposed.
-template <typename DT, int D, int MODE, bool EFAST>
+// HARD windows and SOFT windows of at most kEdgeKeys edge keys (kEdgeTab) start S^T from the
+// query's row of initial values and dP^T from -Delta: a band element then takes a
+// product, an exp2 and a product, where the mask took three more operations and an edge
+// element, which with windows that differ from query to query nearly every one is, fourteen
+// and a reciprocal. 9290 tokens x 16 heads x 64, windows 32 - 512: 62.4 -> 60.4 us. Of that 29
+// are the reads of Q, dO, O and the stores (95 MB); the loop is a chain of LDS, MFMA and exp
+// latencies at 2.2 waves per SIMD (VALU 34 %, LDS 39 %, MFMA 17 % busy).
+template <typename DT, int D, int MODE, int EDGE>
 __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(const BwdParams p) {
     typedef typename DT::vec8 vec8;
+    constexpr bool EFAST = EDGE == kEdgeFast, TAB = EDGE == kEdgeTab;
+    constexpr bool ROWS = MODE == kHard || TAB;  // band scores start from per-query rows
     constexpr int NW = kDqW, BM = kDqBM, NT = 64 * NW;
     constexpr int BN = kDqBN, NRB = BN / 32;
     constexpr int KS = D / 16, ND = D / 32;
@@ -165,7 +203,9 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
     __shared__ int s_red[NW][2];
     __shared__ int s_ltmin[DSALT_MAX_K_LMK / BN];
     // SOFT edge factors ec[j] = exp((kEdgeMid - cst_j) / tau) of the element slots j
-    __shared__ __align__(16) float s_ec[16 * NRB];
+    __shared__ __align__(16) float s_ec[EFAST ? 16 * NRB : 4];
+    __shared__ float s_ini[ROWS ? ini_row(BM) : 1];
+    __shared__ float s_ds[TAB ? ds_row(BM) + 8 : 1];
     extern __shared__ int s_dyn[];
     int *s_lpos = s_dyn;                                          // INT_MAX: empty slot
     float *s_lbias = reinterpret_cast<float *>(s_dyn + p.k_pad);  // log2 units
@@ -186,7 +226,6 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
     if (head >= p.n_heads) return;
     int seq, blk, seq_start, seq_len;
     if (!find_block_desc(p.cu, p.num_seqs, p.total_len, rank, p.n_dqblk, BM, lane, seq, blk, seq_start, seq_len)) return;
-    const int target = seq_start / BM + seq + blk;  // the block's find_block id (ws_minlo index)
     const int wq0 = blk * BM + wave * 32;
     const int i = wq0 + ql;
     const bool qvalid = i < seq_len;
@@ -270,6 +309,12 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
     if (qvalid && hh == 0) {
         float *rec = p.ws_qrec + (size_t)head * kRecFields * p.total_len + tok_i;
         const size_t T = (size_t)p.total_len;
+        if constexpr (TAB) {
+            rec[kTabLse2 * T] = -lse2 * p.inv_c2;
+            rec[kTabDelta * T] = -delta;
+            reinterpret_cast<int *>(rec)[kTabLo * T] = INT_MAX - lo;
+            reinterpret_cast<int *>(rec)[kTabPmax * T] = pmax + 1;
+        } else {
         rec[kRecLse2 * T] = -lse2 * p.inv_c2;  // (S + this) * scale_log2 = S scale_log2 - lse2
         rec[kRecDelta * T] = -delta;
         reinterpret_cast<int *>(rec)[kRecLo * T] = INT_MAX - lo;
@@ -278,6 +323,39 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
         rec[kRecWc * T] = wc;
         reinterpret_cast<int *>(rec)[kRecGLo * T] = INT_MAX - wlo;
         reinterpret_cast<int *>(rec)[kRecGClo * T] = INT_MAX - wclo;
+        }
+    }
+    float edw[2] = {0.f, 0.f};
+    if constexpr (ROWS) {
+        // the query's row, raw units: -inf below the band, log2 sigmoid((w~ - d) / tau) for lo
+        // <= key < corelo, 0 in the core, each minus the LSE; the lane pair splits it
+        constexpr int EH = kIniLen / 2;
+        float *row = s_ini + ini_row(wave * 32 + ql);
+        const int ne = corelo - lo;
+#pragma unroll
+        for (int e = 0; e < EH; ++e) {
+            const int x = hh * EH + e - 4;
+            float bias = 0.f;
+            if constexpr (TAB) {
+                float oms;
+                bias = soft_edge_log2(wc, (float)(i - lo - x), p.inv_tau, oms);
+            }
+            const float v = (x < 0 ? -INFINITY : (x < ne ? bias : 0.f) - lse2) * p.inv_c2;
+            row[e + hh * EH] = v;
+            if constexpr (TAB)
+                if (qvalid && x >= 0 && x < kEdgeKeys)
+                    p.ws_qrec[((size_t)head * kRecFields + kTabIni + x) * p.total_len + tok_i] = v;
+        }
+        if constexpr (TAB) {  // d log2 sigmoid / d w~ of the two edge keys whose dS this lane sums
+            float *ds = s_ds + ds_row(wave * 32 + ql) + 4 + 2 * hh;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int x = 2 * hh + e;
+                soft_edge_log2(wc, (float)(i - lo - x), p.inv_tau, edw[e]);
+                edw[e] = x < ne ? edw[e] * p.inv_tau : 0.f;
+                ds[e] = 0.f;  // no tile writes it where the band holds fewer keys
+            }
+        }
     }
     const int wpmax = wave_max_u(qvalid ? pmax : -1);
     const int whi = min(wq0 + 31, seq_len - 1);
@@ -321,10 +399,11 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
         glo = min(glo, s_red[w][0]);
         gpmax = max(gpmax, s_red[w][1]);
     }
-    if (head == 0 && tid == 0) p.ws_minlo[target] = glo;  // bounds the query scan of the kv pass
+    if (head == 0 && tid < BM / kMinBM && blk * BM + tid * kMinBM < seq_len)  // entries numbered as by find_block
+        p.ws_minlo[seq_start / kMinBM + seq + blk * (BM / kMinBM) + tid] = min(s_red[2 * tid][0], s_red[2 * tid + 1][0]);
     const int n_lt = p.k_pad / BN;
     const uint64_t lmask = __ballot(lane < n_lt && s_ltmin[lane < n_lt ? lane : 0] <= gpmax);
-    const int nb = max((ghi - glo) / BN + 1, NSTAGE - 1);
+    const int nb = max((ghi - glo) / BN + 1, std::max(NSTAGE - 1, BM / BN));
     const int nt = nb + __popcll(lmask);
     auto lmk_tile = [&](int t) {
         uint64_t m = lmask;
@@ -385,6 +464,8 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
     const int A0 = i - ghi + BN - 1 - hh * 4, B0 = lo - ghi + BN - 1 - hh * 4;
     const int nA0 = 4 * (A0 >> 3) + min((A0 & 7) + 1, 4);
     const int nB0 = 4 * ((B0 - 1) >> 3) + min(((B0 - 1) & 7) + 1, 4);
+    // key - lo of element 0 of band tile 0 (tile t: minus BN t)
+    const int X0 = -B0;
 
     // ---- tile loop, in phases of one tile kind: band tiles inside every row's core
     // (keep mask only), SOFT band tiles that reach below a row's core start (a suffix of
@@ -392,6 +473,8 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
     // work is one basic block: S^T/dP^T of the lower 32 keys (MFMA), then the masks, P
     // and dS of that half (VALU) under the S^T/dP^T MFMAs of the upper half, then the
     // upper half's VALU work under the dQ^T MFMAs of the lower half.
+    const float *irow = s_ini + ini_row(wave * 32 + ql) + 4;  // entry of key lo
+    float *drow = s_ds + ds_row(wave * 32 + ql) + 4;
     auto tile = [&](int t, auto kind) {
         constexpr int KIND = decltype(kind)::value;
         if (t + NSTAGE - 1 < nt) issue_tile(t + NSTAGE - 1);
@@ -407,8 +490,22 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
 #pragma unroll
             for (int rb = 0; rb < NRB; ++rb) {
                 f32x16 a0, a1;
+                if constexpr (KIND == kDiagTile || KIND == kRowTile) {
+                    const int x0 = X0 - BN * t + 32 * rb;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) a0[r] = a1[r] = 0.f;
+                    for (int g = 0; g < 4; ++g) {
+                        const float *e4 = irow + 8 * g + min(max(x0, -4 - 8 * g), kEdgeKeys - 8 * g);
+                        a0[4 * g + 0] = e4[0];
+                        a0[4 * g + 1] = e4[1];
+                        a0[4 * g + 2] = e4[2];
+                        a0[4 * g + 3] = e4[3];
+                    }
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) a1[r] = -delta;
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) a0[r] = a1[r] = 0.f;
+                }
 #pragma unroll
                 for (int s = 0; s < KS; ++s) {
                     const vec8 ka = bitcast<vec8>(tile_read_row16<D>(ktile, rb * 32 + ql, 2 * s + hh));
@@ -421,7 +518,37 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
             }
             // logits minus lse2 in log2 units with biases, -inf where not admitted
             f32x16 x[NRB];
-            if constexpr (KIND == kLmkTile) {
+            if constexpr (KIND == kDiagTile || KIND == kRowTile) {
+                // P = 2^(S c) and dS = P dP' from accumulators started from the rows and -Delta
+                const int A = i - tb - hh * 4;  // key <= i  <=> cst <= A
+                const int x0 = X0 - BN * t;
+                uint32_t pk[NRB][8];
+#pragma unroll
+                for (int rb = 0; rb < NRB; ++rb)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        float ds4[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int r = g * 4 + e;
+                            float y = sacc[rb][r] * c;
+                            if constexpr (KIND == kDiagTile) y = (rb * 32 + acc_row_const(r) <= A) ? y : -INFINITY;
+                            ds4[e] = fast_exp2(y) * pacc[rb][r];
+                        }
+                        if constexpr (TAB) {  // the edge keys' dS, for d_w~
+                            const int x = x0 + 32 * rb + 8 * g;  // key - lo of the group
+                            if ((uint32_t)(x + 3) < (uint32_t)(kEdgeKeys + 3)) {
+                                drow[x] = ds4[0];
+                                drow[x + 1] = ds4[1];
+                                drow[x + 2] = ds4[2];
+                                drow[x + 3] = ds4[3];
+                            }
+                        }
+                        pk[rb][2 * g] = DT::pack2(ds4[0], ds4[1]);
+                        pk[rb][2 * g + 1] = DT::pack2(ds4[2], ds4[3]);
+                    }
+                dq_mfma(pk, stage);
+            } else if constexpr (KIND == kLmkTile) {
 #pragma unroll
                 for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
@@ -525,8 +652,8 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
                         for (int r = 0; r < 16; ++r) x[rb][r] = keep_if(keep, rb * 16 + r, fmaf(sacc[rb][r], c, -lse2));
                 }
             }
-            if constexpr (KIND != kEdgeTile) ds_dq(x, pacc, stage);
-            if constexpr (KIND != kEdgeTile && NRB == 2) {
+            if constexpr (KIND == kCoreTile || KIND == kLmkTile) ds_dq(x, pacc, stage);
+            if constexpr ((KIND == kCoreTile || KIND == kLmkTile) && NRB == 2) {
                 __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);  // K/V reads, lower half
                 __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);  // S^T/dP^T MFMAs, lower half
                 __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);  // K/V reads, upper half
@@ -554,9 +681,14 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
 
     tile_barrier<(NSTAGE - 2) * LPT>();  // tile 0 landed (later ones may be in flight)
     int t = 0;
-    for (; t < n_core; ++t) tile(t, std::integral_constant<int, kCoreTile>());
-    if constexpr (MODE == kSoft)
+    if constexpr (ROWS) {
+        // only the first BM / BN tiles hold keys after a query of the workgroup
+        for (; t < BM / BN; ++t) tile(t, std::integral_constant<int, kDiagTile>());
+        for (; t < nb; ++t) tile(t, std::integral_constant<int, kRowTile>());
+    } else {
+        for (; t < n_core; ++t) tile(t, std::integral_constant<int, kCoreTile>());
         for (; t < nb; ++t) tile(t, std::integral_constant<int, kEdgeTile>());
+    }
     for (; t < nt; ++t) tile(t, std::integral_constant<int, kLmkTile>());
 
     if (qvalid) {
@@ -569,7 +701,13 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
         store_row<DT, ND>(p.dq, tok_i * p.dq_st + (int64_t)head * p.dq_sh, p.grad_f32, dqacc, mul, hh);
     }
     if (MODE == kSoft && p.ws_dwh) {
-        const float dwt = half_sum(dw) * p.inv_tau;
+        float dwt;
+        if constexpr (TAB) {
+            __builtin_amdgcn_wave_barrier();  // a wave's LDS operations run in order
+            dwt = half_sum(fmaf(drow[2 * hh], edw[0], drow[2 * hh + 1] * edw[1]));
+        } else {
+            dwt = half_sum(dw) * p.inv_tau;
+        }
         if (hh == 0 && qvalid) p.ws_dwh[tok_i * p.n_heads + head] = dwt;
     }
 }
@@ -586,10 +724,17 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
 // halved the workgroups per CU and measured 1.5 us slower at c3). Per 32-query
 // sub-block: S = Q.K^T and dP = dO.V^T (lane = key column, registers = query rows),
 // P = 2^(S c + bias - lse2) on admitted pairs, dS = P (dP - Delta), then dV^T += dO^T.P
-// and dK^T += Q^T.dS with Q and dO read transposed.
-template <typename DT, int D, int MODE, bool LMK, bool EFAST>
+// and dK^T += Q^T.dS with Q and dO read transposed. kEdgeTab band tiles read each score's
+// initial value from the records (a clamped subtraction picks the field; keys of one query
+// are mostly in one field, so that the reads broadcast) and need no mask, edge factor or
+// tile summary: 86 -> 75 us at 9290 tokens x 16 heads x 64; the D = 128 form went to 0.82 of
+// its time (4627 tokens, 16 heads, 4 K/V heads).
+template <typename DT, int D, int MODE, bool LMK, int EDGE>
 __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1) bwd_kv_kernel(const BwdParams p) {
     typedef typename DT::vec8 vec8;
+    constexpr bool EFAST = EDGE == kEdgeFast && !LMK, TAB = EDGE == kEdgeTab;
+    constexpr int kLse2 = TAB ? (int)kTabLse2 : (int)kRecLse2, kDelta = TAB ? (int)kTabDelta : (int)kRecDelta;
+    constexpr int kPmax = TAB ? (int)kTabPmax : (int)kRecPmax;
     constexpr int NW = LMK ? 4 : kv_waves(D), NT = 64 * NW;  // waves, threads
     constexpr int kBM = kv_bm(D);                            // keys per band workgroup
     constexpr int QT = LMK ? kTN : kv_qt(D);                 // queries per tile
@@ -605,7 +750,9 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
     static_assert(kRecFields % (FPI * NW) == 0, "record fields split evenly over the waves");
 
     __shared__ __align__(1024) char s_tiles[NSTAGE][2][TB];  // [stage][Q, dO], row-swizzled
-    __shared__ __align__(16) char s_rec[NSTAGE][kRecFields][RB];
+    // TAB band: one field of -inf before the records' fields
+    constexpr int PRE = TAB && !LMK ? 1 : 0;
+    __shared__ __align__(16) char s_rec_all[NSTAGE][PRE + kRecFields][RB];
     __shared__ int s_misc[8];
     // band pass: one landmark slot's summed dK and dV rows, handed from the whole wave to
     // the key's two lanes
@@ -665,22 +812,25 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
         const int kb = kblk * kBM;
         kw = kb + wave * 32;
         if (kw + ql < seq_len) key = kw + ql;
-        // last dq query block (kDqBM queries; block ids of the sequence start at
-        // seq_start / kDqBM + seq) whose smallest band start reaches this key block
-        const int dqbase = seq_start / kDqBM + seq;
-        const int nbs = (seq_len + kDqBM - 1) / kDqBM;
-        const int own = (kb + kBM - 1) / kDqBM;  // dq block of the key block's last key
+        // last block of kMinBM queries (their ids in the sequence start at
+        // seq_start / kMinBM + seq) whose smallest band start reaches this key block
+        const int dqbase = seq_start / kMinBM + seq;
+        const int nbs = (seq_len + kMinBM - 1) / kMinBM;
+        const int own = (kb + kBM - 1) / kMinBM;  // dq block of the key block's last key
         int last = own;
         for (int b = own + 1 + tid; b < nbs; b += NT)
             if (p.ws_minlo[dqbase + b] <= kb + kBM - 1) last = max(last, b);
         last = wave_max_u(last);
         if (lane == 0) s_misc[wave] = last;
+        if constexpr (PRE == 1)
+            for (int e = tid; e < NSTAGE * QT; e += NT)
+                reinterpret_cast<float *>(&s_rec_all[e / QT][0][0])[e % QT] = -INFINITY * p.inv_c2;
         __syncthreads();
 #pragma unroll
         for (int w = 0; w < NW; ++w) last = max(last, s_misc[w]);
         last = __builtin_amdgcn_readfirstlane(last);  // wave-uniform: it bounds the tile loops
         q_begin = kb;
-        q_end = min(seq_len, (last + 1) * kDqBM);
+        q_end = min(seq_len, (last + 1) * kMinBM);
     } else {
         if (slot < p.k_lmk) {
             const int64_t pp = p.lmk_pos[head * p.lp_sh + seq * p.lp_ss + slot * p.lp_sk];
@@ -735,7 +885,7 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
     const TileLanes<D, kSwzRow, QT, NW> qlanes(wave, lane, qst);
     const TileLanes<D, kSwzRow, QT, NW> dlanes(wave, lane, dst);
     const uint32_t tiles_lds = lds_addr(&s_tiles[0][0][0]);
-    const uint32_t rec_lds = lds_addr(&s_rec[0][0][0]);
+    const uint32_t rec_lds = lds_addr(&s_rec_all[0][0][0]);
     const int ntile = (q_end > q_begin) ? (q_end - q_begin + QT - 1) / QT : 0;
     auto stage_of = [](int t) { return t % NSTAGE; };  // t >= 0, wave-uniform
     auto issue_tile = [&](int t) {
@@ -753,12 +903,20 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
             const int f = f0 + lane / QT;
             const uint32_t off = (q < seq_len) ? (uint32_t)(((size_t)f * p.total_len + seq_start + q) * 4) : 0xFFFFFF00u;
             asm volatile("buffer_load_dword %0, %1, 0 offen lds" ::"v"(off), "s"(uniform_rsrc(rrs)),
-                         "{m0}"(__builtin_amdgcn_readfirstlane(rec_lds + (st * kRecFields + f0) * RB))
+                         "{m0}"(__builtin_amdgcn_readfirstlane(rec_lds + (st * (PRE + kRecFields) + PRE + f0) * RB))
                          : "memory");
         }
     };
-    auto rec_i = [&](int st, int f, int q) -> const int * { return reinterpret_cast<const int *>(&s_rec[st][f][q * 4]); };
-    auto rec_f = [&](int st, int f, int q) -> const float * { return reinterpret_cast<const float *>(&s_rec[st][f][q * 4]); };
+    // lo(q) <= key <=> rec lo >= nkey. (Lanes without a key form a column that is not stored.)
+    const int nkey = INT_MAX - (kvalid ? key : INT_MAX / 2);
+    auto rec_i = [&](int st, int f, int q) -> const int * { return reinterpret_cast<const int *>(&s_rec_all[st][PRE + f][q * 4]); };
+    auto rec_f = [&](int st, int f, int q) -> const float * { return reinterpret_cast<const float *>(&s_rec_all[st][PRE + f][q * 4]); };
+    // TAB: initial value of the scores of query q (of the tile) at this lane's key: o = the query's
+    // kTabLo record
+    auto rec_ini = [&](int st, int q, int o) -> float {
+        const int x = min(max(o - nkey, -1), kEdgeKeys);  // key - lo
+        return *reinterpret_cast<const float *>(&s_rec_all[st][0][0] + (PRE + x) * RB + q * 4);
+    };
 
     f32x16 dk[ND], dv[ND];
 #pragma unroll
@@ -767,7 +925,6 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
         for (int r = 0; r < 16; ++r) dk[d][r] = dv[d][r] = 0.f;
     float dbias = 0.f;
     const float c = p.scale_log2;
-    const int nkey = INT_MAX - (kvalid ? key : INT_MAX / 2);  // lo(q) <= key <=> rec lo >= nkey
 
 #pragma unroll
     for (int t = 0; t < NSTAGE - 1; ++t)
@@ -850,9 +1007,23 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
         }
     };
     // S and dP (32 queries x 32 keys) of sub-block sb: lane = key column, registers = query rows
-    auto sdp_mfma = [&](const char *qtile, const char *dtile, int sb, f32x16 &sacc, f32x16 &pacc) {
+    auto sdp_mfma = [&](int st, const char *qtile, const char *dtile, int sb, f32x16 &sacc, f32x16 &pacc) {
+        if constexpr (TAB) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sacc[r] = pacc[r] = 0.f;
+            for (int g = 0; g < 4; ++g) {
+                const int qi = sb * 32 + g * 8 + hh * 4;
+                const int4 o = *reinterpret_cast<const int4 *>(rec_i(st, kTabLo, qi));
+                const float4 d4 = *reinterpret_cast<const float4 *>(rec_f(st, kTabDelta, qi));
+                sacc[4 * g] = rec_ini(st, qi, o.x);
+                sacc[4 * g + 1] = rec_ini(st, qi + 1, o.y);
+                sacc[4 * g + 2] = rec_ini(st, qi + 2, o.z);
+                sacc[4 * g + 3] = rec_ini(st, qi + 3, o.w);
+                pacc[4 * g] = d4.x; pacc[4 * g + 1] = d4.y; pacc[4 * g + 2] = d4.z; pacc[4 * g + 3] = d4.w;
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sacc[r] = pacc[r] = 0.f;
+        }
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
             const vec8 qa = bitcast<vec8>(tile_read_row16<D>(qtile, sb * 32 + ql, 2 * s + hh));
@@ -896,7 +1067,7 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
             // lo(q) <= key <=> rec lo >= nkey; records hold INT_MAX - lo >= 0 (0 when out of
             // range), so one unsigned compare against ~0 admits nothing
             const uint32_t nk = (kvalid & live) ? (uint32_t)nkey : 0xFFFFFFFFu;
-            if constexpr (MODE == kSoft && !EFAST) {
+            if constexpr (MODE == kSoft && EDGE == kEdgeExact) {
                 const int gmax_clo = INT_MAX - *rec_i(st, kRecGClo, 0);
                 if (live && gmax_clo > wkmin) {
 #pragma unroll
@@ -919,8 +1090,11 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int qi = g * 8 + hh * 4;
-                const int4 o4 = *reinterpret_cast<const int4 *>(rec_i(st, kRecLo, qi));
-                const uint32_t oa[4] = {(uint32_t)o4.x, (uint32_t)o4.y, (uint32_t)o4.z, (uint32_t)o4.w};
+                uint32_t oa[4] = {0, 0, 0, 0};
+                if constexpr (!TAB) {
+                    const int4 o4 = *reinterpret_cast<const int4 *>(rec_i(st, kRecLo, qi));
+                    oa[0] = o4.x; oa[1] = o4.y; oa[2] = o4.z; oa[3] = o4.w;
+                }
                 int ca[4] = {0, 0, 0, 0};
                 float ra[4] = {0.f, 0.f, 0.f, 0.f};
                 if constexpr (WE) {
@@ -933,7 +1107,7 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int r = g * 4 + e;
-                    bool ok = oa[e] >= nk;
+                    bool ok = TAB || oa[e] >= nk;  // TAB: the initial value admits
                     if constexpr (DIAG) ok = ok & (acc_row_const(r) >= Cj);
                     // masked before the exp (exp2(-inf) = 0): a select, never a branch
                     float pr = fast_exp2(ok ? sc[r] * c : -INFINITY);
@@ -956,6 +1130,16 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
         // queries, plus the products of tile half `half` (0: Q, 1: dO) with the lane's key
         // row `kr` (kreg or vreg): lane = key column, registers = query rows
         auto rec_mfma = [&](int st, int f, int half, const vec8 (&kr)[KS], f32x16 &acc) {
+            if (TAB && f == kLse2) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const int4 o = *reinterpret_cast<const int4 *>(rec_i(st, kTabLo, g * 8 + hh * 4));
+                    acc[4 * g] = rec_ini(st, g * 8 + hh * 4, o.x);
+                    acc[4 * g + 1] = rec_ini(st, g * 8 + hh * 4 + 1, o.y);
+                    acc[4 * g + 2] = rec_ini(st, g * 8 + hh * 4 + 2, o.z);
+                    acc[4 * g + 3] = rec_ini(st, g * 8 + hh * 4 + 3, o.w);
+                }
+            } else
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const float4 v = *reinterpret_cast<const float4 *>(rec_f(st, f, g * 8 + hh * 4));
@@ -975,14 +1159,14 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
             if (t + NSTAGE - 1 < ntile) issue_tile(t + NSTAGE - 1);
             const int st = stage_of(t);
             const int qsb = q_begin + t * QT;
-            const bool live = tile_live(st, qsb);
+            const bool live = TAB || tile_live(st, qsb);
             uint32_t pkp[8], pks[8];
             f32x16 pc;
-            rec_mfma(st, kRecDelta, 1, vreg, pc);
+            rec_mfma(st, kDelta, 1, vreg, pc);
             // S of tile t+1 (landed; past the last tile a stale stage, ignored)
-            rec_mfma(stage_of(t + 1), kRecLse2, 0, kreg, sn);
+            rec_mfma(stage_of(t + 1), kLse2, 0, kreg, sn);
             p_ds1(st, qsb, live, sc, pc, t & 1, we, diag, pkp, pks);
-            if constexpr (!(MODE == kSoft && !EFAST)) {
+            if constexpr (MODE == kHard || EFAST) {
                 __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);  // dP initial values, dO operands
 #pragma unroll
                 for (int m = 0; m < 4; ++m) {
@@ -1007,7 +1191,7 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
         if (ntile >= NSTAGE - 1) tile_barrier<(NSTAGE - 3) * LPT>();
         else tile_barrier<0>();
         f32x16 sA, sB;
-        rec_mfma(0, kRecLse2, 0, kreg, sA);
+        rec_mfma(0, kLse2, 0, kreg, sA);
         put_rq(0);
         using yes = std::true_type;
         using no = std::false_type;
@@ -1083,6 +1267,11 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
 #pragma unroll
             for (int sb = 0; sb < NSB; ++sb) {
                 const int qsb = q0 + sb * 32;
+                if constexpr (TAB) {  // the scores' initial values admit
+                    live[sb] = any = true;
+                    edge[sb] = false;
+                    continue;
+                }
                 const int gmin_lo = INT_MAX - *rec_i(st, kRecGLo, sb * 32);
                 const int gmax_clo = INT_MAX - *rec_i(st, kRecGClo, sb * 32);
                 live[sb] = !((qsb >= q_end) || (qsb + 31 < kw) || (gmin_lo > wkmax));
@@ -1092,8 +1281,8 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
             if (any) {
                 f32x16 sacc[NSB], pacc[NSB];
 #pragma unroll
-                for (int sb = 0; sb < NSB; ++sb) sdp_mfma(qtile, dtile, sb, sacc[sb], pacc[sb]);
-                if (MODE == kSoft && !EFAST) {
+                for (int sb = 0; sb < NSB; ++sb) sdp_mfma(st, qtile, dtile, sb, sacc[sb], pacc[sb]);
+                if (MODE == kSoft && EDGE == kEdgeExact) {
 #pragma unroll
                     for (int sb = 0; sb < NSB; ++sb) {
                         if (!edge[sb]) continue;
@@ -1138,6 +1327,20 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
                         const int qi = sb * 32 + g * 8 + hh * 4;
+                        if constexpr (TAB) {
+                            float pr4[4], ds4[4];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const int r = g * 4 + e;
+                                pr4[e] = fast_exp2(acc_row_const(r) >= Cj ? sacc[sb][r] * c : -INFINITY);
+                                ds4[e] = pr4[e] * pacc[sb][r];
+                            }
+                            pkp[sb][g * 2] = DT::pack2(pr4[0], pr4[1]);
+                            pkp[sb][g * 2 + 1] = DT::pack2(pr4[2], pr4[3]);
+                            pks[sb][g * 2] = DT::pack2(ds4[0], ds4[1]);
+                            pks[sb][g * 2 + 1] = DT::pack2(ds4[2], ds4[3]);
+                            continue;
+                        }
                         float4 l4 = *reinterpret_cast<const float4 *>(rec_f(st, kRecLse2, qi));
                         float4 d4 = *reinterpret_cast<const float4 *>(rec_f(st, kRecDelta, qi));
                         int4 o4 = *reinterpret_cast<const int4 *>(rec_i(st, kRecLo, qi));
@@ -1215,15 +1418,13 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
             const char *qtile = s_tiles[st][0];
             const char *dtile = s_tiles[st][1];
     #pragma unroll
-            for (int sbi = 0; sbi < (LMK ? 1 : 2); ++sbi) {
-                const int sb = LMK ? sbw : sbi;
+            for (int sbi = 0; sbi < 1; ++sbi) {
+                const int sb = sbw;
                 const int qsb = q_begin + t * QT + sb * 32;  // first query of the sub-block
                 // group summaries of the sub-block (wave-uniform LDS reads)
-                const int gmin_lo = INT_MAX - *rec_i(st, kRecGLo, sb * 32);
-                const int gmax_clo = INT_MAX - *rec_i(st, kRecGClo, sb * 32);
                 bool skip = qsb >= q_end;
-                if (!LMK) skip = skip || (qsb + 31 < kw) || (gmin_lo > wkmax);
-                else skip = skip || (gmax_clo <= wkmin);  // pmax < corelo
+                if constexpr (TAB) skip = skip || __ballot(*rec_i(st, kTabPmax, sb * 32 + ql) > wkmin) == 0;
+                else skip = skip || (INT_MAX - *rec_i(st, kRecGClo, sb * 32) <= wkmin);  // pmax < corelo
                 if (skip) continue;
     
                 // S and dP (32 queries x 32 keys): lane = key column, registers = query rows
@@ -1238,49 +1439,24 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
                     pacc = DT::mfma(da, vreg[s], pacc);
                 }
                 // register r holds query q = qsb + hh*4 + acc_row_const(r) of the lane's key
-                const int Cj = (kvalid ? key : INT_MAX / 2) - qsb - hh * 4;  // q >= key <=> cst >= Cj
-                const bool need_hi = LMK || (qsb < wkmax);
-                const bool need_lo = LMK || (gmax_clo > wkmin);
-                const bool need_edge = (MODE == kSoft) && !LMK && need_lo;
                 uint32_t pkp[8], pks[8], plo[8], slo[8];
     #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const int qi = sb * 32 + g * 8 + hh * 4;
-                    const float4 l4 = *reinterpret_cast<const float4 *>(rec_f(st, kRecLse2, qi));
-                    const float4 d4 = *reinterpret_cast<const float4 *>(rec_f(st, kRecDelta, qi));
-                    const int4 o4 = *reinterpret_cast<const int4 *>(rec_i(st, LMK ? kRecPmax : kRecLo, qi));
+                    const float4 l4 = *reinterpret_cast<const float4 *>(rec_f(st, kLse2, qi));
+                    const float4 d4 = *reinterpret_cast<const float4 *>(rec_f(st, kDelta, qi));
+                    const int4 o4 = *reinterpret_cast<const int4 *>(rec_i(st, kPmax, qi));
                     const float la[4] = {l4.x, l4.y, l4.z, l4.w};
                     const float da[4] = {d4.x, d4.y, d4.z, d4.w};
                     const int oa[4] = {o4.x, o4.y, o4.z, o4.w};
-                    int ca[4] = {0, 0, 0, 0};
-                    float wa[4] = {0.f, 0.f, 0.f, 0.f};
-                    if (need_edge) {
-                        const int4 c4 = *reinterpret_cast<const int4 *>(rec_i(st, kRecClo, qi));
-                        const float4 w4 = *reinterpret_cast<const float4 *>(rec_f(st, kRecWc, qi));
-                        ca[0] = c4.x; ca[1] = c4.y; ca[2] = c4.z; ca[3] = c4.w;
-                        wa[0] = w4.x; wa[1] = w4.y; wa[2] = w4.z; wa[3] = w4.w;
-                    }
                     float pr4[4], ds4[4];
     #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const int r = g * 4 + e;
-                        const int cst = acc_row_const(r);
-                        float pr;
-                        if (LMK) {
-                            // landmark admitted: key <= pmax(q) <=> key < rec pmax (key = INT_MAX when empty)
-                            pr = (key < oa[e]) ? fast_exp2(fmaf(sacc[r] + la[e], c, kbias2)) : 0.f;
-                        } else {
-                            const bool ok = (!need_hi | (cst >= Cj)) & (!need_lo | (oa[e] >= nkey)) & kvalid;
-                            float x = (sacc[r] + la[e]) * c;
-                            if (MODE == kSoft && need_edge) {
-                                float oms;
-                                const float edge = soft_edge_log2(wa[e], (float)(cst - Cj), p.inv_tau, oms);
-                                x += (nkey > ca[e]) ? edge : 0.f;  // key < corelo(q)
-                            }
-                            pr = ok ? fast_exp2(x) : 0.f;
-                        }
+                        // landmark admitted: key <= pmax(q) <=> key < rec pmax (key = INT_MAX when empty)
+                        const float pr = (key < oa[e]) ? fast_exp2(fmaf(sacc[r] + la[e], c, kbias2)) : 0.f;
                         const float ds = pr * (pacc[r] + da[e]);
-                        if (LMK) dbias += ds;
+                        dbias += ds;
                         pr4[e] = pr;
                         ds4[e] = ds;
                     }
@@ -1402,7 +1578,7 @@ WsLayout ws_layout(int T, int S, int H, int D, int k) {
     L.qrec = off;
     off += al((size_t)H * kRecFields * T * 4);
     L.minlo = off;
-    off += al((size_t)block_upper_bound(T, S, kDqBM) * 4);
+    off += al((size_t)block_upper_bound(T, S, kMinBM) * 4);
     L.dwh = off;
     off += al((size_t)T * H * 4);
     const size_t kp = (size_t)((k + 63) / 64 * 64);
@@ -1425,29 +1601,32 @@ template <typename DT, int D, int MODE>
 hipError_t launch_typed(const BwdParams &p, hipStream_t stream) {
     // dq writes the per-query records that the key-parallel passes stream
     const size_t dyn = (size_t)p.k_pad * (2 * sizeof(int) + sizeof(float));
-    bool efast = false;
-    if constexpr (MODE == kSoft) efast = dq_edge_fast(p);
-    if (efast)  // instantiated for SOFT only
-        hipLaunchKernelGGL((bwd_dq_kernel<DT, D, MODE, MODE == kSoft>), dim3(p.grid_dq), dim3(64 * kDqW), dyn, stream, p);
-    else
-        hipLaunchKernelGGL((bwd_dq_kernel<DT, D, MODE, false>), dim3(p.grid_dq), dim3(64 * kDqW), dyn, stream, p);
-    if (p.k_lmk > 0)
-        hipLaunchKernelGGL((bwd_kv_kernel<DT, D, MODE, true, false>), dim3(p.n_heads * p.n_lgrp * p.n_lchunk), dim3(256),
-                           0, stream, p);
     // the band pass also sums the landmark partials: each landmark key's dK/dV in its
     // prologue, d_bias in H x S workgroups appended to its grid
     const int grid_kv = p.grid_q + ((p.k_lmk > 0 && p.d_bias) ? p.n_heads * p.num_seqs : 0);
-    // the factored edge path of the band dK/dV kernel exists at D = 64 only (at D = 128 its
-    // second tile loop does not fit the scalar registers)
-    constexpr bool kKvFast = MODE == kSoft && D == 64;
-    bool kv_fast = false;
-    if constexpr (kKvFast) kv_fast = kv_edge_fast(p);
-    if (kv_fast)
-        hipLaunchKernelGGL((bwd_kv_kernel<DT, D, MODE, false, kKvFast>), dim3(grid_kv), dim3(64 * kv_waves(D)), 0,
-                           stream, p);
-    else
-        hipLaunchKernelGGL((bwd_kv_kernel<DT, D, MODE, false, false>), dim3(grid_kv), dim3(64 * kv_waves(D)), 0,
-                           stream, p);
+    const auto run = [&](auto dq_edge, auto lmk_edge, auto kv_edge) {
+        constexpr int DQ = decltype(dq_edge)::value, LM = decltype(lmk_edge)::value, KV = decltype(kv_edge)::value;
+        hipLaunchKernelGGL((bwd_dq_kernel<DT, D, MODE, DQ>), dim3(p.grid_dq), dim3(64 * kDqW), dyn, stream, p);
+        if (p.k_lmk > 0)
+            hipLaunchKernelGGL((bwd_kv_kernel<DT, D, MODE, true, LM>), dim3(p.n_heads * p.n_lgrp * p.n_lchunk), dim3(256),
+                               0, stream, p);
+        hipLaunchKernelGGL((bwd_kv_kernel<DT, D, MODE, false, KV>), dim3(grid_kv), dim3(64 * kv_waves(D)), 0, stream, p);
+    };
+    using exact = std::integral_constant<int, kEdgeExact>;
+    using fast = std::integral_constant<int, kEdgeFast>;
+    using tab = std::integral_constant<int, kEdgeTab>;
+    if constexpr (MODE == kHard) {
+        run(exact(), exact(), exact());
+    } else if (p.win_edge <= (float)kEdgeKeys) {
+        run(tab(), tab(), tab());
+    } else {
+        // the factored edge path of the band dK/dV kernel exists at D = 64 only (at D = 128 its
+        // second tile loop does not fit the scalar registers)
+        using kv_fast = std::conditional_t<D == 64, fast, exact>;
+        if (kv_edge_fast(p)) run(fast(), exact(), kv_fast());  // implies dq_edge_fast
+        else if (dq_edge_fast(p)) run(fast(), exact(), exact());
+        else run(exact(), exact(), exact());
+    }
     return hipGetLastError();
 }
 
