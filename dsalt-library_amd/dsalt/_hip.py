@@ -208,6 +208,10 @@ SELECT_SPLIT_MIN = 4096  # longer sequences can be selected chunk-wise
 
 _lib = None
 
+# torch's accessor of the current stream's raw handle, without a Stream object around it
+_current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
+
 
 def lib() -> ctypes.CDLL:
     """Load libdsalt_hip.so once; raise DsaltError when it has not been built."""
@@ -316,7 +320,9 @@ def require_gpu(*tensors: torch.Tensor) -> torch.device:
 
 
 def stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The raw handle of the current stream of `device` (read on every launch)."""
+    index = device.index
+    return _current_raw_stream(torch.cuda.current_device() if index is None else index)
 
 
 def compute_dtype(dtype: torch.dtype) -> torch.dtype:
@@ -346,6 +352,8 @@ def rope_tables(cos: torch.Tensor, sin: torch.Tensor):
     hit = _ROPE_TABLES.get(key)
     if hit is None:
         c32, s32 = cos.to(torch.float32).contiguous(), sin.to(torch.float32).contiguous()
+        if c32.is_cuda and torch.cuda.is_current_stream_capturing():
+            return c32, s32, False  # the check below cannot synchronise here: whole rows are read
         h = c32.shape[-1] // 2
         half = c32.dim() == 2 and bool(torch.equal(c32[:, :h], c32[:, h:])) and bool(torch.equal(s32[:, :h], s32[:, h:]))
         if len(_ROPE_TABLES) > 64:

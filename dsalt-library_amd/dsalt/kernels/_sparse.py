@@ -14,6 +14,13 @@ import math
 import torch
 
 from .. import _hip
+from ._block_train import eager
+
+
+def no_graph(*tensors) -> bool:
+    """Whether a call on these tensors records nothing: no autograd and nothing else that looks
+    at the autograd function (tracing, functorch transforms, forward mode, subclasses)."""
+    return not torch.is_grad_enabled() and eager(*(t for t in tensors if t is not None))
 
 
 def _forward(ctx, mode: int, q, k, v, lmk_pos, lmk_bias, w, cu_seqlens, tau_win, win_edge,
@@ -25,6 +32,11 @@ def _forward(ctx, mode: int, q, k, v, lmk_pos, lmk_bias, w, cu_seqlens, tau_win,
         raise _hip.DsaltError(f"q must be packed [T, H, D], got {tuple(q.shape)}")
     scale = 1.0 / math.sqrt(q.shape[-1])
     dt = _hip.compute_dtype(q.dtype)
+    if ctx is None:  # nothing is recorded or saved
+        has_lmk = lmk_pos is not None and lmk_pos.shape[-1] > 0
+        return _hip.fwd(mode, _hip.as_kernel_operand(q, dt), _hip.as_kernel_operand(k, dt), _hip.as_kernel_operand(v, dt),
+                        w, lmk_pos if has_lmk else None, lmk_bias if has_lmk else None, cu_seqlens, scale, tau_win,
+                        win_edge, out_dtype=torch.float32 if out_f32 else None, rope=rope)[0]
     q_c = _hip.as_kernel_operand(q.detach(), dt)
     k_c = _hip.as_kernel_operand(k.detach(), dt)
     v_c = _hip.as_kernel_operand(v.detach(), dt)
@@ -83,4 +95,6 @@ def sparse_attention(mode: int, q, k, v, lmk_pos, lmk_bias, w, cu_seqlens,
     """Differentiable DSALT attention returning O [T, H, D] in the compute dtype. With
     ``rope = (cos, sin)`` q is the un-rotated query and the kernel rotates it on load
     (forward only; k must be rotated already)."""
+    if no_graph(q, k, v, lmk_pos, lmk_bias, w, cu_seqlens):
+        return _forward(None, mode, q, k, v, lmk_pos, lmk_bias, w, cu_seqlens, tau_win, win_edge, rope=rope)
     return _SparseAttention.apply(mode, q, k, v, lmk_pos, lmk_bias, w, cu_seqlens, tau_win, win_edge, rope)

@@ -12,6 +12,8 @@ Semantics (dsalt_triton_attn.py:69-169): query i of a sequence attends to keys
 """
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from .. import _hip
@@ -41,8 +43,18 @@ class DSALTAttentionFunction(torch.autograd.Function):
 
 
 def _dynamo_opaque(fn):
+    """fn as a call that torch.compile does not trace into; outside of it, fn itself (the
+    disabled wrapper's frame switch costs microseconds on every call)."""
     disable = getattr(getattr(torch, "_dynamo", None), "disable", None)
-    return disable(fn) if disable is not None else fn
+    if disable is None:
+        return fn
+    opaque = disable(fn)
+
+    @functools.wraps(fn)
+    def call(*args, **kwargs):
+        return opaque(*args, **kwargs) if torch.compiler.is_compiling() else fn(*args, **kwargs)
+
+    return call
 
 
 @_dynamo_opaque
@@ -56,4 +68,7 @@ def dsalt_triton_attention(
     cu_seqlens: torch.Tensor,
 ) -> torch.Tensor:
     """HARD DSALT attention over packed ``[T, H, D]`` q/k/v; returns fp32 ``[T, H, D]``."""
+    if _sparse.no_graph(q, k, v, lmk_indices, lmk_bias, w_sizes, cu_seqlens):
+        return _sparse._forward(None, _hip.MODE_HARD, q, k, v, lmk_indices, lmk_bias, w_sizes, cu_seqlens, 1.0, 4.0,
+                                out_f32=True)
     return DSALTAttentionFunction.apply(q, k, v, lmk_indices, lmk_bias, w_sizes, cu_seqlens)

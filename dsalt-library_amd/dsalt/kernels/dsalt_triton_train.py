@@ -42,5 +42,8 @@ def dsalt_triton_train_attention(q, k, v, lmk_pos, lmk_logw, w_cont, cu_seqlens,
                                  tau_win=1.0, win_edge=4.0, n_max=256, cu_list=None):
     """Differentiable SOFT DSALT attention; returns fp32 ``[T, H, D]``. ``lmk_logw``
     receives d_logw and ``w_cont`` receives d_w~ (summed over heads)."""
+    if _sparse.no_graph(q, k, v, lmk_pos, lmk_logw, w_cont, cu_seqlens):
+        return _sparse._forward(None, _hip.MODE_SOFT, q, k, v, lmk_pos, lmk_logw, w_cont, cu_seqlens, float(tau_win),
+                                float(win_edge), out_f32=True)
     return DSALTTrainFunction.apply(q, k, v, lmk_pos, lmk_logw, w_cont, cu_seqlens,
                                     tau_win, win_edge, n_max, cu_list)

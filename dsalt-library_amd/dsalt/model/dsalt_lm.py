@@ -117,7 +117,9 @@ class DSALTLMHeadModel(nn.Module):
         if max_seqlen is None:
             max_seqlen = input_ids.shape[-1]
         x = self._to_autocast_dtype(self.embed_dropout(self.embed_tokens(input_ids)))
-        cu_list = None if cu_seqlens is None else cu_seqlens.detach().cpu().tolist()
+        cu_list = None
+        if cu_seqlens is not None and not self._device_packing(cu_seqlens, x):
+            cu_list = cu_seqlens.detach().cpu().tolist()
         if labels is None and self._norms_fusable(x):
             # inference: each residual add runs in the pass of the norm that follows it
             delta = None
@@ -138,6 +140,13 @@ class DSALTLMHeadModel(nn.Module):
         loss = _chunked_cross_entropy(x.reshape(-1, self.d_model), self.lm_head.weight,
                                       labels.reshape(-1).long(), self.lm_head_chunk_size)
         return {"loss": loss + self.aux_loss_weight * aux, "logits": None, "aux_loss": aux.detach()}
+
+    def _device_packing(self, cu_seqlens: torch.Tensor, x: torch.Tensor) -> bool:
+        """Whether the layers need no host copy of cu_seqlens (a synchronisation): batches that no
+        selection splits, without the ``_last_P`` diagnostic, on the HIP score route."""
+        return (cu_seqlens.is_cuda and x.dim() == 2 and x.shape[0] <= _hip.SELECT_SPLIT_MIN
+                and all((self.training or not getattr(layer.attn, "_collect_last_P", True))
+                        and getattr(layer.attn, "_hip_scores", False) for layer in self.layers))
 
     def _norms_fusable(self, x: torch.Tensor) -> bool:
         """Whether every residual add and norm of the forward can run as dsalt_add_rms_norm

@@ -45,14 +45,19 @@ from ..kernels._block_train import autocast_dtype, eager, plain
 from ..kernels._lmk_weights import landmark_weights
 from ..kernels._module_attention import module_attention
 from ..kernels._sparse import sparse_attention
+from ..kernels.dsalt_triton_attn import _dynamo_opaque
 from ..kernels.landmark_tokens_ker import hybrid_scores_from_v, hybrid_scores_per_head
 from ..kernels.selectors import _compute_landmark_indices, _landmarks_and_windows
 from ..kernels.window_utils import apply_rotary_emb_packed, build_rope_cache, rotate_packed
 
 
-def _dynamo_opaque(fn):
-    disable = getattr(getattr(torch, "_dynamo", None), "disable", None)
-    return disable(fn) if disable is not None else fn
+def _longest(cu_list: list | None, total_len: int) -> int | None:
+    """A bound on the sequence lengths for the selection: the longest of the host's list of
+    boundaries, without it the whole batch where that is short enough not to be selected
+    chunk-wise, else None (unknown)."""
+    if cu_list is not None:
+        return max((b - a for a, b in zip(cu_list[:-1], cu_list[1:])), default=0)
+    return total_len if total_len <= _hip.SELECT_SPLIT_MIN else None
 
 
 class DSALTAttention(nn.Module):
@@ -303,11 +308,11 @@ class DSALTAttention(nn.Module):
             return False
         if not (self._fused_selector and self._hip_scores and self._fuse_qkv and all(type(m) is nn.Linear for m in lin)):
             return False
-        if not plain(*lin) or not eager(*(p for m in lin for p in m.parameters())):
+        ps = [m.weight for m in lin] + [m.bias for m in lin if m.bias is not None]
+        if not plain(*lin) or not eager(*ps):
             return False
         if any(m.bias is not None for m in lin[:3]) or x.dim() != 2 or x.shape[0] == 0 or x.shape[1] != self.d_model:
             return False
-        ps = [m.weight for m in lin] + ([] if self.win_gate.bias is None else [self.win_gate.bias])
         if any(p.dtype != x.dtype or p.device != x.device or not p.is_contiguous() for p in ps):
             return False
         if self.alpha_w.device != x.device or self.alpha_w.shape != (self.n_heads,):
@@ -379,7 +384,7 @@ class DSALTAttention(nn.Module):
         w_cont = self._window_continuous(x)
         alpha = self._alpha()
         if self._hip_weights(x, v):
-            max_len = None if cu_list is None else max((b - a for a, b in zip(cu_list[:-1], cu_list[1:])), default=0)
+            max_len = _longest(cu_list, total_len)
             v, lmk_logw, lmk_pos, w_disc = landmark_weights(x, v, alpha, w_cont, cu_seqlens, self.k_lmk, max_len,
                                                             self.tau_lmk)
             self._last_selection = (w_disc, lmk_pos)
@@ -411,7 +416,7 @@ class DSALTAttention(nn.Module):
         _hip.require_gpu(x, cu_seqlens)
         if self.training and rope_cs is None and self._one_function(x):
             self._last_P = None
-            max_len = None if cu_list is None else max((b - a for a, b in zip(cu_list[:-1], cu_list[1:])), default=0)
+            max_len = _longest(cu_list, total_len)
             out, lmk_pos, _, w_disc = self._attend(x, cu_seqlens, self.k_lmk, max_len, x_cast=x_cast)
             self._last_selection = (w_disc, lmk_pos)
             return (self._apply_out_proj(out.reshape(total_len, self.d_model)),
@@ -477,8 +482,7 @@ class DSALTAttention(nn.Module):
             # two launches: the norms pass (which also rotates k), then the selection,
             # which forms the scores, the windows and the top-k
             with torch.no_grad():
-                max_len = None if cu_list is None else max((b - a for a, b in zip(cu_list[:-1], cu_list[1:])),
-                                                           default=0)
+                max_len = _longest(cu_list, total_len)
                 w_sizes, lmk_indices, k = _hip.select_hybrid(
                     x.detach(), v_sel.detach(), alpha.detach().float(), self.n_heads, w_cont, cu_seqlens, self.k_lmk,
                     max_seqlen=max_len, gate=gate, rope_k=(k, *self._rope_tables(), cu_seqlens),
