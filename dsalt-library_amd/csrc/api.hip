@@ -632,6 +632,21 @@ int dsalt_norm_train_bwd(const dsalt_norm_train_args *args, void *stream) {
     return DSALT_OK;
 }
 
+int dsalt_group_sum(const float *dk_heads, const float *dv_heads, void *dk, void *dv, int64_t rows, int32_t rep, int32_t d,
+                    int32_t dtype, void *stream) {
+    if (rows < 0 || rep < 1 || d < 4 || d % 4 || d > (1 << 20))
+        return fail(DSALT_ERR_INVALID, "rows >= 0, rep >= 1, d a multiple of 4 (got %lld, %d, %d)", (long long)rows, rep, d);
+    if (!float_dtype(dtype)) return fail(DSALT_ERR_INVALID, "dtype %d is not a float dtype", dtype);
+    if (rows > ((int64_t)1 << 31) / d * 256) return fail(DSALT_ERR_UNSUPPORTED, "rows * d is too large");
+    if (rows == 0) return DSALT_OK;
+    if (!dk_heads || !dv_heads || !dk || !dv) return fail(DSALT_ERR_INVALID, "pointers must be non-NULL");
+    if (!aligned(dk_heads, 16) || !aligned(dv_heads, 16) || !aligned(dk, 16) || !aligned(dv, 16))
+        return fail(DSALT_ERR_INVALID, "pointers must be 16-byte aligned");
+    hipError_t e = dsalt::launch_group_sum(dk_heads, dv_heads, dk, dv, rows, rep, d, dtype, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(DSALT_ERR_LAUNCH, "dsalt_group_sum launch failed: %s", hipGetErrorString(e));
+    return DSALT_OK;
+}
+
 int64_t dsalt_norm_train_workspace_size(int64_t rows, int32_t d) {
     return rows <= 0 || d <= 0 ? 0 : dsalt::norm_train_workspace_bytes(rows, d);
 }
@@ -737,15 +752,16 @@ int dsalt_bwd_rope(const dsalt_bwd_args *a, const dsalt_rope_tables *r, void *st
     int rc = dsalt_bwd_check(a);
     if (rc) return rc;
     if (r) {
-        if (a->mode == DSALT_MODE_DENSE && a->head_dim != 64)
+        if (r->cos && a->mode == DSALT_MODE_DENSE && a->head_dim != 64)
             return fail(DSALT_ERR_UNSUPPORTED, "DSALT_MODE_DENSE un-rotates its gradients at head_dim 64 only (got %d)",
                         a->head_dim);
-        if (!r->cos || !r->sin || !aligned(r->cos, 16) || !aligned(r->sin, 16) || r->rows < 1 ||
-            r->stride < a->head_dim || r->stride % 4)
+        const bool rotate = r->cos || r->sin;
+        if (rotate && (!r->cos || !r->sin || !aligned(r->cos, 16) || !aligned(r->sin, 16) || r->rows < 1 ||
+                       r->stride < a->head_dim || r->stride % 4))
             return fail(DSALT_ERR_INVALID,
                         "RoPE tables need rows >= 1, stride >= head_dim and a multiple of 4, 16-byte alignment "
                         "(rows %d, stride %lld)", r->rows, (long long)r->stride);
-        if (r->round_dtype != a->dtype && r->round_dtype != DSALT_DTYPE_F32)
+        if (rotate && r->round_dtype != a->dtype && r->round_dtype != DSALT_DTYPE_F32)
             return fail(DSALT_ERR_INVALID, "round_dtype must equal dtype or be DSALT_DTYPE_F32 (got %d)", r->round_dtype);
     }
     hipError_t e = dsalt::launch_bwd(*a, r, static_cast<hipStream_t>(stream));

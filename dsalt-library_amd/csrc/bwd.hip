@@ -120,7 +120,7 @@ struct BwdParams {
     int64_t q_st, q_sh, k_st, k_sh, v_st, v_sh, o_st, o_sh, do_st, do_sh, lse_st, lse_sh, w_st;
     int64_t lp_sh, lp_ss, lp_sk, lb_sh, lb_ss, lb_sk;
     int64_t dq_st, dq_sh, dk_st, dk_sh, dv_st, dv_sh;
-    int total_len, num_seqs, n_heads, k_lmk, k_pad, n_qblk, grid_q, n_dqblk, grid_dq, n_lgrp, n_lchunk, grad_f32, o_f32;
+    int total_len, num_seqs, n_heads, k_lmk, k_pad, n_qblk, grid_q, n_dqblk, grid_dq, n_lgrp, n_lchunk, grad_f32, dq_f32, o_f32;
     int kv_rep;  // query heads per K/V head
     float scale, scale_log2, inv_tau, win_edge;
     float inv_c2;  // 1 / scale_log2: log2-unit bias -> raw q.k units
@@ -698,7 +698,7 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
             rotate_acc_transposed<DT, ND>(dqacc, mul, rope, i, hh);
             mul = 1.f;
         }
-        store_row<DT, ND>(p.dq, tok_i * p.dq_st + (int64_t)head * p.dq_sh, p.grad_f32, dqacc, mul, hh);
+        store_row<DT, ND>(p.dq, tok_i * p.dq_st + (int64_t)head * p.dq_sh, p.dq_f32, dqacc, mul, hh);
     }
     if (MODE == kSoft && p.ws_dwh) {
         float dwt;
@@ -1641,6 +1641,42 @@ hipError_t launch_dt(const BwdParams &p, int head_dim, int mode, hipStream_t str
 
 }  // namespace
 
+namespace {
+
+// Gradients of grouped K/V heads: the fp32 per-query-head rows of dK and dV summed over each
+// group's heads in order and rounded once. A thread takes four elements of one K/V head;
+// bound by the bytes (4627 tokens, 16 heads over 4 of 128, fp16: 85 MB).
+template <typename DT>
+__global__ void __launch_bounds__(256) group_sum_kernel(const float4 *__restrict__ dkh, const float4 *__restrict__ dvh,
+                                                        void *dk, void *dv, int64_t n, int rep, int d4) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const int64_t head = i / d4, src = head * rep * d4 + (i - head * d4);  // head: token * n_kv + K/V head
+    const float4 *in = blockIdx.y ? dvh : dkh;
+    float4 t = in[src];
+    for (int h = 1; h < rep; ++h) {
+        const float4 x = in[src + (int64_t)h * d4];
+        t.x += x.x; t.y += x.y; t.z += x.z; t.w += x.w;
+    }
+    void *out = blockIdx.y ? dv : dk;
+    if constexpr (std::is_same<DT, F32>::value) static_cast<float4 *>(out)[i] = t;
+    else static_cast<uint2 *>(out)[i] = make_uint2(DT::pack2(t.x, t.y), DT::pack2(t.z, t.w));
+}
+
+}  // namespace
+
+hipError_t launch_group_sum(const float *dk_heads, const float *dv_heads, void *dk, void *dv, int64_t rows, int rep, int d,
+                            int dtype, hipStream_t stream) {
+    const int64_t n = rows * (d / 4);
+    if (n == 0) return hipSuccess;
+    const dim3 grid((unsigned)((n + 255) / 256), 2);
+    const float4 *a = reinterpret_cast<const float4 *>(dk_heads), *b = reinterpret_cast<const float4 *>(dv_heads);
+    if (dtype == DSALT_DTYPE_BF16) hipLaunchKernelGGL(group_sum_kernel<BF16>, grid, dim3(256), 0, stream, a, b, dk, dv, n, rep, d / 4);
+    else if (dtype == DSALT_DTYPE_F16) hipLaunchKernelGGL(group_sum_kernel<F16>, grid, dim3(256), 0, stream, a, b, dk, dv, n, rep, d / 4);
+    else hipLaunchKernelGGL(group_sum_kernel<F32>, grid, dim3(256), 0, stream, a, b, dk, dv, n, rep, d / 4);
+    return hipGetLastError();
+}
+
 int64_t bwd_workspace_bytes(int total_len, int num_seqs, int n_heads, int head_dim, int k_lmk) {
     const int64_t sparse = (int64_t)ws_layout(total_len, num_seqs, n_heads, head_dim, k_lmk).total;
     // one sequence without landmark slots may also be a dense-mode call
@@ -1671,6 +1707,7 @@ hipError_t launch_bwd(const dsalt_bwd_args &a, const dsalt_rope_tables *rope, hi
     p.dk = a.dk;
     p.dv = a.dv;
     p.grad_f32 = a.grad_dtype == DSALT_DTYPE_F32;
+    p.dq_f32 = p.grad_f32 && !(rope && rope->dq_compute_dtype);
     p.d_bias = a.d_lmk_bias;
     p.d_w = (a.mode == DSALT_MODE_SOFT) ? a.d_w : nullptr;
     p.ws_qrec = reinterpret_cast<float *>(ws + L.qrec);

@@ -68,7 +68,7 @@ struct DenseParams {
     int64_t q_st, q_sh, k_st, k_sh, v_st, v_sh, o_st, o_sh, do_st, do_sh, lse_st, lse_sh, w_st;
     int64_t lb_sh, lb_st;
     int64_t dq_st, dq_sh, dk_st, dk_sh, dv_st, dv_sh;
-    int T, H, n_blk, grid, out_f32, o_f32, grad_f32;
+    int T, H, n_blk, grid, out_f32, o_f32, grad_f32, dq_f32;
     int kv_rep;      // query heads per K/V head
     float c;         // scale * log2(e): raw q.k -> log2-unit logit
     float inv_c;     // 1 / c
@@ -573,7 +573,7 @@ __global__ void __launch_bounds__(128 * dense_bwd_groups(D), 1) dense_dq_kernel(
                 const int dd = d * 32 + g * 8 + hh * 4;
                 const float a0 = dq[d][g * 4] * mul, a1 = dq[d][g * 4 + 1] * mul;
                 const float a2 = dq[d][g * 4 + 2] * mul, a3 = dq[d][g * 4 + 3] * mul;
-                if (p.grad_f32) {
+                if (p.dq_f32) {
                     *reinterpret_cast<float4 *>(static_cast<float *>(p.dq) + off + dd) = make_float4(a0, a1, a2, a3);
                 } else {
                     uint2 val;
@@ -922,6 +922,7 @@ hipError_t launch_dense_bwd(const dsalt_bwd_args &a, const dsalt_rope_tables *ro
     p.dk = a.dk;
     p.dv = a.dv;
     p.grad_f32 = a.grad_dtype == DSALT_DTYPE_F32;
+    p.dq_f32 = p.grad_f32 && !(rope && rope->dq_compute_dtype);
     p.d_lb = a.d_lmk_bias;
     p.d_w = a.d_w;
     char *ws = static_cast<char *>(a.workspace);

@@ -66,6 +66,8 @@ hipError_t launch_swiglu(const void *gate, const void *up, void *out, int64_t n,
 hipError_t launch_add_rms_norm(const void *x, const void *h, void *x_out, void *y, const void *weight, int64_t rows,
                                int d, float eps, int dtype, hipStream_t stream);
 int rms_norm_max_dim();
+hipError_t launch_group_sum(const float *dk_heads, const float *dv_heads, void *dk, void *dv, int64_t rows, int rep, int d,
+                            int dtype, hipStream_t stream);
 hipError_t launch_swiglu_rows(const void *gate_up, const void *d_out, void *out, int64_t rows, int f, int dtype,
                               hipStream_t stream);
 hipError_t launch_norm_train(const dsalt_norm_train_args &a, hipStream_t stream);

@@ -131,7 +131,7 @@ class RopeArgs(ctypes.Structure):
 
 class RopeTables(ctypes.Structure):
     _fields_ = [("cos", c_void_p), ("sin", c_void_p), ("stride", c_int64), ("rows", c_int32), ("half", c_int32),
-                ("round_dtype", c_int32), ("reserved", c_int32)]
+                ("round_dtype", c_int32), ("dq_compute_dtype", c_int32)]
 
 
 class QkvArgs(ctypes.Structure):
@@ -201,7 +201,7 @@ EXPORTED_SYMBOLS = (
     "dsalt_lmk_weights_workspace_size", "dsalt_lmk_weights_args_size", "dsalt_bwd_rope", "dsalt_rope_tables_size",
     "dsalt_select_hybrid_qkv", "dsalt_qkv_args_size", "dsalt_module_grads_v", "dsalt_module_grads_x",
     "dsalt_module_grads_workspace_size", "dsalt_module_grads_args_size", "dsalt_swiglu_rows", "dsalt_norm_train",
-    "dsalt_norm_train_bwd", "dsalt_norm_train_workspace_size", "dsalt_norm_train_args_size",
+    "dsalt_group_sum", "dsalt_norm_train_bwd", "dsalt_norm_train_workspace_size", "dsalt_norm_train_args_size",
 )
 NOALLOC_SCRATCH_BYTES = 76 << 20  # DSALT_NOALLOC_SCRATCH_BYTES
 SELECT_SPLIT_MIN = 4096  # longer sequences can be selected chunk-wise
@@ -247,6 +247,7 @@ def lib() -> ctypes.CDLL:
         ("dsalt_quantize_windows", [c_void_p, c_int64, c_void_p, c_void_p, c_void_p]),
         ("dsalt_norm_train", [ctypes.POINTER(NormTrainArgs), c_void_p]),
         ("dsalt_norm_train_bwd", [ctypes.POINTER(NormTrainArgs), c_void_p]),
+        ("dsalt_group_sum", [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_int32, c_void_p]),
         ("dsalt_swiglu_rows", [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_void_p]),
         ("dsalt_swiglu", [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_void_p]),
         ("dsalt_add_rms_norm", [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_float, c_int32,
@@ -384,6 +385,22 @@ def group_sum(g: torch.Tensor, n_kv: int) -> torch.Tensor:
     return g if n_kv == H else g.view(T, n_kv, H // n_kv, D).sum(2)
 
 
+def group_sum_pair(dk: torch.Tensor, dv: torch.Tensor, n_kv: int, dtype: torch.dtype):
+    """Per-query-head gradients [T, H, D] (fp32, contiguous) summed over each group of H // n_kv
+    heads -> [T, n_kv, D] in dtype (the gradients of K/V heads that several query heads
+    share); one HIP pass for both."""
+    T, H, D = dk.shape
+    dev = require_gpu(dk, dv)
+    if (dk.dtype != torch.float32 or dv.dtype != torch.float32 or dv.shape != dk.shape or H % n_kv
+            or not (dk.is_contiguous() and dv.is_contiguous())):
+        raise DsaltError(f"group_sum_pair needs contiguous fp32 [T, H, D] gradients (got {dk.dtype} {tuple(dk.shape)}, "
+                         f"{dv.dtype} {tuple(dv.shape)})")
+    out = [torch.empty((T, n_kv, D), device=dev, dtype=dtype) for _ in range(2)]
+    _raise(lib().dsalt_group_sum(dk.data_ptr(), dv.data_ptr(), out[0].data_ptr(), out[1].data_ptr(), T * n_kv, H // n_kv, D,
+                                 _SCORE_DTYPES[dtype], stream_handle(dev)), "dsalt_group_sum")
+    return out
+
+
 def _f32_vec(t: torch.Tensor) -> torch.Tensor:
     return t if t.dtype == torch.float32 else t.float()
 
@@ -519,7 +536,7 @@ class BwdLauncher:
         self.args, self._keep, self.results, self.device = _bwd_args(
             mode, q, k, v, out, lse, dout, w, lmk_pos, lmk_bias, cu_seqlens, scale, tau_win, win_edge,
             need_dw, grad_dtype, grads)
-        self._rope, keep = _rope_tables_arg(rope, q.shape[2])
+        self._rope, keep = _rope_tables_arg(rope, q.shape[2], self.results[0].dtype != self.results[1].dtype)
         self._keep += (keep,)
         self._fn = lib().dsalt_bwd_rope
         self._ref = ctypes.byref(self.args)
@@ -528,10 +545,14 @@ class BwdLauncher:
         _raise(self._fn(self._ref, self._rope, stream_handle(self.device)), "dsalt_bwd")
 
 
-def _rope_tables_arg(rope, D: int):
-    """(pointer to a RopeTables block or None, tensors to keep alive) of rope = (cos, sin, dtype)."""
-    if rope is None:
+def _rope_tables_arg(rope, D: int, dq_16: bool = False):
+    """(pointer to a RopeTables block or None, tensors to keep alive) of rope = (cos, sin, dtype);
+    dq_16: dq in the compute dtype besides fp32 dk and dv."""
+    if rope is None and not dq_16:
         return None, None
+    if rope is None:
+        t = RopeTables(dq_compute_dtype=1)
+        return ctypes.byref(t), (t,)
     cos, sin, dtype = rope
     require_gpu(cos, sin)
     cos, sin, half = rope_tables(cos, sin)
@@ -539,19 +560,23 @@ def _rope_tables_arg(rope, D: int):
         raise DsaltError(f"RoPE tables must be [rows, {D}] (got {tuple(cos.shape)}, {tuple(sin.shape)})")
     t = RopeTables()
     t.cos, t.sin, t.stride, t.rows = cos.data_ptr(), sin.data_ptr(), cos.stride(0), cos.shape[0]
-    t.half, t.round_dtype = int(half), _SCORE_DTYPES[dtype]
+    t.half, t.round_dtype, t.dq_compute_dtype = int(half), _SCORE_DTYPES[dtype], int(dq_16)
     return ctypes.byref(t), (t, cos, sin)
 
 
 def _grad_outputs(q: torch.Tensor, dtype: torch.dtype, grads):
-    """dq, dk and dv [T, H, D]: new ones, or the caller's (checked)."""
-    if grads is None:
-        return tuple(torch.empty(q.shape, device=q.device, dtype=dtype) for _ in range(3))
-    for g in grads:
-        if g.shape != q.shape or g.dtype != dtype or g.device != q.device or g.stride(2) != 1:
+    """dq, dk and dv [T, H, D]: the caller's (checked), or new ones where it gives None. Its dq may
+    be in q's dtype where dk and dv are fp32."""
+    out = []
+    for i, g in enumerate(grads or (None, None, None)):
+        if g is None:
+            g = torch.empty(q.shape, device=q.device, dtype=dtype)
+        elif (g.shape != q.shape or g.dtype not in ((dtype, q.dtype) if i == 0 else (dtype,)) or g.device != q.device
+              or g.stride(2) != 1):
             raise DsaltError(f"gradient outputs must be {tuple(q.shape)} {dtype} with unit inner stride, got "
                              f"{tuple(g.shape)} {g.dtype}")
-    return grads
+        out.append(g)
+    return out
 
 
 def _bwd_args(mode, q, k, v, out, lse, dout, w, lmk_pos, lmk_bias, cu_seqlens, scale, tau_win, win_edge,
@@ -742,7 +767,7 @@ class DenseBwdLauncher:
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws_bytes
         a.scale, a.tau_win, a.win_edge = float(scale), float(tau_win), float(win_edge)
         self.args = a
-        self._rope, keep = _rope_tables_arg(rope, D)
+        self._rope, keep = _rope_tables_arg(rope, D, dq.dtype != gdt)
         self._keep = (q, k, v, out, lse, dout, w, lb, ws, keep)
         self.results = (dq, dk, dv, d_lb, d_w)
         self._fn = lib().dsalt_bwd_rope

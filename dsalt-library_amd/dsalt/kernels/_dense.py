@@ -48,7 +48,8 @@ class _DenseAttention(torch.autograd.Function):
         need_dw = ctx.needs_input_grad[3]
         dq, dk, dv, d_lb, d_w = _hip.dense_bwd(q_c, k_c, v_c, out, lse, grad_out, w_f, lb, ctx.dsalt_scale,
                                                ctx.dsalt_tau, ctx.dsalt_edge, need_dw=need_dw, grad_dtype=gdt)
-        dk, dv = _hip.group_sum(dk, n_kv), _hip.group_sum(dv, n_kv)
+        if n_kv != q_c.shape[1]:
+            dk, dv = _hip.group_sum_pair(dk, dv, n_kv, od if od in (torch.float32, q_c.dtype) else torch.float32)
         if not ctx.needs_input_grad[4]:
             d_lb = None
         return (dq.to(od), dk.to(od), dv.to(od),

@@ -77,18 +77,16 @@ class _ModuleAttention(torch.autograd.Function):
         dqkv = torch.empty_like(qkv)
         dq, dk, dv = _split(dqkv, H, n_kv, D)
         # grouped K/V heads: per-query-head gradients in fp32, summed over each group below
-        gdt, grads = (torch.float32, None) if grouped else (od, (dq, dk, dv))
+        gdt, grads = (torch.float32, (dq, None, None)) if grouped else (od, (dq, dk, dv))
         fused = not dense or D == 64  # the dense kernels un-rotate their gradients at D = 64
         rope = (cos, sin, od) if fused else None
         if dense:
-            dq_h, dk_h, dv_h, d_weight, dw = _hip.dense_bwd(q_r, k_r, v_r, out, lse, grad_out, w32, weight, scale,
+            _, dk_h, dv_h, d_weight, dw = _hip.dense_bwd(q_r, k_r, v_r, out, lse, grad_out, w32, weight, scale,
                                                             opt["tau_win"], opt["win_edge"], True, gdt, rope, grads)
         else:
             lp, lw = (pos, weight) if opt["k_lmk"] > 0 else (None, None)
-            dq_h, dk_h, dv_h, d_weight, dw = _hip.bwd(_hip.MODE_SOFT, q_r, k_r, v_r, out, lse, grad_out, w32, lp, lw, cu,
+            _, dk_h, dv_h, d_weight, dw = _hip.bwd(_hip.MODE_SOFT, q_r, k_r, v_r, out, lse, grad_out, w32, lp, lw, cu,
                                                       scale, opt["tau_win"], opt["win_edge"], True, gdt, rope, grads)
-        if grouped:
-            dq.copy_(dq_h)
         g = _hip.ModuleGrads(x.detach(), v, norms, a32, pos, cu, weight if d_weight is None else d_weight,
                              opt["tau_lmk"], dense)
         d_alpha = g.values(dk_h, dv_h, dk, dv, alpha_sigmoid=True)

@@ -64,11 +64,16 @@ def _backward(ctx, grad_out, need_dw: bool):
     # written directly by the kernels, and so do grouped K/V heads (per-query-head dK/dV
     # are summed over each group in fp32)
     n_kv = k_c.shape[1]
-    gdt = torch.float32 if (od == torch.float32 or n_kv != q_c.shape[1]) else q_c.dtype
+    grouped = n_kv != q_c.shape[1]
+    gdt = torch.float32 if (od == torch.float32 or grouped) else q_c.dtype
+    # dq, and the sums of dk and dv, are rounded to q's dtype by the kernels
+    kdt = od if od in (torch.float32, q_c.dtype) else torch.float32
+    grads = (torch.empty(q_c.shape, device=q_c.device, dtype=kdt), None, None) if grouped else None
     dq, dk, dv, d_bias, d_w = _hip.bwd(
         ctx.dsalt_mode, q_c, k_c, v_c, out, lse, grad_out, w_f, lp, lb, cu,
-        ctx.dsalt_scale, ctx.dsalt_tau, ctx.dsalt_edge, need_dw=need_dw, grad_dtype=gdt)
-    dk, dv = _hip.group_sum(dk, n_kv), _hip.group_sum(dv, n_kv)
+        ctx.dsalt_scale, ctx.dsalt_tau, ctx.dsalt_edge, need_dw=need_dw, grad_dtype=gdt, grads=grads)
+    if grouped:
+        dk, dv = _hip.group_sum_pair(dk, dv, n_kv, kdt)
     # the landmark-weight and window gradients stay fp32, as the kernels sum them (autograd
     # casts each to its input's dtype)
     return dq.to(od), dk.to(od), dv.to(od), d_bias, d_w

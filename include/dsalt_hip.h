@@ -201,15 +201,25 @@ int dsalt_bwd_check(const dsalt_bwd_args *args);
  * tables at head_dim 64 only (DSALT_ERR_UNSUPPORTED otherwise: rotate with dsalt_rope).
  */
 typedef struct dsalt_rope_tables {
-    const float *cos, *sin; /* rows of >= head_dim entries, 16-byte aligned */
+    const float *cos, *sin; /* rows of >= head_dim entries, 16-byte aligned; both NULL: no rotation */
     int64_t stride;         /* row stride (elements), a multiple of 4 */
     int32_t rows;
     int32_t half;           /* 1: every row repeats its first half (half of it is read) */
     int32_t round_dtype;    /* what the entries are rounded to: args->dtype, or F32 (not at all) */
-    int32_t reserved;
+    int32_t dq_compute_dtype; /* 1: dq is written in args->dtype also where args->grad_dtype is F32 */
 } dsalt_rope_tables;
 
 int dsalt_bwd_rope(const dsalt_bwd_args *args, const dsalt_rope_tables *rope, void *stream);
+
+/*
+ * Gradients of K/V heads shared by `rep` query heads each: dk and dv [rows, d] (rows = tokens x
+ * K/V heads, dtype BF16, F16 or F32) are the sums of the fp32 per-query-head rows dk_heads
+ * and dv_heads [rows, rep, d] over rep, in order, rounded once. All contiguous and 16-byte
+ * aligned, d a multiple of 4; outputs alias no input. Replaces the sums over repeated heads
+ * that autograd forms for _repeat_kv (dsalt/modules/dsalt_attention.py:236-241).
+ */
+int dsalt_group_sum(const float *dk_heads, const float *dv_heads, void *dk, void *dv, int64_t rows, int32_t rep, int32_t d,
+                    int32_t dtype, void *stream);
 size_t dsalt_rope_tables_size(void);
 
 /*

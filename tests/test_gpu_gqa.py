@@ -102,3 +102,35 @@ def test_gqa_rejects_non_dividing_heads():
     cu = torch.tensor([0, 64], dtype=torch.int32, device=DEV)
     with pytest.raises(hip.DsaltError, match="n_kv dividing H"):
         hip.fwd(hip.MODE_HARD, q, k, k, w, None, None, cu, 0.125)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,n_kv,rep,D", [(1, 1, 2, 64), (37, 3, 5, 128), (515, 2, 8, 64), (9, 4, 1, 4)])
+def test_group_sum_pair(dtype, T, n_kv, rep, D):
+    """Both gradients' fp32 sums over a group's heads, rounded once (the order is the heads')."""
+    print(f"group_sum_pair {dtype} T={T} n_kv={n_kv} rep={rep} D={D}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    a, b = (torch.randn(T, n_kv * rep, D, device="cuda", generator=g) for _ in range(2))
+    for got, x in zip(hip.group_sum_pair(a, b, n_kv, dtype), (a, b)):
+        want = x.view(T, n_kv, rep, D)[:, :, 0]
+        for h in range(1, rep):
+            want = want + x.view(T, n_kv, rep, D)[:, :, h]
+        assert torch.equal(got, want.to(dtype))
+
+
+@pytest.mark.parametrize("mode", [hip.MODE_HARD, hip.MODE_SOFT])
+def test_dq_in_compute_dtype_beside_fp32(mode):
+    """dq written in q's dtype beside fp32 dk and dv is the fp32 dq rounded."""
+    print(f"bwd mixed gradient dtypes {mode}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    T, H, n_kv, D = 300, 4, 2, 64
+    q, dout = (torch.randn(T, H, D, device="cuda", generator=g).bfloat16() for _ in range(2))
+    k, v = (torch.randn(T, n_kv, D, device="cuda", generator=g).bfloat16() for _ in range(2))
+    w = 5 + 40 * torch.rand(T, device="cuda", generator=g)
+    cu = torch.tensor([0, 170, T], dtype=torch.int32, device="cuda")
+    out, lse = hip.fwd(mode, q, k, v, w, None, None, cu, 0.125)
+    args = (mode, q, k, v, out, lse, dout, w, None, None, cu, 0.125)
+    want = hip.bwd(*args, grad_dtype=torch.float32)
+    got = hip.bwd(*args, grad_dtype=torch.float32, grads=(torch.empty_like(q), None, None))
+    assert got[0].dtype == torch.bfloat16 and torch.equal(got[0], want[0].bfloat16())
+    assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
