@@ -22,6 +22,7 @@ from .. import _hip
 class _ModuleAttention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, wq, wk, wv, wg, bg, alpha_w, cos, sin, cu_seqlens, opt, x_cast):
+        ctx.set_materialize_grads(False)  # no zero gradients of the outputs that take none
         cdt, H, n_kv, D = opt["dtype"], opt["n_heads"], opt["n_kv_heads"], opt["head_dim"]
         T, dense, k_lmk = x.shape[0], opt["dense"], opt["k_lmk"]
         xd = x.detach()
@@ -63,6 +64,8 @@ class _ModuleAttention(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out, *_):
+        if grad_out is None:
+            return (None,) * 12
         (x, xb, qkv, q_r, k_r, v_r, w_cat, wg, out, lse, logit, w32, weight, a32, norms, pos, cu, cos,
          sin) = ctx.saved_tensors
         opt, scale, w_dtype, a_dtype = ctx.dsalt
