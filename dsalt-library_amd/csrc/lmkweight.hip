@@ -82,11 +82,12 @@ struct WeightParams {
     float n_min, span;
 };
 
-// log(max(sigmoid(s / tau), 1e-20)) as torch's fp32 ops form it.
+// log(max(sigmoid(s / tau), 1e-20)) as torch's fp32 ops form it (a NaN score gives NaN).
 __device__ __forceinline__ float lmk_weight(float s, float tau) {
     const float sg = 1.f / (1.f + expf(-s / tau));
-    return logf(fmaxf(sg, kSigClamp));
+    return logf(sg < kSigClamp ? kSigClamp : sg);
 }
+
 
 __global__ void __launch_bounds__(kTableThreads) weight_kernel(const WeightParams p) {
     __shared__ float st[4];
@@ -97,6 +98,8 @@ __global__ void __launch_bounds__(kTableThreads) weight_kernel(const WeightParam
         float m, sd;
         const int q = wave == 0 ? 0 : 1 + g;
         hybrid_stat(p.part, p.nblk, 1 + p.n_kv, q, (double)p.T, lane, m, sd);
+        // where a norm is not finite torch's std, and with it every score, is NaN
+        if (!(fabsf(m) < INFINITY)) sd = NAN;
         if (lane == 0) {
             st[2 * wave] = m;
             st[2 * wave + 1] = sd;
@@ -158,7 +161,7 @@ __global__ void __launch_bounds__(kTableThreads) reduce_kernel(const WeightParam
         const float sg = 1.f / (1.f + expf(-s / p.tau));
         const float gw = p.g[p.table ? (int64_t)head * p.T + t : (int64_t)head * p.S * p.k + e];
         // d log(max(sg, c)) / ds = (1 - sg) / tau above the clamp, 0 below it
-        const float ds = sg >= kSigClamp ? gw * (1.f - sg) * p.inv_tau : 0.f;
+        const float ds = sg < kSigClamp ? 0.f : gw * (1.f - sg) * p.inv_tau;
         gz[t] = ds;
         a0 += ds;
         a1 += (double)ds * zv;
@@ -180,6 +183,9 @@ __global__ void __launch_bounds__(kTableThreads) reduce_kernel(const WeightParam
             t1 += s_sum[w][1];
             t2 += s_sum[w][2];
         }
+        // NaN scores are never selected, but through an empty slot's (or an unselected key's) zero
+        // gradient they still make every gradient NaN, as in torch: 0 times NaN
+        if ((sx != sx || sv != sv) && (p.k > 0 || p.table)) t0 = t1 = t2 = NAN;
         p.hsum[3 * head] = t0;
         p.hsum[3 * head + 1] = t1;
         p.hsum[3 * head + 2] = t2;
@@ -192,10 +198,10 @@ __global__ void __launch_bounds__(kTableThreads) reduce_kernel(const WeightParam
 
 // Gradient of norm n (standardised to z = (n - mean) / sd over T tokens) divided by n, from
 // z's gradient dz and the sums A = sum dz, B = sum dz z over the tokens: the row's own
-// gradient is this times the row (0 for a zero row, as torch masks it). A clamped std
-// takes no gradient.
+// gradient is this times the row (0 for a zero row, as torch masks it, and where no
+// gradient comes in, whatever the std). A clamped std takes no gradient.
 __device__ __forceinline__ float norm_coef(float n, float mean, float sd, float dz, double A, double B, int T) {
-    if (n == 0.f) return 0.f;
+    if (n == 0.f || (dz == 0.f && A == 0.0 && B == 0.0)) return 0.f;
     const float z = hybrid_z(n, mean, sd);
     float dn = dz - (float)(A / T);
     if (sd > 1e-6f) dn -= z * (float)(B / (T - 1));

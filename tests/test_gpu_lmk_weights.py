@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 import torch
 
+from dsalt import _hip
 from dsalt.kernels._lmk_weights import landmark_weights
 
 pytestmark = pytest.mark.gpu
@@ -90,3 +91,41 @@ def test_landmark_weights_without_weight_gradient():
     gv = torch.randn_like(v)
     v_out.backward(gv)
     assert x.grad is None and torch.equal(v.grad, gv)
+
+
+@pytest.mark.parametrize("what,T", [("x nan", 70), ("x inf", 70), ("v nan", 70), ("v inf", 70), ("one token", 1)])
+@pytest.mark.parametrize("table", [False, True])
+def test_non_finite_norms_give_nan(what, T, table):
+    """A norm that is not finite, or the std of one token, makes every score NaN: no landmark is
+    selected, a selected one would weigh NaN, and the gradients are NaN where autograd's are
+    (a zero gradient times NaN)."""
+    print(f"landmark weights {what} table={table}", flush=True)
+    g = torch.Generator().manual_seed(T)
+    H, n_kv = 4, 2
+    x, v = torch.randn(T, 64, generator=g).to(DEV), torch.randn(T, n_kv, 64, generator=g).to(DEV)
+    if T > 1:
+        t = x if what[0] == "x" else v.view(T, -1)
+        t[T // 2, 3] = float(what[2:])
+    x, v = x.requires_grad_(), v.requires_grad_()
+    alpha = torch.full((H,), 0.6, device=DEV, requires_grad=True)
+    w = torch.zeros(1, device=DEV).expand(T) if table else torch.ones(T, device=DEV)
+    cu = torch.tensor([0, T], dtype=torch.int32, device=DEV)
+    v_out, weight, pos, _ = landmark_weights(x, v, alpha, w, cu, 3, T, 2.0, table)
+    x64, v64, a64 = (t.detach().double().requires_grad_() for t in (x, v, alpha))
+    ref = reference(x64, v64, a64, pos, [0, T], 2.0, table)
+    if table:  # the reference weighs what is selected; here nothing may be, in the NaN heads
+        ref = torch.where(torch.isfinite(weight), ref, float("-inf"))
+    assert torch.equal(torch.isfinite(ref), torch.isfinite(weight))
+    fin = torch.isfinite(ref).detach()
+    torch.autograd.backward([weight, v_out], [torch.where(fin, 1.0, 0.0), torch.zeros_like(v)])
+    torch.where(fin, ref, 0.0).sum().backward()
+    assert bool(a64.grad.isnan().any())
+    for got, want in ((x, x64), (v, v64), (alpha, a64)):
+        assert torch.equal(got.grad.isnan(), want.grad.isnan())
+    # a slot that names a token whose score is NaN
+    sel = _hip.SelectHybridLauncher(x.detach(), v.detach(), alpha.detach(), H, w, cu, 3, max_seqlen=T, quantize=not table)
+    sel()
+    named = _hip.lmk_weights(sel.norms, alpha.detach(), torch.zeros_like(pos), sel.cu, T, n_kv, 2.0, table)
+    first = named[:, 0] if table else named[:, 0, 0]
+    nan_heads = a64.grad.isnan()
+    assert torch.equal(first.isnan(), nan_heads)

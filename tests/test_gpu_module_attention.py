@@ -213,3 +213,27 @@ def test_training_windows_are_the_rounded_gate(dtype, autocast):
     logit = (x.to(cdt).double() @ w.t() + b).squeeze(-1).to(cdt)
     want = mod.n_min + torch.sigmoid(logit) * (mod.n_max - mod.n_min)
     assert torch.equal(mod._last_selection[0], want.float().floor().clamp(min=1))
+
+
+@pytest.mark.parametrize("T,k", [(1, 0), (1, 4), (70, 0), (70, 4)])
+def test_non_finite_scores_in_training(T, k):
+    """The scores' gradients with one token or an infinite state are autograd's: NaN (0 times
+    NaN) with landmark slots, and without any nothing comes in through them."""
+    print(f"module attention non-finite T={T} k={k}", flush=True)
+    got = {}
+    for hip in (True, False):
+        torch.manual_seed(5)
+        mod = DSALTAttention(256, 4, 8, 100, k, max_seq_len=400, n_kv_heads=2).to(DEV, torch.bfloat16).train()
+        mod._hip_scores = hip  # False: torch's ops
+        x = torch.randn(T, 256, device=DEV).to(torch.bfloat16)
+        if T > 1:
+            x[T // 2, 3] = float("inf")
+        x.requires_grad_()
+        assert mod._one_function(x) == hip
+        mod(x, cu_seqlens=torch.tensor([0, T], dtype=torch.int32, device=DEV))[0].float().sum().backward()
+        got[hip] = {"x": x.grad, **{n: p.grad for n, p in mod.named_parameters()}}
+    for n, want in got[False].items():
+        a = got[True][n]
+        if want is not None:
+            assert torch.equal(a.isnan(), want.isnan()), n
+    assert bool(got[True]["alpha_w"].isnan().all()) == (k > 0)
