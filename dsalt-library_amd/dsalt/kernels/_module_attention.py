@@ -108,8 +108,10 @@ class _ModuleAttention(torch.autograd.Function):
             dx, dwg, dbg = g.states(dx_in, need_x, (wg, logit, dw, od, opt["n_min"], opt["n_max"]))
         if not ctx.needs_input_grad[5]:
             dbg = None
+        if not ctx.needs_input_grad[6] or not (dense or opt["k_lmk"] > 0):
+            d_alpha = None  # without landmark slots alpha takes no part
         return (dx, *dws, dwg if ctx.needs_input_grad[4] else None, dbg,
-                d_alpha.to(a_dtype) if ctx.needs_input_grad[6] else None, *[None] * 5)
+                None if d_alpha is None else d_alpha.to(a_dtype), *[None] * 5)
 
 
 def _split(qkv: torch.Tensor, H: int, n_kv: int, D: int):

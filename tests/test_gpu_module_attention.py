@@ -215,6 +215,18 @@ def test_training_windows_are_the_rounded_gate(dtype, autocast):
     assert torch.equal(mod._last_selection[0], want.float().floor().clamp(min=1))
 
 
+def test_alpha_takes_no_gradient_without_landmarks():
+    """With k_lmk = 0 no weight depends on alpha: its gradient is None (an optimizer leaves it
+    alone), not zeros. The dense variant's table holds a weight for every key, so zeros there."""
+    print("module attention alpha without landmarks", flush=True)
+    mod, x, packed = small_module()
+    mod.k_lmk = 0
+    mod(x, **packed)[0].float().sum().backward()
+    assert mod.alpha_w.grad is None and mod.v_proj.weight.grad is not None
+    mod(x[None])[0].float().sum().backward()
+    assert bool((mod.alpha_w.grad == 0).all())
+
+
 @pytest.mark.parametrize("T,k", [(1, 0), (1, 4), (70, 0), (70, 4)])
 def test_non_finite_scores_in_training(T, k):
     """The scores' gradients with one token or an infinite state are autograd's: NaN (0 times
@@ -236,4 +248,4 @@ def test_non_finite_scores_in_training(T, k):
         a = got[True][n]
         if want is not None:
             assert torch.equal(a.isnan(), want.isnan()), n
-    assert bool(got[True]["alpha_w"].isnan().all()) == (k > 0)
+    assert got[True]["alpha_w"] is None if k == 0 else bool(got[True]["alpha_w"].isnan().all())
