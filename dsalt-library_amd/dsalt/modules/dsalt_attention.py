@@ -278,6 +278,7 @@ class DSALTAttention(nn.Module):
             cu = torch.arange(0, T + 1, T, dtype=torch.int32, device=device)  # [0, T], made on the GPU
             out, lmk_pos, w_cont, _ = self._attend(xs, cu, min(self.k_lmk, T), T, dense=True,
                                                      x_cast=None if x_cast is None else x_cast[0])
+            w_cont = w_cont.to(autocast_dtype(xs))  # rounded to it already: the gate's own type
         else:
             q = self.q_proj(xs).view(T, self.n_heads, self.head_dim)
             k = self.k_proj(xs).view(T, self.n_kv_heads, self.head_dim)

@@ -227,6 +227,22 @@ def test_alpha_takes_no_gradient_without_landmarks():
     assert bool((mod.alpha_w.grad == 0).all())
 
 
+@pytest.mark.parametrize("dtype,autocast", [(torch.bfloat16, False), (torch.float32, False), (torch.float32, True)])
+def test_dense_last_selection_keeps_its_types(dtype, autocast):
+    """The dense variant's _last_selection: windows in the gate's type on either route."""
+    print(f"module attention dense selection {dtype} autocast={autocast}", flush=True)
+    mod, x, _ = small_module(dtype)
+    got = []
+    for hip in (True, False):
+        mod._hip_scores = hip
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+            mod(x[None])
+        got.append(mod._last_selection)
+    (w1, p1), (w2, p2) = got
+    assert w1.dtype == w2.dtype == (torch.bfloat16 if autocast else dtype) and p1.dtype == p2.dtype == torch.int64
+    assert float((w1.double() - w2.double()).abs().max()) <= 2.0 ** (-20 if w1.dtype == torch.float32 else -7) * mod.n_max
+
+
 @pytest.mark.parametrize("T,k", [(1, 0), (1, 4), (70, 0), (70, 4)])
 def test_non_finite_scores_in_training(T, k):
     """The scores' gradients with one token or an infinite state are autograd's: NaN (0 times
