@@ -301,7 +301,7 @@ class DSALTAttention(nn.Module):
         """Whether projections, gate, RoPE, selection and attention of x [T, d] run as one function
         (``module_attention``): the HIP score route; projections that are plain nn.Linear
         modules without hooks (a wrapped, parametrised or hooked one is called as it is, on the
-        route of separate functions), q, k and v without bias; one element type for x and the
+        route of separate functions, and so is a subclass's own step), q, k and v without bias; one element type for x and the
         weights, or fp32 for all of them under a 16-bit autocast; rows that the norms pass
         loads in 16-byte pieces."""
         lin = (self.q_proj, self.k_proj, self.v_proj, self.win_gate)
@@ -310,7 +310,7 @@ class DSALTAttention(nn.Module):
         if not (self._fused_selector and self._hip_scores and self._fuse_qkv and all(type(m) is nn.Linear for m in lin)):
             return False
         ps = [m.weight for m in lin] + [m.bias for m in lin if m.bias is not None]
-        if not plain(*lin) or not eager(*ps):
+        if not plain(*lin) or not eager(*ps) or self._own_steps(*_STEPS):
             return False
         if any(m.bias is not None for m in lin[:3]) or x.dim() != 2 or x.shape[0] == 0 or x.shape[1] != self.d_model:
             return False
@@ -327,6 +327,11 @@ class DSALTAttention(nn.Module):
         return (self.head_dim in (64, 128) and self.n_kv_heads <= _hip.SCORES_MAX_KV and x.stride(1) == 1
                 and x.stride(0) >= self.d_model and x.stride(0) % per == 0 and x.data_ptr() % 16 == 0
                 and self.win_gate.weight.data_ptr() % 16 == 0)
+
+    def _own_steps(self, *names: str) -> bool:
+        """Whether one of these methods of DSALTAttention is replaced, in a subclass, on the class
+        or on this instance."""
+        return any(n in self.__dict__ or getattr(type(self), n) is not _STEPS[n] for n in names)
 
     @_dynamo_opaque
     def _attend(self, x, cu_seqlens, k_lmk, max_seqlen, dense=False, x_cast=None):
@@ -454,8 +459,11 @@ class DSALTAttention(nn.Module):
 
         if self.training:
             self._last_P = None
-            w_cont, lmk_pos, lmk_logw, v_train = self._select_train(x, cu_seqlens, total_len, device, cu_list, v_sel)
-            v = v if v_train is None else v_train
+            if self._own_steps("_train_selectors"):
+                w_cont, lmk_pos, lmk_logw = self._train_selectors(x, cu_seqlens, total_len, device, cu_list, v_sel)
+            else:
+                w_cont, lmk_pos, lmk_logw, v_train = self._select_train(x, cu_seqlens, total_len, device, cu_list, v_sel)
+                v = v if v_train is None else v_train
             out = sparse_attention(_hip.MODE_SOFT, q, k, v, lmk_pos, lmk_logw, w_cont, cu_seqlens,
                                    self.tau_win, float(self.win_edge))
             return self._apply_out_proj(out.reshape(total_len, self.d_model)), aux
@@ -535,3 +543,9 @@ class DSALTAttention(nn.Module):
         logits = torch.matmul(q[seg].transpose(0, 1), k0.transpose(0, 1).transpose(1, 2).contiguous())
         logits = logits * (1.0 / math.sqrt(self.head_dim))
         return logits.masked_fill(~keep, float("-inf")).softmax(dim=-1)
+
+
+# The steps whose work a training forward does without calling them (module_attention,
+# _select_train): where one is replaced, the route that calls it is taken.
+_STEPS = {n: vars(DSALTAttention)[n] for n in ("_project_qkv", "_alpha", "_window_continuous", "_train_selectors",
+                                               "_dense_selectors")}

@@ -172,6 +172,50 @@ def test_hooked_projections_are_called():
     assert mod._one_function(x)
 
 
+class OwnSteps(DSALTAttention):
+    """A subclass with its own balance, windows and landmark weights."""
+
+    def _alpha(self):
+        return torch.sigmoid(3 * self.alpha_w)
+
+    def _window_continuous(self, x):
+        return 0.5 * super()._window_continuous(x)
+
+    def _train_selectors(self, *a, **k):
+        w, pos, logw = super()._train_selectors(*a, **k)
+        return w, pos, logw - 1.0
+
+
+@pytest.mark.parametrize("where", ["subclass", "instance", "class"])
+@pytest.mark.parametrize("dense", [False, True])
+def test_replaced_steps_are_called(where, dense, monkeypatch):
+    """The steps that the one function and the landmark weights' function stand for, replaced in a
+    subclass, on an instance or on the class: each is called."""
+    print(f"module attention own steps {where} dense={dense}", flush=True)
+    mod, x, packed = small_module()
+    seen = []
+
+    def counted(name):
+        step = getattr(OwnSteps, name)
+        return lambda self, *a, **k: (seen.append(name), step(self, *a, **k))[1]
+
+    if where == "subclass":
+        mod.__class__ = type("Counted", (OwnSteps,), {n: counted(n) for n in ("_alpha", "_window_continuous", "_train_selectors")})
+    else:
+        base = {n: getattr(DSALTAttention, n) for n in ("_alpha", "_window_continuous", "_train_selectors")}
+        for n, step in base.items():
+            f = lambda self, *a, _n=n, _s=step, **k: (seen.append(_n), _s(self, *a, **k))[1]  # noqa: E731
+            if where == "class":
+                monkeypatch.setattr(DSALTAttention, n, f)
+            else:
+                mod.__dict__[n] = f.__get__(mod)
+    y = mod(x[None])[0] if dense else mod(x, **packed)[0]
+    y.float().sum().backward()
+    assert {"_alpha", "_window_continuous"} <= set(seen) and ("_train_selectors" in seen) == (not dense)
+    if where == "subclass" and not dense:
+        assert not torch.equal(y, small_module()[0](x, **packed)[0])
+
+
 @pytest.mark.parametrize("frozen", [("q_proj.weight",), ("k_proj.weight", "v_proj.weight", "alpha_w"),
                                     ("win_gate.weight", "win_gate.bias"), ("q_proj.weight", "k_proj.weight", "v_proj.weight")])
 @pytest.mark.parametrize("x_grad", [True, False])
