@@ -53,9 +53,14 @@ class _ModuleAttention(torch.autograd.Function):
                                 opt["tau_win"], opt["win_edge"])
         cast = cdt == torch.float32  # separate fp16 operands; otherwise q and k were rotated in place
         ops = (sel.q_out, sel.k_out, sel.v_out) if cast else (None, None, None)
-        ctx.save_for_backward(x, None if xb is xd else xb, qkv, *ops, w_cat, wg, out, lse, sel.win_logit, sel.win_out,
-                              weight, a32, sel.norms, sel.out, sel.cu, cos, sin)
+        # the weights are saved where x takes a gradient, as four linears would: changed in place
+        # before the backward they are refused then (the backward itself takes w_cat and,
+        # for dx, wg)
+        saved = (wq, wk, wv, wg) if ctx.needs_input_grad[0] else (None,) * 4
+        ctx.save_for_backward(x, None if xb is xd else xb, qkv, *ops, w_cat, out, lse, sel.win_logit, sel.win_out,
+                              weight, a32, sel.norms, sel.out, sel.cu, cos, sin, *saved)
         ctx.dsalt = opt, scale, wq.dtype, alpha_w.dtype
+        ctx.dsalt_gate = None if ctx.needs_input_grad[0] else wg.detach()
         if dense:
             ctx.mark_non_differentiable(sel.out, sel.win_out)
         else:
@@ -66,8 +71,9 @@ class _ModuleAttention(torch.autograd.Function):
     def backward(ctx, grad_out, *_):
         if grad_out is None:
             return (None,) * 12
-        (x, xb, qkv, q_r, k_r, v_r, w_cat, wg, out, lse, logit, w32, weight, a32, norms, pos, cu, cos,
-         sin) = ctx.saved_tensors
+        (x, xb, qkv, q_r, k_r, v_r, w_cat, out, lse, logit, w32, weight, a32, norms, pos, cu, cos, sin,
+         _, _, _, wg) = ctx.saved_tensors
+        wg = ctx.dsalt_gate if wg is None else wg
         opt, scale, w_dtype, a_dtype = ctx.dsalt
         H, n_kv, D, dense, od = opt["n_heads"], opt["n_kv_heads"], opt["head_dim"], opt["dense"], qkv.dtype
         T, grouped = x.shape[0], n_kv != H

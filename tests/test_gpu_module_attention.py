@@ -243,6 +243,28 @@ def test_frozen_parameters_take_no_gradient(frozen, x_grad):
             assert float((g.double() - w).norm()) <= 2 ** -8 * float(w.norm()), n
 
 
+@pytest.mark.parametrize("name", ["q_proj", "k_proj", "v_proj", "win_gate", "alpha_w"])
+@pytest.mark.parametrize("x_grad", [True, False])
+def test_weights_changed_before_the_backward(name, x_grad):
+    """As with linears: a projection's weight changed in place between the passes is refused where
+    it is needed for x's gradient, and taken where x has none."""
+    print(f"module attention changed {name} x_grad={x_grad}", flush=True)
+    mod, x, packed = small_module()
+    x.requires_grad_(x_grad)
+    dy = torch.randn(333, 256, device=DEV).to(x.dtype)
+    ps = [p for n, p in mod.named_parameters() if n != "out_proj.weight"]
+    want = torch.autograd.grad(mod(x, **packed)[0], ps, dy)
+    y = mod(x, **packed)[0]
+    with torch.no_grad():
+        (mod.alpha_w if name == "alpha_w" else getattr(mod, name).weight).mul_(1.5)
+    if x_grad and name != "alpha_w":
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            y.backward(dy)
+    else:
+        for a, b in zip(torch.autograd.grad(y, ps, dy), want):
+            assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype,autocast", [(torch.bfloat16, False), (torch.float16, False), (torch.float32, True)])
 def test_training_windows_are_the_rounded_gate(dtype, autocast):
     """The windows of the norms pass are torch's formula on the correctly rounded logits."""
