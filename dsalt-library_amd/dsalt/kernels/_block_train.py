@@ -37,11 +37,26 @@ def autocast_dtype(x: torch.Tensor) -> torch.dtype:
     return torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
 
 
-def _grads(y: torch.Tensor, inputs, dy: torch.Tensor):
-    """Differentiable gradients of y with respect to the inputs that require one (else None)."""
-    live = [t for t in inputs if t.requires_grad]
-    got = iter(torch.autograd.grad(y, live, dy.to(y.dtype), create_graph=True))
-    return [next(got) if t.requires_grad else None for t in inputs]
+def autocast_state() -> tuple[bool, torch.dtype]:
+    """Autocast as it is here, for ``autocast_as`` in a backward."""
+    return torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda")
+
+
+def autocast_as(state: tuple[bool, torch.dtype]):
+    return torch.autocast("cuda", dtype=state[1], enabled=state[0])
+
+
+def graph_grads(fn, inputs, dys):
+    """Differentiable gradients of fn(*inputs), with the upstream gradients dys of its outputs (None:
+    none), with respect to the inputs that require one (else None). fn sees aliases of the
+    inputs, so that one which depends on another (v on x) gives its own share only."""
+    with torch.enable_grad():
+        alias = [t.view_as(t) if t is not None and t.requires_grad else t for t in inputs]
+        live = [t for t in alias if t is not None and t.requires_grad]
+        pairs = [(y, dy.to(y.dtype)) for y, dy in zip(fn(*alias), dys) if dy is not None and y.requires_grad]
+        got = iter(torch.autograd.grad([y for y, _ in pairs], live, [d for _, d in pairs], create_graph=True,
+                                       allow_unused=True))
+        return [next(got) if t is not None and t.requires_grad else None for t in inputs]
 
 
 class _AddNorm(torch.autograd.Function):
@@ -73,8 +88,7 @@ class _AddNorm(torch.autograd.Function):
             dh = ds.to(h_dtype) if need_h and ds is not None else None
             return ds if need_x else None, dh, None, None, None, None
         if torch.is_grad_enabled():  # a graph of the backward is wanted: torch's own ops
-            y = F.rms_norm(x, x.shape[-1:], weight, eps)
-            dx, dw = _grads(y, (x, weight), dy)
+            dx, dw = graph_grads(lambda x, w: (F.rms_norm(x, x.shape[-1:], w, eps),), (x, weight), (dy,))
             ds = dx if ds is None else ds if dx is None else ds + dx
             dh = ds.to(h_dtype) if need_h else None
             return ds if need_x else None, dh, dw if need_w else None, None, None, None
@@ -125,10 +139,12 @@ class _SwiGLU(torch.autograd.Function):
     def backward(ctx, dy):
         x, wg, wu, wd, gu, a, w_gu, xb, w_d = ctx.saved_tensors
         if torch.is_grad_enabled():  # a graph of the backward is wanted: torch's own ops
+            def ffn(*inputs):
+                xc, g, u, d = (t.to(gu.dtype) for t in inputs)
+                return F.linear(F.silu(F.linear(xc, g)) * F.linear(xc, u), d),
+
             with torch.autocast("cuda", enabled=False):
-                xc, g, u, d = (t.to(gu.dtype) for t in (x, wg, wu, wd))
-                y = F.linear(F.silu(F.linear(xc, g)) * F.linear(xc, u), d)
-                return *_grads(y, (x, wg, wu, wd), dy), None
+                return *graph_grads(ffn, (x, wg, wu, wd), (dy,)), None
         shape, x_dtype, w_dtype, f = x.shape, x.dtype, wg.dtype, wg.shape[0]
         xb = (x.detach() if xb is None else xb).reshape(-1, wg.shape[1])
         w_d = wd.detach() if w_d is None else w_d

@@ -143,6 +143,37 @@ def test_twice_differentiable_and_transformed():
     assert ffn.up_proj.weight.grad is None and ffn.gate_proj.weight.grad is not None
 
 
+def test_second_order_of_dependent_inputs():
+    """A graph of the backward where one input is computed from another (the norm's weight and the
+    feed-forward's weights from x): each gradient counts its own share once."""
+    print("block functions: dependent inputs", flush=True)
+    torch.manual_seed(7)
+    ffn, norm = SwiGLUFFN(64, 72).to(DEV), RMSENorm(64).to(DEV)
+    x = torch.randn(5, 64, device=DEV, requires_grad=True)
+    ws = {n: p.detach() for n, p in ffn.named_parameters()}
+
+    def one():
+        own = {n: p * x.mean() for n, p in ws.items()}
+        w = 1 + x[0]
+        t = RMSENorm(64).to(DEV)
+        t.__dict__["_parameters"] = {"weight": w}
+        s, y = _block_train.add_norm(x, None, t)
+        return torch.func.functional_call(ffn, own, (s + y,))
+
+    def ref():
+        g, u, d = (ws[f"{n}_proj.weight"] * x.mean() for n in ("gate", "up", "down"))
+        h = x + F.rms_norm(x, (64,), 1 + x[0], norm.eps)
+        return F.linear(F.silu(F.linear(h, g)) * F.linear(h, u), d)
+
+    for f in (one, ref):
+        first, = torch.autograd.grad(f().square().sum(), x, create_graph=True)
+        second, = torch.autograd.grad(first.square().sum(), x)
+        if f is one:
+            want = first.detach(), second
+    for a, b in zip(want, (first, second)):
+        assert float((a - b).norm()) <= 1e-4 * float(b.norm())
+
+
 @pytest.mark.parametrize("dtype,autocast", [(FP, True), (BF, False), (BF, True)])
 @pytest.mark.parametrize("checkpoint", [False, True])
 def test_block_matches_separate_ops(dtype, autocast, checkpoint):
