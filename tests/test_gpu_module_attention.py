@@ -331,3 +331,54 @@ def test_non_finite_scores_in_training(T, k):
         if want is not None:
             assert torch.equal(a.isnan(), want.isnan()), n
     assert got[True]["alpha_w"] is None if k == 0 else bool(got[True]["alpha_w"].isnan().all())
+
+
+def second_order(mod, x, packed, dy, autocast=False):
+    """First gradients (with a graph) of x and the parameters, and the gradients of their squares'
+    sum."""
+    ps = [x, *mod.parameters()]
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+        y = mod(x, **packed)[0]
+        first = torch.autograd.grad(y, ps, dy.to(y.dtype), create_graph=True, allow_unused=True)
+        penalty = sum(g.float().square().sum() for g in first if g is not None)
+    return first, torch.autograd.grad(penalty, ps, allow_unused=True)
+
+
+SECOND = {  # H, n_kv, D, dense, dtype, k, autocast
+    "fp32": (4, 4, 64, False, torch.float32, 8, False), "fp32-gqa-d128": (4, 2, 128, False, torch.float32, 8, False),
+    "bf16": (4, 2, 64, False, torch.bfloat16, 8, False), "autocast": (4, 2, 64, False, torch.float32, 8, True),
+    "no-landmarks": (2, 2, 64, False, torch.float32, 0, False), "dense": (4, 2, 64, True, torch.float32, 8, False),
+    "dense-d128": (2, 2, 128, True, torch.float32, 8, False), "dense-autocast": (2, 1, 64, True, torch.float32, 8, True),
+}
+
+
+@pytest.mark.parametrize("case", list(SECOND))
+@pytest.mark.parametrize("route", ["weights"])
+def test_second_order_gradients(case, route):
+    """A graph of the backward holds what torch's projections, gate and landmark weights hold: both
+    the one function and the landmark weights' function ("weights") against torch's ops, whose
+    attention core is a constant in the graph on every route."""
+    H, n_kv, D, dense, dtype, k, autocast = SECOND[case]
+    print(f"module attention second order {case} {route}", flush=True)
+    lens = [130, 77]
+    got = {}
+    for r in (route, "torch"):
+        torch.manual_seed(8)
+        mod = DSALTAttention(H * D, H, 4, 32, k, max_seq_len=300, n_kv_heads=n_kv).to(DEV, dtype).train()
+        mod._fuse_qkv, mod._hip_scores = r == "one", r != "torch"
+        x = torch.randn(sum(lens), H * D, device=DEV).to(dtype)
+        dy = torch.randn(sum(lens), H * D, device=DEV)
+        assert mod._one_function(x) == (r == "one")
+        packed = {} if dense else {"cu_seqlens": torch.tensor([0, 130, 207], dtype=torch.int32, device=DEV)}
+        x, dy = (x[None], dy[None]) if dense else (x, dy)
+        got[r] = second_order(mod, x.detach().requires_grad_(), packed, dy, autocast)
+    # a few roundings of the compute type (the projections' in fp32 take part in fp16 attention)
+    tol = 2e-2 if dtype == torch.bfloat16 or autocast else 2e-3
+    names = ["x", *(n for n, _ in mod.named_parameters())]
+    for order in (0, 1):
+        for n, a, b in zip(names, got[route][order], got["torch"][order]):
+            assert (a is None) == (b is None) and (a is None or a.requires_grad == b.requires_grad), (order, n)
+            if a is None or n == "win_gate.bias":  # a sum of cancelling terms
+                continue
+            a, b = a.detach().double(), b.detach().double()
+            assert float((a - b).norm()) <= tol * float(b.norm()), (order, n, float((a - b).norm() / b.norm()))
