@@ -15,8 +15,11 @@ from __future__ import annotations
 import math
 
 import torch
+import torch.nn.functional as F
 
 from .. import _hip
+from ._block_train import autocast_as, autocast_state, graph_grads
+from ._lmk_weights import torch_weights
 
 
 class _ModuleAttention(torch.autograd.Function):
@@ -61,6 +64,8 @@ class _ModuleAttention(torch.autograd.Function):
                               weight, a32, sel.norms, sel.out, sel.cu, cos, sin, *saved)
         ctx.dsalt = opt, scale, wq.dtype, alpha_w.dtype
         ctx.dsalt_gate = None if ctx.needs_input_grad[0] else wg.detach()
+        # for a graph of the backward only: the parameters themselves, unchecked
+        ctx.dsalt_params, ctx.dsalt_autocast = (wq, wk, wv, wg, bg, alpha_w), autocast_state()
         if dense:
             ctx.mark_non_differentiable(sel.out, sel.win_out)
         else:
@@ -96,6 +101,12 @@ class _ModuleAttention(torch.autograd.Function):
             lp, lw = (pos, weight) if opt["k_lmk"] > 0 else (None, None)
             _, dk_h, dv_h, d_weight, dw = _hip.bwd(_hip.MODE_SOFT, q_r, k_r, v_r, out, lse, grad_out, w32, lp, lw, cu,
                                                       scale, opt["tau_win"], opt["win_edge"], True, gdt, rope, grads)
+        if torch.is_grad_enabled():
+            if grouped:
+                dk, dv = _hip.group_sum_pair(dk_h, dv_h, n_kv, od)
+            if not fused:
+                _hip.rope(dq, dk, cos, sin, cu, transpose=True, q_out=dq, k_out=dk)
+            return (*_graph_grads(ctx, x, v, pos, cu, logit, a32, (dq, dk, dv, dw, d_weight)), *[None] * 5)
         g = _hip.ModuleGrads(x.detach(), v, norms, a32, pos, cu, weight if d_weight is None else d_weight,
                              opt["tau_lmk"], dense)
         d_alpha = g.values(dk_h, dv_h, dk, dv, alpha_sigmoid=True)
@@ -118,6 +129,29 @@ class _ModuleAttention(torch.autograd.Function):
             d_alpha = None  # without landmark slots alpha takes no part
         return (dx, *dws, dwg if ctx.needs_input_grad[4] else None, dbg,
                 None if d_alpha is None else d_alpha.to(a_dtype), *[None] * 5)
+
+
+def _graph_grads(ctx, x, v_saved, pos, cu, logit, a32, core):
+    """The gradients of x and the parameters with a graph, from those of the attention's operands
+    (``core``: un-rotated dq, dk, dv, the windows' and the landmark weights'), which are
+    constants in it, as sparse_attention's are: projections, windows and weights in torch's
+    ops, on the values that the forward had."""
+    opt = ctx.dsalt[0]
+    dq, dk, dv, dw, d_weight = core
+
+    def valued(t, value):  # t's graph at the forward's value
+        return value.to(t.dtype) + (t - t.detach())
+
+    def operands(x, wq, wk, wv, wg, bg, alpha_w):
+        v = valued(F.linear(x, wv).view(v_saved.shape), v_saved)
+        gate = torch.sigmoid(valued(F.linear(x, wg, bg).squeeze(-1), logit))
+        yield from (F.linear(x, wq), F.linear(x, wk), v, opt["n_min"] + gate * (opt["n_max"] - opt["n_min"]))
+        if d_weight is not None:
+            yield torch_weights(x, v, valued(torch.sigmoid(alpha_w), a32), pos, cu, opt["tau_lmk"], opt["dense"])
+
+    with autocast_as(ctx.dsalt_autocast):
+        got = graph_grads(operands, (x, *ctx.dsalt_params), (dq.flatten(1), dk.flatten(1), dv, dw, d_weight))
+    return [g if n else None for g, n in zip(got, ctx.needs_input_grad)]
 
 
 def _split(qkv: torch.Tensor, H: int, n_kv: int, D: int):

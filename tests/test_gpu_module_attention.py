@@ -353,7 +353,7 @@ SECOND = {  # H, n_kv, D, dense, dtype, k, autocast
 
 
 @pytest.mark.parametrize("case", list(SECOND))
-@pytest.mark.parametrize("route", ["weights"])
+@pytest.mark.parametrize("route", ["one", "weights"])
 def test_second_order_gradients(case, route):
     """A graph of the backward holds what torch's projections, gate and landmark weights hold: both
     the one function and the landmark weights' function ("weights") against torch's ops, whose
