@@ -326,6 +326,7 @@ namespace {
 
 int check_operands(const dsalt_scores_args *sa, const dsalt_select_args *a, const dsalt_qkv_args *o) {
     if (!sa->k) return fail(DSALT_ERR_INVALID, "the operands need k (and the RoPE tables) in the score arguments");
+    if (sa->gate_w) return fail(DSALT_ERR_INVALID, "gate_w is not formed with operands: win_w replaces it");
     const bool cast = sa->v_dtype == DSALT_DTYPE_F32 && o->out_dtype == DSALT_DTYPE_F16;
     if (!cast && o->out_dtype != sa->v_dtype)
         return fail(DSALT_ERR_INVALID, "out_dtype must be v_dtype, or F16 for fp32 operands (got %d)", o->out_dtype);
@@ -334,7 +335,6 @@ int check_operands(const dsalt_scores_args *sa, const dsalt_select_args *a, cons
         const bool low = o->win_dtype == DSALT_DTYPE_BF16 || o->win_dtype == DSALT_DTYPE_F16;
         if (o->win_dtype != sa->x_dtype && !(low && sa->x_dtype == DSALT_DTYPE_F32))
             return fail(DSALT_ERR_INVALID, "win_dtype must be x_dtype, or a 16-bit type for fp32 x (got %d)", o->win_dtype);
-        if (sa->gate_w) return fail(DSALT_ERR_INVALID, "win_w replaces gate_w");
         if (!o->win_logit || !o->win_out) return fail(DSALT_ERR_INVALID, "win_w needs win_logit and win_out");
         if (!aligned(o->win_w, 16) || !aligned(o->win_b, sa->x_dtype == DSALT_DTYPE_F32 ? 4 : 2))
             return fail(DSALT_ERR_INVALID, "win_w must be 16-byte aligned, win_b to its element");

@@ -908,6 +908,10 @@ class SelectHybridLauncher:
             norms_f32 = autocast_norms()
         if gate_linear is not None and (gate is not None or w_cont is not None):
             raise DsaltError("gate_linear replaces gate and w_cont: pass neither with it")
+        if rope_q is not None and gate_linear is not None:
+            raise DsaltError("the norms pass that rotates q forms no gate_linear: pass window")
+        if window is not None and (rope_q is None or gate is not None or w_cont is not None):
+            raise DsaltError("window goes with rope_q and replaces gate and w_cont")
         self.device = require_gpu(x, v, alpha, cu_seqlens, gate_linear[0] if gate_linear is not None else
                                   window[0] if window is not None else w_cont if gate is None else gate[0])
         x, v, alpha = _score_operands(x, v, alpha, n_heads)

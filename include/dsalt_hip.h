@@ -389,7 +389,7 @@ int dsalt_select_hybrid(const dsalt_scores_args *scores, const dsalt_select_args
  * win_dtype. win_w [d_model] (16-byte aligned) and win_b [1] (may be NULL) in x_dtype;
  * win_logit and win_out [T] fp32. Replaces _window_continuous
  * (dsalt/modules/dsalt_attention.py:270-276); `select` takes its windows from win_out
- * (w = win_out; scores->gate_w must be NULL).
+ * (w = win_out). scores->gate_w must be NULL, with win_w and without.
  */
 typedef struct dsalt_qkv_args {
     int32_t out_dtype;

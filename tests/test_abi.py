@@ -6,6 +6,7 @@ import os
 import re
 
 import pytest
+import torch
 
 import dsalt._hip as hip
 
@@ -319,6 +320,33 @@ def test_dense_mode_checks():
                        (dict(num_seqs=1, k_lmk=0, lmk_pos=None, scale=-0.125), "scale > 0")):
         rc, msg = _check(_fake_fwd(mode=hip.MODE_DENSE, **kw))
         assert rc != 0 and needle in msg, (kw, rc, msg)
+
+
+def test_operand_form_rejects_the_gate_logits():
+    """The norms pass that writes the attention's operands has no gate_w form: with or without its
+    own window gate, gate_w is refused (its logits would never be written), on the host and in
+    the launcher; so is a window gate without the operands."""
+    lib = hip.lib()
+    a = _scores_args(scores=0, k=0x110000, k_out=0x120000, rope_cos=0x130000, rope_sin=0x140000, rope_rows=300,
+                     rope_stride=64, k_stride_t=512, k_stride_h=64, k_out_stride_t=512, k_out_stride_h=64,
+                     gate_w=0x60000, gate_out=0x80000)
+    sel = hip.SelectArgs()
+    sel.total_len, sel.num_seqs, sel.n_heads, sel.k_lmk = a.total_len, 1, a.n_heads, 4
+    sel.w_logit, sel.w_logit_dtype, sel.w_out, sel.w_logit_stride = 0x80000, a.x_dtype, 0x90000, 1
+    sel.cu_seqlens, sel.lmk_pos, sel.n_min, sel.n_max = 0x3000, 0x4000, 8, 64
+    for win in (0, 0x70000):
+        o = hip.QkvArgs()
+        o.out_dtype, o.win_w, o.win_logit, o.win_out, o.win_dtype = a.v_dtype, win, 0x200000, 0x210000, a.x_dtype
+        assert lib.dsalt_select_hybrid_qkv(ctypes.byref(a), ctypes.byref(sel), ctypes.byref(o), None) == 1
+        assert "gate_w" in lib.dsalt_last_error().decode()
+    x, v, q = torch.zeros(4, 64), torch.zeros(4, 1, 64), torch.zeros(4, 1, 64)
+    cu, w = torch.tensor([0, 4]), torch.zeros(1, 64)
+    args = (x, v, torch.ones(1), 1)
+    with pytest.raises(hip.DsaltError, match="gate_linear"):
+        hip.SelectHybridLauncher(*args, None, cu, 2, gate_linear=(w, None, 1, 2), rope_q=q)
+    for bad in (dict(), dict(rope_q=q, gate=(x[:, 0], 1, 2))):
+        with pytest.raises(hip.DsaltError, match="window goes with rope_q"):
+            hip.SelectHybridLauncher(*args, None, cu, 2, window=(w, None, x.dtype, 1, 2), **bad)
 
 
 def test_select_hybrid_rejects_before_launching():
