@@ -4,6 +4,8 @@ residual add alone, and the SwiGLU feed-forward as one function each
 """
 from __future__ import annotations
 
+import functools
+
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
@@ -44,6 +46,19 @@ def autocast_state() -> tuple[bool, torch.dtype]:
 
 def autocast_as(state: tuple[bool, torch.dtype]):
     return torch.autocast("cuda", dtype=state[1], enabled=state[0])
+
+
+def without_autocast(backward):
+    """A backward whose operands have their types already: an autocast that is on where it runs
+    (a backward called inside one, maybe of another type than the forward's) changes nothing."""
+    @functools.wraps(backward)
+    def call(ctx, *grads):
+        if not torch.is_autocast_enabled("cuda"):
+            return backward(ctx, *grads)
+        with torch.autocast("cuda", enabled=False):
+            return backward(ctx, *grads)
+
+    return call
 
 
 def graph_grads(fn, inputs, dys):
@@ -136,6 +151,7 @@ class _SwiGLU(torch.autograd.Function):
         return y.view(*x.shape[:-1], wd.shape[0])
 
     @staticmethod
+    @without_autocast
     def backward(ctx, dy):
         x, wg, wu, wd, gu, a, w_gu, xb, w_d = ctx.saved_tensors
         if torch.is_grad_enabled():  # a graph of the backward is wanted: torch's own ops
@@ -143,8 +159,7 @@ class _SwiGLU(torch.autograd.Function):
                 xc, g, u, d = (t.to(gu.dtype) for t in inputs)
                 return F.linear(F.silu(F.linear(xc, g)) * F.linear(xc, u), d),
 
-            with torch.autocast("cuda", enabled=False):
-                return *graph_grads(ffn, (x, wg, wu, wd), (dy,)), None
+            return *graph_grads(ffn, (x, wg, wu, wd), (dy,)), None
         shape, x_dtype, w_dtype, f = x.shape, x.dtype, wg.dtype, wg.shape[0]
         xb = (x.detach() if xb is None else xb).reshape(-1, wg.shape[1])
         w_d = wd.detach() if w_d is None else w_d

@@ -18,7 +18,7 @@ import torch
 import torch.nn.functional as F
 
 from .. import _hip
-from ._block_train import autocast_as, autocast_state, graph_grads
+from ._block_train import autocast_as, autocast_state, graph_grads, without_autocast
 from ._lmk_weights import torch_weights
 
 
@@ -73,6 +73,7 @@ class _ModuleAttention(torch.autograd.Function):
         return out, sel.out, sel.win_out, sel.w_out
 
     @staticmethod
+    @without_autocast
     def backward(ctx, grad_out, *_):
         if grad_out is None:
             return (None,) * 12

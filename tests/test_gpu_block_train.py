@@ -7,6 +7,7 @@ import torch.nn.functional as F
 from dsalt import _hip
 from dsalt.kernels import _block_train
 from dsalt.kernels.RMSENorm import RMSENorm
+from dsalt.modules import DSALTAttention
 from dsalt.modules.dsalt_transformer import DSALTTransformerBlock, SwiGLUFFN
 
 pytestmark = pytest.mark.gpu
@@ -141,6 +142,34 @@ def test_twice_differentiable_and_transformed():
     ffn.zero_grad()
     ffn(x).sum().backward()
     assert ffn.up_proj.weight.grad is None and ffn.gate_proj.weight.grad is not None
+
+
+@pytest.mark.parametrize("fwd", [None, HF, BF])
+@pytest.mark.parametrize("bwd", [HF, BF])
+@pytest.mark.parametrize("part", ["ffn", "attention"])
+def test_backward_inside_autocast(part, fwd, bwd):
+    """A backward called inside an autocast, of the forward's type or another, gives the gradients
+    that it gives outside."""
+    print(f"{part}: backward inside autocast fwd={fwd} bwd={bwd}", flush=True)
+    torch.manual_seed(5)
+    if part == "ffn":
+        mod = SwiGLUFFN(128, 264).to(DEV)
+        run = mod
+    else:
+        mod = DSALTAttention(128, 2, 4, 30, 4, max_seq_len=100).to(DEV).train()
+        mod._apply_out_proj = lambda o: o  # torch's linear follows the autocast around its backward
+        cu = torch.tensor([0, 75], dtype=torch.int32, device=DEV)
+        run = lambda x: mod(x, cu_seqlens=cu)[0]  # noqa: E731
+    x = torch.randn(75, 128, device=DEV, requires_grad=True)
+    got = []
+    for inside in (False, True):
+        with torch.autocast("cuda", dtype=fwd or BF, enabled=fwd is not None):
+            y = run(x)
+        with torch.autocast("cuda", dtype=bwd, enabled=inside):
+            got.append(torch.autograd.grad(y, [x, *(p for n, p in mod.named_parameters() if "out_proj" not in n)],
+                                           torch.ones_like(y)))
+    for a, b in zip(*got):
+        assert a.dtype == b.dtype and torch.equal(a, b)
 
 
 def test_second_order_of_dependent_inputs():
