@@ -145,10 +145,12 @@ class _SwiGLU(torch.autograd.Function):
             w_d = wd.detach().to(dtype)
         gu = torch.mm(xb, w_gu.t())
         a = _hip.swiglu_rows(gu)
-        y = torch.mm(a, w_d.t())
+        # not a view of the GEMM's result: torch lets no one modify a view from a function in place
+        y = torch.empty((*x.shape[:-1], w_d.shape[0]), device=x.device, dtype=dtype)
+        torch.mm(a, w_d.t(), out=y.view(-1, w_d.shape[0]))
         cast = xb.dtype != x.dtype
         ctx.save_for_backward(x, wg, wu, wd, gu, a, w_gu, xb if cast else None, w_d if w_d.dtype != wd.dtype else None)
-        return y.view(*x.shape[:-1], wd.shape[0])
+        return y
 
     @staticmethod
     @without_autocast

@@ -172,6 +172,29 @@ def test_backward_inside_autocast(part, fwd, bwd):
         assert a.dtype == b.dtype and torch.equal(a, b)
 
 
+@pytest.mark.parametrize("dtype,autocast", [(FP, True), (BF, False)])
+@pytest.mark.parametrize("shape", [(40, 128), (1, 40, 128)])
+def test_outputs_can_be_modified_in_place(dtype, autocast, shape):
+    """Hooks that scale the feed-forward's or the attention's output in place, as on torch's ops."""
+    print(f"block in place {dtype} {shape}", flush=True)
+    torch.manual_seed(2)
+    block = DSALTTransformerBlock(128, 2, 4, 30, 4, 100, 264).to(DEV, dtype).train()
+    x = torch.randn(shape, device=DEV).to(dtype)
+    packed = {} if len(shape) == 3 else {"cu_seqlens": torch.tensor([0, 40], dtype=torch.int32, device=DEV)}
+    got = []
+    for inplace in (True, False):
+        hooks = [block.ffn.register_forward_hook(lambda m, a, o: o.mul_(2) if inplace else o * 2),
+                 block.attn.register_forward_hook(lambda m, a, o: (o[0].mul_(2) if inplace else o[0] * 2, o[1]))]
+        xx = x.clone().requires_grad_()
+        with torch.autocast("cuda", dtype=BF, enabled=autocast):
+            y, _ = block(xx, **packed)
+        got.append([y.detach(), *torch.autograd.grad(y.float().sum(), [xx, *block.parameters()])])
+        for hk in hooks:
+            hk.remove()
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
 def test_second_order_of_dependent_inputs():
     """A graph of the backward where one input is computed from another (the norm's weight and the
     feed-forward's weights from x): each gradient counts its own share once."""
