@@ -12,7 +12,8 @@
 // element is produced by exactly one thread, in a fixed order.
 //
 // Kernels, launched in this order on one stream:
-//   dq      query-parallel, kDqW waves x 32 queries per workgroup, the forward's tiling
+//   dq      query-parallel, two waves (long sequences: see launch_dq) x 32 queries per
+//           workgroup, the forward's tiling
 //           (band tiles of kDqBN keys, then gathered landmark tiles); S^T, dP^T and dQ^T
 //           on MFMA. Computes
 //           Delta = rowsum(O * dO) for its queries and writes dQ, the per-head soft-edge
@@ -50,11 +51,8 @@ constexpr int kv_bm(int d) { return 32 * kv_waves(d); }  // keys per band kv wor
 constexpr int kv_qt(int d) { return d == 64 ? 32 : 64; }
 constexpr int kv_stages(int) { return 4; }
 constexpr int kTN = 64;     // queries per lmk_kv tile
-constexpr int kDqW = 4;     // waves per dq workgroup
-constexpr int kDqBM = 32 * kDqW;  // queries per dq workgroup (32 per wave)
 constexpr int kDqBN = 32;   // keys per dq tile
 constexpr int kMinBM = 64;  // queries per smallest-band-start entry (bounds the scan of kv)
-constexpr int kDqStages = 4;  // dq LDS ring depth
 constexpr int kLC = 512;  // queries per lmk_kv chunk (chunks are numbered like query blocks)
 
 // Tile kinds of the dq loop phases (kDiagTile, kRowTile: initial-value rows, see below).
@@ -67,6 +65,10 @@ enum { kCoreTile = 0, kEdgeTile = 1, kLmkTile = 2, kDiagTile = 3, kRowTile = 4 }
 // edges form them per element: as factors while those stay in the fp32 range (kEdgeFast),
 // else one exp per element (kEdgeExact). HARD windows have no edge (kEdgeExact).
 enum { kEdgeExact = 0, kEdgeFast = 1, kEdgeTab = 2 };
+// Two-stage rings of dq (see launch_dq); four waves for long sequences.
+constexpr bool dq_two_stages(int d, int mode, int edge) { return d == 64 || mode == kHard || edge == kEdgeTab; }
+constexpr int kDqLong = 1024;    // mean sequence length and
+constexpr int kDqWide = 256;     // four-wave workgroups from which dq takes them
 constexpr int kEdgeKeys = 4;
 // dq: a query's row of initial values holds keys lo - 4 .. lo + 7 (read four consecutive keys
 // at a time from a start clamped to lo - 4 .. lo + 4); rows start in 32 different banks
@@ -127,6 +129,15 @@ struct BwdParams {
     RopeRows rope; // q and k were rotated with these tables: dq and dk are returned un-rotated
 };
 
+// The kernel argument at byte offset `off`, read here (see late_rope_rows).
+template <typename T>
+__device__ __forceinline__ T late_arg(size_t off) {
+    typedef const __attribute__((address_space(4))) char *kptr;
+    uint64_t a = (uint64_t)(kptr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(a));
+    return *(const __attribute__((address_space(4))) T *)(a + off);
+}
+
 __device__ __forceinline__ uint4 ld16(const uint16_t *p) { return *reinterpret_cast<const uint4 *>(p); }
 
 // A operand of a k-step over 16 tokens from a transposed tile row: 4 tokens at `at` and
@@ -171,32 +182,29 @@ __device__ __forceinline__ void pack_block(const f32x16 &x, uint32_t (&pk)[8]) {
 // ==================================================================================
 // dq: query-parallel dQ (band + landmarks) and per-head soft-edge d_w~
 // ==================================================================================
-// The forward's structure: one workgroup = kDqW waves x 32 queries of one (sequence,
-// head); K and V tiles of kDqBN keys stream through a kDqStages-deep LDS ring by direct
-// global->LDS loads (band tiles from the diagonal down, then the gathered landmark
-// tiles). Four waves share a ring of four stages (32 KB at D = 64), so that with the rows below
-// three workgroups, 12 waves, fit a CU's LDS as they fit its registers (two waves on three
-// stages: 5 workgroups, 10 waves). Per tile a wave
+// The forward's structure: one workgroup = NW waves x 32 queries of one (sequence, head);
+// K and V tiles of kDqBN keys stream through an NSTAGE-deep LDS ring by direct global->LDS
+// loads (band tiles from the diagonal down, then the gathered landmark tiles); launch_dq
+// picks NW and NSTAGE. Per tile a wave
 // computes S^T = K.Q^T and dP^T = V.dO^T (lane = query column), P = 2^(S c + bias - lse2)
 // on admitted pairs, dS = P (dP - Delta), and dQ^T += K^T.dS^T with K read transposed.
-// HARD windows and SOFT windows of at most kEdgeKeys edge keys (kEdgeTab) start S^T from the
-// query's row of initial values and dP^T from -Delta: a band element then takes a
-// product, an exp2 and a product, where the mask took three more operations and an edge
-// element, which with windows that differ from query to query nearly every one is, fourteen
-// and a reciprocal. 9290 tokens x 16 heads x 64, windows 32 - 512: 62.4 -> 60.4 us. Of that 29
-// are the reads of Q, dO, O and the stores (95 MB); the loop is a chain of LDS, MFMA and exp
-// latencies at 2.2 waves per SIMD (VALU 34 %, LDS 39 %, MFMA 17 % busy).
-template <typename DT, int D, int MODE, int EDGE>
-__global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(const BwdParams p) {
+// SOFT windows of at most kEdgeKeys edge keys (kEdgeTab) start S^T from the query's row of
+// initial values and dP^T from -Delta: a band element then takes a product, an exp2 and a
+// product, where the mask took three more operations and an edge element, which with
+// windows that differ from query to query nearly every one is, fourteen and a reciprocal.
+// 9290 tokens x 16 heads x 64, windows 32 - 512: 67.1 -> 62.1 us, of which 29 are the reads of
+// Q, dO, O and the stores (95 MB); the loop is a chain of LDS, MFMA and exp latencies. HARD
+// bands take the bit mask: from rows they measured the same at D = 64 and 1 - 5 % slower
+// at 128 in batches that do not fill the chip.
+template <typename DT, int D, int MODE, int EDGE, int NW, int NSTAGE>
+__global__ void __launch_bounds__(64 * NW, D == 64 ? 3 : 2) bwd_dq_kernel(const BwdParams p) {
     typedef typename DT::vec8 vec8;
     constexpr bool EFAST = EDGE == kEdgeFast, TAB = EDGE == kEdgeTab;
-    constexpr bool ROWS = MODE == kHard || TAB;  // band scores start from per-query rows
-    constexpr int NW = kDqW, BM = kDqBM, NT = 64 * NW;
+    constexpr int BM = 32 * NW, NT = 64 * NW;  // queries (32 per wave), threads
     constexpr int BN = kDqBN, NRB = BN / 32;
     constexpr int KS = D / 16, ND = D / 32;
     typedef TileN<D, BN, NW> Tile;
     constexpr int TB = Tile::BYTES;
-    constexpr int NSTAGE = kDqStages;
     constexpr int LPT = 2 * Tile::LOADS_PER_WAVE;
 
     __shared__ __align__(1024) char s_tiles[NSTAGE][2][TB];  // [stage][K, V], both row-swizzled
@@ -204,7 +212,7 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
     __shared__ int s_ltmin[DSALT_MAX_K_LMK / BN];
     // SOFT edge factors ec[j] = exp((kEdgeMid - cst_j) / tau) of the element slots j
     __shared__ __align__(16) float s_ec[EFAST ? 16 * NRB : 4];
-    __shared__ float s_ini[ROWS ? ini_row(BM) : 1];
+    __shared__ float s_ini[TAB ? ini_row(BM) : 1];
     __shared__ float s_ds[TAB ? ds_row(BM) + 8 : 1];
     extern __shared__ int s_dyn[];
     int *s_lpos = s_dyn;                                          // INT_MAX: empty slot
@@ -224,6 +232,11 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
     int head, rank;
     head_rank(blockIdx.x, p.grid_dq, p.n_heads, p.n_dqblk, head, rank);
     if (head >= p.n_heads) return;
+    // find_block numbers blocks with gaps. Sequences of a block each leave every second number
+    // empty, and a regular gap leaves shader engines idle (144 x 64 tokens: 49 us, 34 with the
+    // even numbers first)
+    if (p.num_seqs > 64 && p.total_len <= BM * p.num_seqs)
+        rank = 2 * rank < p.n_dqblk ? 2 * rank : 2 * (rank - (p.n_dqblk + 1) / 2) + 1;
     int seq, blk, seq_start, seq_len;
     if (!find_block_desc(p.cu, p.num_seqs, p.total_len, rank, p.n_dqblk, BM, lane, seq, blk, seq_start, seq_len)) return;
     const int wq0 = blk * BM + wave * 32;
@@ -326,7 +339,7 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
         }
     }
     float edw[2] = {0.f, 0.f};
-    if constexpr (ROWS) {
+    if constexpr (TAB) {
         // the query's row, raw units: -inf below the band, log2 sigmoid((w~ - d) / tau) for lo
         // <= key < corelo, 0 in the core, each minus the LSE; the lane pair splits it
         constexpr int EH = kIniLen / 2;
@@ -335,26 +348,21 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
 #pragma unroll
         for (int e = 0; e < EH; ++e) {
             const int x = hh * EH + e - 4;
-            float bias = 0.f;
-            if constexpr (TAB) {
-                float oms;
-                bias = soft_edge_log2(wc, (float)(i - lo - x), p.inv_tau, oms);
-            }
+            float oms;
+            const float bias = soft_edge_log2(wc, (float)(i - lo - x), p.inv_tau, oms);
             const float v = (x < 0 ? -INFINITY : (x < ne ? bias : 0.f) - lse2) * p.inv_c2;
             row[e + hh * EH] = v;
-            if constexpr (TAB)
-                if (qvalid && x >= 0 && x < kEdgeKeys)
-                    p.ws_qrec[((size_t)head * kRecFields + kTabIni + x) * p.total_len + tok_i] = v;
+            if (qvalid && x >= 0 && x < kEdgeKeys)
+                p.ws_qrec[((size_t)head * kRecFields + kTabIni + x) * p.total_len + tok_i] = v;
         }
-        if constexpr (TAB) {  // d log2 sigmoid / d w~ of the two edge keys whose dS this lane sums
-            float *ds = s_ds + ds_row(wave * 32 + ql) + 4 + 2 * hh;
+        // d log2 sigmoid / d w~ of the two edge keys whose dS this lane sums
+        float *ds = s_ds + ds_row(wave * 32 + ql) + 4 + 2 * hh;
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int x = 2 * hh + e;
-                soft_edge_log2(wc, (float)(i - lo - x), p.inv_tau, edw[e]);
-                edw[e] = x < ne ? edw[e] * p.inv_tau : 0.f;
-                ds[e] = 0.f;  // no tile writes it where the band holds fewer keys
-            }
+        for (int e = 0; e < 2; ++e) {
+            const int x = 2 * hh + e;
+            soft_edge_log2(wc, (float)(i - lo - x), p.inv_tau, edw[e]);
+            edw[e] = x < ne ? edw[e] * p.inv_tau : 0.f;
+            ds[e] = 0.f;  // no tile writes it where the band holds fewer keys
         }
     }
     const int wpmax = wave_max_u(qvalid ? pmax : -1);
@@ -535,14 +543,12 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
                             if constexpr (KIND == kDiagTile) y = (rb * 32 + acc_row_const(r) <= A) ? y : -INFINITY;
                             ds4[e] = fast_exp2(y) * pacc[rb][r];
                         }
-                        if constexpr (TAB) {  // the edge keys' dS, for d_w~
-                            const int x = x0 + 32 * rb + 8 * g;  // key - lo of the group
-                            if ((uint32_t)(x + 3) < (uint32_t)(kEdgeKeys + 3)) {
-                                drow[x] = ds4[0];
-                                drow[x + 1] = ds4[1];
-                                drow[x + 2] = ds4[2];
-                                drow[x + 3] = ds4[3];
-                            }
+                        const int x = x0 + 32 * rb + 8 * g;  // key - lo of the group
+                        if ((uint32_t)(x + 3) < (uint32_t)(kEdgeKeys + 3)) {  // the edge keys' dS, for d_w~
+                            drow[x] = ds4[0];
+                            drow[x + 1] = ds4[1];
+                            drow[x + 2] = ds4[2];
+                            drow[x + 3] = ds4[3];
                         }
                         pk[rb][2 * g] = DT::pack2(ds4[0], ds4[1]);
                         pk[rb][2 * g + 1] = DT::pack2(ds4[2], ds4[3]);
@@ -681,7 +687,7 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
 
     tile_barrier<(NSTAGE - 2) * LPT>();  // tile 0 landed (later ones may be in flight)
     int t = 0;
-    if constexpr (ROWS) {
+    if constexpr (TAB) {
         // only the first BM / BN tiles hold keys after a query of the workgroup
         for (; t < BM / BN; ++t) tile(t, std::integral_constant<int, kDiagTile>());
         for (; t < nb; ++t) tile(t, std::integral_constant<int, kRowTile>());
@@ -692,15 +698,19 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
     for (; t < nt; ++t) tile(t, std::integral_constant<int, kLmkTile>());
 
     if (qvalid) {
-        float mul = p.scale;
+        float mul = late_arg<float>(offsetof(BwdParams, scale));
         const RopeRows rope = late_rope_rows(offsetof(BwdParams, rope));
         if (rope.cos) {
             rotate_acc_transposed<DT, ND>(dqacc, mul, rope, i, hh);
             mul = 1.f;
         }
-        store_row<DT, ND>(p.dq, tok_i * p.dq_st + (int64_t)head * p.dq_sh, p.dq_f32, dqacc, mul, hh);
+        const int64_t row = tok_i * late_arg<int64_t>(offsetof(BwdParams, dq_st)) +
+                            (int64_t)head * late_arg<int64_t>(offsetof(BwdParams, dq_sh));
+        store_row<DT, ND>(late_arg<void *>(offsetof(BwdParams, dq)), row, late_arg<int>(offsetof(BwdParams, dq_f32)), dqacc,
+                          mul, hh);
     }
-    if (MODE == kSoft && p.ws_dwh) {
+    float *const dwh = late_arg<float *>(offsetof(BwdParams, ws_dwh));
+    if (MODE == kSoft && dwh) {
         float dwt;
         if constexpr (TAB) {
             __builtin_amdgcn_wave_barrier();  // a wave's LDS operations run in order
@@ -708,7 +718,7 @@ __global__ void __launch_bounds__(64 * kDqW, D == 64 ? 3 : 2) bwd_dq_kernel(cons
         } else {
             dwt = half_sum(dw) * p.inv_tau;
         }
-        if (hh == 0 && qvalid) p.ws_dwh[tok_i * p.n_heads + head] = dwt;
+        if (hh == 0 && qvalid) dwh[tok_i * late_arg<int>(offsetof(BwdParams, n_heads)) + head] = dwt;
     }
 }
 
@@ -1597,6 +1607,32 @@ WsLayout ws_layout(int T, int S, int H, int D, int k) {
 inline bool dq_edge_fast(const BwdParams &p) { return (p.win_edge + 1.f + 16.f * (kDqBN / 32)) * p.inv_tau < 80.f; }
 inline bool kv_edge_fast(const BwdParams &p) { return (p.win_edge + 33.f) * p.inv_tau < 80.f; }
 
+// Two waves on a ring of two stages wherever their registers allow it: the ring is then small
+// enough that registers, not LDS, bound the waves on a CU (D = 64: 12 waves, 10 with three
+// stages; D = 128: 8 waves, 6), and a sequence of up to 64 tokens leaves no wave idle.
+// dq (SOFT, rows) in us at ~9200 tokens, two waves x two stages against two x three and four
+// x four: D = 64, 16 heads, sequences of 32: 40 / 43 / 55, of 128: 37 / 40 / 55, eight of 1161:
+// 62 / 66 / 66; D = 128, 8 heads: 41 / 54 / 56, 38 / 46 / 60, 57 / 81 / 65. SOFT edges wider
+// than kEdgeKeys at D = 128 need too many registers for two stages: three, and for long
+// sequences that give every CU a workgroup of them, four waves on four (16 heads, two x
+// three against four x four: one sequence of 8192 133 / 112, four of 2048 116 / 106, 12 of 768
+// 114 / 112, 36 of 256 82 / 87, 72 of 128 73 / 121; 8 heads, one of 2048: 34 / 38).
+template <typename DT, int D, int MODE, int EDGE>
+void launch_dq(BwdParams p, size_t dyn, hipStream_t stream) {
+    const auto run = [&](auto waves, auto stages) {
+        constexpr int NW = decltype(waves)::value, NS = decltype(stages)::value;
+        p.n_dqblk = block_upper_bound(p.total_len, p.num_seqs, 32 * NW);
+        p.grid_dq = (int)(((int64_t)p.n_dqblk * p.n_heads + 7) / 8 * 8);
+        hipLaunchKernelGGL((bwd_dq_kernel<DT, D, MODE, EDGE, NW, NS>), dim3(p.grid_dq), dim3(64 * NW), dyn, stream, p);
+    };
+    using two = std::integral_constant<int, 2>;
+    using three = std::integral_constant<int, 3>;
+    using four = std::integral_constant<int, 4>;
+    if constexpr (dq_two_stages(D, MODE, EDGE)) run(two(), two());
+    else if (p.total_len / p.num_seqs >= kDqLong && p.total_len / 128 * p.n_heads >= kDqWide) run(four(), four());
+    else run(two(), three());
+}
+
 template <typename DT, int D, int MODE>
 hipError_t launch_typed(const BwdParams &p, hipStream_t stream) {
     // dq writes the per-query records that the key-parallel passes stream
@@ -1606,7 +1642,7 @@ hipError_t launch_typed(const BwdParams &p, hipStream_t stream) {
     const int grid_kv = p.grid_q + ((p.k_lmk > 0 && p.d_bias) ? p.n_heads * p.num_seqs : 0);
     const auto run = [&](auto dq_edge, auto lmk_edge, auto kv_edge) {
         constexpr int DQ = decltype(dq_edge)::value, LM = decltype(lmk_edge)::value, KV = decltype(kv_edge)::value;
-        hipLaunchKernelGGL((bwd_dq_kernel<DT, D, MODE, DQ>), dim3(p.grid_dq), dim3(64 * kDqW), dyn, stream, p);
+        launch_dq<DT, D, MODE, DQ>(p, dyn, stream);
         if (p.k_lmk > 0)
             hipLaunchKernelGGL((bwd_kv_kernel<DT, D, MODE, true, LM>), dim3(p.n_heads * p.n_lgrp * p.n_lchunk), dim3(256),
                                0, stream, p);
@@ -1738,8 +1774,6 @@ hipError_t launch_bwd(const dsalt_bwd_args &a, const dsalt_rope_tables *rope, hi
     p.n_lchunk = block_upper_bound(a.total_len, a.num_seqs, kLC);
     p.n_qblk = block_upper_bound(a.total_len, a.num_seqs, kv_bm(a.head_dim));
     p.grid_q = (int)(((int64_t)p.n_qblk * a.n_heads + 7) / 8 * 8);
-    p.n_dqblk = block_upper_bound(a.total_len, a.num_seqs, kDqBM);
-    p.grid_dq = (int)(((int64_t)p.n_dqblk * a.n_heads + 7) / 8 * 8);
     p.scale = a.scale;
     p.scale_log2 = a.scale * kLog2e;
     p.inv_c2 = 1.f / p.scale_log2;
