@@ -74,6 +74,11 @@ def graph_grads(fn, inputs, dys):
         return [next(got) if t is not None and t.requires_grad else None for t in inputs]
 
 
+def valued(t: torch.Tensor, value: torch.Tensor) -> torch.Tensor:
+    """t's graph at the value that the forward had (a parameter may have changed since)."""
+    return value.to(t.dtype) + (t - t.detach())
+
+
 class _AddNorm(torch.autograd.Function):
     """(x_out, y): the sum (x itself without h) and its norm, in x's dtype or only rounded to
     `cast` (cast_only); with both, y_cast is a third output that takes no gradient."""
@@ -149,29 +154,36 @@ class _SwiGLU(torch.autograd.Function):
         y = torch.empty((*x.shape[:-1], w_d.shape[0]), device=x.device, dtype=dtype)
         torch.mm(a, w_d.t(), out=y.view(-1, w_d.shape[0]))
         cast = xb.dtype != x.dtype
-        ctx.save_for_backward(x, wg, wu, wd, gu, a, w_gu, xb if cast else None, w_d if w_d.dtype != wd.dtype else None)
+        # the weights are saved where a gradient needs them, as three linears would: changed in place
+        # before the backward they are refused then (the backward itself takes w_gu and w_d)
+        need_x, need_g, need_u = ctx.needs_input_grad[:3]
+        saved = (wg, wu) if need_x else (None, None)
+        ctx.save_for_backward(x, *saved, wd if need_x or need_g or need_u else None, gu, a, w_gu, xb if cast else None,
+                              w_d if w_d.dtype != wd.dtype else None)
+        ctx.dsalt_params = wg, wu, wd  # for a graph of the backward: the parameters, unchecked
         return y
 
     @staticmethod
     @without_autocast
     def backward(ctx, dy):
-        x, wg, wu, wd, gu, a, w_gu, xb, w_d = ctx.saved_tensors
+        x, _, _, wd, gu, a, w_gu, xb, w_d = ctx.saved_tensors
         if torch.is_grad_enabled():  # a graph of the backward is wanted: torch's own ops
             def ffn(*inputs):
                 xc, g, u, d = (t.to(gu.dtype) for t in inputs)
-                return F.linear(F.silu(F.linear(xc, g)) * F.linear(xc, u), d),
+                xc, f = xc.reshape(-1, xc.shape[-1]), g.shape[0]
+                h = F.silu(valued(F.linear(xc, g), gu[:, :f])) * valued(F.linear(xc, u), gu[:, f:])
+                return F.linear(h, d).view(dy.shape),
 
-            return *graph_grads(ffn, (x, wg, wu, wd), (dy,)), None
-        shape, x_dtype, w_dtype, f = x.shape, x.dtype, wg.dtype, wg.shape[0]
-        xb = (x.detach() if xb is None else xb).reshape(-1, wg.shape[1])
-        w_d = wd.detach() if w_d is None else w_d
-        dy = dy.reshape(-1, w_d.shape[0])
+            return *graph_grads(ffn, (x, *ctx.dsalt_params), (dy,)), None
+        shape, x_dtype, w_dtype, f = x.shape, x.dtype, ctx.dsalt_params[0].dtype, a.shape[1]
+        xb = (x.detach() if xb is None else xb).reshape(-1, shape[-1])
+        dy = dy.reshape(-1, dy.shape[-1])
         need_x, need_g, need_u, need_d = ctx.needs_input_grad[:4]
         dx = dg = du = dwd = None
         if need_d:
             dwd = torch.mm(dy.t(), a).to(w_dtype)
         if need_x or need_g or need_u:
-            dgu = _hip.swiglu_rows(gu, torch.mm(dy, w_d))
+            dgu = _hip.swiglu_rows(gu, torch.mm(dy, wd.detach() if w_d is None else w_d))
             if need_g and need_u:
                 dg, du = torch.mm(dgu.t(), xb).to(w_dtype).split(f)
             else:

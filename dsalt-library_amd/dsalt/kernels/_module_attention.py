@@ -18,7 +18,7 @@ import torch
 import torch.nn.functional as F
 
 from .. import _hip
-from ._block_train import autocast_as, autocast_state, graph_grads, without_autocast
+from ._block_train import autocast_as, autocast_state, graph_grads, valued, without_autocast
 from ._lmk_weights import torch_weights
 
 
@@ -139,9 +139,6 @@ def _graph_grads(ctx, x, v_saved, pos, cu, logit, a32, core):
     ops, on the values that the forward had."""
     opt = ctx.dsalt[0]
     dq, dk, dv, dw, d_weight = core
-
-    def valued(t, value):  # t's graph at the forward's value
-        return value.to(t.dtype) + (t - t.detach())
 
     def operands(x, wq, wk, wv, wg, bg, alpha_w):
         v = valued(F.linear(x, wv).view(v_saved.shape), v_saved)

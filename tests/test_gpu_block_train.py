@@ -172,6 +172,27 @@ def test_backward_inside_autocast(part, fwd, bwd):
         assert a.dtype == b.dtype and torch.equal(a, b)
 
 
+@pytest.mark.parametrize("name", ["gate_proj", "up_proj", "down_proj"])
+@pytest.mark.parametrize("x_grad", [True, False])
+def test_weights_changed_before_the_backward(name, x_grad):
+    """As with linears: gate's and up's weights are refused where x takes a gradient, down's always
+    (its input takes one), and the others are free to change."""
+    print(f"swiglu changed {name} x_grad={x_grad}", flush=True)
+    torch.manual_seed(5)
+    ffn = SwiGLUFFN(64, 72).to(DEV)
+    x = torch.randn(9, 64, device=DEV).requires_grad_(x_grad)
+    want = torch.autograd.grad(ffn(x).sum(), list(ffn.parameters()))
+    y = ffn(x)
+    with torch.no_grad():
+        getattr(ffn, name).weight.mul_(1.5)
+    if x_grad or name == "down_proj":
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            y.sum().backward()
+    else:
+        for a, b in zip(torch.autograd.grad(y.sum(), list(ffn.parameters())), want):
+            assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype,autocast", [(FP, True), (BF, False)])
 @pytest.mark.parametrize("shape", [(40, 128), (1, 40, 128)])
 def test_outputs_can_be_modified_in_place(dtype, autocast, shape):
