@@ -328,14 +328,14 @@ __global__ void __launch_bounds__(64 * NW, D == 64 ? 3 : 2) bwd_dq_kernel(const 
             reinterpret_cast<int *>(rec)[kTabLo * T] = INT_MAX - lo;
             reinterpret_cast<int *>(rec)[kTabPmax * T] = pmax + 1;
         } else {
-        rec[kRecLse2 * T] = -lse2 * p.inv_c2;  // (S + this) * scale_log2 = S scale_log2 - lse2
-        rec[kRecDelta * T] = -delta;
-        reinterpret_cast<int *>(rec)[kRecLo * T] = INT_MAX - lo;
-        reinterpret_cast<int *>(rec)[kRecClo * T] = INT_MAX - corelo;
-        reinterpret_cast<int *>(rec)[kRecPmax * T] = pmax + 1;
-        rec[kRecWc * T] = wc;
-        reinterpret_cast<int *>(rec)[kRecGLo * T] = INT_MAX - wlo;
-        reinterpret_cast<int *>(rec)[kRecGClo * T] = INT_MAX - wclo;
+            rec[kRecLse2 * T] = -lse2 * p.inv_c2;  // (S + this) * scale_log2 = S scale_log2 - lse2
+            rec[kRecDelta * T] = -delta;
+            reinterpret_cast<int *>(rec)[kRecLo * T] = INT_MAX - lo;
+            reinterpret_cast<int *>(rec)[kRecClo * T] = INT_MAX - corelo;
+            reinterpret_cast<int *>(rec)[kRecPmax * T] = pmax + 1;
+            rec[kRecWc * T] = wc;
+            reinterpret_cast<int *>(rec)[kRecGLo * T] = INT_MAX - wlo;
+            reinterpret_cast<int *>(rec)[kRecGClo * T] = INT_MAX - wclo;
         }
     }
     float edw[2] = {0.f, 0.f};
@@ -1427,6 +1427,7 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
             const int st = stage_of(t);
             const char *qtile = s_tiles[st][0];
             const char *dtile = s_tiles[st][1];
+            // one pass; as an if the compiler takes 26 registers more (D = 128: 30 AGPRs)
     #pragma unroll
             for (int sbi = 0; sbi < 1; ++sbi) {
                 const int sb = sbw;

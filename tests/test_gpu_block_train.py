@@ -271,9 +271,13 @@ def test_block_matches_separate_ops(dtype, autocast, checkpoint):
             y, _ = block(xx, cu_seqlens=cu, cu_list=[0, 200, 333], gradient_checkpointing=checkpoint)
         assert y.dtype == dtype
         y.backward(dy.to(y.dtype))
-        out.append([y.detach(), xx.grad] + [p.grad for n, p in block.named_parameters() if "alpha" not in n])
+        out.append({"y": y.detach(), "x": xx.grad, **{n: p.grad for n, p in block.named_parameters()}})
         for hk in hooks:
             hk.remove()
-    for a, b in zip(*out):
+    for n, a in out[0].items():
+        b = out[1][n]
         assert a.dtype == b.dtype
-        assert float((a.double() - b.double()).norm()) <= 2.0 ** -5 * float(b.double().norm())
+        # each of the separate ops rounds once more on the way (2^-9 a time, five to eight of them);
+        # the gate's bias and alpha sum cancelling terms over the tokens and the slots
+        share = 2.0 ** -5 if n in ("attn.win_gate.bias", "attn.alpha_w") else 2.0 ** -7
+        assert float((a.double() - b.double()).norm()) <= share * float(b.double().norm()), n

@@ -136,7 +136,7 @@ def test_module_training_equals_composed_route(case):
     for name, a in got["one"].items():
         b = got["composed"][name]
         if a is None or b is None:  # no landmark: alpha takes no gradient
-            assert k == 0 and name == "alpha_w"
+            assert a is None and b is None and k == 0 and name == "alpha_w"
             continue
         assert a.dtype == b.dtype
         if name == "win_gate.bias":  # a sum of cancelling terms: on the scale of its weight's gradient
@@ -382,3 +382,71 @@ def test_second_order_gradients(case, route):
                 continue
             a, b = a.detach().double(), b.detach().double()
             assert float((a - b).norm()) <= tol * float(b.norm()), (order, n, float((a - b).norm() / b.norm()))
+
+
+def test_fp32_windows():
+    """fp32 modules form their windows in the norms pass too: expf within 2 ulp, a division, a
+    product and a sum rounded once each, all relative to at most n_max: 2^-21 n_max."""
+    print("module attention fp32 windows", flush=True)
+    mod, x, _ = small_module(torch.float32)
+    with torch.no_grad():
+        mod.win_gate.weight.mul_(8)
+        mod(x[None])
+    logit = x.double() @ mod.win_gate.weight.double().squeeze(0) + mod.win_gate.bias.double()
+    want = mod.n_min + torch.sigmoid(logit) * (mod.n_max - mod.n_min)
+    assert float((mod._last_selection[0].double() - want).abs().max()) <= 2.0 ** -21 * mod.n_max
+
+
+# tokens per workgroup of the states' pass (8, 16 from 4096 tokens, 32 from 16384; the last
+# workgroup partly filled) and rows of one, exactly and just over 256 column chunks
+@pytest.mark.parametrize("T,d,H,n_kv,dtype", [
+    (33, 64, 2, 2, torch.bfloat16), (4095, 2048, 2, 1, torch.bfloat16), (4099, 2056, 2, 1, torch.float16),
+    (16387, 72, 3, 3, torch.bfloat16), (4097, 1028, 2, 2, torch.float32), (16384, 1024, 2, 1, torch.float32)])
+def test_module_grads_at_the_edges_of_its_shapes(T, d, H, n_kv, dtype):
+    """dsalt_module_grads_v and _x against float64 autograd of the scores, the weights and the gate."""
+    print(f"module grads T={T} d={d} H={H}/{n_kv} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(T + d)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(DEV)  # noqa: E731
+    D, k, tau, n_min, n_max = 64, 12, 2.0, 4.0, 60.0
+    lens = [T // 3, T - T // 3]
+    cu = torch.tensor([0, lens[0], T], dtype=torch.int32, device=DEV)
+    x, v = rnd(T, d).to(dtype), rnd(T, n_kv, D).to(dtype)
+    aw = rnd(H)
+    alpha = torch.sigmoid(aw)
+    sel = _hip.SelectHybridLauncher(x, v, alpha, H, 1 + 30 * torch.rand(T, generator=g).to(DEV), cu, k,
+                                    max_seqlen=max(lens), norms_f32=True)
+    sel()
+    _hip.lmk_weights(sel.norms, alpha, sel.out, sel.cu, T, n_kv, tau)
+    dlw = rnd(H, 2, k) * 0.1
+    dk_h, dv_h, dx_in, dw = rnd(T, H, D).to(dtype), rnd(T, H, D).to(dtype), rnd(T, d).to(dtype), rnd(T) * 0.1
+    wg = (rnd(1, d) / d ** 0.5).to(dtype)
+    logit = rnd(T).to(dtype).float()
+    m = _hip.ModuleGrads(x, v, sel.norms, alpha, sel.out, sel.cu, dlw, tau, False)
+    dk, dv = torch.empty(T, n_kv, D, device=DEV, dtype=dtype), torch.empty(T, n_kv, D, device=DEV, dtype=dtype)
+    da = m.values(dk_h, dv_h, dk, dv, alpha_sigmoid=True)
+    dx, dwg, dbg = m.states(dx_in, True, (wg, logit, dw, dtype, n_min, n_max))
+
+    x64, v64, a64 = (t.detach().double().requires_grad_() for t in (x, v, aw))
+    sig = torch.sigmoid(a64)
+    z = [(n - n.mean(0)) / n.std(0) for n in (x64.norm(dim=-1), v64.norm(dim=-1))]
+    s = sig * z[1].repeat_interleave(H // n_kv, 1) + (1 - sig) * z[0].unsqueeze(1)
+    tok = cu[:-1].long().view(1, 2, 1) + sel.out.clamp(min=0)
+    filled = sel.out >= 0
+    logw = torch.log(torch.sigmoid(s.t().gather(1, tok.view(H, -1)).view(tok.shape) / tau))
+    logw[filled].backward(dlw[filled].double())
+    assert bool(filled.any()) and bool(filled.all()) == (T > 33)
+    sg = torch.sigmoid(logit.double()).to(dtype).double()  # the gate as the forward rounded it
+    dl = dw.double() * (n_max - n_min) * sg * (1 - sg)
+    want = {"dx": x64.grad + dx_in.double() + dl[:, None] * wg.double(),
+            "dv": v64.grad + dv_h.double().view(T, n_kv, -1, D).sum(2), "dwg": (dl @ x.double())[None], "dbg": dl.sum()[None],
+            "da": a64.grad}
+    if n_kv != H:
+        want["dk"] = dk_h.double().view(T, n_kv, -1, D).sum(2)
+    # fp32 sums: 1e-4 of the largest value where the standardised norms take part (see the weights'
+    # own test), 1e-5 of the terms' sum for the gate's; each result rounded once
+    ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -23}[dtype]
+    terms = {"dwg": dl.abs() @ x.double().abs(), "dbg": dl.abs().sum()}
+    for n, w in want.items():
+        got = {"dx": dx, "dv": dv, "dwg": dwg, "dbg": dbg, "da": da, "dk": dk}[n].double()
+        bar = ulp * w.abs() + (1e-5 * terms[n] if n in terms else 1e-4 * w.abs().max())
+        assert bool(((got - w).abs() <= bar).all()), (n, float(((got - w).abs() - bar).max()))
