@@ -331,7 +331,11 @@ class DSALTAttention(nn.Module):
     def _own_steps(self, *names: str) -> bool:
         """Whether one of these methods of DSALTAttention is replaced, in a subclass, on the class
         or on this instance."""
-        return any(n in self.__dict__ or getattr(type(self), n) is not _STEPS[n] for n in names)
+        own, cls = self.__dict__, type(self)
+        for n in names:
+            if getattr(cls, n) is not _STEPS[n] or n in own:
+                return True
+        return False
 
     @_dynamo_opaque
     def _attend(self, x, cu_seqlens, k_lmk, max_seqlen, dense=False, x_cast=None):
