@@ -12,20 +12,19 @@
 // element is produced by exactly one thread, in a fixed order.
 //
 // Kernels, launched in this order on one stream:
-//   dq      query-parallel, two waves (long sequences: see launch_dq) x 32 queries per
-//           workgroup, the forward's tiling
-//           (band tiles of kDqBN keys, then gathered landmark tiles); S^T, dP^T and dQ^T
-//           on MFMA. Computes
-//           Delta = rowsum(O * dO) for its queries and writes dQ, the per-head soft-edge
-//           d_w~, the per-query records of the key-parallel passes and (head 0) the
-//           smallest band start of each 64 queries, which bounds the scan of `kv` (workspace).
+//   dq      query-parallel, two waves (or four: see launch_dq) x 32 queries per workgroup,
+//           the forward's tiling (band tiles of kDqBN keys, then gathered landmark tiles);
+//           S^T, dP^T and dQ^T on MFMA. Computes Delta = rowsum(O * dO) for its queries and
+//           writes dQ, the per-head soft-edge d_w~, the per-query records of the key-parallel
+//           passes and (head 0) the smallest band start of each 64 queries, which bounds the
+//           scan of `kv` (workspace).
 //   lmk_kv  key-parallel over landmark slots: one workgroup per (head, 64 slots, chunk of
 //           512 queries of one sequence); 4 waves = 2 slot groups x 2 query sub-blocks scan
 //           the chunk's queries in 64-query LDS tiles. Writes landmark dK/dV and d_bias
 //           partials per chunk (workspace).
 //   kv      key-parallel band dK/dV, kv_waves(D) waves x 32 keys per workgroup, scanning
-//           kv_qt(D)-query LDS tiles from the key block to the last dq query block whose
-//           band reaches it; keys that are landmark positions start from their landmark
+//           kv_qt(D)-query LDS tiles from the key block to the last 64 queries whose band
+//           reaches it; keys that are landmark positions start from their landmark
 //           dK/dV (the lmk_kv chunk partials summed in chunk order in the prologue); its
 //           head-0 workgroups reduce d_w~ over heads, and H x S workgroups appended to its
 //           grid sum the d_bias partials of each (head, sequence).
@@ -826,7 +825,7 @@ __global__ void __launch_bounds__(LMK ? 256 : 64 * kv_waves(D), D == 64 ? 2 : 1)
         // seq_start / kMinBM + seq) whose smallest band start reaches this key block
         const int dqbase = seq_start / kMinBM + seq;
         const int nbs = (seq_len + kMinBM - 1) / kMinBM;
-        const int own = (kb + kBM - 1) / kMinBM;  // dq block of the key block's last key
+        const int own = (kb + kBM - 1) / kMinBM;  // the key block's last key's own
         int last = own;
         for (int b = own + 1 + tid; b < nbs; b += NT)
             if (p.ws_minlo[dqbase + b] <= kb + kBM - 1) last = max(last, b);

@@ -20,7 +20,8 @@
 // result. Deterministic: no atomics, every element is written by one thread. Bound: the
 // apply pass streams x, v and d_v_in (read), d_x and d_v (written): 95 MB in 24.0 us (4.0
 // TB/s) at 9290 tokens x 1024 in bf16; weight_kernel (4.7 us) and reduce_kernel (5.3 us) are
-// latency.
+// latency. Both walk the sequences: 4.7 and 6.5 us up to 8 of them, 25 and 32 at 300 (9300
+// tokens), 148 and 198 at 2000 (10000 tokens; each of H x S workgroups re-sums the partials).
 // The module's own function (dsalt_module_grads_v / _x) splits the apply pass around the
 // projections' GEMMs:
 //   grads_v_kernel  one wave per token: dv = value-norm share + the attention's dv (summed over
@@ -31,8 +32,8 @@
 // One pass over x, dx_in and dx (19.3 us at that shape; grads_v 13.0, gate 8.8) instead of
 // torch's outer-product GEMM, GEMV, bias sum and three additions over [T, d].
 // A training step of the module at that shape: 1985 us with torch's ops (152 launches, GPU
-// busy 1391 us), 1146 with the weights here (46, 888), 718 with everything between x and
-// the attention's output as one function (23, 651).
+// busy 1391 us), 1146 with the weights here (46, 888), 716 with everything between x and
+// the attention's output as one function (23, 662).
 #include "common.h"
 #include "hybrid.h"
 #include "launch.h"
@@ -345,7 +346,9 @@ constexpr int kXBatch = 4;      // tokens whose rows a thread loads together
 
 // Tokens per workgroup: a thread walks its share of them in latency-bound steps, so small
 // batches take few (1001 tokens x 1024: 126 workgroups), large ones more (fewer rows of
-// partial sums for gate_kernel).
+// partial sums for gate_kernel). With 8 / 16 / 32 the two kernels take, at d = 1024 in bf16, 2048
+// tokens 14.4 / 16.2 / 20.4 us, 4096 18.3 / 16.6 / 21.9, 9290 37.4 / 27.8 / 26.7, 16384 53.3 /
+// 36.8 / 32.4; at d = 4096, 2048 29 / 39 / 64, 9290 75 / 56 / 75, 16384 125 / 105 / 112.
 inline int x_tokens(int T) { return T >= 16384 ? 32 : T >= 4096 ? 16 : 8; }
 
 __device__ __forceinline__ float round_win(float v, int dt) {

@@ -3,8 +3,9 @@
 Drop-in for dsalt/kernels/dsalt_triton_train.py: same entry point
 ``dsalt_triton_train_attention(q, k, v, lmk_pos, lmk_logw, w_cont, cu_seqlens,
 tau_win=1.0, win_edge=4.0, n_max=256, cu_list=None)`` and the same
-``DSALTTrainFunction`` (fp32 output; gradients dq, dk, dv, d_logw, d_w~ in q's dtype,
-:751-760). The module name is kept for import compatibility; nothing here uses Triton.
+``DSALTTrainFunction`` (fp32 output; gradients dq, dk, dv in q's dtype, :751-760; d_logw
+and d_w~ fp32 as the kernels sum them, which autograd casts to their inputs' dtypes). The
+module name is kept for import compatibility; nothing here uses Triton.
 
 Semantics (dsalt_triton_train.py:116-198): band ``0 <= d = i - j <= w~(i)`` with logit
 bias 0 in the core ``d <= w~ - win_edge`` and ``log sigmoid((w~ - d) / tau_win)`` on the

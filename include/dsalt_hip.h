@@ -384,9 +384,9 @@ int dsalt_select_hybrid(const dsalt_scores_args *scores, const dsalt_select_args
  * v_out = NULL (v is its own operand). The k_out of `scores` has out_dtype. Outputs alias
  * no input when out_dtype != v_dtype; q_out may alias q otherwise.
  * Windows (win_w NULL: none): logit = x . win_w + win_b[0] over operands rounded to
- * win_dtype (x_dtype, or a 16-bit type for fp32 x: autocast), fp32 sums in a fixed order,
- * rounded to win_dtype; w~ = n_min + sigmoid(logit) (n_max - n_min), every step rounded to
- * win_dtype. win_w [d_model] (16-byte aligned) and win_b [1] (may be NULL) in x_dtype;
+ * win_dtype (x_dtype, or a 16-bit type for fp32 x: autocast), products summed in fp64 in a
+ * fixed order, one rounding to win_dtype; w~ = n_min + sigmoid(logit) (n_max - n_min), every
+ * step rounded to win_dtype. win_w [d_model] (16-byte aligned) and win_b [1] (may be NULL) in x_dtype;
  * win_logit and win_out [T] fp32. Replaces _window_continuous
  * (dsalt/modules/dsalt_attention.py:270-276); `select` takes its windows from win_out
  * (w = win_out). scores->gate_w must be NULL, with win_w and without.
