@@ -89,7 +89,6 @@ __device__ __forceinline__ float lmk_weight(float s, float tau) {
     return logf(sg < kSigClamp ? kSigClamp : sg);
 }
 
-
 __global__ void __launch_bounds__(kTableThreads) weight_kernel(const WeightParams p) {
     __shared__ float st[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;

@@ -301,9 +301,9 @@ class DSALTAttention(nn.Module):
         """Whether projections, gate, RoPE, selection and attention of x [T, d] run as one function
         (``module_attention``): the HIP score route; projections that are plain nn.Linear
         modules without hooks (a wrapped, parametrised or hooked one is called as it is, on the
-        route of separate functions, and so is a subclass's own step), q, k and v without bias; one element type for x and the
-        weights, or fp32 for all of them under a 16-bit autocast; rows that the norms pass
-        loads in 16-byte pieces."""
+        route of separate functions, and so is a replaced step), q, k and v without bias; one
+        element type for x and the weights, or fp32 for all of them under a 16-bit autocast; rows
+        that the norms pass loads in 16-byte pieces."""
         lin = (self.q_proj, self.k_proj, self.v_proj, self.win_gate)
         if not eager(x, self.alpha_w):
             return False
